@@ -34,6 +34,7 @@ EXPORTED_SYMBOLS = (
     "hp_npairs_projected", "hp_npairs_xy_z", "hp_marked_npairs_3d", "hp_npairs_per_object_3d",
     "hp_marked_npairs_xy_z", "hp_npairs_jackknife_3d", "hp_npairs_jackknife_xy_z", "hp_marked_backward",
     "hp_segment_sum_scratch", "hp_segment_sum", "hp_debug_bin_lookup", "hp_debug_hilbert",
+    "hp_debug_tile_lookup",
     "hp_npairs_3d_noalloc", "hp_zheng07_tangent",
 )
 
@@ -130,6 +131,10 @@ def library():
                                         ctypes.POINTER(ctypes.c_double), ctypes.c_int64,
                                         ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32)]
     lib.hp_debug_bin_lookup.restype = ctypes.c_int
+    lib.hp_debug_tile_lookup.argtypes = [ctypes.POINTER(ctypes.c_double), ctypes.c_int32,
+                                         ctypes.POINTER(ctypes.c_double), ctypes.c_int64, ctypes.c_int32,
+                                         ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32)]
+    lib.hp_debug_tile_lookup.restype = ctypes.c_int
     lib.hp_debug_hilbert.argtypes = [ctypes.c_uint32, ctypes.c_uint32, ctypes.c_uint32, ctypes.c_int32]
     lib.hp_debug_hilbert.restype = ctypes.c_uint32
     _LIB = lib
@@ -153,3 +158,17 @@ def debug_bin_lookup(r2, d):
         r2.ctypes.data_as(P(ctypes.c_double)), len(r2), d.ctypes.data_as(P(ctypes.c_double)),
         len(d), out.ctypes.data_as(P(ctypes.c_int32)), info.ctypes.data_as(P(ctypes.c_int32))))
     return out, dict(shift=int(info[0]), base=int(info[1]), nb=int(info[2]), multi=int(info[3]))
+
+
+def debug_tile_lookup(r2, d, off=0):
+    """Host evaluation of the matrix-core kernels' lookup with each d's high word
+    off by `off` units: bins (-1: evaluated exactly), and whether the edges fit."""
+    r2 = np.ascontiguousarray(r2, dtype=np.float64)
+    d = np.ascontiguousarray(d, dtype=np.float64)
+    out = np.zeros(len(d), dtype=np.int32)
+    info = np.zeros(3, dtype=np.int32)
+    P = ctypes.POINTER
+    check(library().hp_debug_tile_lookup(
+        r2.ctypes.data_as(P(ctypes.c_double)), len(r2), d.ctypes.data_as(P(ctypes.c_double)), len(d), off,
+        out.ctypes.data_as(P(ctypes.c_int32)), info.ctypes.data_as(P(ctypes.c_int32))))
+    return out, bool(info[0])

@@ -14,7 +14,8 @@ OUT = os.path.join(HERE, "_lib", "libhalopair.so")
 # the pair kernel's variants are instantiated one mode per translation unit
 # (pairs_mode_*.hip) so that they compile in parallel
 SOURCES = ["cellbuild.hip", "pairs.hip", "reduce.hip", "capi.hip"] + [
-    "pairs_mode_%s.hip" % m for m in ("count3d", "proj", "xyz", "obj", "wxyz", "jack", "jackxy", "wsum", "jac", "tan")]
+    "pairs_mode_%s.hip" % m for m in ("count3d", "proj", "xyz", "obj", "wxyz", "jack", "jackxy", "wsum", "jac", "tan")] + [
+    "pairs_tile_%s.hip" % m for m in ("count3d", "proj", "xyz", "wxyz", "obj", "jac", "tan", "wsum")]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 

@@ -21,7 +21,7 @@
 
 namespace hp {
 int launch_reduce_sums_s(const double* partial, int nr, int np, const MockGeom* geom, int nmocks, int side,
-                         int64_t max_groups, double* scratch, double* sums, hipStream_t s);
+                         int64_t max_groups, int parts_sh, double* scratch, double* sums, hipStream_t s);
 int launch_reduce_evals_s(const uint64_t* pevals, const MockGeom* geom, int nmocks, int side, int64_t max_groups,
                           uint64_t* scratch, int64_t* evals, hipStream_t s);
 int64_t reduce_scratch_elems(int64_t max_groups_per_mock, int nmocks, int nb);
@@ -111,6 +111,62 @@ static Table make_table(const std::vector<double>& e_in, int K) {
     return T;
 }
 
+// The matrix-core kernels' bucket table: 8-byte entries (high word of the only
+// edge that can lie in the bucket, plus one; edges below the bucket).  Their
+// high word may be off by one, so an edge must not end a bucket (the next
+// bucket's entry would not know it).  The coarsest buckets that part the edges
+// make the smallest table.
+struct TileTable {
+    TileSpec spec{};
+    std::vector<uint32_t> t;  // 2 words per entry
+};
+
+static TileTable make_tile_table(const std::vector<double>& e, int K) {
+    TileTable T;
+    double first_pos = INFINITY;
+    for (int k = 0; k < K; k++)
+        if (e[k] > 0.0 && e[k] < first_pos) first_pos = e[k];
+    const double last = K > 0 ? e[K - 1] : 0.0;
+    if (!(first_pos < INFINITY) || !(last < INFINITY)) return T;
+    for (int shift = 20; shift >= 3; shift--) {
+        // bucket 0: everything far below the first positive edge (and the zero
+        // edges); bucket 1 parts it from the first positive edge's
+        const int64_t base = std::max<int64_t>((int64_t)(hiword(first_pos) >> shift) - 2, 0);
+        const int64_t nb = (int64_t)(hiword(last) >> shift) - base + 2;
+        if (nb > kTableMax) break;  // finer ones need more still
+        bool fits = true;
+        for (int k = 0; k < K && fits; k++) {
+            const uint32_t h = hiword(e[(size_t)k]);
+            if (((h + 1) >> shift) != (h >> shift)) fits = false;
+        }
+        uint32_t n = 8;
+        while ((int64_t)n < nb) n *= 2;
+        T.t.assign(2 * (size_t)n, 0u);
+        for (int64_t b = 0; b < nb && fits; b++) {
+            const double lo = b == 0 ? 0.0 : from_hiword((uint32_t)((base + b) << shift));
+            const double hi = b + 1 < nb ? from_hiword((uint32_t)((base + b + 1) << shift)) : INFINITY;
+            const int below = (int)(std::lower_bound(e.data(), e.data() + K, lo) - e.data());
+            const int upto = b + 1 == nb ? K : (int)(std::lower_bound(e.data(), e.data() + K, hi) - e.data());
+            if (upto - below > 1) fits = false;
+            // ... nor start the bucket after one that holds an edge
+            if (upto - below == 1 && upto < K && (int64_t)((hiword(e[(size_t)upto]) - 1) >> shift) == base + b)
+                fits = false;
+            const size_t at = (size_t)((base + b) & (n - 1));
+            T.t[2 * at] = hiword(e[(size_t)below]) + 1;
+            T.t[2 * at + 1] = (uint32_t)below;
+        }
+        if (!fits) continue;
+        T.spec.lo = (uint32_t)(base << shift);
+        T.spec.hi = (uint32_t)((base + nb - 1) << shift);
+        T.spec.sh3 = (uint32_t)shift - 3;
+        T.spec.mask = n - 1;
+        T.spec.ok = 1;
+        return T;
+    }
+    T.t.clear();
+    return T;
+}
+
 static int lookup_host(const Table& T, double d) {
     const uint32_t hi = hiword(d);
     const uint32_t t = hi > T.spec.basesh ? hi - T.spec.basesh : 0u;
@@ -142,6 +198,9 @@ struct Plan {
     size_t o_tfirst[2] = {0, 0};
     std::vector<MockGeom> geom;
     Table tr, tp;
+    TileTable ttr, ttp;  // radial / rp and pi bins for the matrix-core kernels
+    size_t o_ttr = 0, o_ttp = 0;
+    int parts_sh = 0;    // log2 of their work items per lane group
     int Kr = 0, Kp = 0, nb_count = 0;
     // workspace layout (byte offsets)
     size_t o_geom = 0, o_er = 0, o_ep = 0, o_tr = 0, o_tp = 0;
@@ -154,6 +213,8 @@ struct Plan {
     size_t o_rows[2] = {0, 0};       // packed coordinate rows of each side with a row-major order
     int row_stride[2] = {4, 4}, row_nw[2] = {0, 0};
     size_t o_keys_row = 0;           // row-major keys of a side sorted in both orders
+    bool tiles = false;  // matrix-core kernels on the curve-ordered rows
+    size_t o_crow[2] = {0, 0}, o_cw[2] = {0, 0}, o_cperm[2] = {0, 0}, o_cubes[2] = {0, 0};
     bool sym = false;  // auto-count (unweighted or tangent): symmetric evaluation
     int crep = 1;
     bool tangent = false;
@@ -171,6 +232,13 @@ struct Plan {
 
 static size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
+#ifndef HP_TILE_ITEMS
+#define HP_TILE_ITEMS 16
+#endif
+#ifndef HP_CUBE_R
+#define HP_CUBE_R 0.6
+#define HP_CUBE_G 0.5
+#endif
 constexpr double kCellTarget = 4096.0;  // most stream points per default fine cell
 constexpr int kHilbertMaxBits = 8;   // lane-ordering grid <= 256^3 cells per mock
 constexpr int kCountReplicas = 256;  // count accumulator copies per mock
@@ -181,7 +249,23 @@ static int bits_for(uint64_t range) {
     return b;
 }
 
-static int make_plan(const hp_request* r, int kind, Plan& P) {
+// Mode of the pair kernel of a request.
+static int mode_of(const Plan& P, int kind, int wfunc) {
+    switch (kind) {
+        case HP_NPAIRS_3D: return kModeCount3D;
+        case HP_NPAIRS_PROJECTED: return kModeProj;
+        case HP_NPAIRS_XY_Z: return kModeXYZ;
+        case HP_NPAIRS_PER_OBJECT_3D: return kModeObj;
+        case HP_MARKED_NPAIRS_XY_Z: return kModeWXYZ;
+        case HP_NPAIRS_JACKKNIFE_3D: return kModeJack;
+        case HP_NPAIRS_JACKKNIFE_XY_Z: return kModeJackXY;
+    }
+    return P.tangent ? kModeTan : ((wfunc == 1 && P.nw == 1 && (P.rows1 || P.rows2)) ? kModeJac : kModeWSum);
+}
+
+// tiles: the matrix-core kernels may be chosen (else the others, which need
+// less workspace when the samples differ)
+static int make_plan(const hp_request* r, int kind, Plan& P, bool tiles = true) {
     if (!r) return fail("null request");
     P.kind = kind;
     P.flags = r->flags;
@@ -236,12 +320,14 @@ static int make_plan(const hp_request* r, int kind, Plan& P) {
 
     std::vector<double> er = suffix_min(r->r2, P.Kr);
     P.tr = make_table(er, P.Kr);
+    P.ttr = make_tile_table(er, P.Kr);
     double Rxy = sqrt(er[(size_t)P.Kr - 1]);
     double Rz = Rxy;
     int shape = 0;
     if (xyz) {
         std::vector<double> ep = suffix_min(r->p2, P.Kp);
         P.tp = make_table(ep, P.Kp);
+        P.ttp = make_tile_table(ep, P.Kp);
         Rz = sqrt(ep[(size_t)P.Kp - 1]);
         shape = 1;
     } else if (kind == HP_NPAIRS_PROJECTED) {
@@ -250,6 +336,7 @@ static int make_plan(const hp_request* r, int kind, Plan& P) {
         P.tp.spec.nbins = 1;
         P.tp.spec.nb = 1;
         P.tp.t.assign(1, TabEntry{INFINITY, 0u, 0u});
+        P.ttp = make_tile_table(P.tp.e, 1);
         Rz = sqrt(r->p2[0]);
         shape = 1;
     } else {
@@ -260,6 +347,20 @@ static int make_plan(const hp_request* r, int kind, Plan& P) {
     }
     if (!(Rxy == Rxy) || !(Rz == Rz)) return fail("bins must not be NaN");
     P.nb_count = xyz ? P.Kr * P.Kp : P.Kr;
+
+    // The matrix-core kernels (pairs_tile.h) take what their bucket tables and the
+    // LDS hold: bins that buckets of 1/16 octave or finer part, and a wave's
+    // histogram beside its stage at 7 waves per CU or more.  Wider or denser
+    // binnings and the jackknife tables stay with pairs_kernel.h.
+    const int mode = mode_of(P, kind, r->wfunc);
+    {
+        const int wb = tile_wave_bytes(mode, P.Kr, P.Kp, P.nw, P.counts ? 1 : 0);
+        P.tiles = tiles && mode != kModeTan && mode != kModeWXYZ && P.ttr.spec.ok && (P.Kp == 0 || P.ttp.spec.ok) && wb > 0 && wb <= 23 * 1024 &&
+                  !std::getenv("HALOPAIR_NO_TILES");
+        // one u32 (rp, pi) cell must hold every pair of a group, counted twice
+        for (int m = 0; m < P.M; m++)
+            if (kind == HP_NPAIRS_XY_Z && r->mocks[m].n1 >= (1 << 25)) P.tiles = false;
+    }
 
     // ---- per-mock geometry
     P.geom.resize((size_t)P.M);
@@ -307,6 +408,25 @@ static int make_plan(const hp_request* r, int kind, Plan& P) {
         while (mb < kHilbertMaxBits && (double)(1 << mb) < 1.25 * cbrt(nlane)) mb++;
         G.mbits = mb;
         for (int d = 0; d < 3; d++) G.inv_hcell[d] = (double)(1 << mb) / G.period[d];
+        if (P.tiles) {
+            // cubes of the curve: an edge near half the search length, but not
+            // far below the size of a lane group (cell hints set the edge)
+            double want = 0.0;
+            for (int d = 0; d < 3; d++) {
+                const double R = (d < 2) ? Rxy : Rz, L = hm.period[d];
+                const double grp = L * cbrt(64.0 / std::max(nlane, 64.0));
+                double b = hm.cell[d] > 0.0 ? hm.cell[d] : std::max(R * HP_CUBE_R, grp * HP_CUBE_G);
+                want += log2(L / b) / 3.0;
+            }
+            G.cbits = (int32_t)std::min<double>(mb, std::max(1.0, floor(want + 0.5)));
+            while (G.cbits > 1 && (double)((int64_t)1 << (3 * G.cbits)) > 4.0 * std::max(nlane, 512.0)) G.cbits--;
+            ncells = (int64_t)1 << (3 * G.cbits);
+            for (int d = 0; d < 3; d++) {
+                G.ndiv[d] = 1 << G.cbits;
+                G.cell[d] = G.period[d] / (double)G.ndiv[d];
+                G.inv_cell[d] = 1.0 / G.cell[d];
+            }
+        }
         const float eps = (float)(1e-5 * Lmax);
         G.eps = eps;
         G.search[0] = (float)(Rxy * (1.0 + 1e-6)) + eps;
@@ -372,6 +492,8 @@ static int make_plan(const hp_request* r, int kind, Plan& P) {
     P.o_ep = take(P.tp.e.size() * 8);
     P.o_tr = take(P.tr.t.size() * sizeof(TabEntry));
     P.o_tp = take(P.tp.t.size() * sizeof(TabEntry));
+    P.o_ttr = take(P.ttr.t.size() * 4);
+    P.o_ttp = take(P.ttp.t.size() * 4);
     P.o_tfirst[0] = take(((size_t)P.M + 1) * 4);
     P.o_tfirst[1] = take(((size_t)P.M + 1) * 4);
     const size_t consts_end = off;
@@ -381,9 +503,11 @@ static int make_plan(const hp_request* r, int kind, Plan& P) {
     // sorted sides: pass A lanes = (0, Hilbert), stream = (s2, RowMajor);
     // pass B lanes = (s2, Hilbert), stream = (0, RowMajor)
     const int s2 = P.same ? 0 : 1;
-    P.sorted[0][kHilbert].needed = true;
-    P.sorted[s2][kRowMajor].needed = true;
-    if (P.rows2) {
+    if (!P.tiles) {
+        P.sorted[0][kHilbert].needed = true;
+        P.sorted[s2][kRowMajor].needed = true;
+    }
+    if (P.rows2 && !P.tiles) {
         P.sorted[s2][kHilbert].needed = true;
         P.sorted[0][kRowMajor].needed = true;
     }
@@ -406,6 +530,22 @@ static int make_plan(const hp_request* r, int kind, Plan& P) {
             if (o == kRowMajor) S.cs = take((size_t)(P.total_cells + 1) * 4);
         }
     }
+    if (P.tiles) {
+        for (int s = 0; s <= s2; s++) {
+            const size_t n = (size_t)std::max<int64_t>(P.n[s], 1);
+            nmax = std::max<int64_t>(nmax, (int64_t)n);
+            P.o_crow[s] = take(n * 32);
+            if (P.weighted()) P.o_cw[s] = take(n * 8 * (size_t)P.nw);
+            P.o_cperm[s] = take(n * 4);
+            // packed input rows, for column inputs
+            if ((s == 0 ? r->stride1 : r->stride2) <= 1) P.o_rows[s] = take(n * 32);
+            P.row_stride[s] = 4;
+            P.row_nw[s] = 0;
+        }
+        // the stream side's cubes; the swapped pass streams side 0
+        P.o_cubes[s2] = take((size_t)P.total_cells * 8);
+        if (P.rows2 && s2) P.o_cubes[0] = take((size_t)P.total_cells * 8);
+    }
     // digit counts per tile: room for the smaller tiles whichever size runs
     const int64_t ntiles = (nmax + kSortTile - 1) / kSortTile + P.M + 1;
     P.o_keys[0] = take((size_t)nmax * 4);
@@ -416,17 +556,23 @@ static int make_plan(const hp_request* r, int kind, Plan& P) {
     P.o_tiles = take((size_t)ntiles * kRadixDigits * 4);
     P.o_digits = take((size_t)kRadixDigits * 4);
     const int64_t gA = std::max<int64_t>(P.ngroups[0], 1);
+    // Small requests split each lane group into work items until the chip has
+    // HP_TILE_ITEMS waves per CU to run (rows per lane point are written once,
+    // so those stay whole).
+    if (P.tiles && mode != kModeObj && mode != kModeJac)
+        while (P.parts_sh < 4 && (gA << P.parts_sh) < 256 * HP_TILE_ITEMS) P.parts_sh++;
+    const int64_t gP = gA << P.parts_sh;  // rows of FP64 partials
     // count accumulators: up to kCountReplicas copies per mock (a group adds
     // into copy group % crep), so the atomics of many groups spread over cache
     // lines; wide histograms (xy_z) spread over their own bins already
     P.crep = (int)std::max<int64_t>(
         1, std::min<int64_t>({(int64_t)kCountReplicas, P.max_groups[0], (int64_t)(2048 / std::max(P.nb_count, 1))}));
     if (P.counts) P.o_pcount = take((size_t)P.M * (size_t)P.crep * (size_t)P.nb_count * 8);
-    if (P.sums) P.o_psum = take((size_t)gA * (size_t)P.nb_count * 8);
-    if (P.tangent) P.o_ptan = take((size_t)gA * (size_t)P.Kr * 8);
+    if (P.sums) P.o_psum = take((size_t)gP * (size_t)P.nb_count * 8);
+    if (P.tangent) P.o_ptan = take((size_t)gP * (size_t)P.Kr * 8);
     P.o_pevals = take((size_t)gA * 8);
     P.o_queue = take(64 * 4);  // work-queue counters of the pair launches
-    const int64_t red = reduce_scratch_elems(std::max<int64_t>(P.max_groups[0], 1), P.M,
+    const int64_t red = reduce_scratch_elems(std::max<int64_t>(P.max_groups[0], 1) << P.parts_sh, P.M,
                                              P.nb_count);  // sums (Kr or Kr * Kp) and evals (1)
     P.o_red = take((size_t)red * 8);
     // auto-count with shared weights: rows2 = rows1 + seam corrections, no swapped pass
@@ -441,7 +587,7 @@ static int make_plan(const hp_request* r, int kind, Plan& P) {
     // packed rows (x, y, z, Hilbert position[, up to 4 weights]) of every side
     // the stream side is built from: one random row read per point in the gather
     for (int s = 0; s < 2; s++) {
-        if (!P.sorted[s][kRowMajor].needed) continue;
+        if (P.tiles || !P.sorted[s][kRowMajor].needed) continue;
         const bool pack_w = P.weighted() && P.nw <= 4;
         P.row_nw[s] = pack_w ? P.nw : 0;
         P.row_stride[s] = pack_w ? 8 : 4;
@@ -462,12 +608,16 @@ static int make_plan(const hp_request* r, int kind, Plan& P) {
     P.tr.spec.table_off = (int64_t)P.o_tr;
     P.tp.spec.edges_off = (int64_t)P.o_ep;
     P.tp.spec.table_off = (int64_t)P.o_tp;
+    P.ttr.spec.off = (int64_t)P.o_ttr;
+    P.ttp.spec.off = (int64_t)P.o_ttp;
     P.consts.assign(consts_end, 0);
     std::memcpy(P.consts.data() + P.o_geom, P.geom.data(), sizeof(MockGeom) * (size_t)P.M);
     std::memcpy(P.consts.data() + P.o_er, P.tr.e.data(), P.tr.e.size() * 8);
     std::memcpy(P.consts.data() + P.o_ep, P.tp.e.data(), P.tp.e.size() * 8);
     std::memcpy(P.consts.data() + P.o_tr, P.tr.t.data(), P.tr.t.size() * sizeof(TabEntry));
     std::memcpy(P.consts.data() + P.o_tp, P.tp.t.data(), P.tp.t.size() * sizeof(TabEntry));
+    if (P.ttr.spec.ok) std::memcpy(P.consts.data() + P.o_ttr, P.ttr.t.data(), P.ttr.t.size() * 4);
+    if (P.ttp.spec.ok) std::memcpy(P.consts.data() + P.o_ttp, P.ttp.t.data(), P.ttp.t.size() * 4);
     for (int s = 0; s < 2; s++) std::memcpy(P.consts.data() + P.o_tfirst[s], P.tfirst[s].data(), P.tfirst[s].size() * 4);
     return 0;
 }
@@ -515,11 +665,11 @@ struct PhaseRange {
     ~PhaseRange() { end(); }
 };
 
-static int run(const hp_request* r, int kind) {
+static int run(const hp_request* r, int kind, bool tiles = true) {
     PhaseRange phase;
     phase.begin("halopair: plan");
     Plan P;
-    if (make_plan(r, kind, P)) return -1;
+    if (make_plan(r, kind, P, tiles)) return -1;
     if (!r->workspace) return fail("workspace must not be null");
     if (r->workspace_bytes < P.total) return fail("workspace too small");
     if (P.n[0] > 0 && (!r->x1 || !r->y1 || !r->z1)) return fail("sample1 coordinates must not be null");
@@ -571,6 +721,26 @@ static int run(const hp_request* r, int kind) {
     phase.begin("halopair: cell build");
     if (r->build_events[0] && hipEventRecord(static_cast<hipEvent_t>(r->build_events[0]), s) != hipSuccess)
         return fail("event record failed");
+    // matrix-core kernels: one curve-ordered copy of each side, the stream side's with its cubes
+    SortedSide curve[2] = {};
+    for (int sd = 0; P.tiles && sd < (P.same ? 1 : 2); sd++) {
+        SortedSide& C = curve[sd];
+        C.x = reinterpret_cast<double*>(ws + P.o_crow[sd]);
+        C.w = P.weighted() ? reinterpret_cast<double*>(ws + P.o_cw[sd]) : nullptr;
+        C.perm = reinterpret_cast<uint32_t*>(ws + P.o_cperm[sd]);
+        C.cubes = P.o_cubes[sd] ? reinterpret_cast<uint2*>(ws + P.o_cubes[sd]) : nullptr;
+        C.xs = 4;
+        PackedRows rows;
+        // (N, 3) rows are gathered in place, columns through packed rows
+        if (XS[sd] == 1 && P.n[sd] > 0) rows.p = reinterpret_cast<double*>(ws + P.o_rows[sd]);
+        SortTiles st;
+        st.first = reinterpret_cast<const uint32_t*>(ws + P.o_tfirst[sd]);
+        st.tile = P.tile[sd];
+        st.ntiles = P.ntiles[sd];
+        if (build_curve_side(dgeom, P.M, sd, X[sd], Y[sd], Z[sd], P.weighted() ? W[sd] : nullptr, P.nw, P.n[sd],
+                             P.total_cells, P.bits_hilbert, sb, st, C, status, s, rows, XS[sd]))
+            return fail("cell build launch failed");
+    }
     for (int sd = 0; sd < 2; sd++) {
         for (int o = 0; o < 2; o++) {
             const Side& S = P.sorted[sd][o];
@@ -604,7 +774,7 @@ static int run(const hp_request* r, int kind) {
     }
     // the order keys: the fourth word of each row of side 0's row-major copy
     const uint64_t* hkey =
-        (P.sym && P.n[0] > 0) ? reinterpret_cast<const uint64_t*>(ws + P.sorted[0][kRowMajor].x) + 3 : nullptr;
+        (P.sym && P.n[0] > 0 && !P.tiles) ? reinterpret_cast<const uint64_t*>(ws + P.sorted[0][kRowMajor].x) + 3 : nullptr;
     if (r->build_events[1] && hipEventRecord(static_cast<hipEvent_t>(r->build_events[1]), s) != hipSuccess)
         return fail("event record failed");
 
@@ -619,9 +789,18 @@ static int run(const hp_request* r, int kind) {
     L.ngroups = P.ngroups[0];
     L.lane = lane_ptrs(ws, P.sorted[0][kHilbert], X[0], Y[0], Z[0], P.weighted() ? W[0] : nullptr, XS[0]);
     L.strm = side_ptrs(ws, P.sorted[s2][kRowMajor]);
+    if (P.tiles) {
+        L.lane = curve[0];
+        L.strm = curve[s2];
+        L.sym = P.sym ? 1 : 0;
+    }
     L.nw = P.nw;
     L.br = P.tr.spec;
     L.bp = P.tp.spec;
+    L.tr = P.ttr.spec;
+    L.tr.ok = P.tiles ? 1 : 0;
+    L.tp = P.ttp.spec;
+    L.parts_sh = P.parts_sh;
     L.ws = ws;
     L.wfunc = r->wfunc;
     L.waves = r->tile_waves;
@@ -631,32 +810,21 @@ static int run(const hp_request* r, int kind) {
     L.pcount = P.counts ? reinterpret_cast<uint64_t*>(ws + P.o_pcount) : nullptr;
     L.psum = P.sums ? reinterpret_cast<double*>(ws + P.o_psum) : nullptr;
     L.ptan = P.tangent ? reinterpret_cast<double*>(ws + P.o_ptan) : nullptr;
-    L.pevals = reinterpret_cast<uint64_t*>(ws + P.o_pevals);
+    // candidate evaluations per group, only when the caller asked for them
+    L.pevals = r->evals ? reinterpret_cast<uint64_t*>(ws + P.o_pevals) : nullptr;
+    if (L.pevals) launch_fill_u32(reinterpret_cast<uint32_t*>(L.pevals), 0u, P.ngroups[0] * 2, s);
     L.queue = reinterpret_cast<uint32_t*>(ws + P.o_queue);
-    switch (kind) {
-        case HP_NPAIRS_3D: L.mode = kModeCount3D; break;
-        case HP_NPAIRS_PROJECTED: L.mode = kModeProj; break;
-        case HP_NPAIRS_XY_Z: L.mode = kModeXYZ; break;
-        case HP_NPAIRS_PER_OBJECT_3D:
-            L.mode = kModeObj;
-            L.orows = r->counts;
-            break;
-        case HP_MARKED_NPAIRS_XY_Z: L.mode = kModeWXYZ; break;
-        case HP_NPAIRS_JACKKNIFE_3D:
-        case HP_NPAIRS_JACKKNIFE_XY_Z:
-            L.mode = (kind == HP_NPAIRS_JACKKNIFE_XY_Z) ? kModeJackXY : kModeJack;
-            L.jacc = reinterpret_cast<double*>(ws + P.o_jacc);
-            L.nsamp = P.nsamp;
-            L.jslots = P.jslots;
-            launch_fill_u32(reinterpret_cast<uint32_t*>(L.jacc), 0u, (int64_t)P.M * (P.nsamp + 1) * P.nb_count * 2,
-                            s);
-            break;
-        default:
-            L.mode = P.tangent ? kModeTan
-                               : ((r->wfunc == 1 && P.nw == 1 && (P.rows1 || P.rows2)) ? kModeJac : kModeWSum);
-            L.also_count = P.counts ? 1 : 0;
-            L.rows = P.rows1 ? r->rows1 : nullptr;
-            break;
+    L.mode = mode_of(P, kind, r->wfunc);
+    if (kind == HP_NPAIRS_PER_OBJECT_3D) L.orows = r->counts;
+    if (P.jack) {
+        L.jacc = reinterpret_cast<double*>(ws + P.o_jacc);
+        L.nsamp = P.nsamp;
+        L.jslots = P.jslots;
+        launch_fill_u32(reinterpret_cast<uint32_t*>(L.jacc), 0u, (int64_t)P.M * (P.nsamp + 1) * P.nb_count * 2, s);
+    }
+    if (kind == HP_MARKED_NPAIRS_3D) {
+        L.also_count = P.counts ? 1 : 0;
+        L.rows = P.rows1 ? r->rows1 : nullptr;
     }
     double* corr = nullptr;
     if (P.elim) {
@@ -694,6 +862,10 @@ static int run(const hp_request* r, int kind) {
         B.ngroups = P.ngroups[s2];
         B.lane = lane_ptrs(ws, P.sorted[s2][kHilbert], X[s2], Y[s2], Z[s2], W[s2], XS[s2]);
         B.strm = side_ptrs(ws, P.sorted[0][kRowMajor]);
+        if (P.tiles) {
+            B.lane = curve[s2];
+            B.strm = curve[0];
+        }
         B.rows = r->rows2;
         B.pcount = nullptr;
         B.psum = nullptr;
@@ -716,12 +888,12 @@ static int run(const hp_request* r, int kind) {
             return fail("jackknife reduction launch failed");
     }
     if (P.sums) {
-        if (launch_reduce_sums_s(L.psum, P.Kr, P.mxyz ? P.Kp : 0, dgeom, P.M, 0, P.max_groups[0],
+        if (launch_reduce_sums_s(L.psum, P.Kr, P.mxyz ? P.Kp : 0, dgeom, P.M, 0, P.max_groups[0], P.parts_sh,
                                  reinterpret_cast<double*>(red), r->sums, s))
             return fail("reduction launch failed");
     }
     if (P.tangent) {
-        if (launch_reduce_sums_s(L.ptan, P.Kr, 0, dgeom, P.M, 0, P.max_groups[0], reinterpret_cast<double*>(red),
+        if (launch_reduce_sums_s(L.ptan, P.Kr, 0, dgeom, P.M, 0, P.max_groups[0], P.parts_sh, reinterpret_cast<double*>(red),
                                  r->tangents, s))
             return fail("reduction launch failed");
     }
@@ -787,6 +959,13 @@ int hp_npairs_3d_noalloc(const hp_request* req) {
         return fail("hp_npairs_3d_noalloc takes no workspace (workspace must be NULL and workspace_bytes 0)");
     Plan P;
     if (make_plan(req, HP_NPAIRS_3D, P)) return -1;
+    bool tiles = true;
+    if (P.total > (size_t)HP_NOALLOC_SCRATCH_BYTES) {
+        // the other kernels' sorted copies of two different samples are smaller
+        P = Plan();
+        if (make_plan(req, HP_NPAIRS_3D, P, false)) return -1;
+        tiles = false;
+    }
     if (P.total > (size_t)HP_NOALLOC_SCRATCH_BYTES)
         return fail("hp_npairs_3d_noalloc: the request needs " + std::to_string(P.total) +
                     " bytes of scratch, more than the library's fixed " +
@@ -797,7 +976,7 @@ int hp_npairs_3d_noalloc(const hp_request* req) {
     hp_request r = *req;
     r.workspace = ptr;
     r.workspace_bytes = (size_t)HP_NOALLOC_SCRATCH_BYTES;
-    return run(&r, HP_NPAIRS_3D);
+    return run(&r, HP_NPAIRS_3D, tiles);
 }
 int hp_npairs_projected(const hp_request* req) { return run(req, HP_NPAIRS_PROJECTED); }
 int hp_npairs_xy_z(const hp_request* req) { return run(req, HP_NPAIRS_XY_Z); }
@@ -861,6 +1040,28 @@ int hp_debug_bin_lookup(const double* r2, int32_t K, const double* d, int64_t n,
         info[1] = T.spec.base;
         info[2] = T.spec.nb;
         info[3] = T.spec.multi;
+    }
+    return 0;
+}
+
+// Host-only: the matrix-core kernels' lookup for d whose high word is off by
+// `off` units: the bin, or -1 where the kernels evaluate the pair exactly.
+int hp_debug_tile_lookup(const double* r2, int32_t K, const double* d, int64_t n, int32_t off, int32_t* out,
+                         int32_t* info) {
+    if (!r2 || !d || !out || K < 1) return fail("bad arguments");
+    std::vector<double> e = suffix_min(r2, K);
+    const TileTable T = make_tile_table(e, K);
+    if (info) {
+        info[0] = T.spec.ok;
+        info[1] = (int32_t)T.spec.sh3 + 3;
+        info[2] = (int32_t)T.spec.mask + 1;
+    }
+    for (int64_t i = 0; i < n && T.spec.ok; i++) {
+        const int32_t h = (int32_t)hiword(d[i]) + off;
+        const int32_t c = std::max((int32_t)T.spec.lo, std::min(h, (int32_t)T.spec.hi));
+        const size_t at = (size_t)(((uint32_t)c >> (T.spec.sh3 + 3)) & T.spec.mask);
+        const uint32_t edge = T.t[2 * at], t = edge - (uint32_t)h;
+        out[i] = t <= 2u ? -1 : (int32_t)(T.t[2 * at + 1] + (edge < (uint32_t)h ? 1u : 0u));
     }
     return 0;
 }

@@ -435,6 +435,45 @@ int sort_tile(int64_t n) {
     return n >= kSortLargeMin ? kSortTileLarge : kSortTile;
 }
 
+// The counting-sort passes of one order: keys from kin0 (or sb.keys[0]), the
+// permutation into perm; returns the buffer that ends up with the sorted keys,
+// or null on a bad tile shape.
+static uint32_t* sort_passes(const uint32_t* kin0, const MockGeom* geom, int nmocks, int side, int key_bits,
+                             SortBufs sb, SortTiles st, uint32_t* perm, bool global_ids, hipStream_t s) {
+    const int tile = st.tile, ntiles = st.ntiles;
+    if ((tile != kSortTile && tile != kSortTileLarge) || ntiles <= 0) return nullptr;
+    const int passes = key_bits <= 0 ? 1 : (key_bits + kRadixBits - 1) / kRadixBits;
+    int cur = 0;
+    for (int pass = 0; pass < passes; pass++) {
+        const int shift = pass * kRadixBits;
+        const uint32_t* kin = (pass == 0 && kin0) ? kin0 : sb.keys[cur];
+        if (tile == kSortTileLarge)
+            hipLaunchKernelGGL(k_radix_hist<kSortTileLarge>, dim3(ntiles), dim3(256), 0, s, kin, geom, st.first,
+                               nmocks, side, shift, sb.tile_counts, ntiles);
+        else
+            hipLaunchKernelGGL(k_radix_hist<kSortTile>, dim3(ntiles), dim3(256), 0, s, kin, geom, st.first, nmocks,
+                               side, shift, sb.tile_counts, ntiles);
+        hipLaunchKernelGGL(k_radix_scan, dim3(kRadixDigits), dim3(256), 0, s, sb.tile_counts, ntiles,
+                           sb.digit_totals);
+        // the last pass writes the permutation straight into perm, and (when
+        // asked) the global cell ids for the cell-start table
+        const bool last = pass == passes - 1;
+        uint32_t* vdst = last ? perm : sb.vals[cur ^ 1];
+        const uint32_t* vsrc = pass == 0 ? (const uint32_t*)nullptr : sb.vals[cur];
+        const int add_off = (last && global_ids) ? 1 : 0;
+        if (tile == kSortTileLarge)
+            hipLaunchKernelGGL((k_radix_scatter<kSortTileLarge, 8>), dim3(ntiles), dim3(512), 0, s, kin, vsrc,
+                               sb.keys[cur ^ 1], vdst, geom, st.first, nmocks, side, shift, add_off, sb.tile_counts,
+                               sb.digit_totals, ntiles);
+        else
+            hipLaunchKernelGGL((k_radix_scatter<kSortTile, 4>), dim3(ntiles), dim3(256), 0, s, kin, vsrc,
+                               sb.keys[cur ^ 1], vdst, geom, st.first, nmocks, side, shift, add_off, sb.tile_counts,
+                               sb.digit_totals, ntiles);
+        cur ^= 1;
+    }
+    return sb.keys[cur];
+}
+
 int build_sorted_side(const MockGeom* geom, int nmocks, int side, Order order, const double* x, const double* y,
                       const double* z, const double* w, int nw, int64_t n, int64_t total_cells, int key_bits,
                       SortBufs sb, SortTiles st, SortedSide out, int32_t* status, hipStream_t s, PackedRows rows,
@@ -448,38 +487,8 @@ int build_sorted_side(const MockGeom* geom, int nmocks, int side, Order order, c
     if (!keys_in)
         hipLaunchKernelGGL(k_keys, dim3(nb), dim3(256), 0, s, geom, nmocks, side, (int)order, x, y, z, n, sb.keys[0],
                            status, order == kHilbert ? keys_row_out : (uint32_t*)nullptr, w, nw, rows, xs);
-    const int tile = st.tile, ntiles = st.ntiles;
-    if (tile != kSortTile && tile != kSortTileLarge) return -1;
-    if (ntiles <= 0) return -1;
-    const int passes = key_bits <= 0 ? 1 : (key_bits + kRadixBits - 1) / kRadixBits;
-    int cur = 0;
-    for (int pass = 0; pass < passes; pass++) {
-        const int shift = pass * kRadixBits;
-        const uint32_t* kin = (pass == 0 && keys_in) ? keys_in : sb.keys[cur];
-        if (tile == kSortTileLarge)
-            hipLaunchKernelGGL(k_radix_hist<kSortTileLarge>, dim3(ntiles), dim3(256), 0, s, kin, geom, st.first,
-                               nmocks, side, shift, sb.tile_counts, ntiles);
-        else
-            hipLaunchKernelGGL(k_radix_hist<kSortTile>, dim3(ntiles), dim3(256), 0, s, kin, geom, st.first, nmocks,
-                               side, shift, sb.tile_counts, ntiles);
-        hipLaunchKernelGGL(k_radix_scan, dim3(kRadixDigits), dim3(256), 0, s, sb.tile_counts, ntiles,
-                           sb.digit_totals);
-        // the last pass writes the permutation straight into out.perm, and
-        // (row-major) the global cell ids for the cell-start table
-        const bool last = pass == passes - 1;
-        uint32_t* vdst = last ? out.perm : sb.vals[cur ^ 1];
-        const uint32_t* vsrc = pass == 0 ? (const uint32_t*)nullptr : sb.vals[cur];
-        const int add_off = (last && order == kRowMajor) ? 1 : 0;
-        if (tile == kSortTileLarge)
-            hipLaunchKernelGGL((k_radix_scatter<kSortTileLarge, 8>), dim3(ntiles), dim3(512), 0, s, kin, vsrc,
-                               sb.keys[cur ^ 1], vdst, geom, st.first, nmocks, side, shift, add_off, sb.tile_counts,
-                               sb.digit_totals, ntiles);
-        else
-            hipLaunchKernelGGL((k_radix_scatter<kSortTile, 4>), dim3(ntiles), dim3(256), 0, s, kin, vsrc,
-                               sb.keys[cur ^ 1], vdst, geom, st.first, nmocks, side, shift, add_off, sb.tile_counts,
-                               sb.digit_totals, ntiles);
-        cur ^= 1;
-    }
+    const uint32_t* keys = sort_passes(keys_in, geom, nmocks, side, key_bits, sb, st, out.perm, order == kRowMajor, s);
+    if (!keys) return -1;
     if (check("sort")) return -1;
     // The lane side (Hilbert order) is read once per group through the
     // permutation; only the stream side needs sorted copies.
@@ -487,9 +496,72 @@ int build_sorted_side(const MockGeom* geom, int nmocks, int side, Order order, c
         // the gather of the packed rows and the cell starts in one pass
         if (!rows.p) return -1;  // the row-major gather reads the packed rows
         hipLaunchKernelGGL(k_gather, dim3((unsigned)((n + 1 + 255) / 256)), dim3(256), 0, s, out.perm, n, rows, w,
-                           nw, out.x, out.w, want_hkey ? 1 : 0, sb.keys[cur], total_cells, out.cell_start);
+                           nw, out.x, out.w, want_hkey ? 1 : 0, keys, total_cells, out.cell_start);
     }
     return check("gather");
+}
+
+// The curve-ordered rows of one side (see build_curve_side), and the rows of
+// every cube that holds points: a cube of the 2^cbits grid is one stretch of the
+// sorted keys, so the point at its start and the one at its end write its entry
+// (the other entries were cleared).
+__global__ void k_gather_curve(const uint32_t* __restrict__ perm, const uint32_t* __restrict__ keys, int64_t n,
+                               const MockGeom* __restrict__ geom, int nmocks, int side, const double* __restrict__ x,
+                               const double* __restrict__ y, const double* __restrict__ z, int64_t xs, PackedRows rows,
+                               const double* __restrict__ w, int nw, double* __restrict__ orow,
+                               double* __restrict__ ow, uint2* __restrict__ cubes) {
+    const int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (q >= n) return;
+    const int64_t p = perm[q];
+    double px, py, pz;
+    if (rows.p) {
+        const double4 c = *reinterpret_cast<const double4*>(rows.p + p * rows.stride);
+        px = c.x;
+        py = c.y;
+        pz = c.z;
+    } else {
+        px = x[p * xs];
+        py = y[p * xs];
+        pz = z[p * xs];
+    }
+    reinterpret_cast<double4*>(orow)[q] = make_double4(px, py, pz, __longlong_as_double((long long)p));
+    if (ow)
+        for (int k = 0; k < nw; k++) ow[q * nw + k] = w[p * nw + k];
+    if (!cubes) return;
+    const int qf = __builtin_amdgcn_readfirstlane((int)q);
+    const int64_t mf = mock_of_point(geom, nmocks, side, qf);
+    const int64_t ml = mock_of_point(geom, nmocks, side, min((int64_t)qf + 63, n - 1));
+    const int64_t m = (mf == ml) ? mf : mock_of_point(geom, nmocks, side, q);
+    const MockGeom& G = geom[m];
+    const int sh = G.mbits - G.cbits;
+    const uint32_t h = keys[q] >> (3 * sh);
+    const int64_t q0 = G.p_off[side], q1 = q0 + G.n[side];
+    const bool first = q == q0 || (keys[q - 1] >> (3 * sh)) != h;
+    const bool last = q + 1 == q1 || (keys[q + 1] >> (3 * sh)) != h;
+    if (!first && !last) return;
+    bool bad = false;
+    const int hn = 1 << G.mbits;
+    const int cx = cell_index(px, G.inv_hcell[0], hn, bad, G.period[0], 0) >> sh;
+    const int cy = cell_index(py, G.inv_hcell[1], hn, bad, G.period[1], 0) >> sh;
+    const int cz = cell_index(pz, G.inv_hcell[2], hn, bad, G.period[2], 0) >> sh;
+    uint2* c = cubes + G.cell_off + ((((int64_t)cx << G.cbits) + cy) << G.cbits) + cz;
+    if (first) c->x = (uint32_t)q;
+    if (last) c->y = (uint32_t)(q + 1);
+}
+
+int build_curve_side(const MockGeom* geom, int nmocks, int side, const double* x, const double* y, const double* z,
+                     const double* w, int nw, int64_t n, int64_t total_cells, int key_bits, SortBufs sb, SortTiles st,
+                     SortedSide out, int32_t* status, hipStream_t s, PackedRows rows, int64_t xs) {
+    if (out.cubes && launch_fill_u32(reinterpret_cast<uint32_t*>(out.cubes), 0u, 2 * total_cells, s)) return -1;
+    if (n <= 0) return 0;
+    const unsigned nb = (unsigned)((n + 255) / 256);
+    hipLaunchKernelGGL(k_keys, dim3(nb), dim3(256), 0, s, geom, nmocks, side, (int)kHilbert, x, y, z, n, sb.keys[0],
+                       status, (uint32_t*)nullptr, (const double*)nullptr, 0, rows, xs);
+    const uint32_t* keys = sort_passes(nullptr, geom, nmocks, side, key_bits, sb, st, out.perm, false, s);
+    if (!keys) return -1;
+    hipLaunchKernelGGL(k_gather_curve, dim3(nb), dim3(256), 0, s, out.perm, keys, n, geom, nmocks, side, x, y, z, xs,
+                       rows, w, nw, out.x, out.w, out.cubes);
+    return check("curve");
 }
 
 }  // namespace hp

@@ -26,7 +26,7 @@ struct alignas(64) MockGeom {
     int32_t ndiv[3];      // cells per dimension
     int32_t pbc;
     int32_t mbits;        // bits per dimension of the lane-ordering (Hilbert) grid
-    int32_t pad;
+    int32_t cbits;        // curve builds: bits per dimension of the cube grid (<= mbits; ndiv = 2^cbits)
     int64_t p_off[2];     // first point of this mock on each side
     int64_t n[2];         // points of this mock on each side
     int64_t cell_off;     // first global cell id of this mock
@@ -54,6 +54,16 @@ struct BinSpec {
     int32_t multi;   // 1 if some bucket holds more than one edge
     int64_t edges_off;  // byte offset of e[0..K+1] in the workspace
     int64_t table_off;  // byte offset of TabEntry table[nb]
+};
+
+// Bucket table of the matrix-core kernels (pairs_tile.h), indexed by the high
+// word h of a squared distance: entry ((clamp(h, lo, hi) >> shift) & mask).
+struct TileSpec {
+    int64_t off;     // byte offset of the (edge + 1, k) entries in the workspace
+    uint32_t lo, hi; // clamp: first value of the lowest and of the highest bucket
+    uint32_t sh3;    // shift - 3 (entries are 8 bytes)
+    uint32_t mask;   // entries - 1 (a power of two)
+    int32_t ok;      // the edges fit such a table
 };
 
 // One bucket of the table: k = number of edges strictly below the bucket's
@@ -89,6 +99,7 @@ struct SortedSide {
     double* w;          // (n, nw) row-major, or nullptr
     uint32_t* perm;     // sorted position -> original index
     uint32_t* cell_start;  // row-major order only: [total_cells + 1]
+    uint2* cubes;       // curve order with rows: [total_cells] first and past-the-last row of each cube
     int64_t xs;         // doubles between consecutive points of x, y, z (4: the sorted 32-byte rows)
 };
 
@@ -133,6 +144,16 @@ int build_sorted_side(const MockGeom* geom, int nmocks, int side, Order order,
                       bool want_hkey = false, uint32_t* keys_row_out = nullptr,
                       const uint32_t* keys_in = nullptr, int64_t xs = 1);
 
+// The Hilbert-ordered copy of one side for the matrix-core kernels: rows of 32
+// bytes (x, y, z, input index) in curve order (out.x), the weight rows (out.w)
+// and, per cube of a 2^cube_bits grid in row-major order, the rows it holds
+// (out.cubes): a cube is one stretch of the curve.  One sort serves as the lane
+// order and as the stream order.  `rows`: packed rows of the input (the key
+// pass writes them), or none: the gather reads the caller's coordinates.
+int build_curve_side(const MockGeom* geom, int nmocks, int side, const double* x, const double* y, const double* z,
+                     const double* w, int nw, int64_t n, int64_t total_cells, int key_bits, SortBufs sb, SortTiles st,
+                     SortedSide out, int32_t* status, hipStream_t s, PackedRows rows, int64_t xs);
+
 // pairs.hip
 struct PairLaunch {
     int mode;              // kModeCount3D ...
@@ -148,6 +169,9 @@ struct PairLaunch {
     int nw;
     BinSpec br;            // radial / rp bins
     BinSpec bp;            // pi bins (xy_z) or pi_max (projected, nbins = 1)
+    int sym;               // matrix-core kernels: symmetric auto-count
+    TileSpec tr, tp;       // the radial / rp and the pi bins for the matrix-core kernels
+    int parts_sh;          // ... log2 of the work items per lane group (FP64 partials: one row each)
     const void* ws;        // workspace base (edges / tables)
     uint64_t* pcount;      // [nmocks][crep][nbins_count], zeroed, accumulated with atomics
     int crep;              // count replicas per mock (spread the atomics over cache lines)
@@ -176,6 +200,9 @@ struct PairLaunch {
     // by launch_pairs before every launch)
     uint32_t* queue;
 };
+// LDS bytes of one wave of the matrix-core kernels for a mode, or -1 when they
+// have no such mode
+int tile_wave_bytes(int mode, int K, int Kp, int nw, int also);
 enum Mode : int { kModeCount3D = 0, kModeProj = 1, kModeXYZ = 2, kModeWSum = 3, kModeJac = 4, kModeTan = 5,
                   kModeObj = 6, kModeWXYZ = 7, kModeJack = 8, kModeJackXY = 9 };
 constexpr int kJackSlots = 16;  // most subsample tags a wave keeps in LDS

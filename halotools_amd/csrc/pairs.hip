@@ -2,7 +2,11 @@
 // dispatch to the per-mode launchers.  The kernel itself is pairs_kernel.h.
 #include <cstdlib>
 
-#include "pairs_kernel.h"
+#include "pairs_tile.h"
+
+#ifndef HP_TILE_TAIL
+#define HP_TILE_TAIL 8  // sixteenths of the resident waves whose groups go out in quarters at the end
+#endif
 
 namespace hp {
 
@@ -17,6 +21,15 @@ extern template int launch_mode<kModeJackXY>(const PairArgs&, int, int, int, int
 extern template int launch_mode<kModeWSum>(const PairArgs&, int, int, int, int, hipStream_t);
 extern template int launch_mode<kModeJac>(const PairArgs&, int, int, int, int, hipStream_t);
 extern template int launch_mode<kModeTan>(const PairArgs&, int, int, int, int, hipStream_t);
+
+extern template int launch_tiles_mode<kModeCount3D>(const TileArgs&, int, int64_t, int, int, int, hipStream_t);
+extern template int launch_tiles_mode<kModeProj>(const TileArgs&, int, int64_t, int, int, int, hipStream_t);
+extern template int launch_tiles_mode<kModeXYZ>(const TileArgs&, int, int64_t, int, int, int, hipStream_t);
+extern template int launch_tiles_mode<kModeWXYZ>(const TileArgs&, int, int64_t, int, int, int, hipStream_t);
+extern template int launch_tiles_mode<kModeObj>(const TileArgs&, int, int64_t, int, int, int, hipStream_t);
+extern template int launch_tiles_mode<kModeJac>(const TileArgs&, int, int64_t, int, int, int, hipStream_t);
+extern template int launch_tiles_mode<kModeTan>(const TileArgs&, int, int64_t, int, int, int, hipStream_t);
+extern template int launch_tiles_mode<kModeWSum>(const TileArgs&, int, int64_t, int, int, int, hipStream_t);
 
 static int align16(int v) { return (v + 15) & ~15; }
 
@@ -70,6 +83,109 @@ static int jack_slots(const PairLaunch& L, int kc) {
     return std::max(0, std::min(L.jslots, 24576 / jrow - 1));
 }
 
+static int num_compute_units() {
+    static int n = 0;  // of the device, queried once
+    if (n == 0) {
+        int dev = 0, v = 0;
+        if (hipGetDevice(&dev) == hipSuccess &&
+            hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
+            n = v;
+        else
+            n = 256;
+    }
+    return n;
+}
+
+// LDS layout of one wave of the matrix-core kernels: the stage, the weights of
+// staged and lane points (and the lanes' z for (rp, pi) bins), the histogram.
+static int tile_layout(int mode, int K, int Kp, int nw, int also, TileArgs& A) {
+    const bool xy = (mode == kModeXYZ || mode == kModeWXYZ || mode == kModeProj);
+    A.w_off = align16(kTileBytes);
+    A.lw_off = A.w_off + align16(nw * kSlots * 8);
+    A.hist_off = A.lw_off + nw * 512 + (xy ? 512 : 0);
+    A.cnt_off = A.hist_off;
+    int h = -1;
+    switch (mode) {
+        case kModeCount3D:
+        case kModeProj: h = (K + 1) * 128; break;
+        case kModeXYZ: h = K * Kp * 4; break;
+        case kModeWXYZ: h = K * Kp * 8; break;
+        case kModeObj: h = (K + 1) * 256; break;
+        case kModeJac:
+            h = (K + 1) * 512;
+            if (also) { A.cnt_off = A.hist_off + h; h += (K + 1) * 128; }
+            break;
+        case kModeWSum:
+            h = (K + 1) * 128;
+            if (also) { A.cnt_off = A.hist_off + h; h += (K + 1) * 128; }
+            break;
+        case kModeTan:
+            A.cnt_off = A.hist_off + 256;
+            h = (K + 1) * (also ? 384 : 256);
+            break;
+        default: return -1;
+    }
+    A.wave_bytes = align16(A.hist_off + h);
+    return A.wave_bytes;
+}
+
+int tile_wave_bytes(int mode, int K, int Kp, int nw, int also) {
+    TileArgs A;
+    if ((int64_t)K * std::max(Kp, 1) > 65536) return -1;
+    return tile_layout(mode, K, Kp, nw, also, A);
+}
+
+// Matrix-core kernels: workgroup shape (the waves per workgroup that keep the
+// most waves resident) and work items.
+static int launch_tiles(const PairLaunch& L, int lds_per_block, hipStream_t s) {
+    TileArgs A;
+    A.L = L;
+    A.tr = L.tr;
+    A.tp = L.tp;
+    const bool xy = (L.mode == kModeXYZ || L.mode == kModeWXYZ || L.mode == kModeProj);
+    const int also = L.also_count ? 1 : 0;
+    const int prod = (L.wfunc == 1 && L.nw == 1) ? 1 : 0;
+    if (tile_layout(L.mode, L.br.nbins, L.bp.nbins, L.nw, also, A) < 0) return -1;
+    A.tp_off = align16(8 * ((int)L.tr.mask + 1));
+    A.tab_bytes = A.tp_off + (xy ? align16(8 * ((int)L.tp.mask + 1)) : 0);
+    constexpr int kLdsPerCU = 160 * 1024, reg_waves = 4 * HP_TILE_WPS;
+    int waves = 0, best = 0;
+    for (const int w : {4, 8, 2, 1}) {
+        if (L.waves > 0 && w != L.waves) continue;
+        const int bytes = A.tab_bytes + w * A.wave_bytes;
+        if (bytes > lds_per_block) continue;
+        const int res = std::min(w * (kLdsPerCU / bytes), reg_waves);
+        if (res > best) { best = res; waves = w; }
+    }
+    if (best == 0 && L.waves > 0) {
+        PairLaunch M = L;
+        M.waves = 0;  // the shape asked for does not fit: take the best one
+        return launch_tiles(M, lds_per_block, s);
+    }
+    if (best == 0) return -2;
+    A.parts_sh = L.parts_sh;
+    A.tail_sh = L.parts_sh;
+    A.tail = L.ngroups;
+    const bool counts = (L.mode == kModeCount3D || L.mode == kModeProj || L.mode == kModeXYZ);
+    if (counts && L.parts_sh < 2) {
+        A.tail_sh = 2;
+        A.tail = L.ngroups - std::min<int64_t>(L.ngroups, (int64_t)num_compute_units() * best * HP_TILE_TAIL / 16);
+    }
+    const int64_t items = (A.tail << A.parts_sh) + ((L.ngroups - A.tail) << A.tail_sh);
+    const int smem = A.tab_bytes + waves * A.wave_bytes;
+    switch (L.mode) {
+        case kModeCount3D: return launch_tiles_mode<kModeCount3D>(A, waves, items, smem, also, 0, s);
+        case kModeProj: return launch_tiles_mode<kModeProj>(A, waves, items, smem, also, 0, s);
+        case kModeXYZ: return launch_tiles_mode<kModeXYZ>(A, waves, items, smem, also, 0, s);
+        case kModeWXYZ: return launch_tiles_mode<kModeWXYZ>(A, waves, items, smem, also, prod, s);
+        case kModeObj: return launch_tiles_mode<kModeObj>(A, waves, items, smem, also, 0, s);
+        case kModeJac: return launch_tiles_mode<kModeJac>(A, waves, items, smem, also, L.swap, s);
+        case kModeTan: return launch_tiles_mode<kModeTan>(A, waves, items, smem, also, 0, s);
+        case kModeWSum: return launch_tiles_mode<kModeWSum>(A, waves, items, smem, also, prod, s);
+    }
+    return -1;
+}
+
 int launch_pairs(const PairLaunch& L, hipStream_t s) {
     PairArgs A;
     A.L = L;
@@ -92,15 +208,9 @@ int launch_pairs(const PairLaunch& L, hipStream_t s) {
             lds_per_block = 64 * 1024;
     }
     const int kLdsPerBlock = lds_per_block;
-    static int num_cus = 0;  // compute units of the device (queried once)
-    if (num_cus == 0) {
-        int dev = 0, v = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
-            num_cus = v;
-        else
-            num_cus = 256;
-    }
+    const int num_cus = num_compute_units();
+    // the plan chose the kernels: their sorted copies differ
+    if (L.tr.ok) return launch_tiles(L, kLdsPerBlock, s);
     // product marks (weight_func_id 1, one weight per point) have a compiled-in variant
     const int prod = (L.wfunc == 1 && L.nw == 1) ? 1 : 0;
     // waves per SIMD the kernels' registers allow (their launch bounds; the

@@ -1,0 +1,907 @@
+// pairs_tile.h -- pair kernels on the FP64 matrix cores (replace the j-loops of
+// PC/cpairs/npairs_3d_engine.pyx:103-182 and its siblings for the common bin
+// layouts; the kernels of pairs_kernel.h take every other request).
+//
+// One wavefront takes a group of 64 lane points consecutive along the Hilbert
+// curve, as four sub-groups of 16.  Stream points near the group's box are
+// staged in LDS in coordinates relative to the box centre (the periodic shift
+// folded in); staged points near a sub-group's own, smaller box are dealt to
+// it in tiles of 16, and one v_mfma_f64_16x16x4 forms the 256 squared
+// distances |a|^2 + |b|^2 - 2 a.b of a tile (planar ones for (rp, pi) bins).
+//
+// Exactness.  The matrix product's rounding is far below one unit of the high
+// word of the distance (20 mantissa bits) except for very close pairs, so the
+// bin follows from the high word alone unless it lies within one unit of an
+// edge's or below the group's rounding floor; those pairs are evaluated again
+// with the reference's arithmetic, (x1 - shift) - x2 and dx*dx + dy*dy + dz*dz
+// in FP64, and binned with its "<=".  Every pair therefore lands in the bin
+// the reference puts it in.
+//
+// What bounds it: instruction issue.  The MFMA (65 cycles per 256 pairs; it does
+// not overlap other waves' VALU work here) replaces 8 FP64 instructions of 4.5
+// cycles per 64 pairs, the bin takes 7 instructions and two LDS accesses instead
+// of 12 and two, and sub-groups of 16 evaluate 2.4 pairs per pair in range where
+// groups of 64 evaluated 4.4 (1M clustered points, 20 edges to 50 Mpc/h: 6.3e8
+// instead of 1.18e9 evaluations).  Measured against the kernels of pairs_kernel.h
+// on the whole call: that count 1192 -> 782 us, 20k x 20k 344 -> 228 us, 2M
+// (rp, pi) 2782 -> 2192 us, 150k x 1M projected 1011 -> 528 us, 200k generic
+// marks 935 -> 574 us, per-object rows of 1M 1621 -> 1324 us.
+#pragma once
+
+#include "pairs_kernel.h"
+
+namespace hp {
+
+typedef double dbl4 __attribute__((ext_vector_type(4)));
+
+#ifndef HP_TILE_WPS
+#define HP_TILE_WPS 4
+#endif
+constexpr int kSub = 16;                   // lane points of a sub-group, stream points of a tile
+constexpr int kStage = 192;                // staged stream points per wave: 128 are dealt at a time
+constexpr int kDeal = 128;
+constexpr int kSlots = kStage + 1;         // and one that no pair bins
+constexpr int kIdOff = 4 * kSlots * 8;     // after x, y, z, squared norm: stream index and image of each
+constexpr int kListOff = kIdOff + kStage * 4;            // slots dealt to a sub-group, two tiles of padding
+constexpr int kMarkOff = kListOff + kDeal + 3 * kSub;    // 64: starts of stretches
+constexpr int kInfoOff = (kMarkOff + 64 + 15) / 16 * 16; // the sub-groups' boxes and the group's box
+constexpr int kTileBytes = kInfoOff + 4 * 32 + 32;
+constexpr double kFar = 1.0e300;           // squared norm of a point that no pair bins
+
+struct TileArgs {
+    PairLaunch L;
+    TileSpec tr, tp;
+    int tp_off;      // LDS byte offset of the pi table
+    int w_off;       // byte offset of the staged weights in a wave's LDS area
+    int lw_off;      // ... of the lane points' weights
+    int hist_off;    // ... of its histogram
+    int cnt_off;     // ... of the count rows of a marked pass
+    int wave_bytes;
+    int tab_bytes;
+    int parts_sh;    // log2 of the work items per lane group (cubes dealt round-robin)
+    int tail_sh;     // ... of the groups from `tail` on
+    int64_t tail;
+};
+
+typedef const __attribute__((address_space(4))) TileArgs kernarg_tile_args;  // as the kernel receives them
+
+// DPP moves: row rotations (all 16 lanes of a row), prefix steps over the wave
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_or_zero(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_ror(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+// minimum and maximum over each 16-lane row
+__device__ __forceinline__ float row_min(float v) {
+    v = fminf(v, dpp_ror<0x128>(v));
+    v = fminf(v, dpp_ror<0x124>(v));
+    v = fminf(v, dpp_ror<0x122>(v));
+    return fminf(v, dpp_ror<0x121>(v));
+}
+__device__ __forceinline__ float row_max(float v) {
+    v = fmaxf(v, dpp_ror<0x128>(v));
+    v = fmaxf(v, dpp_ror<0x124>(v));
+    v = fmaxf(v, dpp_ror<0x122>(v));
+    return fmaxf(v, dpp_ror<0x121>(v));
+}
+// of the four rows' values (uniform)
+__device__ __forceinline__ float lane_f(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ __forceinline__ float rows_min(float v) {
+    return fminf(fminf(lane_f(v, 0), lane_f(v, 16)), fminf(lane_f(v, 32), lane_f(v, 48)));
+}
+__device__ __forceinline__ float rows_max(float v) {
+    return fmaxf(fmaxf(lane_f(v, 0), lane_f(v, 16)), fmaxf(lane_f(v, 32), lane_f(v, 48)));
+}
+__device__ __forceinline__ double unid(double v) {
+    return __hiloint2double(uni(__double2hiint(v)), uni(__double2loint(v)));
+}
+// inclusive prefix sum and running maximum over the wave; values >= 0
+__device__ __forceinline__ int wave_prefix(int v) {
+    v += dpp_or_zero<0x111, 0xf>(v);
+    v += dpp_or_zero<0x112, 0xf>(v);
+    v += dpp_or_zero<0x114, 0xf>(v);
+    v += dpp_or_zero<0x118, 0xf>(v);
+    v += dpp_or_zero<0x142, 0xa>(v);
+    v += dpp_or_zero<0x143, 0xc>(v);
+    return v;
+}
+__device__ __forceinline__ int wave_scan_max(int v) {
+    v = max(v, dpp_or_zero<0x111, 0xf>(v));
+    v = max(v, dpp_or_zero<0x112, 0xf>(v));
+    v = max(v, dpp_or_zero<0x114, 0xf>(v));
+    v = max(v, dpp_or_zero<0x118, 0xf>(v));
+    v = max(v, dpp_or_zero<0x142, 0xa>(v));
+    v = max(v, dpp_or_zero<0x143, 0xc>(v));
+    return v;
+}
+// lane I of the lane's row
+template <int I>
+__device__ __forceinline__ double row_bcast(double v) {
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), 0x150 + I, 0xf, 0xf, false),
+                            __builtin_amdgcn_mov_dpp(__double2loint(v), 0x150 + I, 0xf, 0xf, false));
+}
+// clamp to [lo, hi] in one instruction (lo <= hi)
+__device__ __forceinline__ int med3i(int v, int lo, int hi) {
+    int r;
+    asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "v"(lo), "v"(hi));
+    return r;
+}
+// an entry of a bucket table at a byte offset of the workgroup's LDS
+__device__ __forceinline__ uint2 lds_entry(uint32_t off) {
+    typedef __attribute__((address_space(3))) const unsigned long long lds_u64;
+    const unsigned long long v = *(lds_u64*)(uintptr_t)off;
+    return make_uint2((uint32_t)v, (uint32_t)(v >> 32));
+}
+// t = e - c, kout = k + (e < c): one subtraction with borrow, one addition with carry
+__device__ __forceinline__ void sub_borrow(uint32_t e, uint32_t c, uint32_t k, uint32_t& t, uint32_t& kout) {
+    asm("v_sub_co_u32_e32 %0, vcc, %2, %3\n\tv_addc_co_u32_e32 %1, vcc, 0, %4, vcc"
+        : "=&v"(t), "=v"(kout)
+        : "v"(e), "v"(c), "v"(k)
+        : "vcc");
+}
+
+// VAR: product marks compiled in (kModeWSum, kModeWXYZ); the swapped Jacobian
+// pass (kModeJac: lanes are sample 2, the stream is sample 1).  ALSO: plain
+// counts beside the sums.
+template <int MODE, int VAR, int ALSO, int WAVES>
+__global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArgs A) {
+    constexpr bool SWAP = (MODE == kModeJac) && VAR;
+    constexpr bool PROD = (MODE == kModeWSum || MODE == kModeWXYZ) && VAR;
+    constexpr bool XY = (MODE == kModeXYZ || MODE == kModeWXYZ || MODE == kModeProj);
+    constexpr bool F64 = (MODE == kModeWSum || MODE == kModeWXYZ || MODE == kModeJac || MODE == kModeTan);
+    constexpr bool TAN = (MODE == kModeTan);
+    extern __shared__ __align__(16) unsigned char lds[];
+    const PairLaunch& L = A.L;
+    const int lane = threadIdx.x & 63;
+    const int wid = uni(threadIdx.x >> 6);
+    const int K = L.br.nbins, Kp = XY ? L.bp.nbins : 1;
+    const int nw = !F64 ? 0 : (TAN ? 2 : ((MODE == kModeJac || PROD) ? 1 : L.nw));
+    unsigned char* const wsm = lds + A.tab_bytes + wid * A.wave_bytes;
+    // entries of the tables: k becomes the byte offset of the bin's row (column)
+    {
+        const uint2* gt = reinterpret_cast<const uint2*>(static_cast<const char*>(L.ws) + A.tr.off);
+        uint2* st = reinterpret_cast<uint2*>(lds);
+        for (int i = threadIdx.x; i <= (int)A.tr.mask; i += WAVES * 64) st[i] = gt[i];
+        if (XY) {
+            const uint2* gp = reinterpret_cast<const uint2*>(static_cast<const char*>(L.ws) + A.tp.off);
+            uint2* sp = reinterpret_cast<uint2*>(lds + A.tp_off);
+            for (int i = threadIdx.x; i <= (int)A.tp.mask; i += WAVES * 64) sp[i] = gp[i];
+        }
+    }
+    double* const SX = reinterpret_cast<double*>(wsm);  // x[kSlots], y, z, n
+    uint32_t* const ID = reinterpret_cast<uint32_t*>(wsm + kIdOff);
+    uint8_t* const list = wsm + kListOff;
+    uint8_t* const mark = wsm + kMarkOff;
+    float* const info = reinterpret_cast<float*>(wsm + kInfoOff);  // per sub-group: low x, y, z, high x, y, z; the group's
+    double* const SWT = reinterpret_cast<double*>(wsm + A.w_off);   // staged weights: [nw][kSlots]
+    double* const LWT = reinterpret_cast<double*>(wsm + A.lw_off);  // lane points' weights: [nw][64]
+    unsigned char* const hist = wsm + A.hist_off;
+    for (int i = lane; i < (A.wave_bytes - A.hist_off) / 4; i += 64) reinterpret_cast<uint32_t*>(hist)[i] = 0u;
+    __syncthreads();  // no block-level synchronisation below
+
+    // XCD-interleaved block order, as the other count kernels (pairs_kernel.h)
+    int64_t b = blockIdx.x;
+    {
+        constexpr int64_t C = HP_XCD_CHUNK;
+        const int64_t full = ((int64_t)gridDim.x / (8 * C)) * (8 * C);
+        if (b < full) b = ((b >> 3) / C) * (8 * C) + (b & 7) * C + ((b >> 3) % C);
+    }
+    int64_t item = b * WAVES + wid;
+    int psh = A.parts_sh;
+    int64_t g = item >> psh;
+    if (g >= A.tail) {
+        // the last groups go out in smaller items, which even out the end of the launch
+        item -= A.tail << psh;
+        psh = A.tail_sh;
+        g = A.tail + (item >> psh);
+    }
+    const int parts = 1 << psh;
+    const int part = uni((int)(item & (parts - 1)));
+    if (g >= L.ngroups) return;
+
+    constexpr int SD = SWAP ? 1 : 0;  // the lanes' side of the geometry, the stream's
+    constexpr int SS = 1 - SD;
+    const int m = uni(L.group_mock[g]);
+    const MockGeom* const geom = L.geom + m;
+    const int64_t gl = g - geom->group_off[SD];
+    const int64_t p0 = geom->p_off[SD] + gl * kGroup;
+    const int64_t left = geom->n[SD] - gl * kGroup;
+    const int cnt = uni((int)(left < kGroup ? left : kGroup));
+    const bool act = lane < cnt;
+    const float r2xy = geom->r2xy;
+    const float Rz = geom->search[2];
+    const bool sym = L.sym != 0;
+
+    // ---- the group's box, and the lane points relative to its centre
+    float hx, hy, hz;     // half sizes, with the eps margin
+    double cx, cy, cz;
+    double Bf[4], NA[4];  // per sub-group: the tile's B operand and |a|^2
+    uint32_t floor_hi;    // pairs below this high word are evaluated exactly
+    uint32_t floor_pi = 0u;  // ... (rp, pi): below this high word of dz^2
+    {
+        const float INF = __builtin_inff();
+        const float eps = geom->eps;
+        const double4 pr = reinterpret_cast<const double4*>(L.lane.x)[p0 + (act ? lane : 0)];
+        const double px = pr.x, py = pr.y, pz = pr.z;
+        // boxes of the sub-groups, one 16-lane row of the wave each
+        float xl = row_min(act ? f32_down(px) : INF) - eps, xh = row_max(act ? f32_up(px) : -INF) + eps;
+        float yl = row_min(act ? f32_down(py) : INF) - eps, yh = row_max(act ? f32_up(py) : -INF) + eps;
+        float zl = row_min(act ? f32_down(pz) : INF) - eps, zh = row_max(act ? f32_up(pz) : -INF) + eps;
+        const float bxlo = rows_min(xl), bylo = rows_min(yl), bzlo = rows_min(zl);
+        const float bxhi = rows_max(xh), byhi = rows_max(yh), bzhi = rows_max(zh);
+        const float fx = unif(0.5f * (bxlo + bxhi)), fy = unif(0.5f * (bylo + byhi)), fz = unif(0.5f * (bzlo + bzhi));
+        cx = unid((double)fx);
+        cy = unid((double)fy);
+        cz = unid((double)fz);
+        // half sizes of the box about its (rounded) centre; the eps margin covers the rounding
+        hx = unif(0.5f * (bxhi - bxlo));
+        hy = unif(0.5f * (byhi - bylo));
+        hz = unif(0.5f * (bzhi - bzlo));
+        const double ax = px - cx, ay = py - cy, az = pz - cz;
+        const double na = !act ? kFar : (XY ? ax * ax + ay * ay : ax * ax + ay * ay + az * az);
+        if ((lane & 15) == 0) {
+            float* const f = info + (lane >> 4) * 8;
+            f[0] = xl - fx; f[1] = yl - fy; f[2] = zl - fz; f[3] = xh - fx; f[4] = yh - fy; f[5] = zh - fz;
+        }
+        if (lane == 0) {
+            float* const f = info + 32;
+            f[0] = bxlo; f[1] = bylo; f[2] = bzlo; f[3] = bxhi; f[4] = byhi; f[5] = bzhi;
+            // the slot that fills up a tile
+            SX[kStage] = 0.0;
+            SX[kSlots + kStage] = 0.0;
+            SX[2 * kSlots + kStage] = 0.0;
+            SX[3 * kSlots + kStage] = kFar;
+        }
+        if (F64) {
+            const double* w = L.lane.w + (p0 + (act ? lane : 0)) * nw;
+            for (int c = 0; c < nw; c++) LWT[c * 64 + lane] = w[c];
+            if (lane == 0)
+                for (int c = 0; c < nw; c++) SWT[c * kSlots + kStage] = 0.0;
+        }
+        // B operand: lane l holds component l / 16 of point l % 16 of the sub-group
+        SX[lane] = act ? -2.0 * ax : 0.0;
+        SX[kSlots + lane] = act ? -2.0 * ay : 0.0;
+        SX[2 * kSlots + lane] = (act && !XY) ? -2.0 * az : 0.0;
+        SX[3 * kSlots + lane] = na;
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            const double v = SX[min(lane >> 4, 2) * kSlots + s * kSub + (lane & 15)];
+            Bf[s] = (lane >> 4) == 3 ? 1.0 : v;
+            NA[s] = SX[3 * kSlots + s * kSub + (lane & 15)];
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (XY) {
+            // the lane points' z, read by the tiles
+            reinterpret_cast<double*>(wsm + A.lw_off)[nw * 64 + lane] = az;
+        }
+        // Rounding of |a|^2 + |b|^2 - 2 a.b: below 2^-47 (|a|^2 + |b|^2), with
+        // |a| <= h (half the box diagonal) and |b| <= h + R.  One unit of the
+        // high word of d is at least 2^-21 d, so the rounding stays within a
+        // unit for d >= 2^-26 S; the floor takes twice that.  The rounding of
+        // the centre and of the periodic shift (2^-52 of the box) is covered
+        // by the second term (dz^2 has only that one).
+        const float h = sqrtf(hx * hx + hy * hy + (XY ? 0.f : hz * hz)) * 1.001f, hr = h + geom->search[0] * 1.001f;
+        const double Lmax = fmax(fmax(geom->period[0], geom->period[1]), geom->period[2]);
+        const double fl2 = Lmax * Lmax * 3.5527136788005009e-15;                          // 2^-48
+        const double fl = (double)(h * h + hr * hr) * 2.9802322387695312e-08 + fl2;      // 2^-25
+        floor_hi = (uint32_t)uni((int)(__double2hiint(fl) + 1));
+        if (XY) floor_pi = (uint32_t)uni((int)(__double2hiint(fl2) + 1));
+    }
+
+    bool self_done = false;
+    const uint32_t sbase = (uint32_t)uni((int)geom->p_off[SS]);
+    const int tlo = (int)A.tr.lo, thi = (int)A.tr.hi;
+    const uint32_t tsh = A.tr.sh3, tmask = A.tr.mask << 3;
+    const int plo = (int)A.tp.lo, phi = (int)A.tp.hi;
+    const uint32_t psh3 = A.tp.sh3, pmask = A.tp.mask << 3;
+    const int lrow = ((lane & 3) << 2) | ((lane >> 2) & 3);   // list position of this lane's A row
+    const int brow = ((lane >> 4) << 2) | (lane & 3);         // list position of the D row this lane's row broadcasts
+    const double* const comp = SX + (lane >> 4) * kSlots;     // the component this lane holds of the A operand
+    // histogram columns: u32 rows of 32 columns, f64 rows of 16 (no two lanes of
+    // one LDS pass on one address); per lane point for object rows and Jacobians
+    const uint32_t col4 = (uint32_t)(lane & 31) * 4u, col8 = (uint32_t)(lane & 15) * 8u;
+    uint64_t evals = 0;
+
+    // Exact bin of the pair (lane point j of the group, staged slot): the first
+    // edge not below the distance, scanning from edge k (and q along pi).  Rarely
+    // taken: what it needs is loaded here, not kept in registers through the
+    // kernel (the empty asm hides that it is the same).  rev: the pair's other
+    // orientation, (x2 + shift) - x1.
+    auto exact_bin = [&](int j, int slot, bool self, uint32_t k, uint32_t& kp, bool rev) __attribute__((always_inline)) -> uint32_t {
+        kernarg_tile_args* ap = (kernarg_tile_args*)__builtin_amdgcn_kernarg_segment_ptr();
+        const MockGeom* gp = geom;
+        asm volatile("" : "+s"(ap), "+s"(gp));
+        const double* ge = reinterpret_cast<const double*>(static_cast<const char*>(ap->L.ws) + ap->L.br.edges_off);
+        const int64_t first = gp->p_off[SD] + gl * kGroup;
+        const double* pl = ap->L.lane.x + (first + min(j, cnt - 1)) * 4;
+        double px = pl[0], py = pl[1], pz = pl[2];
+        const double* r;
+        int tx = 0, ty = 0, tz = 0;
+        if (self) {
+            r = ap->L.lane.x + (first + min(slot, cnt - 1)) * 4;
+        } else {
+            const uint32_t id = ID[slot];
+            const int img = (int)(id >> 27);
+            r = ap->L.strm.x + (gp->p_off[SS] + (int64_t)(id & 0x7ffffffu)) * 4;
+            tx = img / 9 - 1;
+            ty = (img / 3) % 3 - 1;
+            tz = img % 3 - 1;
+        }
+        double qx = r[0], qy = r[1], qz = r[2];
+        // the image of the stream point lies at q + t L; the reference shifts the sample-1 point
+        if ((!SWAP && !rev) || (SWAP && rev)) {
+            if (tx) px = px - (double)tx * gp->period[0];
+            if (ty) py = py - (double)ty * gp->period[1];
+            if (tz) pz = pz - (double)tz * gp->period[2];
+        } else {
+            if (tx) qx = qx + (double)tx * gp->period[0];
+            if (ty) qy = qy + (double)ty * gp->period[1];
+            if (tz) qz = qz + (double)tz * gp->period[2];
+        }
+        const double dx = px - qx, dy = py - qy, dz = pz - qz;
+        if (XY) {
+            const double* gq = reinterpret_cast<const double*>(static_cast<const char*>(ap->L.ws) + ap->L.bp.edges_off);
+            const double dz2 = dz * dz;
+            uint32_t q = 0;
+            while (gq[q] < dz2) ++q;
+            kp = q;
+            const double dxy = dx * dx + dy * dy;
+            while (ge[k] < dxy) ++k;
+        } else {
+            const double dsq = dx * dx + dy * dy + dz * dz;
+            while (ge[k] < dsq) ++k;
+        }
+        return k;
+    };
+
+    // ---- staged points: deal them to the sub-groups, evaluate the tiles
+    // self: the slots hold the group's own points
+    int qlen = 0;
+    auto process = [&](bool self) __attribute__((always_inline)) {
+        float fx[2], fy[2], fz[2];
+        uint64_t in[2], plain[2];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int slot = h * 64 + lane;
+            in[h] = (uint64_t)__ballot(slot < qlen);
+            fx[h] = (float)SX[slot];
+            fy[h] = (float)SX[kSlots + slot];
+            fz[h] = (float)SX[2 * kSlots + slot];
+            plain[h] = sym ? (uint64_t)__ballot((ID[slot] >> 27) == 13u) & in[h] : 0ull;
+        }
+        // symmetric counts: the shifted points (once), then the unshifted ones
+        // (twice); other counts: every point once
+        const bool two = sym && !self;
+        for (int sc = two ? 0 : 4; sc < 8; sc++) {
+            const int s = sc & 3;
+            uint64_t mk[2];
+#pragma unroll
+            for (int h = 0; h < 2; h++) mk[h] = !two ? in[h] : (sc < 4 ? in[h] & ~plain[h] : plain[h]);
+            if ((mk[0] | mk[1]) == 0) {
+                sc |= 3;  // none of this class
+                continue;
+            }
+            uint32_t inc = (two && sc >= 4) ? 2u : 1u;
+            int n;
+            if (self) {
+                n = min(qlen, (s + 1) * kSub);  // the group's points up to this sub-group
+                list[lane] = (uint8_t)lane;
+            } else {
+                // staged points near the sub-group's box
+                const float4 b0 = *reinterpret_cast<const float4*>(info + 8 * s);
+                const float2 b1 = *reinterpret_cast<const float2*>(info + 8 * s + 4);
+                n = 0;
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const float gx = fmaxf(0.f, fmaxf(fx[h] - b0.w, b0.x - fx[h]));
+                    const float gy = fmaxf(0.f, fmaxf(fy[h] - b1.x, b0.y - fy[h]));
+                    const float gz = fmaxf(0.f, fmaxf(fz[h] - b1.y, b0.z - fz[h]));
+                    const float gxy = __builtin_fmaf(gy, gy, gx * gx);
+                    const bool near = XY ? (gxy <= r2xy && gz <= Rz) : (__builtin_fmaf(gz, gz, gxy) <= r2xy);
+                    const uint64_t mm = (uint64_t)__ballot(near) & mk[h];
+                    const uint32_t r = __builtin_amdgcn_mbcnt_hi((uint32_t)(mm >> 32),
+                                                                 __builtin_amdgcn_mbcnt_lo((uint32_t)mm, (uint32_t)n));
+                    if (__builtin_amdgcn_inverse_ballot_w64(mm)) list[r] = (uint8_t)(h * 64 + lane);
+                    n += __builtin_popcountll(mm);
+                }
+                if (lane < kSub) list[n + lane] = (uint8_t)kStage;
+                evals += (uint64_t)n * kSub;
+            }
+            __builtin_amdgcn_wave_barrier();
+            const double bs = s == 0 ? Bf[0] : (s == 1 ? Bf[1] : (s == 2 ? Bf[2] : Bf[3]));
+            const double ns = s == 0 ? NA[0] : (s == 1 ? NA[1] : (s == 2 ? NA[2] : NA[3]));
+            const dbl4 cc = {ns, ns, ns, ns};
+            // this sub-group's lane points: weights and z
+            const int lj = s * kSub + (lane & 15);
+            double lw[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+            if (F64) {
+#pragma unroll
+                for (int c = 0; c < 5; c++)
+                    if (c < nw) lw[c] = LWT[c * 64 + lj];
+            }
+            if (TAN && sym && !self && sc < 4) {
+                // symmetric sums are doubled at the end: a shifted pair counts from both sides
+                lw[0] *= 0.5;
+                lw[1] *= 0.5;
+            }
+            double za = 0.0;
+            if (XY) za = LWT[nw * 64 + lj];
+            // operands one tile ahead, their slots two
+            double a = comp[list[lrow]];
+            int slot2 = list[kSub + lrow];
+            for (int t0 = 0; t0 < n; t0 += kSub) {
+                // rows: staged points list[t0 + 4 (lane / 16) + i]; columns: the sub-group's points
+                const double a1 = comp[slot2];
+                slot2 = list[t0 + 2 * kSub + lrow];
+                double zb = 0.0, wb[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+                if (XY || F64) {
+                    const int bslot = list[t0 + brow];
+                    if (XY) zb = SX[2 * kSlots + bslot];
+                    if (F64) {
+#pragma unroll
+                        for (int c = 0; c < 5; c++)
+                            if (c < nw) wb[c] = SWT[c * kSlots + bslot];
+                    }
+                }
+                const dbl4 D = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bs, cc, 0, 0, 0);
+                a = a1;
+                int hi[4], hp[4];
+                uint2 ent[4], enp[4];
+                uint32_t t[4], k[4], tp[4], kp[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) hi[i] = __double2hiint(D[i]);
+                bool diag = false;
+                if (self) {
+                    inc = 2u;
+                    diag = t0 == s * kSub;
+                    if (diag) {
+                        // inside a sub-group: ordered pairs, without a point and itself
+                        inc = 1u;
+#pragma unroll
+                        for (int i = 0; i < 4; i++)
+                            if ((lane >> 4) * 4 + i == (lane & 15)) hi[i] = 0x7e000000;
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const uint32_t off = ((uint32_t)med3i(hi[i], tlo, thi) >> tsh) & tmask;
+                    ent[i] = lds_entry(off);
+                }
+                if (XY) {
+                    double dz[4];
+                    dz[0] = row_bcast<0>(zb) - za;
+                    dz[1] = row_bcast<1>(zb) - za;
+                    dz[2] = row_bcast<2>(zb) - za;
+                    dz[3] = row_bcast<3>(zb) - za;
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        hp[i] = __double2hiint(dz[i] * dz[i]);
+                        const uint32_t off = (((uint32_t)med3i(hp[i], plo, phi) >> psh3) & pmask) + (uint32_t)A.tp_off;
+                        enp[i] = lds_entry(off);
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < 4; i++) sub_borrow(ent[i].x, (uint32_t)hi[i], ent[i].y, t[i], k[i]);
+                uint32_t tm = min(min(t[0], t[1]), min(t[2], t[3]));
+                const int hm = min(min(hi[0], hi[1]), min(hi[2], hi[3]));
+                bool odd = tm <= 2u || hm < (int)floor_hi;
+                if (XY) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) sub_borrow(enp[i].x, (uint32_t)hp[i], enp[i].y, tp[i], kp[i]);
+                    const uint32_t pm = min(min(tp[0], tp[1]), min(tp[2], tp[3]));
+                    const int qm = min(min(hp[0], hp[1]), min(hp[2], hp[3]));
+                    odd = odd || pm <= 2u || qm < (int)floor_pi;
+                }
+                if (__builtin_expect((uint64_t)__ballot(odd) != 0, 0)) {
+#pragma unroll 1
+                    for (int i = 0; i < 4; i++) {
+                        const uint32_t ti = i == 0 ? t[0] : (i == 1 ? t[1] : (i == 2 ? t[2] : t[3]));
+                        const int hv = i == 0 ? hi[0] : (i == 1 ? hi[1] : (i == 2 ? hi[2] : hi[3]));
+                        const uint32_t ek = i == 0 ? ent[0].y : (i == 1 ? ent[1].y : (i == 2 ? ent[2].y : ent[3].y));
+                        bool oi = ti <= 2u || hv < (int)floor_hi;
+                        if (XY) {
+                            const uint32_t pi = i == 0 ? tp[0] : (i == 1 ? tp[1] : (i == 2 ? tp[2] : tp[3]));
+                            const int hq = i == 0 ? hp[0] : (i == 1 ? hp[1] : (i == 2 ? hp[2] : hp[3]));
+                            oi = (oi || pi <= 2u || hq < (int)floor_pi) && hv < 0x7e000000;
+                        }
+                        if (oi) {
+                            const int slot = list[t0 + (lane >> 4) * 4 + i];
+                            const uint32_t kb = hv < (int)floor_hi || ek == 0u ? 0u : ek - 1u;
+                            uint32_t kq = 0u;
+                            uint32_t kk = exact_bin(s * kSub + (lane & 15), slot, self, kb, kq, false);
+                            if (MODE == kModeJac && !SWAP && L.corr != nullptr) {
+                                // Auto-count with one set of weights: the sample-2 rows take
+                                // the pair's other orientation, which across the periodic seam
+                                // may round into another bin; those disagreements are recorded,
+                                // so rows2 = rows1 + corr (as pairs_kernel.h does for every
+                                // shifted pair; only these can differ).
+                                const uint32_t id = ID[slot];
+                                uint32_t dummy = 0u;
+                                const uint32_t kr = exact_bin(s * kSub + (lane & 15), slot, self, kb, dummy, true);
+                                if (kr != kk && (id >> 27) != 13u && s * kSub + (lane & 15) < cnt) {
+                                    const int64_t sr = (int64_t)sbase + (int64_t)(id & 0x7ffffffu);
+                                    const int64_t q = __double_as_longlong(L.strm.x[sr * 4 + 3]);
+                                    double* crow = L.corr + q * K;
+                                    if (kk < (uint32_t)K)
+                                        __hip_atomic_fetch_add(crow + kk, lw[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                                    if (kr < (uint32_t)K)
+                                        __hip_atomic_fetch_add(crow + kr, -lw[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                                }
+                            }
+#pragma unroll
+                            for (int u = 0; u < 4; u++)
+                                if (i == u) {
+                                    k[u] = kk;
+                                    if (XY) kp[u] = kq;
+                                }
+                        }
+                    }
+                }
+                // ---- accumulate
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    // the row's stream weights (all lanes: a broadcast reads none that is masked off)
+                    double sw[5];
+                    if constexpr (F64) {
+#pragma unroll
+                        for (int c = 0; c < 5; c++)
+                            sw[c] = c >= nw ? 0.0
+                                            : (i == 0 ? row_bcast<0>(wb[c])
+                                                      : (i == 1 ? row_bcast<1>(wb[c])
+                                                                : (i == 2 ? row_bcast<2>(wb[c]) : row_bcast<3>(wb[c]))));
+                    }
+                    if constexpr (MODE == kModeCount3D) {
+                        __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hist + ((k[i] << 7) + col4)), inc,
+                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    } else if constexpr (MODE == kModeProj) {
+                        // beyond pi_max: the trash row
+                        const uint32_t kk = kp[i] == 0u ? k[i] : (uint32_t)K;
+                        __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hist + ((kk << 7) + col4)), inc,
+                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    } else if constexpr (MODE == kModeXYZ || MODE == kModeWXYZ) {
+                        // one [K][Kp] histogram per wave; pairs beyond an edge skip it
+                        if (k[i] < (uint32_t)K && kp[i] < (uint32_t)Kp) {
+                            const uint32_t cell = k[i] * (uint32_t)Kp + kp[i];
+                            if constexpr (MODE == kModeXYZ) {
+                                __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hist) + cell, inc, __ATOMIC_RELAXED,
+                                                       __HIP_MEMORY_SCOPE_WORKGROUP);
+                            } else {
+                                const double v = PROD ? lw[0] * sw[0] : wfunc_eval(L.wfunc, lw, sw);
+                                __hip_atomic_fetch_add(reinterpret_cast<double*>(hist) + cell, v, __ATOMIC_RELAXED,
+                                                       __HIP_MEMORY_SCOPE_WORKGROUP);
+                            }
+                        }
+                    } else if constexpr (MODE == kModeObj) {
+                        __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hist + ((k[i] << 8) + (uint32_t)lj * 4u)), 1u,
+                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    } else {
+                        if constexpr (MODE == kModeJac) {
+                            __hip_atomic_fetch_add(reinterpret_cast<double*>(hist + ((k[i] << 9) + (uint32_t)lj * 8u)),
+                                                   sw[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        } else if constexpr (MODE == kModeTan) {
+                            // pair terms w_i w_j and t_i w_j + w_i t_j (t = dw/dtheta); the
+                            // group's own pairs: ordered ones inside a sub-group count half
+                            if (k[i] < (uint32_t)K) {
+                                double wj = sw[0], tj = sw[1];
+                                if (diag) {
+                                    wj *= 0.5;
+                                    tj *= 0.5;
+                                }
+                                const double v = lw[0] * wj;
+                                const double tv = __builtin_fma(lw[0], tj, lw[1] * wj);
+                                unsigned char* const r = hist + k[i] * (ALSO ? 384u : 256u);
+                                __hip_atomic_fetch_add(reinterpret_cast<double*>(r + col8), v, __ATOMIC_RELAXED,
+                                                       __HIP_MEMORY_SCOPE_WORKGROUP);
+                                __hip_atomic_fetch_add(reinterpret_cast<double*>(r + 128 + col8), tv, __ATOMIC_RELAXED,
+                                                       __HIP_MEMORY_SCOPE_WORKGROUP);
+                                if (ALSO)
+                                    __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(r + 256 + col4), inc,
+                                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                            }
+                        } else if constexpr (MODE == kModeWSum) {
+                            const double v = PROD ? lw[0] * sw[0] : wfunc_eval(L.wfunc, lw, sw);
+                            __hip_atomic_fetch_add(reinterpret_cast<double*>(hist + ((k[i] << 7) + col8)), v,
+                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        }
+                        if constexpr (ALSO && MODE != kModeTan)
+                            __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(wsm + A.cnt_off + ((k[i] << 7) + col4)), 1u,
+                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    }
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+        // what was not dealt moves to the front
+        const int rest = self ? 0 : max(qlen - kDeal, 0);
+        if (rest > 0 && lane < rest) {
+            const int f = kDeal + lane;
+            const double x = SX[f], y = SX[kSlots + f], z = SX[2 * kSlots + f], nn = SX[3 * kSlots + f];
+            const uint32_t id = ID[f];
+            SX[lane] = x;
+            SX[kSlots + lane] = y;
+            SX[2 * kSlots + lane] = z;
+            SX[3 * kSlots + lane] = nn;
+            ID[lane] = id;
+            if (F64)
+                for (int c = 0; c < nw; c++) SWT[c * kSlots + lane] = SWT[c * kSlots + f];
+        }
+        __builtin_amdgcn_wave_barrier();
+        qlen = rest;
+    };
+
+    // ---- the cubes of the curve near the group.  A lane takes one cube of the
+    // window and looks up the stretch of rows it holds; the stretches of 64 cubes
+    // form one list of rows, which is walked 64 rows at a time: a scan over the
+    // starts gives each lane its stretch.  Symmetric counts drop the rows before
+    // the group's end here (unshifted cubes), a whole stretch at a time.
+    const double4* const SR = reinterpret_cast<const double4*>(L.strm.x) + sbase;
+    int cube0 = -64;                // the next 64 cubes of the window
+    int cimg = 0;                   // the lane's cube: its image
+    bool seam = false;              // some cube of the list is a periodic image
+    int pre = 0, end = 0, run = 0;  // the lane's stretch: its place [pre, end) in the list, first row - pre
+    int at = 0, total = 0;          // list position of the next rows, rows in the list
+    // the next 64 rows: false when the group has no more.  The list is made
+    // rarely: what that needs is loaded here.
+    auto next = [&]() __attribute__((always_inline)) -> bool {
+        at += 64;
+        while (at >= total) {
+            const MockGeom* gp = geom;
+            asm volatile("" : "+s"(gp));
+            const int nc = gp->ndiv[0];  // cubes per dimension
+            const int pbc = gp->pbc;
+            const float Rx = gp->search[0];
+            const float cxf = (float)gp->cell[0], cyf = (float)gp->cell[1], czf = (float)gp->cell[2];
+            const float bxlo = unif(info[32]), bylo = unif(info[33]), bzlo = unif(info[34]);
+            const float bxhi = unif(info[35]), byhi = unif(info[36]), bzhi = unif(info[37]);
+            const int j0 = pbc ? -nc : 0, j1 = pbc ? 2 * nc - 1 : nc - 1;
+            const int jx0 = uni(max((int)floorf((bxlo - Rx) / cxf), j0)), jx1 = uni(min((int)floorf((bxhi + Rx) / cxf), j1));
+            const int jy0 = uni(max((int)floorf((bylo - Rx) / cyf), j0)), jy1 = uni(min((int)floorf((byhi + Rx) / cyf), j1));
+            const int jz0 = uni(max((int)floorf((bzlo - Rz) / czf), j0)), jz1 = uni(min((int)floorf((bzhi + Rz) / czf), j1));
+            const int wy = jy1 - jy0 + 1, wz = jz1 - jz0 + 1;
+            const int ncubes = (jx1 >= jx0 && wy > 0 && wz > 0) ? (jx1 - jx0 + 1) * wy * wz : 0;
+            cube0 += 64;
+            if ((cube0 << psh) + part >= ncubes) return false;
+            const int ci = ((cube0 + lane) << psh) + part;
+            const int cxy = ci / wz;
+            const int jx = jx0 + cxy / wy, jy = jy0 + cxy % wy, jz = jz0 + ci % wz;
+            const float gx = fmaxf(0.f, fmaxf((float)jx * cxf - bxhi, bxlo - (float)(jx + 1) * cxf));
+            const float gy = fmaxf(0.f, fmaxf((float)jy * cyf - byhi, bylo - (float)(jy + 1) * cyf));
+            const float gz = fmaxf(0.f, fmaxf((float)jz * czf - bzhi, bzlo - (float)(jz + 1) * czf));
+            at = 0;
+            total = 0;
+            const bool has = ci < ncubes && (XY ? gx * gx + gy * gy : gx * gx + gy * gy + gz * gz) <= r2xy;
+            if ((uint64_t)__ballot(has) == 0) continue;
+            const int tx = jx < 0 ? -1 : (jx >= nc ? 1 : 0), ty = jy < 0 ? -1 : (jy >= nc ? 1 : 0),
+                      tz = jz < 0 ? -1 : (jz >= nc ? 1 : 0);
+            cimg = (tx + 1) * 9 + (ty + 1) * 3 + (tz + 1);
+            int len = 0;
+            run = 0;
+            if (has) {
+                const uint2 c = L.strm.cubes[gp->cell_off + ((int64_t)(jx - tx * nc) * nc + (jy - ty * nc)) * nc +
+                                             (jz - tz * nc)];
+                run = (int)c.x;
+                if (sym && cimg == 13) run = max(run, (int)(gp->p_off[SD] + gl * kGroup + cnt));
+                len = max((int)c.y - run, 0);
+            }
+            seam = (uint64_t)__ballot(len > 0 && cimg != 13) != 0;
+            pre = wave_prefix(len);
+            total = __builtin_amdgcn_readlane(pre, 63);
+            end = len > 0 ? pre : -1;
+            pre -= len;
+            run -= pre + (int)sbase;
+        }
+        return true;
+    };
+    // this lane's row of the list (relative to the mock's first) and its image;
+    // a row past the end repeats the last one
+    auto fetch = [&](uint32_t& jj, int& img) __attribute__((always_inline)) {
+        mark[lane] = 0;
+        __builtin_amdgcn_wave_barrier();
+        if (pre < at + 64 && end > at) mark[max(pre - at, 0)] = (uint8_t)lane;
+        __builtin_amdgcn_wave_barrier();
+        const int sg = wave_scan_max((int)mark[lane]) << 2;
+        jj = (uint32_t)(min(at + lane, total - 1) + __builtin_amdgcn_ds_bpermute(sg, run));
+        img = seam ? __builtin_amdgcn_ds_bpermute(sg, cimg) : 13;
+    };
+    bool more = next();
+    double4 row = make_double4(0.0, 0.0, 0.0, 0.0);
+    uint32_t jn = 0;
+    int imgn = 13, nn = 0;  // the rows being loaded: indices, images, how many
+    bool seamn = false;
+    if (more) {
+        fetch(jn, imgn);
+        nn = total - at;
+        seamn = seam;
+        row = SR[jn];
+    }
+    for (;;) {
+        bool self = false;
+        if (more) {
+            const double4 sr = row;
+            const uint32_t jj = jn;
+            const int img = imgn, nrow = nn;
+            double x = sr.x - cx, y = sr.y - cy, z = sr.z - cz;
+            if (seamn) {
+                const MockGeom* gp = geom;
+                asm volatile("" : "+s"(gp));
+                const int tx = img / 9 - 1, ty = (img / 3) % 3 - 1, tz = img % 3 - 1;
+                x = sr.x - (cx - (double)tx * gp->period[0]);
+                y = sr.y - (cy - (double)ty * gp->period[1]);
+                z = sr.z - (cz - (double)tz * gp->period[2]);
+            }
+            more = next();
+            if (more) {
+                fetch(jn, imgn);
+                nn = total - at;
+                seamn = seam;
+                row = SR[jn];
+            }
+            const float gx = fmaxf(0.f, fabsf((float)x) - hx);
+            const float gy = fmaxf(0.f, fabsf((float)y) - hy);
+            const float gz = fmaxf(0.f, fabsf((float)z) - hz);
+            const float gxy = __builtin_fmaf(gy, gy, gx * gx);
+            const bool ok = lane < nrow && (XY ? (gxy <= r2xy && gz <= Rz) : (__builtin_fmaf(gz, gz, gxy) <= r2xy));
+            const uint64_t mk = (uint64_t)__ballot(ok);
+            if (ok) {
+                const uint32_t slot = __builtin_amdgcn_mbcnt_hi(
+                    (uint32_t)(mk >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mk, (uint32_t)qlen));
+                SX[slot] = x;
+                SX[kSlots + slot] = y;
+                SX[2 * kSlots + slot] = z;
+                SX[3 * kSlots + slot] = XY ? x * x + y * y : x * x + y * y + z * z;
+                ID[slot] = jj | ((uint32_t)img << 27);
+                if (F64) {
+                    const double* w = L.strm.w + ((int64_t)sbase + jj) * nw;
+                    for (int c = 0; c < nw; c++) SWT[c * kSlots + slot] = w[c];
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+            qlen += __builtin_popcountll(mk);
+        } else if (qlen == 0) {
+            if (!sym || part != 0 || self_done) break;
+            // symmetric counts, last: the group's own points.  Each unordered
+            // pair of different sub-groups counts twice, the ordered pairs inside
+            // a sub-group once, each point with itself (distance 0: bin 0) once.
+            const double4 pr = reinterpret_cast<const double4*>(L.lane.x)[p0 + (act ? lane : 0)];
+            const double ax = pr.x - cx, ay = pr.y - cy, az = pr.z - cz;
+            SX[lane] = act ? ax : 0.0;
+            SX[kSlots + lane] = act ? ay : 0.0;
+            SX[2 * kSlots + lane] = act ? az : 0.0;
+            SX[3 * kSlots + lane] = !act ? kFar : (XY ? ax * ax + ay * ay : ax * ax + ay * ay + az * az);
+            if (F64)
+                for (int c = 0; c < nw; c++) SWT[c * kSlots + lane] = LWT[c * 64 + lane];
+            evals += (uint64_t)cnt * cnt;
+            if constexpr (MODE == kModeTan) {
+                if (act) {
+                    const double w = LWT[lane], t = LWT[64 + lane];
+                    __hip_atomic_fetch_add(reinterpret_cast<double*>(hist + col8), 0.5 * (w * w), __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_WORKGROUP);
+                    __hip_atomic_fetch_add(reinterpret_cast<double*>(hist + 128 + col8), w * t, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_WORKGROUP);
+                }
+                if (ALSO && lane == 0) *reinterpret_cast<uint32_t*>(hist + 256) += (uint32_t)cnt;
+            } else {
+                if (lane == 0) *reinterpret_cast<uint32_t*>(hist) += (uint32_t)cnt;
+            }
+            __builtin_amdgcn_wave_barrier();
+            qlen = cnt;
+            self = true;
+            self_done = true;
+        }
+        if (qlen >= kDeal || !more) process(self);
+    }
+    __builtin_amdgcn_wave_barrier();
+
+    // ---- the group's results
+    // columns are summed starting at a lane's own one (a bank per lane), counts
+    // go to the mock's accumulators
+    uint64_t* const cacc =
+        L.pcount ? L.pcount + ((int64_t)m * L.crep + (int64_t)(gl % L.crep)) * ((MODE == kModeXYZ) ? K * Kp : K) : nullptr;
+    if constexpr (MODE == kModeXYZ) {
+        const uint32_t* h = reinterpret_cast<const uint32_t*>(hist);
+        for (int k = lane; k < K * Kp; k += 64)
+            if (h[k]) __hip_atomic_fetch_add(cacc + k, (uint64_t)h[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else if constexpr (MODE == kModeCount3D || MODE == kModeProj || ALSO) {
+        const uint32_t* h = reinterpret_cast<const uint32_t*>(wsm + A.cnt_off);
+        const int step = TAN ? 96 : 32;
+        for (int k = lane; k < K; k += 64) {
+            uint64_t tot = 0;
+            for (int c = 0; c < 32; c++) tot += h[k * step + ((c + lane) & 31)];
+            if (tot) __hip_atomic_fetch_add(cacc + k, tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    if constexpr (MODE == kModeWXYZ) {
+        const double* h = reinterpret_cast<const double*>(hist);
+        double* dst = L.psum + ((g << psh) + part) * (int64_t)K * Kp;
+        for (int k = lane; k < K * Kp; k += 64) dst[k] = h[k];
+    }
+    if constexpr (MODE == kModeWSum || MODE == kModeTan) {
+        const double* h = reinterpret_cast<const double*>(hist);
+        const int step = TAN ? (ALSO ? 48 : 32) : 16;
+        const double sc = (TAN && sym) ? 2.0 : 1.0;
+        for (int k = lane; k < K; k += 64) {
+            double v = 0.0, tv = 0.0;
+            for (int c = 0; c < 16; c++) {
+                v += h[k * step + ((c + lane) & 15)];
+                if (TAN) tv += h[k * step + 16 + ((c + lane) & 15)];
+            }
+            const int64_t at_ = ((g << psh) + part) * K + k;
+            if (L.psum) L.psum[at_] = sc * v;
+            if (TAN) L.ptan[at_] = sc * tv;
+        }
+    }
+    if constexpr (MODE == kModeObj || MODE == kModeJac) {
+        if (act) {
+            // the lane point's row at its input position
+            const int64_t q = __double_as_longlong(L.lane.x[(p0 + lane) * 4 + 3]);
+            if constexpr (MODE == kModeObj) {
+                int64_t* r = L.orows + q * K;
+                int64_t sum = 0;
+                for (int k = 0; k < K; k++) {
+                    sum += (int64_t)reinterpret_cast<const uint32_t*>(hist)[k * 64 + lane];
+                    r[k] = sum;
+                }
+            } else if (L.rows) {
+                double* r = L.rows + q * K;
+                for (int k = 0; k < K; k++) r[k] = reinterpret_cast<const double*>(hist)[k * 64 + lane];
+            }
+        }
+        if constexpr (MODE == kModeJac && !SWAP) {
+            if (L.psum) {
+                const double w = act ? LWT[lane] : 0.0;
+                for (int k = 0; k < K; k++) {
+                    const double tot = wave_sum_f64(act ? w * reinterpret_cast<const double*>(hist)[k * 64 + lane] : 0.0);
+                    if (lane == 0) L.psum[g * K + k] = tot;
+                }
+            }
+        }
+    }
+    if (L.pevals && lane == 0)
+        __hip_atomic_fetch_add(reinterpret_cast<unsigned long long*>(L.pevals + g), (unsigned long long)evals,
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+template <int MODE, int VAR, int ALSO, int WAVES>
+static int launch_tiles_w(const TileArgs& A, int64_t items, int smem, hipStream_t s) {
+    hipLaunchKernelGGL((k_tiles<MODE, VAR, ALSO, WAVES>), dim3((unsigned)((items + WAVES - 1) / WAVES)),
+                       dim3(WAVES * 64), (size_t)smem, s, A);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+template <int MODE, int VAR, int ALSO>
+static int launch_tiles_v(const TileArgs& A, int waves, int64_t items, int smem, hipStream_t s) {
+    if (items <= 0) return 0;
+    if (waves == 8) return launch_tiles_w<MODE, VAR, ALSO, 8>(A, items, smem, s);
+    if (waves == 4) return launch_tiles_w<MODE, VAR, ALSO, 4>(A, items, smem, s);
+    if (waves == 2) return launch_tiles_w<MODE, VAR, ALSO, 2>(A, items, smem, s);
+    return launch_tiles_w<MODE, VAR, ALSO, 1>(A, items, smem, s);
+}
+
+// One launch of mode MODE; each mode is instantiated in its own translation
+// unit (pairs_tile_*.hip).
+template <int MODE>
+int launch_tiles_mode(const TileArgs& A, int waves, int64_t items, int smem, int also, int var, hipStream_t s) {
+    if constexpr (MODE == kModeWSum || MODE == kModeJac) {
+        if (var)
+            return also ? launch_tiles_v<MODE, 1, 1>(A, waves, items, smem, s)
+                        : launch_tiles_v<MODE, 1, 0>(A, waves, items, smem, s);
+        return also ? launch_tiles_v<MODE, 0, 1>(A, waves, items, smem, s)
+                    : launch_tiles_v<MODE, 0, 0>(A, waves, items, smem, s);
+    } else if constexpr (MODE == kModeWXYZ) {
+        return var ? launch_tiles_v<MODE, 1, 0>(A, waves, items, smem, s)
+                   : launch_tiles_v<MODE, 0, 0>(A, waves, items, smem, s);
+    } else if constexpr (MODE == kModeTan) {
+        return also ? launch_tiles_v<MODE, 0, 1>(A, waves, items, smem, s)
+                    : launch_tiles_v<MODE, 0, 0>(A, waves, items, smem, s);
+    } else {
+        return launch_tiles_v<MODE, 0, 0>(A, waves, items, smem, s);
+    }
+}
+
+}  // namespace hp

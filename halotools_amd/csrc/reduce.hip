@@ -16,10 +16,11 @@ constexpr int kChunk = 512;  // groups per stage-1 block
 
 template <typename T>
 __global__ void __launch_bounds__(256) k_reduce_s1(const T* __restrict__ partial, int nb, const MockGeom* __restrict__ geom,
-                                                   int side, int nchunk_max, T* __restrict__ s1) {
+                                                   int side, int nchunk_max, T* __restrict__ s1, int psh) {
     __shared__ T sh[256];
     const int m = blockIdx.y, c = blockIdx.x;
-    const int64_t go = geom[m].group_off[side], ng = geom[m].ngroups[side];
+    // 2^psh partial rows per lane group
+    const int64_t go = geom[m].group_off[side] << psh, ng = geom[m].ngroups[side] << psh;
     const int64_t r0 = (int64_t)c * kChunk;
     const int64_t r1 = r0 + kChunk < ng ? r0 + kChunk : ng;
     T* out = s1 + ((int64_t)m * nchunk_max + c) * nb;
@@ -48,10 +49,10 @@ __global__ void __launch_bounds__(256) k_reduce_s1(const T* __restrict__ partial
 // dims: nr (and np for the 2-D xy_z histogram; np = 0 means 1-D).
 template <typename T, typename TO>
 __global__ void __launch_bounds__(256) k_reduce_s2(const T* __restrict__ s1, int nr, int np, const MockGeom* __restrict__ geom,
-                                                   int side, int nchunk_max, TO* __restrict__ out) {
+                                                   int side, int nchunk_max, TO* __restrict__ out, int psh) {
     const int m = blockIdx.x;
     const int nb = np > 0 ? nr * np : nr;
-    const int64_t ng = geom[m].ngroups[side];
+    const int64_t ng = geom[m].ngroups[side] << psh;
     const int nchunks = (int)((ng + kChunk - 1) / kChunk);
     TO* o = out + (int64_t)m * nb;
     for (int b = threadIdx.x; b < nb; b += blockDim.x) {
@@ -161,10 +162,10 @@ static int64_t nchunk_w(int64_t max_groups) { return (max_groups + kChunkW - 1) 
 
 __global__ void __launch_bounds__(256) k_reduce_w1(const double* __restrict__ partial, int nb,
                                                    const MockGeom* __restrict__ geom, int side, int nchunk_max,
-                                                   double* __restrict__ s1) {
+                                                   double* __restrict__ s1, int psh) {
     const int m = blockIdx.y, c = blockIdx.x;
     const int b = blockIdx.z * 256 + threadIdx.x;
-    const int64_t go = geom[m].group_off[side], ng = geom[m].ngroups[side];
+    const int64_t go = geom[m].group_off[side] << psh, ng = geom[m].ngroups[side] << psh;
     const int64_t r0 = (int64_t)c * kChunkW;
     if (b >= nb || r0 >= ng) return;
     const int64_t r1 = r0 + kChunkW < ng ? r0 + kChunkW : ng;
@@ -175,12 +176,12 @@ __global__ void __launch_bounds__(256) k_reduce_w1(const double* __restrict__ pa
 
 __global__ void __launch_bounds__(256) k_reduce_w2(const double* __restrict__ s1, int nb,
                                                    const MockGeom* __restrict__ geom, int side, int nchunk_max,
-                                                   double* __restrict__ out) {
+                                                   double* __restrict__ out, int psh) {
     __shared__ double sh[4][64];
     const int m = blockIdx.y;
     const int bl = threadIdx.x & 63, stripe = threadIdx.x >> 6;
     const int b = blockIdx.x * 64 + bl;
-    const int64_t ng = geom[m].ngroups[side];
+    const int64_t ng = geom[m].ngroups[side] << psh;
     const int nchunks = (int)((ng + kChunkW - 1) / kChunkW);
     double acc = 0.0;
     if (b < nb)
@@ -211,30 +212,32 @@ int64_t reduce_scratch_elems(int64_t max_groups_per_mock, int nmocks, int nb) {
     return nc * nmocks * (int64_t)nb;
 }
 
-// FP64 partial histograms [groups][nr] (2-D: [groups][nr * np]) -> cumulative sums per mock
+// FP64 partial histograms [groups << parts_sh][nr] (2-D: [...][nr * np]) -> cumulative sums per mock
 int launch_reduce_sums_s(const double* partial, int nr, int np, const MockGeom* geom, int nmocks, int side,
-                         int64_t max_groups, double* scratch, double* sums, hipStream_t s) {
+                         int64_t max_groups, int parts_sh, double* scratch, double* sums, hipStream_t s) {
     const int nb = np > 0 ? nr * np : nr;
+    max_groups <<= parts_sh;
     if (np > 0 && nb > kWideCells) {
         const int nc = (int)(nchunk_w(max_groups) > 0 ? nchunk_w(max_groups) : 1);
         hipLaunchKernelGGL(k_reduce_w1, dim3(nc, nmocks, (nb + 255) / 256), dim3(256), 0, s, partial, nb, geom, side,
-                           nc, scratch);
+                           nc, scratch, parts_sh);
         hipLaunchKernelGGL(k_reduce_w2, dim3((nb + 63) / 64, nmocks), dim3(256), 0, s, scratch, nb, geom, side, nc,
-                           sums);
+                           sums, parts_sh);
         hipLaunchKernelGGL(k_prefix_2d, dim3(nmocks), dim3(256), 0, s, sums, nr, np);
         return hipGetLastError() == hipSuccess ? 0 : -1;
     }
     const int nc = (int)(nchunk_of(max_groups) > 0 ? nchunk_of(max_groups) : 1);
-    hipLaunchKernelGGL(k_reduce_s1<double>, dim3(nc, nmocks), dim3(256), 0, s, partial, nb, geom, side, nc, scratch);
+    hipLaunchKernelGGL(k_reduce_s1<double>, dim3(nc, nmocks), dim3(256), 0, s, partial, nb, geom, side, nc, scratch, parts_sh);
     hipLaunchKernelGGL((k_reduce_s2<double, double>), dim3(nmocks), dim3(256), 0, s, scratch, nr, np, geom, side, nc,
-                       sums);
+                       sums, parts_sh);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int launch_reduce_evals_s(const uint64_t* pevals, const MockGeom* geom, int nmocks, int side, int64_t max_groups,
                           uint64_t* scratch, int64_t* evals, hipStream_t s) {
     const int nc = (int)(nchunk_of(max_groups) > 0 ? nchunk_of(max_groups) : 1);
-    hipLaunchKernelGGL(k_reduce_s1<uint64_t>, dim3(nc, nmocks), dim3(256), 0, s, pevals, 1, geom, side, nc, scratch);
+    hipLaunchKernelGGL(k_reduce_s1<uint64_t>, dim3(nc, nmocks), dim3(256), 0, s, pevals, 1, geom, side, nc, scratch,
+                       0);
     hipLaunchKernelGGL(k_reduce_plain, dim3(nmocks), dim3(64), 0, s, scratch, geom, side, nc, evals);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }

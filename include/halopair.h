@@ -231,6 +231,10 @@ int hp_segment_sum(const double* values, const int64_t* offsets, int32_t nmocks,
 /* The kernels' bucketed bin lookup: out[i] = number of suffix-minimum edges of r2 below d[i];
  * info = {shift, base, table entries, multi}. */
 int hp_debug_bin_lookup(const double* r2, int32_t K, const double* d, int64_t n, int32_t* out, int32_t* info);
+/* The matrix-core pair kernels' lookup when the high word of d[i] is off by `off` units: out[i] = the bin,
+ * or -1 where the kernels evaluate the pair exactly; info = {1 if the edges fit such a table, shift, entries}. */
+int hp_debug_tile_lookup(const double* r2, int32_t K, const double* d, int64_t n, int32_t off, int32_t* out,
+                         int32_t* info);
 /* Hilbert index of cell (x, y, z) on a 2^bits grid: the lane-group order of the pair kernels. */
 uint32_t hp_debug_hilbert(uint32_t x, uint32_t y, uint32_t z, int32_t bits);
 

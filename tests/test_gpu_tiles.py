@@ -1,0 +1,123 @@
+"""Matrix-core pair kernels at the sizes where they can go wrong: sub-groups of
+16, groups of 64, dealt parts of 128, split groups, pairs at and next to bin
+edges, coincident points, periodic images; against the oracle (counts bit-exact,
+sums to 1e-12, the bound of the other kernels: FP64 sums of up to ~1e6 positive
+terms in another order) and against the general kernels."""
+import numpy as np
+import pytest
+
+from oracle import mesh as ORC
+
+pytestmark = pytest.mark.gpu
+
+L = 100.0
+RB = np.logspace(-1, np.log10(20.0), 12)
+PI = np.array([0.0, 2.0, 7.5, 20.0])
+
+
+@pytest.fixture(scope="module")
+def mo(gpu):
+    import halotools_amd.mock_observables as mo
+    return mo
+
+
+def _points(n, kind, seed):
+    rng = np.random.default_rng([7, n, seed])
+    p = rng.uniform(0, L, (n, 3))
+    if kind == "clumps":   # pairs far below the first edge, and exact duplicates
+        p = np.mod(p[rng.integers(0, max(1, n // 6), n)] + rng.normal(size=(n, 3)) * 0.01, L)
+        p[n // 2:n // 2 + n // 10] = p[:n // 10]
+    elif kind == "lattice":  # separations exactly on and next to edges
+        p = rng.integers(0, 40, (n, 3)) * 2.5
+    elif kind == "seam":   # everything next to the box faces and corners
+        p = np.mod(rng.normal(size=(n, 3)) * 3.0, L)
+    elif kind == "slab":   # wide, flat groups
+        p[:, 2] = rng.uniform(0, 0.01, n)
+    return p
+
+
+CASES = [(n, 0, k) for n in (1, 2, 15, 16, 17, 63, 64, 65, 128, 129, 200, 1000) for k in ("uniform", "clumps")] + \
+        [(3000, 0, k) for k in ("uniform", "clumps", "lattice", "seam", "slab")] + \
+        [(1, 64, "uniform"), (17, 1, "seam"), (65, 2000, "uniform"), (2000, 65, "clumps"), (1500, 1500, "lattice"),
+         (20000, 9000, "uniform")]
+
+
+@pytest.mark.parametrize("period", [L, None], ids=["box", "open"])
+@pytest.mark.parametrize("n1,n2,kind", CASES)
+def test_counts(mo, n1, n2, kind, period):
+    p1 = _points(n1, kind, 0)
+    p2 = p1 if n2 == 0 else _points(n2, kind, 1)
+    rb = np.array([2.5, 5.0, 7.5, 10.0, 12.5]) if kind == "lattice" else RB
+    kw = dict(period=period)
+    got = mo.npairs_3d(p1, p2, rb, **kw)
+    assert np.array_equal(got, ORC.npairs_3d(p1, p2, rb, **kw))
+    assert np.array_equal(mo.npairs_xy_z(p1, p2, rb, PI, **kw), ORC.npairs_xy_z(p1, p2, rb, PI, **kw))
+    assert np.array_equal(mo.npairs_projected(p1, p2, rb, 7.5, **kw), ORC.npairs_projected(p1, p2, rb, 7.5, **kw))
+    assert np.array_equal(mo.npairs_per_object_3d(p1, p2, rb, **kw), ORC.npairs_per_object_3d(p1, p2, rb, **kw))
+
+
+@pytest.mark.parametrize("wfunc,nw", [(1, 1), (2, 1), (5, 2), (9, 2), (12, 4), (17, 5)])
+@pytest.mark.parametrize("n1,n2,kind", [(65, 0, "clumps"), (129, 40, "uniform"), (1000, 0, "seam"),
+                                        (1500, 700, "lattice")])
+def test_sums(mo, n1, n2, kind, wfunc, nw):
+    p1 = _points(n1, kind, 0)
+    p2 = p1 if n2 == 0 else _points(n2, kind, 1)
+    rb = np.array([2.5, 5.0, 7.5, 10.0, 12.5]) if kind == "lattice" else RB
+    rng = np.random.default_rng(3)
+    w1 = rng.uniform(0.1, 1, (len(p1), nw))
+    w2 = w1 if n2 == 0 else rng.uniform(0.1, 1, (len(p2), nw))
+    if nw == 5:
+        w1[:, 4] = np.round(w1[:, 4] * 3)
+        w2[:, 4] = np.round(w2[:, 4] * 3)
+    kw = dict(period=L, weights1=w1, weights2=w2, weight_func_id=wfunc)
+    np.testing.assert_allclose(mo.marked_npairs_3d(p1, p2, rb, **kw), ORC.marked_npairs_3d(p1, p2, rb, **kw),
+                               rtol=1e-12, atol=1e-300)
+    if wfunc < 16:
+        np.testing.assert_allclose(mo.marked_npairs_xy_z(p1, p2, rb, PI, **kw),
+                                   ORC.marked_npairs_xy_z(p1, p2, rb, PI, **kw), rtol=1e-12, atol=1e-300)
+
+
+@pytest.mark.parametrize("layout", ["rows", "columns", "f32", "sliced"])
+def test_layouts_and_general_kernels_agree(mo, gpu, layout, monkeypatch):
+    import torch
+    p = torch.as_tensor(_points(5000, "clumps", 2), device=gpu)
+    if layout == "columns":
+        p = p.t().contiguous().t()
+    elif layout == "f32":
+        p = p.to(torch.float32).clamp(0, float(np.nextafter(np.float32(L), np.float32(0))))
+    elif layout == "sliced":
+        p = torch.cat([p, p], dim=1)[::2, 1:4]
+    got = [mo.npairs_3d(p, p, RB, period=L), mo.npairs_xy_z(p, p, RB, PI, period=L),
+           mo.npairs_per_object_3d(p, p, RB, period=L), mo.npairs_projected(p, p, RB, 3.0, period=L)]
+    monkeypatch.setenv("HALOPAIR_NO_TILES", "1")
+    ref = [mo.npairs_3d(p, p, RB, period=L), mo.npairs_xy_z(p, p, RB, PI, period=L),
+           mo.npairs_per_object_3d(p, p, RB, period=L), mo.npairs_projected(p, p, RB, 3.0, period=L)]
+    for a, b in zip(got, ref):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("same", [True, False])
+def test_jacobian_rows_and_seam_corrections(gpu, same, monkeypatch):
+    # weights that are small integers: both kernels' row sums are exact, so the rows agree bit for bit
+    import torch
+
+    from halotools_amd import _device as D
+    from halotools_amd import _engine as E
+    rng = np.random.default_rng(5)
+    p1 = _points(1200, "lattice", 0) + 0.1 * rng.integers(0, 2, (1200, 3))
+    p2 = _points(700, "lattice", 1)
+    t1, t2 = [torch.as_tensor(np.mod(p, L), device=gpu) for p in (p1, p2)]
+    w1 = torch.as_tensor(rng.integers(1, 9, (1200, 1)).astype(float), device=gpu)
+    w2 = torch.as_tensor(rng.integers(1, 9, (700, 1)).astype(float), device=gpu)
+    r2 = np.array([2.4, 2.5, 5.0, 7.5, 12.4]) ** 2
+    mock = dict(n1=1200, n2=700, period=[L] * 3, pbc=True)
+
+    def run():
+        res = D.run(E.HP_MARKED_NPAIRS_3D, [mock], t1.unbind(1), (t1 if same else t2).unbind(1), r2, same=same, w1=w1,
+                    w2=None if same else w2, nw=1, wfunc=1, want_counts=False, want_sums=True, rows1=True, rows2=True,
+                    also_counts=True, device=gpu)
+        return res.rows1, res.rows2, res.sums, res.counts
+    got = run()
+    monkeypatch.setenv("HALOPAIR_NO_TILES", "1")
+    for a, b in zip(got, run()):
+        assert torch.equal(a, b)
