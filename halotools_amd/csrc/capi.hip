@@ -355,11 +355,14 @@ static int make_plan(const hp_request* r, int kind, Plan& P, bool tiles = true) 
     const int mode = mode_of(P, kind, r->wfunc);
     {
         const int wb = tile_wave_bytes(mode, P.Kr, P.Kp, P.nw, P.counts ? 1 : 0);
-        P.tiles = tiles && mode != kModeTan && mode != kModeWXYZ && P.ttr.spec.ok && (P.Kp == 0 || P.ttp.spec.ok) && wb > 0 && wb <= 23 * 1024 &&
+        P.tiles = tiles && P.ttr.spec.ok && (P.Kp == 0 || P.ttp.spec.ok) && wb > 0 && wb <= 23 * 1024 &&
                   !std::getenv("HALOPAIR_NO_TILES");
         // one u32 (rp, pi) cell must hold every pair of a group, counted twice
-        for (int m = 0; m < P.M; m++)
-            if (kind == HP_NPAIRS_XY_Z && r->mocks[m].n1 >= (1 << 25)) P.tiles = false;
+        // and a staged point's id holds 26 bits of row
+        for (int m = 0; m < P.M; m++) {
+            const int64_t most = std::max(r->mocks[m].n1, P.same ? (int64_t)0 : r->mocks[m].n2);
+            if (most >= (1 << 26) || (kind == HP_NPAIRS_XY_Z && most >= (1 << 25))) P.tiles = false;
+        }
     }
 
     // ---- per-mock geometry

@@ -98,17 +98,22 @@ static int num_compute_units() {
 
 // LDS layout of one wave of the matrix-core kernels: the stage, the weights of
 // staged and lane points (and the lanes' z for (rp, pi) bins), the histogram.
-static int tile_layout(int mode, int K, int Kp, int nw, int also, TileArgs& A) {
+static int tile_layout(int mode, int K, int Kp, int nw, int also, int var, TileArgs& A) {
     const bool xy = (mode == kModeXYZ || mode == kModeWXYZ || mode == kModeProj);
-    A.w_off = align16(kTileBytes);
-    A.lw_off = A.w_off + align16(nw * kSlots * 8);
+    A.lw_off = align16(deal_of(mode, var) == 64 ? Stage<64>::kTileBytes : Stage<128>::kTileBytes);
+    A.ccol_sh = 0;
     A.hist_off = A.lw_off + nw * 512 + (xy ? 512 : 0);
     A.cnt_off = A.hist_off;
     int h = -1;
     switch (mode) {
         case kModeCount3D:
         case kModeProj: h = (K + 1) * 128; break;
-        case kModeXYZ: h = K * Kp * 4; break;
+        case kModeXYZ:
+            // few cells (wp: one pi bin) in up to 32 columns, so that the lanes of
+            // one LDS pass rarely meet on one cell
+            while (A.ccol_sh < 5 && (K * Kp * 4 << (A.ccol_sh + 1)) <= 4096) A.ccol_sh++;
+            h = K * Kp * 4 << A.ccol_sh;
+            break;
         case kModeWXYZ: h = K * Kp * 8; break;
         case kModeObj: h = (K + 1) * 256; break;
         case kModeJac:
@@ -120,8 +125,8 @@ static int tile_layout(int mode, int K, int Kp, int nw, int also, TileArgs& A) {
             if (also) { A.cnt_off = A.hist_off + h; h += (K + 1) * 128; }
             break;
         case kModeTan:
-            A.cnt_off = A.hist_off + 256;
-            h = (K + 1) * (also ? 384 : 256);
+            A.cnt_off = A.hist_off + 16 * (int)kTanCols;
+            h = (K + 1) * (also ? 24 : 16) * (int)kTanCols;
             break;
         default: return -1;
     }
@@ -129,10 +134,21 @@ static int tile_layout(int mode, int K, int Kp, int nw, int also, TileArgs& A) {
     return A.wave_bytes;
 }
 
+// The kernel's VAR for a request (pairs_tile.h).
+static int tile_var(int mode, int K, int Kp, int wfunc, int nw, int swap) {
+    switch (mode) {
+        case kModeXYZ: return K * Kp > 256 ? 1 : 0;  // cells in one column or two: their LDS bounds the waves
+        case kModeWSum:
+        case kModeWXYZ: return (wfunc == 1 && nw == 1) ? 1 : (nw == 2 ? 2 : 0);
+        case kModeJac: return swap;
+    }
+    return 0;
+}
+
 int tile_wave_bytes(int mode, int K, int Kp, int nw, int also) {
     TileArgs A;
     if ((int64_t)K * std::max(Kp, 1) > 65536) return -1;
-    return tile_layout(mode, K, Kp, nw, also, A);
+    return tile_layout(mode, K, Kp, nw, also, tile_var(mode, K, Kp, 0, nw, 0), A);
 }
 
 // Matrix-core kernels: workgroup shape (the waves per workgroup that keep the
@@ -144,10 +160,11 @@ static int launch_tiles(const PairLaunch& L, int lds_per_block, hipStream_t s) {
     A.tp = L.tp;
     const bool xy = (L.mode == kModeXYZ || L.mode == kModeWXYZ || L.mode == kModeProj);
     const int also = L.also_count ? 1 : 0;
-    const int prod = (L.wfunc == 1 && L.nw == 1) ? 1 : 0;
-    if (tile_layout(L.mode, L.br.nbins, L.bp.nbins, L.nw, also, A) < 0) return -1;
-    A.tp_off = align16(8 * ((int)L.tr.mask + 1));
-    A.tab_bytes = A.tp_off + (xy ? align16(8 * ((int)L.tp.mask + 1)) : 0);
+    const int var = tile_var(L.mode, L.br.nbins, L.bp.nbins, L.wfunc, L.nw, L.swap);
+    if (tile_layout(L.mode, L.br.nbins, L.bp.nbins, L.nw, also, var, A) < 0) return -1;
+    // tables of 2^n entries, the pi table at a multiple of its size
+    A.tp_off = xy ? 8 * (int)std::max(L.tr.mask + 1, L.tp.mask + 1) : 0;
+    A.tab_bytes = xy ? A.tp_off + 8 * ((int)L.tp.mask + 1) : 8 * ((int)L.tr.mask + 1);
     constexpr int kLdsPerCU = 160 * 1024, reg_waves = 4 * HP_TILE_WPS;
     int waves = 0, best = 0;
     for (const int w : {4, 8, 2, 1}) {
@@ -174,14 +191,14 @@ static int launch_tiles(const PairLaunch& L, int lds_per_block, hipStream_t s) {
     const int64_t items = (A.tail << A.parts_sh) + ((L.ngroups - A.tail) << A.tail_sh);
     const int smem = A.tab_bytes + waves * A.wave_bytes;
     switch (L.mode) {
-        case kModeCount3D: return launch_tiles_mode<kModeCount3D>(A, waves, items, smem, also, 0, s);
-        case kModeProj: return launch_tiles_mode<kModeProj>(A, waves, items, smem, also, 0, s);
-        case kModeXYZ: return launch_tiles_mode<kModeXYZ>(A, waves, items, smem, also, 0, s);
-        case kModeWXYZ: return launch_tiles_mode<kModeWXYZ>(A, waves, items, smem, also, prod, s);
-        case kModeObj: return launch_tiles_mode<kModeObj>(A, waves, items, smem, also, 0, s);
-        case kModeJac: return launch_tiles_mode<kModeJac>(A, waves, items, smem, also, L.swap, s);
-        case kModeTan: return launch_tiles_mode<kModeTan>(A, waves, items, smem, also, 0, s);
-        case kModeWSum: return launch_tiles_mode<kModeWSum>(A, waves, items, smem, also, prod, s);
+        case kModeCount3D: return launch_tiles_mode<kModeCount3D>(A, waves, items, smem, also, var, s);
+        case kModeProj: return launch_tiles_mode<kModeProj>(A, waves, items, smem, also, var, s);
+        case kModeXYZ: return launch_tiles_mode<kModeXYZ>(A, waves, items, smem, also, var, s);
+        case kModeWXYZ: return launch_tiles_mode<kModeWXYZ>(A, waves, items, smem, also, var, s);
+        case kModeObj: return launch_tiles_mode<kModeObj>(A, waves, items, smem, also, var, s);
+        case kModeJac: return launch_tiles_mode<kModeJac>(A, waves, items, smem, also, var, s);
+        case kModeTan: return launch_tiles_mode<kModeTan>(A, waves, items, smem, also, var, s);
+        case kModeWSum: return launch_tiles_mode<kModeWSum>(A, waves, items, smem, also, var, s);
     }
     return -1;
 }

@@ -34,28 +34,50 @@ namespace hp {
 
 typedef double dbl4 __attribute__((ext_vector_type(4)));
 
+#ifndef HP_TAN_COLS
+#define HP_TAN_COLS 8
+#endif
+constexpr uint32_t kTanCols = HP_TAN_COLS;
 #ifndef HP_TILE_WPS
 #define HP_TILE_WPS 4
 #endif
 constexpr int kSub = 16;                   // lane points of a sub-group, stream points of a tile
-constexpr int kStage = 192;                // staged stream points per wave: 128 are dealt at a time
-constexpr int kDeal = 128;
-constexpr int kSlots = kStage + 1;         // and one that no pair bins
-constexpr int kIdOff = 4 * kSlots * 8;     // after x, y, z, squared norm: stream index and image of each
-constexpr int kListOff = kIdOff + kStage * 4;            // slots dealt to a sub-group, two tiles of padding
-constexpr int kMarkOff = kListOff + kDeal + 3 * kSub;    // 64: starts of stretches
-constexpr int kInfoOff = (kMarkOff + 64 + 15) / 16 * 16; // the sub-groups' boxes and the group's box
-constexpr int kTileBytes = kInfoOff + 4 * 32 + 32;
+// Staged stream points dealt at a time: 128, or 64 where the histogram leaves
+// little LDS, so that more waves fit a CU (forward-mode pass of 64 mocks: 9.4 ->
+// 12 waves per CU and 45.9 -> 42.6 ms; 1M marked (rp, pi) sums 1782 -> 1720 us;
+// the 1M count, whose tiles fill less well with 64, loses 813 -> 860 us).
+// Wide (rp, pi) counts (2M points, 656 cells: 12 -> 16 waves) take 64 (var 1), wp's
+// few cells 128.
+constexpr int deal_of(int mode, int var) {
+    return (mode == kModeTan || mode == kModeWXYZ || mode == kModeObj || mode == kModeJac ||
+            (mode == kModeXYZ && var == 1))
+               ? 64
+               : 128;
+}
+// LDS layout of one wave ahead of its weights and histogram
+template <int kDeal>
+struct Stage {
+static constexpr int kStage = kDeal + 64;         // staged points
+static constexpr int kSlots = kStage + 1;         // and one that no pair bins
+static constexpr int kIdOff = 4 * kSlots * 8;     // after x, y, z, squared norm: stream index and image of each
+static constexpr int kListOff = kIdOff + (kSlots + 3) / 4 * 16;            // slots dealt to a sub-group, two tiles of padding
+static constexpr int kMarkOff = kListOff + kDeal + 3 * kSub;    // 64: starts of stretches
+static constexpr int kInfoOff = (kMarkOff + 64 + 15) / 16 * 16; // boxes of the sub-groups and the group, the cube window
+static constexpr int kTileBytes = kInfoOff + 4 * 32 + 32 + 48;
+};
+constexpr int kImgShift = 26;              // a staged point's id: row of its mock, image above
+constexpr uint32_t kRowMask = (1u << kImgShift) - 1u;
+constexpr int kHere = 1 | (1 << 2) | (1 << 4);  // the unshifted image
 constexpr double kFar = 1.0e300;           // squared norm of a point that no pair bins
 
 struct TileArgs {
     PairLaunch L;
     TileSpec tr, tp;
-    int tp_off;      // LDS byte offset of the pi table
-    int w_off;       // byte offset of the staged weights in a wave's LDS area
-    int lw_off;      // ... of the lane points' weights
+    int tp_off;      // LDS byte offset of the pi table, a multiple of its size
+    int lw_off;      // byte offset of the lane points' weights in a wave's LDS area
     int hist_off;    // ... of its histogram
     int cnt_off;     // ... of the count rows of a marked pass
+    int ccol_sh;     // log2 of the columns of the (rp, pi) count cells
     int wave_bytes;
     int tab_bytes;
     int parts_sh;    // log2 of the work items per lane group (cubes dealt round-robin)
@@ -64,6 +86,7 @@ struct TileArgs {
 };
 
 typedef const __attribute__((address_space(4))) TileArgs kernarg_tile_args;  // as the kernel receives them
+typedef const __attribute__((address_space(4))) MockGeom const_geom;         // scalar loads
 
 // DPP moves: row rotations (all 16 lanes of a row), prefix steps over the wave
 template <int CTRL, int ROWS>
@@ -145,22 +168,26 @@ __device__ __forceinline__ void sub_borrow(uint32_t e, uint32_t c, uint32_t k, u
         : "vcc");
 }
 
-// VAR: product marks compiled in (kModeWSum, kModeWXYZ); the swapped Jacobian
-// pass (kModeJac: lanes are sample 2, the stream is sample 1).  ALSO: plain
+// VAR: product marks compiled in (kModeWSum, kModeWXYZ: 1; 2: two weights per
+// point); the swapped Jacobian pass (kModeJac: lanes are sample 2, the stream is
+// sample 1).  ALSO: plain
 // counts beside the sums.
 template <int MODE, int VAR, int ALSO, int WAVES>
 __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArgs A) {
     constexpr bool SWAP = (MODE == kModeJac) && VAR;
-    constexpr bool PROD = (MODE == kModeWSum || MODE == kModeWXYZ) && VAR;
+    constexpr bool PROD = (MODE == kModeWSum || MODE == kModeWXYZ) && VAR == 1;
     constexpr bool XY = (MODE == kModeXYZ || MODE == kModeWXYZ || MODE == kModeProj);
     constexpr bool F64 = (MODE == kModeWSum || MODE == kModeWXYZ || MODE == kModeJac || MODE == kModeTan);
     constexpr bool TAN = (MODE == kModeTan);
+    constexpr int kDeal = deal_of(MODE, VAR), kDealH = kDeal / 64;
+    using ST = Stage<kDeal>;
+    constexpr int kStage = ST::kStage, kSlots = ST::kSlots;
     extern __shared__ __align__(16) unsigned char lds[];
     const PairLaunch& L = A.L;
     const int lane = threadIdx.x & 63;
     const int wid = uni(threadIdx.x >> 6);
     const int K = L.br.nbins, Kp = XY ? L.bp.nbins : 1;
-    const int nw = !F64 ? 0 : (TAN ? 2 : ((MODE == kModeJac || PROD) ? 1 : L.nw));
+    const int nw = !F64 ? 0 : (TAN ? 2 : ((MODE == kModeJac || PROD) ? 1 : (VAR == 2 ? 2 : L.nw)));
     unsigned char* const wsm = lds + A.tab_bytes + wid * A.wave_bytes;
     // entries of the tables: k becomes the byte offset of the bin's row (column)
     {
@@ -174,11 +201,10 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
         }
     }
     double* const SX = reinterpret_cast<double*>(wsm);  // x[kSlots], y, z, n
-    uint32_t* const ID = reinterpret_cast<uint32_t*>(wsm + kIdOff);
-    uint8_t* const list = wsm + kListOff;
-    uint8_t* const mark = wsm + kMarkOff;
-    float* const info = reinterpret_cast<float*>(wsm + kInfoOff);  // per sub-group: low x, y, z, high x, y, z; the group's
-    double* const SWT = reinterpret_cast<double*>(wsm + A.w_off);   // staged weights: [nw][kSlots]
+    uint32_t* const ID = reinterpret_cast<uint32_t*>(wsm + ST::kIdOff);
+    uint8_t* const list = wsm + ST::kListOff;
+    uint8_t* const mark = wsm + ST::kMarkOff;
+    float* const info = reinterpret_cast<float*>(wsm + ST::kInfoOff);  // per sub-group: low x, y, z, high x, y, z; the group's
     double* const LWT = reinterpret_cast<double*>(wsm + A.lw_off);  // lane points' weights: [nw][64]
     unsigned char* const hist = wsm + A.hist_off;
     for (int i = lane; i < (A.wave_bytes - A.hist_off) / 4; i += 64) reinterpret_cast<uint32_t*>(hist)[i] = 0u;
@@ -207,7 +233,7 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
     constexpr int SD = SWAP ? 1 : 0;  // the lanes' side of the geometry, the stream's
     constexpr int SS = 1 - SD;
     const int m = uni(L.group_mock[g]);
-    const MockGeom* const geom = L.geom + m;
+    const_geom* const geom = (const_geom*)(L.geom + m);
     const int64_t gl = g - geom->group_off[SD];
     const int64_t p0 = geom->p_off[SD] + gl * kGroup;
     const int64_t left = geom->n[SD] - gl * kGroup;
@@ -251,17 +277,31 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
         if (lane == 0) {
             float* const f = info + 32;
             f[0] = bxlo; f[1] = bylo; f[2] = bzlo; f[3] = bxhi; f[4] = byhi; f[5] = bzhi;
+            // the window of cubes (the eps margin of the box covers the rounding here)
+            const int nc = geom->ndiv[0];
+            const int j0 = geom->pbc ? -nc : 0, j1 = geom->pbc ? 2 * nc - 1 : nc - 1;
+            const float R = geom->search[0];
+            const float ix = (float)geom->inv_cell[0], iy = (float)geom->inv_cell[1], iz = (float)geom->inv_cell[2];
+            const int jx0 = max((int)floorf((bxlo - R) * ix), j0), jx1 = min((int)floorf((bxhi + R) * ix), j1);
+            const int jy0 = max((int)floorf((bylo - R) * iy), j0), jy1 = min((int)floorf((byhi + R) * iy), j1);
+            const int jz0 = max((int)floorf((bzlo - Rz) * iz), j0), jz1 = min((int)floorf((bzhi + Rz) * iz), j1);
+            const int wy = jy1 - jy0 + 1, wz = jz1 - jz0 + 1;
+            int* const w = reinterpret_cast<int*>(info) + 40;
+            w[0] = jx0; w[1] = jy0; w[2] = jz0; w[3] = wy; w[4] = wz;
+            w[5] = (jx1 >= jx0 && wy > 0 && wz > 0) ? (jx1 - jx0 + 1) * wy * wz : 0;
+            f[14] = 1.0f / (float)wy;
+            f[15] = 1.0f / (float)wz;
+            f[16] = (float)geom->cell[0]; f[17] = (float)geom->cell[1]; f[18] = (float)geom->cell[2];
             // the slot that fills up a tile
             SX[kStage] = 0.0;
             SX[kSlots + kStage] = 0.0;
             SX[2 * kSlots + kStage] = 0.0;
             SX[3 * kSlots + kStage] = kFar;
+            ID[kStage] = 0u;
         }
         if (F64) {
             const double* w = L.lane.w + (p0 + (act ? lane : 0)) * nw;
             for (int c = 0; c < nw; c++) LWT[c * 64 + lane] = w[c];
-            if (lane == 0)
-                for (int c = 0; c < nw; c++) SWT[c * kSlots + kStage] = 0.0;
         }
         // B operand: lane l holds component l / 16 of point l % 16 of the sub-group
         SX[lane] = act ? -2.0 * ax : 0.0;
@@ -299,40 +339,36 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
     const int tlo = (int)A.tr.lo, thi = (int)A.tr.hi;
     const uint32_t tsh = A.tr.sh3, tmask = A.tr.mask << 3;
     const int plo = (int)A.tp.lo, phi = (int)A.tp.hi;
-    const uint32_t psh3 = A.tp.sh3, pmask = A.tp.mask << 3;
+    const uint32_t psh3 = A.tp.sh3, pmask = A.tp.mask << 3, ptab = (uint32_t)A.tp_off;
     const int lrow = ((lane & 3) << 2) | ((lane >> 2) & 3);   // list position of this lane's A row
     const int brow = ((lane >> 4) << 2) | (lane & 3);         // list position of the D row this lane's row broadcasts
     const double* const comp = SX + (lane >> 4) * kSlots;     // the component this lane holds of the A operand
     // histogram columns: u32 rows of 32 columns, f64 rows of 16 (no two lanes of
     // one LDS pass on one address); per lane point for object rows and Jacobians
     const uint32_t col4 = (uint32_t)(lane & 31) * 4u, col8 = (uint32_t)(lane & 15) * 8u;
+    constexpr uint32_t TC = kTanCols, TR = 8u * TC;  // forward mode: columns of the W, dW and count rows
+    const uint32_t tcol8 = (uint32_t)(lane & (TC - 1)) * 8u, tcol4 = (uint32_t)(lane & (2 * TC - 1)) * 4u;
+    const uint32_t ccol = (uint32_t)A.ccol_sh, ccl = (uint32_t)(lane & ((1 << A.ccol_sh) - 1));
     uint64_t evals = 0;
+    const double* const SWm = F64 ? L.strm.w + (int64_t)sbase * nw : nullptr;
 
     // Exact bin of the pair (lane point j of the group, staged slot): the first
     // edge not below the distance, scanning from edge k (and q along pi).  Rarely
     // taken: what it needs is loaded here, not kept in registers through the
     // kernel (the empty asm hides that it is the same).  rev: the pair's other
     // orientation, (x2 + shift) - x1.
-    auto exact_bin = [&](int j, int slot, bool self, uint32_t k, uint32_t& kp, bool rev) __attribute__((always_inline)) -> uint32_t {
+    auto exact_bin = [&](int j, int slot, uint32_t k, uint32_t& kp, bool rev) __attribute__((always_inline)) -> uint32_t {
         kernarg_tile_args* ap = (kernarg_tile_args*)__builtin_amdgcn_kernarg_segment_ptr();
-        const MockGeom* gp = geom;
+        const_geom* gp = geom;
         asm volatile("" : "+s"(ap), "+s"(gp));
         const double* ge = reinterpret_cast<const double*>(static_cast<const char*>(ap->L.ws) + ap->L.br.edges_off);
         const int64_t first = gp->p_off[SD] + gl * kGroup;
         const double* pl = ap->L.lane.x + (first + min(j, cnt - 1)) * 4;
         double px = pl[0], py = pl[1], pz = pl[2];
-        const double* r;
-        int tx = 0, ty = 0, tz = 0;
-        if (self) {
-            r = ap->L.lane.x + (first + min(slot, cnt - 1)) * 4;
-        } else {
-            const uint32_t id = ID[slot];
-            const int img = (int)(id >> 27);
-            r = ap->L.strm.x + (gp->p_off[SS] + (int64_t)(id & 0x7ffffffu)) * 4;
-            tx = img / 9 - 1;
-            ty = (img / 3) % 3 - 1;
-            tz = img % 3 - 1;
-        }
+        const uint32_t id = ID[slot];
+        const int img = (int)(id >> kImgShift);
+        const double* r = ap->L.strm.x + (gp->p_off[SS] + (int64_t)(id & kRowMask)) * 4;
+        const int tx = (img & 3) - 1, ty = ((img >> 2) & 3) - 1, tz = (img >> 4) - 1;
         double qx = r[0], qy = r[1], qz = r[2];
         // the image of the stream point lies at q + t L; the reference shifts the sample-1 point
         if ((!SWAP && !rev) || (SWAP && rev)) {
@@ -364,26 +400,29 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
     // self: the slots hold the group's own points
     int qlen = 0;
     auto process = [&](bool self) __attribute__((always_inline)) {
-        float fx[2], fy[2], fz[2];
-        uint64_t in[2], plain[2];
+        float fx[kDealH], fy[kDealH], fz[kDealH];
+        uint64_t in[kDealH], plain[kDealH];
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
+        for (int h = 0; h < kDealH; h++) {
             const int slot = h * 64 + lane;
             in[h] = (uint64_t)__ballot(slot < qlen);
             fx[h] = (float)SX[slot];
             fy[h] = (float)SX[kSlots + slot];
             fz[h] = (float)SX[2 * kSlots + slot];
-            plain[h] = sym ? (uint64_t)__ballot((ID[slot] >> 27) == 13u) & in[h] : 0ull;
+            plain[h] = sym ? (uint64_t)__ballot((ID[slot] >> kImgShift) == (uint32_t)kHere) & in[h] : 0ull;
         }
         // symmetric counts: the shifted points (once), then the unshifted ones
         // (twice); other counts: every point once
         const bool two = sym && !self;
         for (int sc = two ? 0 : 4; sc < 8; sc++) {
             const int s = sc & 3;
-            uint64_t mk[2];
+            uint64_t mk[kDealH], any = 0;
 #pragma unroll
-            for (int h = 0; h < 2; h++) mk[h] = !two ? in[h] : (sc < 4 ? in[h] & ~plain[h] : plain[h]);
-            if ((mk[0] | mk[1]) == 0) {
+            for (int h = 0; h < kDealH; h++) {
+                mk[h] = !two ? in[h] : (sc < 4 ? in[h] & ~plain[h] : plain[h]);
+                any |= mk[h];
+            }
+            if (any == 0) {
                 sc |= 3;  // none of this class
                 continue;
             }
@@ -392,13 +431,14 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
             if (self) {
                 n = min(qlen, (s + 1) * kSub);  // the group's points up to this sub-group
                 list[lane] = (uint8_t)lane;
+                if (lane < 2 * kSub) list[64 + lane] = (uint8_t)kStage;
             } else {
                 // staged points near the sub-group's box
                 const float4 b0 = *reinterpret_cast<const float4*>(info + 8 * s);
                 const float2 b1 = *reinterpret_cast<const float2*>(info + 8 * s + 4);
                 n = 0;
 #pragma unroll
-                for (int h = 0; h < 2; h++) {
+                for (int h = 0; h < kDealH; h++) {
                     const float gx = fmaxf(0.f, fmaxf(fx[h] - b0.w, b0.x - fx[h]));
                     const float gy = fmaxf(0.f, fmaxf(fy[h] - b1.x, b0.y - fy[h]));
                     const float gz = fmaxf(0.f, fmaxf(fz[h] - b1.y, b0.z - fz[h]));
@@ -410,7 +450,8 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                     if (__builtin_amdgcn_inverse_ballot_w64(mm)) list[r] = (uint8_t)(h * 64 + lane);
                     n += __builtin_popcountll(mm);
                 }
-                if (lane < kSub) list[n + lane] = (uint8_t)kStage;
+                if (n == 0) continue;
+                if (lane < 2 * kSub) list[n + lane] = (uint8_t)kStage;
                 evals += (uint64_t)n * kSub;
             }
             __builtin_amdgcn_wave_barrier();
@@ -432,6 +473,15 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
             }
             double za = 0.0;
             if (XY) za = LWT[nw * 64 + lj];
+            // stream weights of the D row this lane's row broadcasts
+            double wn[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+            auto load_weights = [&](int slot) __attribute__((always_inline)) {
+                const double* w = SWm + (uint32_t)((ID[slot] & kRowMask) * (uint32_t)nw);
+#pragma unroll
+                for (int c = 0; c < 5; c++)
+                    if (c < nw) wn[c] = w[c];
+            };
+            if (F64) load_weights(list[brow]);
             // operands one tile ahead, their slots two
             double a = comp[list[lrow]];
             int slot2 = list[kSub + lrow];
@@ -439,16 +489,17 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                 // rows: staged points list[t0 + 4 (lane / 16) + i]; columns: the sub-group's points
                 const double a1 = comp[slot2];
                 slot2 = list[t0 + 2 * kSub + lrow];
-                double zb = 0.0, wb[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-                if (XY || F64) {
-                    const int bslot = list[t0 + brow];
-                    if (XY) zb = SX[2 * kSlots + bslot];
-                    if (F64) {
+                double zb = 0.0, wb[5];
+                if (XY) zb = SX[2 * kSlots + list[t0 + brow]];
+                if (F64) {
+                    // this tile's stream weights were loaded a tile ago
 #pragma unroll
-                        for (int c = 0; c < 5; c++)
-                            if (c < nw) wb[c] = SWT[c * kSlots + bslot];
-                    }
+                    for (int c = 0; c < 5; c++) wb[c] = wn[c];
+                    load_weights(list[t0 + kSub + brow]);
                 }
+                // (the next operands' reads go out before the product, which would otherwise
+                // hold them back: its result registers are reused at once)
+                __builtin_amdgcn_sched_barrier(0);
                 const dbl4 D = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bs, cc, 0, 0, 0);
                 a = a1;
                 int hi[4], hp[4];
@@ -482,7 +533,7 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
                         hp[i] = __double2hiint(dz[i] * dz[i]);
-                        const uint32_t off = (((uint32_t)med3i(hp[i], plo, phi) >> psh3) & pmask) + (uint32_t)A.tp_off;
+                        const uint32_t off = (((uint32_t)med3i(hp[i], plo, phi) >> psh3) & pmask) | ptab;
                         enp[i] = lds_entry(off);
                     }
                 }
@@ -514,7 +565,7 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                             const int slot = list[t0 + (lane >> 4) * 4 + i];
                             const uint32_t kb = hv < (int)floor_hi || ek == 0u ? 0u : ek - 1u;
                             uint32_t kq = 0u;
-                            uint32_t kk = exact_bin(s * kSub + (lane & 15), slot, self, kb, kq, false);
+                            uint32_t kk = exact_bin(s * kSub + (lane & 15), slot, kb, kq, false);
                             if (MODE == kModeJac && !SWAP && L.corr != nullptr) {
                                 // Auto-count with one set of weights: the sample-2 rows take
                                 // the pair's other orientation, which across the periodic seam
@@ -523,9 +574,9 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                                 // shifted pair; only these can differ).
                                 const uint32_t id = ID[slot];
                                 uint32_t dummy = 0u;
-                                const uint32_t kr = exact_bin(s * kSub + (lane & 15), slot, self, kb, dummy, true);
-                                if (kr != kk && (id >> 27) != 13u && s * kSub + (lane & 15) < cnt) {
-                                    const int64_t sr = (int64_t)sbase + (int64_t)(id & 0x7ffffffu);
+                                const uint32_t kr = exact_bin(s * kSub + (lane & 15), slot, kb, dummy, true);
+                                if (kr != kk && (id >> kImgShift) != (uint32_t)kHere && s * kSub + (lane & 15) < cnt) {
+                                    const int64_t sr = (int64_t)sbase + (int64_t)(id & kRowMask);
                                     const int64_t q = __double_as_longlong(L.strm.x[sr * 4 + 3]);
                                     double* crow = L.corr + q * K;
                                     if (kk < (uint32_t)K)
@@ -567,9 +618,9 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                     } else if constexpr (MODE == kModeXYZ || MODE == kModeWXYZ) {
                         // one [K][Kp] histogram per wave; pairs beyond an edge skip it
                         if (k[i] < (uint32_t)K && kp[i] < (uint32_t)Kp) {
-                            const uint32_t cell = k[i] * (uint32_t)Kp + kp[i];
+                            const uint32_t cell = __umul24(k[i], (uint32_t)Kp) + kp[i];
                             if constexpr (MODE == kModeXYZ) {
-                                __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hist) + cell, inc, __ATOMIC_RELAXED,
+                                __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hist) + ((cell << ccol) + ccl), inc, __ATOMIC_RELAXED,
                                                        __HIP_MEMORY_SCOPE_WORKGROUP);
                             } else {
                                 const double v = PROD ? lw[0] * sw[0] : wfunc_eval(L.wfunc, lw, sw);
@@ -595,13 +646,13 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                                 }
                                 const double v = lw[0] * wj;
                                 const double tv = __builtin_fma(lw[0], tj, lw[1] * wj);
-                                unsigned char* const r = hist + k[i] * (ALSO ? 384u : 256u);
-                                __hip_atomic_fetch_add(reinterpret_cast<double*>(r + col8), v, __ATOMIC_RELAXED,
+                                unsigned char* const r = hist + __umul24(k[i], ALSO ? 3 * TR : 2 * TR);
+                                __hip_atomic_fetch_add(reinterpret_cast<double*>(r + tcol8), v, __ATOMIC_RELAXED,
                                                        __HIP_MEMORY_SCOPE_WORKGROUP);
-                                __hip_atomic_fetch_add(reinterpret_cast<double*>(r + 128 + col8), tv, __ATOMIC_RELAXED,
+                                __hip_atomic_fetch_add(reinterpret_cast<double*>(r + TR + tcol8), tv, __ATOMIC_RELAXED,
                                                        __HIP_MEMORY_SCOPE_WORKGROUP);
                                 if (ALSO)
-                                    __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(r + 256 + col4), inc,
+                                    __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(r + 2 * TR + tcol4), inc,
                                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                             }
                         } else if constexpr (MODE == kModeWSum) {
@@ -628,8 +679,6 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
             SX[2 * kSlots + lane] = z;
             SX[3 * kSlots + lane] = nn;
             ID[lane] = id;
-            if (F64)
-                for (int c = 0; c < nw; c++) SWT[c * kSlots + lane] = SWT[c * kSlots + f];
         }
         __builtin_amdgcn_wave_barrier();
         qlen = rest;
@@ -651,45 +700,48 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
     auto next = [&]() __attribute__((always_inline)) -> bool {
         at += 64;
         while (at >= total) {
-            const MockGeom* gp = geom;
+            const_geom* gp = geom;
             asm volatile("" : "+s"(gp));
-            const int nc = gp->ndiv[0];  // cubes per dimension
-            const int pbc = gp->pbc;
-            const float Rx = gp->search[0];
-            const float cxf = (float)gp->cell[0], cyf = (float)gp->cell[1], czf = (float)gp->cell[2];
-            const float bxlo = unif(info[32]), bylo = unif(info[33]), bzlo = unif(info[34]);
-            const float bxhi = unif(info[35]), byhi = unif(info[36]), bzhi = unif(info[37]);
-            const int j0 = pbc ? -nc : 0, j1 = pbc ? 2 * nc - 1 : nc - 1;
-            const int jx0 = uni(max((int)floorf((bxlo - Rx) / cxf), j0)), jx1 = uni(min((int)floorf((bxhi + Rx) / cxf), j1));
-            const int jy0 = uni(max((int)floorf((bylo - Rx) / cyf), j0)), jy1 = uni(min((int)floorf((byhi + Rx) / cyf), j1));
-            const int jz0 = uni(max((int)floorf((bzlo - Rz) / czf), j0)), jz1 = uni(min((int)floorf((bzhi + Rz) / czf), j1));
-            const int wy = jy1 - jy0 + 1, wz = jz1 - jz0 + 1;
-            const int ncubes = (jx1 >= jx0 && wy > 0 && wz > 0) ? (jx1 - jx0 + 1) * wy * wz : 0;
+            const int cb = gp->cbits, nc = 1 << cb;  // cubes per dimension
+            const int* const w = reinterpret_cast<const int*>(info) + 40;
+            const int wy = w[3], wz = w[4], ncubes = uni(w[5]);
             cube0 += 64;
             if ((cube0 << psh) + part >= ncubes) return false;
+            // cube ci of the window: z fastest (quotients from reciprocals: exact
+            // for the few thousand cubes of a window, and one more test for more)
             const int ci = ((cube0 + lane) << psh) + part;
-            const int cxy = ci / wz;
-            const int jx = jx0 + cxy / wy, jy = jy0 + cxy % wy, jz = jz0 + ci % wz;
-            const float gx = fmaxf(0.f, fmaxf((float)jx * cxf - bxhi, bxlo - (float)(jx + 1) * cxf));
-            const float gy = fmaxf(0.f, fmaxf((float)jy * cyf - byhi, bylo - (float)(jy + 1) * cyf));
-            const float gz = fmaxf(0.f, fmaxf((float)jz * czf - bzhi, bzlo - (float)(jz + 1) * czf));
+            int cxy = (int)((float)ci * info[47]);
+            int jz = ci - cxy * wz;
+            if (jz < 0) { jz += wz; cxy--; }
+            if (jz >= wz) { jz -= wz; cxy++; }
+            int jx = (int)((float)cxy * info[46]);
+            int jy = cxy - jx * wy;
+            if (jy < 0) { jy += wy; jx--; }
+            if (jy >= wy) { jy -= wy; jx++; }
+            jx += w[0];
+            jy += w[1];
+            jz += w[2];
+            const float cxf = info[48], cyf = info[49], czf = info[50];
+            const float gx = fmaxf(0.f, fmaxf((float)jx * cxf - info[35], info[32] - (float)(jx + 1) * cxf));
+            const float gy = fmaxf(0.f, fmaxf((float)jy * cyf - info[36], info[33] - (float)(jy + 1) * cyf));
+            const float gz = fmaxf(0.f, fmaxf((float)jz * czf - info[37], info[34] - (float)(jz + 1) * czf));
             at = 0;
             total = 0;
             const bool has = ci < ncubes && (XY ? gx * gx + gy * gy : gx * gx + gy * gy + gz * gz) <= r2xy;
             if ((uint64_t)__ballot(has) == 0) continue;
-            const int tx = jx < 0 ? -1 : (jx >= nc ? 1 : 0), ty = jy < 0 ? -1 : (jy >= nc ? 1 : 0),
-                      tz = jz < 0 ? -1 : (jz >= nc ? 1 : 0);
-            cimg = (tx + 1) * 9 + (ty + 1) * 3 + (tz + 1);
+            // image: 0, 1, 2 for -L, 0, +L per dimension, two bits each
+            const int ux = (jx >> cb) + 1, uy = (jy >> cb) + 1, uz = (jz >> cb) + 1;
+            cimg = ux | (uy << 2) | (uz << 4);
             int len = 0;
             run = 0;
             if (has) {
-                const uint2 c = L.strm.cubes[gp->cell_off + ((int64_t)(jx - tx * nc) * nc + (jy - ty * nc)) * nc +
-                                             (jz - tz * nc)];
+                const int cm = nc - 1;
+                const uint2 c = (L.strm.cubes + gp->cell_off)[(uint32_t)(((((jx & cm) << cb) + (jy & cm)) << cb) + (jz & cm))];
                 run = (int)c.x;
-                if (sym && cimg == 13) run = max(run, (int)(gp->p_off[SD] + gl * kGroup + cnt));
+                if (sym && cimg == kHere) run = max(run, (int)(gp->p_off[SD] + gl * kGroup + cnt));
                 len = max((int)c.y - run, 0);
             }
-            seam = (uint64_t)__ballot(len > 0 && cimg != 13) != 0;
+            seam = (uint64_t)__ballot(len > 0 && cimg != kHere) != 0;
             pre = wave_prefix(len);
             total = __builtin_amdgcn_readlane(pre, 63);
             end = len > 0 ? pre : -1;
@@ -707,12 +759,12 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
         __builtin_amdgcn_wave_barrier();
         const int sg = wave_scan_max((int)mark[lane]) << 2;
         jj = (uint32_t)(min(at + lane, total - 1) + __builtin_amdgcn_ds_bpermute(sg, run));
-        img = seam ? __builtin_amdgcn_ds_bpermute(sg, cimg) : 13;
+        img = seam ? __builtin_amdgcn_ds_bpermute(sg, cimg) : kHere;
     };
     bool more = next();
     double4 row = make_double4(0.0, 0.0, 0.0, 0.0);
     uint32_t jn = 0;
-    int imgn = 13, nn = 0;  // the rows being loaded: indices, images, how many
+    int imgn = kHere, nn = 0;  // the rows being loaded: indices, images, how many
     bool seamn = false;
     if (more) {
         fetch(jn, imgn);
@@ -728,12 +780,11 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
             const int img = imgn, nrow = nn;
             double x = sr.x - cx, y = sr.y - cy, z = sr.z - cz;
             if (seamn) {
-                const MockGeom* gp = geom;
+                const_geom* gp = geom;
                 asm volatile("" : "+s"(gp));
-                const int tx = img / 9 - 1, ty = (img / 3) % 3 - 1, tz = img % 3 - 1;
-                x = sr.x - (cx - (double)tx * gp->period[0]);
-                y = sr.y - (cy - (double)ty * gp->period[1]);
-                z = sr.z - (cz - (double)tz * gp->period[2]);
+                x = sr.x - __builtin_fma((double)(1 - (img & 3)), gp->period[0], cx);
+                y = sr.y - __builtin_fma((double)(1 - ((img >> 2) & 3)), gp->period[1], cy);
+                z = sr.z - __builtin_fma((double)(1 - (img >> 4)), gp->period[2], cz);
             }
             more = next();
             if (more) {
@@ -755,11 +806,7 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                 SX[kSlots + slot] = y;
                 SX[2 * kSlots + slot] = z;
                 SX[3 * kSlots + slot] = XY ? x * x + y * y : x * x + y * y + z * z;
-                ID[slot] = jj | ((uint32_t)img << 27);
-                if (F64) {
-                    const double* w = L.strm.w + ((int64_t)sbase + jj) * nw;
-                    for (int c = 0; c < nw; c++) SWT[c * kSlots + slot] = w[c];
-                }
+                ID[slot] = jj | ((uint32_t)img << kImgShift);
             }
             __builtin_amdgcn_wave_barrier();
             qlen += __builtin_popcountll(mk);
@@ -774,18 +821,18 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
             SX[kSlots + lane] = act ? ay : 0.0;
             SX[2 * kSlots + lane] = act ? az : 0.0;
             SX[3 * kSlots + lane] = !act ? kFar : (XY ? ax * ax + ay * ay : ax * ax + ay * ay + az * az);
-            if (F64)
-                for (int c = 0; c < nw; c++) SWT[c * kSlots + lane] = LWT[c * 64 + lane];
+            // (the lanes' rows are the stream's: one sample)
+            ID[lane] = (uint32_t)(p0 + (act ? lane : 0) - (int64_t)sbase) | ((uint32_t)kHere << kImgShift);
             evals += (uint64_t)cnt * cnt;
             if constexpr (MODE == kModeTan) {
                 if (act) {
                     const double w = LWT[lane], t = LWT[64 + lane];
-                    __hip_atomic_fetch_add(reinterpret_cast<double*>(hist + col8), 0.5 * (w * w), __ATOMIC_RELAXED,
+                    __hip_atomic_fetch_add(reinterpret_cast<double*>(hist + tcol8), 0.5 * (w * w), __ATOMIC_RELAXED,
                                            __HIP_MEMORY_SCOPE_WORKGROUP);
-                    __hip_atomic_fetch_add(reinterpret_cast<double*>(hist + 128 + col8), w * t, __ATOMIC_RELAXED,
+                    __hip_atomic_fetch_add(reinterpret_cast<double*>(hist + TR + tcol8), w * t, __ATOMIC_RELAXED,
                                            __HIP_MEMORY_SCOPE_WORKGROUP);
                 }
-                if (ALSO && lane == 0) *reinterpret_cast<uint32_t*>(hist + 256) += (uint32_t)cnt;
+                if (ALSO && lane == 0) *reinterpret_cast<uint32_t*>(hist + 2 * TR) += (uint32_t)cnt;
             } else {
                 if (lane == 0) *reinterpret_cast<uint32_t*>(hist) += (uint32_t)cnt;
             }
@@ -805,14 +852,17 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
         L.pcount ? L.pcount + ((int64_t)m * L.crep + (int64_t)(gl % L.crep)) * ((MODE == kModeXYZ) ? K * Kp : K) : nullptr;
     if constexpr (MODE == kModeXYZ) {
         const uint32_t* h = reinterpret_cast<const uint32_t*>(hist);
-        for (int k = lane; k < K * Kp; k += 64)
-            if (h[k]) __hip_atomic_fetch_add(cacc + k, (uint64_t)h[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int k = lane; k < K * Kp; k += 64) {
+            uint64_t tot = 0;
+            for (int c = 0; c < (1 << ccol); c++) tot += h[(k << ccol) + ((c + lane) & ((1 << ccol) - 1))];
+            if (tot) __hip_atomic_fetch_add(cacc + k, tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
     } else if constexpr (MODE == kModeCount3D || MODE == kModeProj || ALSO) {
         const uint32_t* h = reinterpret_cast<const uint32_t*>(wsm + A.cnt_off);
-        const int step = TAN ? 96 : 32;
+        constexpr int step = TAN ? 3 * (int)TR / 4 : 32, nc = TAN ? 2 * (int)TC : 32;
         for (int k = lane; k < K; k += 64) {
             uint64_t tot = 0;
-            for (int c = 0; c < 32; c++) tot += h[k * step + ((c + lane) & 31)];
+            for (int c = 0; c < nc; c++) tot += h[k * step + ((c + lane) & (nc - 1))];
             if (tot) __hip_atomic_fetch_add(cacc + k, tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
@@ -823,13 +873,14 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
     }
     if constexpr (MODE == kModeWSum || MODE == kModeTan) {
         const double* h = reinterpret_cast<const double*>(hist);
-        const int step = TAN ? (ALSO ? 48 : 32) : 16;
+        constexpr int nc = TAN ? (int)TC : 16;
+        constexpr int step = TAN ? (ALSO ? 3 : 2) * (int)TC : 16;
         const double sc = (TAN && sym) ? 2.0 : 1.0;
         for (int k = lane; k < K; k += 64) {
             double v = 0.0, tv = 0.0;
-            for (int c = 0; c < 16; c++) {
-                v += h[k * step + ((c + lane) & 15)];
-                if (TAN) tv += h[k * step + 16 + ((c + lane) & 15)];
+            for (int c = 0; c < nc; c++) {
+                v += h[k * step + ((c + lane) & (nc - 1))];
+                if (TAN) tv += h[k * step + nc + ((c + lane) & (nc - 1))];
             }
             const int64_t at_ = ((g << psh) + part) * K + k;
             if (L.psum) L.psum[at_] = sc * v;
@@ -887,6 +938,11 @@ static int launch_tiles_v(const TileArgs& A, int waves, int64_t items, int smem,
 // unit (pairs_tile_*.hip).
 template <int MODE>
 int launch_tiles_mode(const TileArgs& A, int waves, int64_t items, int smem, int also, int var, hipStream_t s) {
+    if constexpr (MODE == kModeWSum) {
+        if (var == 2)
+            return also ? launch_tiles_v<MODE, 2, 1>(A, waves, items, smem, s)
+                        : launch_tiles_v<MODE, 2, 0>(A, waves, items, smem, s);
+    }
     if constexpr (MODE == kModeWSum || MODE == kModeJac) {
         if (var)
             return also ? launch_tiles_v<MODE, 1, 1>(A, waves, items, smem, s)
@@ -894,6 +950,10 @@ int launch_tiles_mode(const TileArgs& A, int waves, int64_t items, int smem, int
         return also ? launch_tiles_v<MODE, 0, 1>(A, waves, items, smem, s)
                     : launch_tiles_v<MODE, 0, 0>(A, waves, items, smem, s);
     } else if constexpr (MODE == kModeWXYZ) {
+        if (var == 2) return launch_tiles_v<MODE, 2, 0>(A, waves, items, smem, s);
+        return var ? launch_tiles_v<MODE, 1, 0>(A, waves, items, smem, s)
+                   : launch_tiles_v<MODE, 0, 0>(A, waves, items, smem, s);
+    } else if constexpr (MODE == kModeXYZ) {
         return var ? launch_tiles_v<MODE, 1, 0>(A, waves, items, smem, s)
                    : launch_tiles_v<MODE, 0, 0>(A, waves, items, smem, s);
     } else if constexpr (MODE == kModeTan) {
