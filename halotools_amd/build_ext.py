@@ -15,7 +15,7 @@ OUT = os.path.join(HERE, "_lib", "libhalopair.so")
 # (pairs_mode_*.hip) so that they compile in parallel
 SOURCES = ["cellbuild.hip", "pairs.hip", "reduce.hip", "capi.hip"] + [
     "pairs_mode_%s.hip" % m for m in ("count3d", "proj", "xyz", "obj", "wxyz", "jack", "jackxy", "wsum", "jac", "tan")] + [
-    "pairs_tile_%s.hip" % m for m in ("count3d", "proj", "xyz", "wxyz", "obj", "jac", "tan", "wsum")]
+    "pairs_tile_%s.hip" % m for m in ("count3d", "proj", "xyz", "wxyz", "obj", "jac", "jack", "tan", "wsum")]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 

@@ -348,6 +348,7 @@ static int make_plan(const hp_request* r, int kind, Plan& P, bool tiles = true) 
     if (!(Rxy == Rxy) || !(Rz == Rz)) return fail("bins must not be NaN");
     P.nb_count = xyz ? P.Kr * P.Kp : P.Kr;
 
+    // (the jackknife tables of an auto-count; cross-counts stay with pairs_kernel.h)
     // The matrix-core kernels (pairs_tile.h) take what their bucket tables and the
     // LDS hold: bins that buckets of 1/16 octave or finer part, and a wave's
     // histogram beside its stage at 7 waves per CU or more.  Wider or denser
@@ -355,7 +356,7 @@ static int make_plan(const hp_request* r, int kind, Plan& P, bool tiles = true) 
     const int mode = mode_of(P, kind, r->wfunc);
     {
         const int wb = tile_wave_bytes(mode, P.Kr, P.Kp, P.nw, P.counts ? 1 : 0);
-        P.tiles = tiles && P.ttr.spec.ok && (P.Kp == 0 || P.ttp.spec.ok) && wb > 0 && wb <= 23 * 1024 &&
+        P.tiles = tiles && !(P.jack && !P.same) && P.ttr.spec.ok && (P.Kp == 0 || P.ttp.spec.ok) && wb > 0 && wb <= 23 * 1024 &&
                   !std::getenv("HALOPAIR_NO_TILES");
         // one u32 (rp, pi) cell must hold every pair of a group, counted twice
         // and a staged point's id holds 26 bits of row
@@ -586,7 +587,7 @@ static int make_plan(const hp_request* r, int kind, Plan& P, bool tiles = true) 
     }
     // unweighted auto-counts evaluate each unshifted unordered pair once; they
     // need every row-major point's position in the Hilbert order
-    P.sym = P.same && !P.obj && (!P.marked || P.tangent);
+    P.sym = P.same && !P.obj && (!P.marked || P.tangent) && !(P.jack && P.tiles);
     // packed rows (x, y, z, Hilbert position[, up to 4 weights]) of every side
     // the stream side is built from: one random row read per point in the gather
     for (int s = 0; s < 2; s++) {
@@ -796,6 +797,9 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
         L.lane = curve[0];
         L.strm = curve[s2];
         L.sym = P.sym ? 1 : 0;
+        // (a sample's Jacobian rows add up in one order whether its second sample is
+        // known to be the same or not)
+        L.own = (P.same && !P.sym && mode_of(P, kind, r->wfunc) != kModeJac) ? 1 : 0;
     }
     L.nw = P.nw;
     L.br = P.tr.spec;
@@ -823,6 +827,7 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
         L.jacc = reinterpret_cast<double*>(ws + P.o_jacc);
         L.nsamp = P.nsamp;
         L.jslots = P.jslots;
+        L.unit = r->w1 ? 0 : 1;
         launch_fill_u32(reinterpret_cast<uint32_t*>(L.jacc), 0u, (int64_t)P.M * (P.nsamp + 1) * P.nb_count * 2, s);
     }
     if (kind == HP_MARKED_NPAIRS_3D) {
@@ -887,7 +892,8 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
             return fail("reduction launch failed");
     }
     if (P.jack) {
-        if (launch_jack_finish(L.jacc, P.Kr, kind == HP_NPAIRS_JACKKNIFE_XY_Z ? P.Kp : 0, P.M, P.nsamp, r->sums, s))
+        if (launch_jack_finish(L.jacc, P.Kr, kind == HP_NPAIRS_JACKKNIFE_XY_Z ? P.Kp : 0, P.M, P.nsamp, P.tiles,
+                               r->sums, s))
             return fail("jackknife reduction launch failed");
     }
     if (P.sums) {

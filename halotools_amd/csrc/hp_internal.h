@@ -170,6 +170,7 @@ struct PairLaunch {
     BinSpec br;            // radial / rp bins
     BinSpec bp;            // pi bins (xy_z) or pi_max (projected, nbins = 1)
     int sym;               // matrix-core kernels: symmetric auto-count
+    int own;               // ... one sample, but every ordered pair from its first point
     TileSpec tr, tp;       // the radial / rp and the pi bins for the matrix-core kernels
     int parts_sh;          // ... log2 of the work items per lane group (FP64 partials: one row each)
     const void* ws;        // workspace base (edges / tables)
@@ -195,6 +196,7 @@ struct PairLaunch {
     // accumulated with atomics; lane and stream weights are (w, tag) rows
     double* jacc;
     int nsamp;
+    int unit;              // jackknife: every weight is 1
     int jslots;            // LDS rows per wave for subsample tags (<= kJackSlots)
     // persistent launches: one work-queue counter per XCD (8 words, zeroed
     // by launch_pairs before every launch)
@@ -218,7 +220,8 @@ int launch_rows_dot(const double* rows, int nr, const double* gsuffix, const int
 int launch_add_rows(const double* a, const double* b, double* out, int64_t n, hipStream_t s);
 int launch_pack_jack(const double* w, const int32_t* tags, int64_t n, int nsamp, double* out, int32_t* status,
                      hipStream_t s);
-int launch_jack_finish(double* acc, int nr, int np, int nmocks, int nsamp, double* out, hipStream_t s);
+// total: row 0 (all pairs) is the sum of the subsample rows
+int launch_jack_finish(double* acc, int nr, int np, int nmocks, int nsamp, bool total, double* out, hipStream_t s);
 int launch_zheng07_tangent(const double* logm, const int64_t* mock_id, const double* logMmin, double sigma,
                            int64_t n, double* wt, hipStream_t s);
 

@@ -27,6 +27,7 @@ extern template int launch_tiles_mode<kModeProj>(const TileArgs&, int, int64_t, 
 extern template int launch_tiles_mode<kModeXYZ>(const TileArgs&, int, int64_t, int, int, int, hipStream_t);
 extern template int launch_tiles_mode<kModeWXYZ>(const TileArgs&, int, int64_t, int, int, int, hipStream_t);
 extern template int launch_tiles_mode<kModeObj>(const TileArgs&, int, int64_t, int, int, int, hipStream_t);
+extern template int launch_tiles_mode<kModeJack>(const TileArgs&, int, int64_t, int, int, int, hipStream_t);
 extern template int launch_tiles_mode<kModeJac>(const TileArgs&, int, int64_t, int, int, int, hipStream_t);
 extern template int launch_tiles_mode<kModeTan>(const TileArgs&, int, int64_t, int, int, int, hipStream_t);
 extern template int launch_tiles_mode<kModeWSum>(const TileArgs&, int, int64_t, int, int, int, hipStream_t);
@@ -116,6 +117,7 @@ static int tile_layout(int mode, int K, int Kp, int nw, int also, int var, TileA
             break;
         case kModeWXYZ: h = K * Kp * 8; break;
         case kModeObj: h = (K + 1) * 256; break;
+        case kModeJack: h = (K + 1) * (var ? 512 : 256); break;
         case kModeJac:
             h = (K + 1) * 512;
             if (also) { A.cnt_off = A.hist_off + h; h += (K + 1) * 128; }
@@ -135,12 +137,13 @@ static int tile_layout(int mode, int K, int Kp, int nw, int also, int var, TileA
 }
 
 // The kernel's VAR for a request (pairs_tile.h).
-static int tile_var(int mode, int K, int Kp, int wfunc, int nw, int swap) {
+static int tile_var(int mode, int K, int Kp, int wfunc, int nw, int swap, int unit) {
     switch (mode) {
         case kModeXYZ: return K * Kp > 256 ? 1 : 0;  // cells in one column or two: their LDS bounds the waves
         case kModeWSum:
         case kModeWXYZ: return (wfunc == 1 && nw == 1) ? 1 : (nw == 2 ? 2 : 0);
         case kModeJac: return swap;
+        case kModeJack: return unit ? 0 : 1;
     }
     return 0;
 }
@@ -148,7 +151,7 @@ static int tile_var(int mode, int K, int Kp, int wfunc, int nw, int swap) {
 int tile_wave_bytes(int mode, int K, int Kp, int nw, int also) {
     TileArgs A;
     if ((int64_t)K * std::max(Kp, 1) > 65536) return -1;
-    return tile_layout(mode, K, Kp, nw, also, tile_var(mode, K, Kp, 0, nw, 0), A);
+    return tile_layout(mode, K, Kp, nw, also, tile_var(mode, K, Kp, 0, nw, 0, 0), A);
 }
 
 // Matrix-core kernels: workgroup shape (the waves per workgroup that keep the
@@ -160,7 +163,7 @@ static int launch_tiles(const PairLaunch& L, int lds_per_block, hipStream_t s) {
     A.tp = L.tp;
     const bool xy = (L.mode == kModeXYZ || L.mode == kModeWXYZ || L.mode == kModeProj);
     const int also = L.also_count ? 1 : 0;
-    const int var = tile_var(L.mode, L.br.nbins, L.bp.nbins, L.wfunc, L.nw, L.swap);
+    const int var = tile_var(L.mode, L.br.nbins, L.bp.nbins, L.wfunc, L.nw, L.swap, L.unit);
     if (tile_layout(L.mode, L.br.nbins, L.bp.nbins, L.nw, also, var, A) < 0) return -1;
     // tables of 2^n entries, the pi table at a multiple of its size
     A.tp_off = xy ? 8 * (int)std::max(L.tr.mask + 1, L.tp.mask + 1) : 0;
@@ -196,6 +199,7 @@ static int launch_tiles(const PairLaunch& L, int lds_per_block, hipStream_t s) {
         case kModeXYZ: return launch_tiles_mode<kModeXYZ>(A, waves, items, smem, also, var, s);
         case kModeWXYZ: return launch_tiles_mode<kModeWXYZ>(A, waves, items, smem, also, var, s);
         case kModeObj: return launch_tiles_mode<kModeObj>(A, waves, items, smem, also, var, s);
+        case kModeJack: return launch_tiles_mode<kModeJack>(A, waves, items, smem, also, var, s);
         case kModeJac: return launch_tiles_mode<kModeJac>(A, waves, items, smem, also, var, s);
         case kModeTan: return launch_tiles_mode<kModeTan>(A, waves, items, smem, also, var, s);
         case kModeWSum: return launch_tiles_mode<kModeWSum>(A, waves, items, smem, also, var, s);

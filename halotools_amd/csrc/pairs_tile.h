@@ -50,7 +50,7 @@ constexpr int kSub = 16;                   // lane points of a sub-group, stream
 // few cells 128.
 constexpr int deal_of(int mode, int var) {
     return (mode == kModeTan || mode == kModeWXYZ || mode == kModeObj || mode == kModeJac ||
-            (mode == kModeXYZ && var == 1))
+            mode == kModeJack || (mode == kModeXYZ && var == 1))
                ? 64
                : 128;
 }
@@ -177,7 +177,11 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
     constexpr bool SWAP = (MODE == kModeJac) && VAR;
     constexpr bool PROD = (MODE == kModeWSum || MODE == kModeWXYZ) && VAR == 1;
     constexpr bool XY = (MODE == kModeXYZ || MODE == kModeWXYZ || MODE == kModeProj);
-    constexpr bool F64 = (MODE == kModeWSum || MODE == kModeWXYZ || MODE == kModeJac || MODE == kModeTan);
+    // jackknife tables of an auto-count: per-lane-point rows as the per-object
+    // counts (VAR 0: unit weights, u32) or the Jacobian (VAR 1: FP64 sums of the
+    // stream weights), added up by the lane points' tags at the end
+    constexpr bool JK = (MODE == kModeJack);
+    constexpr bool F64 = (MODE == kModeWSum || MODE == kModeWXYZ || MODE == kModeJac || MODE == kModeTan || (JK && VAR));
     constexpr bool TAN = (MODE == kModeTan);
     constexpr int kDeal = deal_of(MODE, VAR), kDealH = kDeal / 64;
     using ST = Stage<kDeal>;
@@ -187,7 +191,8 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
     const int lane = threadIdx.x & 63;
     const int wid = uni(threadIdx.x >> 6);
     const int K = L.br.nbins, Kp = XY ? L.bp.nbins : 1;
-    const int nw = !F64 ? 0 : (TAN ? 2 : ((MODE == kModeJac || PROD) ? 1 : (VAR == 2 ? 2 : L.nw)));
+    const int nw = !F64 ? 0 : (TAN ? 2 : ((MODE == kModeJac || PROD || JK) ? 1 : (VAR == 2 ? 2 : L.nw)));
+    const int wst = JK ? 2 : nw;  // doubles per weight row (jackknife: weight and tag)
     unsigned char* const wsm = lds + A.tab_bytes + wid * A.wave_bytes;
     // entries of the tables: k becomes the byte offset of the bin's row (column)
     {
@@ -242,6 +247,7 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
     const float r2xy = geom->r2xy;
     const float Rz = geom->search[2];
     const bool sym = L.sym != 0;
+    const bool own = L.own != 0;  // one sample, every ordered pair from its first point: the group's own points come last
 
     // ---- the group's box, and the lane points relative to its centre
     float hx, hy, hz;     // half sizes, with the eps margin
@@ -300,7 +306,7 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
             ID[kStage] = 0u;
         }
         if (F64) {
-            const double* w = L.lane.w + (p0 + (act ? lane : 0)) * nw;
+            const double* w = L.lane.w + (p0 + (act ? lane : 0)) * wst;
             for (int c = 0; c < nw; c++) LWT[c * 64 + lane] = w[c];
         }
         // B operand: lane l holds component l / 16 of point l % 16 of the sub-group
@@ -350,7 +356,7 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
     const uint32_t tcol8 = (uint32_t)(lane & (TC - 1)) * 8u, tcol4 = (uint32_t)(lane & (2 * TC - 1)) * 4u;
     const uint32_t ccol = (uint32_t)A.ccol_sh, ccl = (uint32_t)(lane & ((1 << A.ccol_sh) - 1));
     uint64_t evals = 0;
-    const double* const SWm = F64 ? L.strm.w + (int64_t)sbase * nw : nullptr;
+    const double* const SWm = F64 ? L.strm.w + (int64_t)sbase * wst : nullptr;
 
     // Exact bin of the pair (lane point j of the group, staged slot): the first
     // edge not below the distance, scanning from edge k (and q along pi).  Rarely
@@ -429,7 +435,7 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
             uint32_t inc = (two && sc >= 4) ? 2u : 1u;
             int n;
             if (self) {
-                n = min(qlen, (s + 1) * kSub);  // the group's points up to this sub-group
+                n = sym ? min(qlen, (s + 1) * kSub) : qlen;  // the group's points (up to this sub-group)
                 list[lane] = (uint8_t)lane;
                 if (lane < 2 * kSub) list[64 + lane] = (uint8_t)kStage;
             } else {
@@ -476,7 +482,7 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
             // stream weights of the D row this lane's row broadcasts
             double wn[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
             auto load_weights = [&](int slot) __attribute__((always_inline)) {
-                const double* w = SWm + (uint32_t)((ID[slot] & kRowMask) * (uint32_t)nw);
+                const double* w = SWm + (uint32_t)((ID[slot] & kRowMask) * (uint32_t)wst);
 #pragma unroll
                 for (int c = 0; c < 5; c++)
                     if (c < nw) wn[c] = w[c];
@@ -509,7 +515,7 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                 for (int i = 0; i < 4; i++) hi[i] = __double2hiint(D[i]);
                 bool diag = false;
                 if (self) {
-                    inc = 2u;
+                    inc = sym ? 2u : 1u;
                     diag = t0 == s * kSub;
                     if (diag) {
                         // inside a sub-group: ordered pairs, without a point and itself
@@ -585,6 +591,27 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                                         __hip_atomic_fetch_add(crow + kr, -lw[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                                 }
                             }
+                            if constexpr (JK) {
+                                // A pair of two tags gives half of its weight to each.  The rows
+                                // give all of an ordered pair's to its lane point's tag, which is
+                                // the same where the pair's other order lands in the same bin;
+                                // across the periodic seam it may not, and half moves over.
+                                const uint32_t id = ID[slot];
+                                uint32_t dummy = 0u;
+                                const uint32_t kr = exact_bin(lj, slot, kb, dummy, true);
+                                if (kr != kk && (id >> kImgShift) != (uint32_t)kHere && lj < cnt) {
+                                    const double* wi = L.lane.w + (p0 + lj) * 2;
+                                    const double v = 0.5 * wi[0] * L.strm.w[((int64_t)sbase + (int64_t)(id & kRowMask)) * 2];
+                                    const int t = (int)wi[1];
+                                    double* r = L.jacc + ((int64_t)m * (L.nsamp + 1) + t) * K;
+                                    if (t >= 1 && t <= L.nsamp) {
+                                        if (kk < (uint32_t)K)
+                                            __hip_atomic_fetch_add(r + kk, -v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                                        if (kr < (uint32_t)K)
+                                            __hip_atomic_fetch_add(r + kr, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                                    }
+                                }
+                            }
 #pragma unroll
                             for (int u = 0; u < 4; u++)
                                 if (i == u) {
@@ -628,11 +655,11 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                                                        __HIP_MEMORY_SCOPE_WORKGROUP);
                             }
                         }
-                    } else if constexpr (MODE == kModeObj) {
+                    } else if constexpr (MODE == kModeObj || (JK && !VAR)) {
                         __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hist + ((k[i] << 8) + (uint32_t)lj * 4u)), 1u,
                                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                     } else {
-                        if constexpr (MODE == kModeJac) {
+                        if constexpr (MODE == kModeJac || JK) {
                             __hip_atomic_fetch_add(reinterpret_cast<double*>(hist + ((k[i] << 9) + (uint32_t)lj * 8u)),
                                                    sw[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                         } else if constexpr (MODE == kModeTan) {
@@ -761,6 +788,7 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
         jj = (uint32_t)(min(at + lane, total - 1) + __builtin_amdgcn_ds_bpermute(sg, run));
         img = seam ? __builtin_amdgcn_ds_bpermute(sg, cimg) : kHere;
     };
+    const uint32_t own0 = (uint32_t)(p0 - (int64_t)sbase);  // the group's first row, in one sample
     bool more = next();
     double4 row = make_double4(0.0, 0.0, 0.0, 0.0);
     uint32_t jn = 0;
@@ -797,7 +825,8 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
             const float gy = fmaxf(0.f, fabsf((float)y) - hy);
             const float gz = fmaxf(0.f, fabsf((float)z) - hz);
             const float gxy = __builtin_fmaf(gy, gy, gx * gx);
-            const bool ok = lane < nrow && (XY ? (gxy <= r2xy && gz <= Rz) : (__builtin_fmaf(gz, gz, gxy) <= r2xy));
+            // (the group's own rows wait for the end)
+            const bool ok = lane < nrow && !(own && jj - own0 < (uint32_t)cnt && img == kHere) && (XY ? (gxy <= r2xy && gz <= Rz) : (__builtin_fmaf(gz, gz, gxy) <= r2xy));
             const uint64_t mk = (uint64_t)__ballot(ok);
             if (ok) {
                 const uint32_t slot = __builtin_amdgcn_mbcnt_hi(
@@ -811,10 +840,11 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
             __builtin_amdgcn_wave_barrier();
             qlen += __builtin_popcountll(mk);
         } else if (qlen == 0) {
-            if (!sym || part != 0 || self_done) break;
-            // symmetric counts, last: the group's own points.  Each unordered
-            // pair of different sub-groups counts twice, the ordered pairs inside
-            // a sub-group once, each point with itself (distance 0: bin 0) once.
+            if (!(sym || own) || part != 0 || self_done) break;
+            // One sample, last: the group's own points.  Symmetric counts take each
+            // unordered pair of different sub-groups twice and the ordered pairs
+            // inside a sub-group once, other passes every ordered pair once; each
+            // point with itself (distance 0: bin 0) is added here.
             const double4 pr = reinterpret_cast<const double4*>(L.lane.x)[p0 + (act ? lane : 0)];
             const double ax = pr.x - cx, ay = pr.y - cy, az = pr.z - cz;
             SX[lane] = act ? ax : 0.0;
@@ -833,8 +863,25 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                                            __HIP_MEMORY_SCOPE_WORKGROUP);
                 }
                 if (ALSO && lane == 0) *reinterpret_cast<uint32_t*>(hist + 2 * TR) += (uint32_t)cnt;
+            } else if constexpr (MODE == kModeObj || (JK && !VAR)) {
+                if (act) reinterpret_cast<uint32_t*>(hist)[lane] += 1u;
+            } else if constexpr (MODE == kModeJac || JK) {
+                if (act) reinterpret_cast<double*>(hist)[lane] += LWT[lane];
+            } else if constexpr (MODE == kModeWSum || MODE == kModeWXYZ) {
+                if (act) {
+                    double w[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                    for (int c = 0; c < 5; c++)
+                        if (c < nw) w[c] = LWT[c * 64 + lane];
+                    const double v = PROD ? w[0] * w[0] : wfunc_eval(L.wfunc, w, w);
+                    __hip_atomic_fetch_add(reinterpret_cast<double*>(hist + (MODE == kModeWSum ? col8 : 0u)), v,
+                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                }
             } else {
                 if (lane == 0) *reinterpret_cast<uint32_t*>(hist) += (uint32_t)cnt;
+            }
+            if constexpr (ALSO && MODE != kModeTan) {
+                if (lane == 0) *reinterpret_cast<uint32_t*>(wsm + A.cnt_off) += (uint32_t)cnt;
             }
             __builtin_amdgcn_wave_barrier();
             qlen = cnt;
@@ -885,6 +932,41 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
             const int64_t at_ = ((g << psh) + part) * K + k;
             if (L.psum) L.psum[at_] = sc * v;
             if (TAN) L.ptan[at_] = sc * tv;
+        }
+    }
+    if constexpr (JK) {
+        // sums of the lane points' rows by tag, one distinct tag at a time: lane
+        // k adds up bin k of the points that carry it.  (A group of very many
+        // tags leaves the loop and adds point by point.)
+        const int tag = act ? (int)L.lane.w[(p0 + lane) * 2 + 1] : 0;
+        const double wl = (VAR && act) ? LWT[lane] : 1.0;
+        uint64_t todo = (uint64_t)__ballot(act && tag >= 1 && tag <= L.nsamp);
+        auto value = [&](int k, int j) __attribute__((always_inline)) -> double {
+            if (VAR) return LWT[j] * reinterpret_cast<const double*>(hist)[k * 64 + j];
+            return (double)reinterpret_cast<const uint32_t*>(hist)[k * 64 + j];
+        };
+        for (int round = 0; round < 8 && todo; round++) {
+            const int t = __builtin_amdgcn_readlane(tag, __builtin_ctzll(todo));
+            const uint64_t mine = (uint64_t)__ballot(tag == t) & todo;
+            todo &= ~mine;
+            double* r = L.jacc + ((int64_t)m * (L.nsamp + 1) + t) * K;
+            for (int k0 = 0; k0 < K; k0 += 64) {
+                const int k = k0 + lane;
+                double sum = 0.0;
+                for (int c = 0; c < 64; c++) {
+                    const int j = (c + lane) & 63;  // a bank per lane
+                    if (((mine >> j) & 1) && k < K) sum += value(k, j);
+                }
+                if (k < K && sum != 0.0) __hip_atomic_fetch_add(r + k, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        if (todo && ((todo >> lane) & 1)) {
+            double* r = L.jacc + ((int64_t)m * (L.nsamp + 1) + tag) * K;
+            for (int k = 0; k < K; k++) {
+                const double v = VAR ? wl * reinterpret_cast<const double*>(hist)[k * 64 + lane]
+                                     : (double)reinterpret_cast<const uint32_t*>(hist)[k * 64 + lane];
+                if (v != 0.0) __hip_atomic_fetch_add(r + k, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
         }
     }
     if constexpr (MODE == kModeObj || MODE == kModeJac) {
@@ -953,7 +1035,7 @@ int launch_tiles_mode(const TileArgs& A, int waves, int64_t items, int smem, int
         if (var == 2) return launch_tiles_v<MODE, 2, 0>(A, waves, items, smem, s);
         return var ? launch_tiles_v<MODE, 1, 0>(A, waves, items, smem, s)
                    : launch_tiles_v<MODE, 0, 0>(A, waves, items, smem, s);
-    } else if constexpr (MODE == kModeXYZ) {
+    } else if constexpr (MODE == kModeXYZ || MODE == kModeJack) {
         return var ? launch_tiles_v<MODE, 1, 0>(A, waves, items, smem, s)
                    : launch_tiles_v<MODE, 0, 0>(A, waves, items, smem, s);
     } else if constexpr (MODE == kModeTan) {

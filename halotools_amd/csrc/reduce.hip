@@ -405,6 +405,23 @@ int launch_pack_jack(const double* w, const int32_t* tags, int64_t n, int nsamp,
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+// Row 0 of each mock's table as the sum of its subsample rows (every point
+// carries one tag), in a fixed order: 8 strided sums per bin, then those in order.
+__global__ void __launch_bounds__(256) k_jack_total(double* __restrict__ acc, int nr, int nsamp) {
+    __shared__ double sh[8][32];
+    double* t = acc + (int64_t)blockIdx.y * (nsamp + 1) * nr;
+    const int b = blockIdx.x * 32 + (threadIdx.x & 31), g = threadIdx.x >> 5;
+    double sum = 0.0;
+    if (b < nr)
+        for (int s = 1 + g; s <= nsamp; s += 8) sum += t[(int64_t)s * nr + b];
+    sh[g][threadIdx.x & 31] = sum;
+    __syncthreads();
+    if (g == 0 && b < nr) {
+        for (int i = 1; i < 8; i++) sum += sh[i][threadIdx.x];
+        t[b] = sum;
+    }
+}
+
 // Inclusive prefix of every (mock, subsample) table row: over bins (1-D) or
 // over pi then rp (2-D, the order of k_reduce_s2).
 __global__ void __launch_bounds__(256) k_jack_prefix(double* __restrict__ acc, int nr, int np) {
@@ -440,14 +457,15 @@ __global__ void k_jack_out(const double* __restrict__ acc, int64_t nb, int nsamp
     }
 }
 
-int launch_jack_finish(double* acc, int nr, int np, int nmocks, int nsamp, double* out, hipStream_t s) {
+int launch_jack_finish(double* acc, int nr, int np, int nmocks, int nsamp, bool total, double* out, hipStream_t s) {
+    if (total) hipLaunchKernelGGL(k_jack_total, dim3((nr + 31) / 32, nmocks), dim3(256), 0, s, acc, nr, nsamp);
     const int64_t rows = (int64_t)nmocks * (nsamp + 1);
     const int64_t nb = np > 0 ? (int64_t)nr * np : nr;
     hipLaunchKernelGGL(k_jack_prefix, dim3((unsigned)rows), dim3(np > 0 ? 256 : 64), 0, s, acc, nr, np);
-    const int64_t total = rows * nb;
-    int64_t blocks = (total + 255) / 256;
+    const int64_t cells = rows * nb;
+    int64_t blocks = (cells + 255) / 256;
     if (blocks > 8192) blocks = 8192;
-    hipLaunchKernelGGL(k_jack_out, dim3((unsigned)blocks), dim3(256), 0, s, acc, nb, nsamp, total, out);
+    hipLaunchKernelGGL(k_jack_out, dim3((unsigned)blocks), dim3(256), 0, s, acc, nb, nsamp, cells, out);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

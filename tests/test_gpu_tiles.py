@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from oracle import mesh as ORC
+from tests.test_gpu_autodiff import _seam_pair
 
 pytestmark = pytest.mark.gpu
 
@@ -121,3 +122,24 @@ def test_jacobian_rows_and_seam_corrections(gpu, same, monkeypatch):
     monkeypatch.setenv("HALOPAIR_NO_TILES", "1")
     for a, b in zip(got, run()):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("tags", ["one", "slabs", "random"])
+@pytest.mark.parametrize("n", [1, 64, 65, 700])
+def test_jackknife_tables(mo, n, tags):
+    rng = np.random.default_rng(n)
+    p = rng.uniform(0, 1, (n, 3))
+    r = 0.1
+    if n > 20:
+        x, y, r = _seam_pair()  # its two orders fall into different bins
+        p[3], p[17] = [x, 0.5, 0.5], [y, 0.5, 0.5]
+    ns = {"one": 1, "slabs": 4, "random": 40}[tags]
+    t = {"one": np.ones(n, int), "slabs": 1 + np.minimum((p[:, 0] * 4).astype(int), 3),
+         "random": rng.integers(1, ns + 1, n)}[tags]
+    rb = np.array([0.5 * r, r, 0.2])
+    got = mo.npairs_jackknife_3d(p, p, rb, t, t, ns, period=1.0)
+    assert np.array_equal(got, ORC.npairs_jackknife(p, p, rb, t, t, ns, period=1.0))
+    w = rng.uniform(0.1, 1, n)
+    got = mo.npairs_jackknife_3d(p, p, rb, t, t, ns, period=1.0, weights1=w, weights2=w)
+    ref = ORC.npairs_jackknife(p, p, rb, t, t, ns, period=1.0, weights1=w, weights2=w)
+    np.testing.assert_allclose(got, ref, rtol=0, atol=1e-12 * ref.max())
