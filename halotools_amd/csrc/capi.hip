@@ -214,6 +214,8 @@ struct Plan {
     int row_stride[2] = {4, 4}, row_nw[2] = {0, 0};
     size_t o_keys_row = 0;           // row-major keys of a side sorted in both orders
     bool tiles = false;  // matrix-core kernels on the curve-ordered rows
+    bool small = false;  // ... built by the launches for small requests
+    size_t o_small[2] = {0, 0};
     size_t o_crow[2] = {0, 0}, o_cw[2] = {0, 0}, o_cperm[2] = {0, 0}, o_cubes[2] = {0, 0};
     bool sym = false;  // auto-count (unweighted or tangent): symmetric evaluation
     int crep = 1;
@@ -494,6 +496,10 @@ static int make_plan(const hp_request* r, int kind, Plan& P, bool tiles = true) 
     P.o_geom = take(sizeof(MockGeom) * (size_t)P.M);
     P.o_er = take(P.tr.e.size() * 8);
     P.o_ep = take(P.tp.e.size() * 8);
+    if (P.tiles) {
+        P.tr.t.clear();  // the general kernels' tables stay behind
+        P.tp.t.clear();
+    }
     P.o_tr = take(P.tr.t.size() * sizeof(TabEntry));
     P.o_tp = take(P.tp.t.size() * sizeof(TabEntry));
     P.o_ttr = take(P.ttr.t.size() * 4);
@@ -534,12 +540,19 @@ static int make_plan(const hp_request* r, int kind, Plan& P, bool tiles = true) 
             if (o == kRowMajor) S.cs = take((size_t)(P.total_cells + 1) * 4);
         }
     }
+    P.small = P.tiles && P.M == 1 && P.n[0] <= kSmallMax && P.n[s2] <= kSmallMax && P.bits_hilbert <= 2 * kSmallBits;
     if (P.tiles) {
         for (int s = 0; s <= s2; s++) {
             const size_t n = (size_t)std::max<int64_t>(P.n[s], 1);
             nmax = std::max<int64_t>(nmax, (int64_t)n);
             P.o_crow[s] = take(n * 32);
             if (P.weighted()) P.o_cw[s] = take(n * 8 * (size_t)P.nw);
+            if (P.small) {
+                // keys, keys and indices after the first pass, digit counts of both
+                const size_t tiles_ = (n + kSmallTile - 1) / kSmallTile;
+                P.o_small[s] = take(n * 12 + 2 * tiles_ * kSmallDigits * 4 + 256);
+                continue;
+            }
             P.o_cperm[s] = take(n * 4);
             // packed input rows, for column inputs
             if ((s == 0 ? r->stride1 : r->stride2) <= 1) P.o_rows[s] = take(n * 32);
@@ -694,9 +707,9 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
     char* ws = static_cast<char*>(r->workspace);
     const MockGeom* dgeom = reinterpret_cast<const MockGeom*>(ws + P.o_geom);
 
-    if (launch_store_bytes(ws, P.consts.data(), P.consts.size(), s)) return fail("constant upload failed");
     int32_t* status = r->status ? r->status : reinterpret_cast<int32_t*>(ws + P.o_status);
-    launch_fill_u32(reinterpret_cast<uint32_t*>(status), 0u, 1, s);
+    if (launch_store_bytes(ws, P.consts.data(), P.consts.size(), reinterpret_cast<uint32_t*>(status), s))
+        return fail("constant upload failed");
 
     const double* X[2] = {r->x1, P.same ? r->x1 : r->x2};
     // doubles between consecutive points of each sample's coordinate arrays
@@ -727,6 +740,7 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
         return fail("event record failed");
     // matrix-core kernels: one curve-ordered copy of each side, the stream side's with its cubes
     SortedSide curve[2] = {};
+    SmallBuild small = {};
     for (int sd = 0; P.tiles && sd < (P.same ? 1 : 2); sd++) {
         SortedSide& C = curve[sd];
         C.x = reinterpret_cast<double*>(ws + P.o_crow[sd]);
@@ -734,6 +748,25 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
         C.perm = reinterpret_cast<uint32_t*>(ws + P.o_cperm[sd]);
         C.cubes = P.o_cubes[sd] ? reinterpret_cast<uint2*>(ws + P.o_cubes[sd]) : nullptr;
         C.xs = 4;
+        if (P.small) {
+            SmallSide& S = small.s[sd];
+            const size_t n = (size_t)std::max<int64_t>(P.n[sd], 1);
+            C.perm = nullptr;
+            S.x = X[sd];
+            S.y = Y[sd];
+            S.z = Z[sd];
+            S.w = P.weighted() ? W[sd] : nullptr;
+            S.xs = XS[sd];
+            S.n = (int)P.n[sd];
+            S.counts = reinterpret_cast<uint32_t*>(ws + P.o_small[sd]);
+            S.key0 = S.counts + 2 * ((n + kSmallTile - 1) / kSmallTile) * kSmallDigits;
+            S.key1 = S.key0 + n;
+            S.val1 = S.key1 + n;
+            S.row = C.x;
+            S.ow = C.w;
+            S.cubes = C.cubes;
+            continue;
+        }
         PackedRows rows;
         // (N, 3) rows are gathered in place, columns through packed rows
         if (XS[sd] == 1 && P.n[sd] > 0) rows.p = reinterpret_cast<double*>(ws + P.o_rows[sd]);
@@ -744,6 +777,15 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
         if (build_curve_side(dgeom, P.M, sd, X[sd], Y[sd], Z[sd], P.weighted() ? W[sd] : nullptr, P.nw, P.n[sd],
                              P.total_cells, P.bits_hilbert, sb, st, C, status, s, rows, XS[sd]))
             return fail("cell build launch failed");
+    }
+    if (P.small) {
+        small.geom = dgeom;
+        small.status = status;
+        small.nw = P.nw;
+        small.total_cells = P.total_cells;
+        small.clear = P.counts ? reinterpret_cast<uint32_t*>(ws + P.o_pcount) : nullptr;
+        small.clear_words = P.counts ? (int64_t)P.crep * P.nb_count * 2 : 0;
+        if (build_curve_small(small, P.same ? 1 : 2, s)) return fail("cell build launch failed");
     }
     for (int sd = 0; sd < 2; sd++) {
         for (int o = 0; o < 2; o++) {
@@ -784,7 +826,11 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
 
     const int s2 = P.same ? 0 : 1;
     int32_t* gm0 = reinterpret_cast<int32_t*>(ws + P.o_gm[0]);
-    if (launch_group_mock(dgeom, P.M, 0, gm0, P.ngroups[0], s)) return fail("group table launch failed");
+    if (P.M > 1 || !P.tiles) {
+        if (launch_group_mock(dgeom, P.M, 0, gm0, P.ngroups[0], s)) return fail("group table launch failed");
+    } else {
+        gm0 = nullptr;  // one mock
+    }
 
     PairLaunch L;
     std::memset(&L, 0, sizeof(L));
@@ -842,7 +888,7 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
         launch_fill_u32(reinterpret_cast<uint32_t*>(corr), 0u, P.n[0] * (int64_t)P.Kr * 2, s);
     }
     L.crep = P.crep;
-    if (P.counts)
+    if (P.counts && !P.small)
         launch_fill_u32(reinterpret_cast<uint32_t*>(L.pcount), 0u, (int64_t)P.M * P.crep * P.nb_count * 2, s);
     int rc = 0;
     phase.begin("halopair: pair kernels");
@@ -861,7 +907,11 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
         // pass B: lanes are sample 2, the stream is sample 1 (same arithmetic,
         // (x1 - x2shift) - x2, with the shift applied to the sample-1 point)
         int32_t* gm1 = reinterpret_cast<int32_t*>(ws + P.o_gm[1]);
-        if (launch_group_mock(dgeom, P.M, s2, gm1, P.ngroups[s2], s)) return fail("group table launch failed");
+        if (P.M > 1 || !P.tiles) {
+            if (launch_group_mock(dgeom, P.M, s2, gm1, P.ngroups[s2], s)) return fail("group table launch failed");
+        } else {
+            gm1 = nullptr;
+        }
         PairLaunch B = L;
         B.mode = kModeJac;
         B.swap = 1;

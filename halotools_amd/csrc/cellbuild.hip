@@ -22,24 +22,27 @@ namespace hp {
 // ----------------------------------------------------------------- utilities
 struct ByteChunk {
     uint32_t* dst;
+    uint32_t* clear;      // a word to set to zero, or null
     uint32_t nwords;
-    uint32_t words[508];  // 2032 bytes of payload per launch
+    uint32_t words[900];  // 3600 bytes of payload per launch (kernel arguments hold 4 KB)
 };
 
 __global__ void k_store_words(const ByteChunk c) {
     for (uint32_t i = threadIdx.x; i < c.nwords; i += blockDim.x) c.dst[i] = c.words[i];
+    if (c.clear && threadIdx.x == 0) *c.clear = 0u;
 }
 
-int launch_store_bytes(void* dst, const void* src, size_t nbytes, hipStream_t s) {
+int launch_store_bytes(void* dst, const void* src, size_t nbytes, uint32_t* clear, hipStream_t s) {
     // Carries a host blob into device memory through kernel arguments: no
     // memcpy API, so the upload is legal inside HIP-graph capture.
     const size_t nwords_total = (nbytes + 3) / 4;
     const uint8_t* bytes = static_cast<const uint8_t*>(src);
-    for (size_t w0 = 0; w0 < nwords_total; w0 += 508) {
+    for (size_t w0 = 0; w0 < nwords_total; w0 += 900) {
         ByteChunk c;
-        const size_t nw = nwords_total - w0 < 508 ? nwords_total - w0 : 508;
+        const size_t nw = nwords_total - w0 < 900 ? nwords_total - w0 : 900;
         c.dst = static_cast<uint32_t*>(dst) + w0;
         c.nwords = static_cast<uint32_t>(nw);
+        c.clear = w0 == 0 ? clear : nullptr;
         const size_t b0 = w0 * 4;
         const size_t nb = (b0 + nw * 4 <= nbytes) ? nw * 4 : nbytes - b0;
         std::memset(c.words, 0, sizeof(c.words));
@@ -562,6 +565,156 @@ int build_curve_side(const MockGeom* geom, int nmocks, int side, const double* x
     hipLaunchKernelGGL(k_gather_curve, dim3(nb), dim3(256), 0, s, out.perm, keys, n, geom, nmocks, side, x, y, z, xs,
                        rows, w, nw, out.x, out.w, out.cubes);
     return check("curve");
+}
+
+// ------------------------------------------------------------ small builds
+// A request of up to kSmallMax points a side is bound by launches and their
+// latency: three kernels build both sides (20k x 20k: 166 -> 54 us of kernels
+// per call, of which the pair kernel is 26).  At most 64 tiles a side, so a
+// workgroup adds up the digit counts of the tiles before its own itself (no
+// scan launch), and the first pass counts the second pass's digits by atomics.
+__global__ void __launch_bounds__(256) k_small_keys(const SmallBuild B) {
+    __shared__ uint32_t h[kSmallDigits];
+    const SmallSide& S = B.s[blockIdx.y];
+    const MockGeom& G = B.geom[0];
+    const int tile = blockIdx.x, tiles = (S.n + kSmallTile - 1) / kSmallTile;
+    // clear what later kernels add into: this side's cubes, the second pass's
+    // counts, the caller's accumulators
+    const int64_t gt = (int64_t)blockIdx.x * 256 + threadIdx.x, gn = (int64_t)gridDim.x * 256;
+    if (S.cubes)
+        for (int64_t i = gt; i < B.total_cells; i += gn) S.cubes[i] = make_uint2(0x7fffffffu, 0u);
+    for (int64_t i = gt; i < (int64_t)tiles * kSmallDigits; i += gn) S.counts[(int64_t)tiles * kSmallDigits + i] = 0u;
+    if (blockIdx.y == 0)
+        for (int64_t i = gt; i < B.clear_words; i += gn) B.clear[i] = 0u;
+    if (tile >= tiles) return;
+    for (int i = threadIdx.x; i < kSmallDigits; i += 256) h[i] = 0u;
+    __syncthreads();
+    const int hb = G.mbits, hn = 1 << hb;
+    bool bad = false;
+#pragma unroll
+    for (int r = 0; r < kSmallTile / 256; r++) {
+        const int p = tile * kSmallTile + r * 256 + threadIdx.x;
+        if (p >= S.n) break;
+        const double v[3] = {S.x[p * S.xs], S.y[p * S.xs], S.z[p * S.xs]};
+        uint32_t c[3];
+        for (int d = 0; d < 3; d++) {
+            bool dummy = false;
+            if (!(v[d] == v[d]) || v[d] > 1.0e300 || v[d] < -1.0e300) bad = true;
+            if (G.pbc && (v[d] < 0.0 || v[d] > G.period[d])) bad = true;
+            c[d] = (uint32_t)cell_index(v[d], G.inv_hcell[d], hn, dummy, G.period[d], 0);
+        }
+        const uint32_t key = hilbert3(c[0], c[1], c[2], hb);
+        S.key0[p] = key;
+        atomicAdd(&h[key & (kSmallDigits - 1)], 1u);
+    }
+    if (bad) atomicOr(B.status, 1);
+    __syncthreads();
+    for (int i = threadIdx.x; i < kSmallDigits; i += 256) S.counts[(int64_t)tile * kSmallDigits + i] = h[i];
+}
+
+// One stable pass over 9 bits; PASS 1 (the last) writes the points' rows and
+// their cubes' first and last rows.
+template <int PASS>
+__global__ void __launch_bounds__(kSmallDigits) k_small_scatter(const SmallBuild B) {
+    constexpr int WAVES = kSmallDigits / 64, kRounds = kSmallTile / WAVES / 64;
+    __shared__ uint32_t wcnt[WAVES][kSmallDigits];
+    __shared__ uint32_t scan[kSmallDigits];
+    const SmallSide& S = B.s[blockIdx.y];
+    const int tile = blockIdx.x, tiles = (S.n + kSmallTile - 1) / kSmallTile;
+    if (tile >= tiles) return;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int tn = min(kSmallTile, S.n - tile * kSmallTile);
+    const uint32_t* kin = PASS ? S.key1 : S.key0;
+    for (int w = 0; w < WAVES; w++) wcnt[w][tid] = 0u;
+    // this digit's keys in earlier tiles, and in all
+    const uint32_t* cnt = S.counts + (int64_t)PASS * tiles * kSmallDigits + tid;
+    uint32_t before = 0, all = 0;
+#pragma unroll 8
+    for (int t = 0; t < tiles; t++) {
+        const uint32_t c = cnt[(int64_t)t * kSmallDigits];
+        before += t < tile ? c : 0u;
+        all += c;
+    }
+    __syncthreads();
+    const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    uint32_t kk[kRounds], rk[kRounds];
+#pragma unroll
+    for (int r = 0; r < kRounds; r++) {
+        const int li = wv * (kSmallTile / WAVES) + r * 64 + lane;
+        const bool valid = li < tn;
+        const uint32_t key = valid ? kin[tile * kSmallTile + li] : 0u;
+        const uint32_t d = key & (kSmallDigits - 1);
+        uint64_t peers = __ballot(valid);
+#pragma unroll
+        for (int bit = 0; bit < kSmallBits; bit++) {
+            const bool on = (d >> bit) & 1u;
+            const uint64_t bm = __ballot(on);
+            peers &= on ? bm : ~bm;
+        }
+        const uint32_t ahead = (uint32_t)__popcll(peers & lt);
+        const uint32_t c = valid ? wcnt[wv][d] : 0u;
+        __builtin_amdgcn_wave_barrier();
+        if (valid && ahead == 0) wcnt[wv][d] = c + (uint32_t)__popcll(peers);
+        __builtin_amdgcn_wave_barrier();
+        kk[r] = key;
+        rk[r] = c + ahead;
+    }
+    // exclusive prefix of the digit totals, then this digit's place for every wave
+    scan[tid] = all;
+    __syncthreads();
+    for (int off = 1; off < kSmallDigits; off <<= 1) {
+        const uint32_t u = tid >= off ? scan[tid - off] : 0u;
+        __syncthreads();
+        scan[tid] += u;
+        __syncthreads();
+    }
+    uint32_t run = scan[tid] - all + before;
+    for (int w = 0; w < WAVES; w++) {
+        const uint32_t c = wcnt[w][tid];
+        wcnt[w][tid] = run;
+        run += c;
+    }
+    __syncthreads();
+    const MockGeom& G = B.geom[0];
+#pragma unroll
+    for (int r = 0; r < kRounds; r++) {
+        const int li = wv * (kSmallTile / WAVES) + r * 64 + lane;
+        if (li >= tn) break;
+        const uint32_t pos = wcnt[wv][kk[r] & (kSmallDigits - 1)] + rk[r];
+        if (PASS == 0) {
+            const uint32_t high = kk[r] >> kSmallBits;
+            S.key1[pos] = high;
+            S.val1[pos] = (uint32_t)(tile * kSmallTile + li);
+            atomicAdd(S.counts + ((int64_t)tiles + pos / kSmallTile) * kSmallDigits + (high & (kSmallDigits - 1)), 1u);
+        } else {
+            const int64_t p = S.val1[tile * kSmallTile + li];
+            const double px = S.x[p * S.xs], py = S.y[p * S.xs], pz = S.z[p * S.xs];
+            reinterpret_cast<double4*>(S.row)[pos] = make_double4(px, py, pz, __longlong_as_double((long long)p));
+            if (S.ow)
+                for (int k = 0; k < B.nw; k++) S.ow[(int64_t)pos * B.nw + k] = S.w[p * B.nw + k];
+            if (S.cubes) {
+                bool bad = false;
+                const int hn = 1 << G.mbits, sh = G.mbits - G.cbits;
+                const int cx = cell_index(px, G.inv_hcell[0], hn, bad, G.period[0], 0) >> sh;
+                const int cy = cell_index(py, G.inv_hcell[1], hn, bad, G.period[1], 0) >> sh;
+                const int cz = cell_index(pz, G.inv_hcell[2], hn, bad, G.period[2], 0) >> sh;
+                uint2* c = S.cubes + (((((int64_t)cx << G.cbits) + cy) << G.cbits) + cz);
+                atomicMin(&c->x, pos);
+                atomicMax(&c->y, pos + 1u);
+            }
+        }
+    }
+}
+
+int build_curve_small(const SmallBuild& b, int sides, hipStream_t s) {
+    const int most = sides > 1 ? (b.s[0].n > b.s[1].n ? b.s[0].n : b.s[1].n) : b.s[0].n;
+    const unsigned tiles = (unsigned)((most + kSmallTile - 1) / kSmallTile);
+    // (at least a few workgroups for the clearing)
+    hipLaunchKernelGGL(k_small_keys, dim3(tiles < 16 ? 16 : tiles, sides), dim3(256), 0, s, b);
+    if (tiles == 0) return check("small");
+    hipLaunchKernelGGL(k_small_scatter<0>, dim3(tiles, sides), dim3(kSmallDigits), 0, s, b);
+    hipLaunchKernelGGL(k_small_scatter<1>, dim3(tiles, sides), dim3(kSmallDigits), 0, s, b);
+    return check("small");
 }
 
 }  // namespace hp

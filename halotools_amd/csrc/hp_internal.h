@@ -118,7 +118,8 @@ struct PackedRows {
 
 // ------------------------------------------------------------------ launchers
 // cellbuild.hip
-int launch_store_bytes(void* dst, const void* src, size_t nbytes, hipStream_t s);
+// clear: a word set to zero by the way, or null
+int launch_store_bytes(void* dst, const void* src, size_t nbytes, uint32_t* clear, hipStream_t s);
 int launch_fill_u32(uint32_t* p, uint32_t v, int64_t n, hipStream_t s);
 int launch_group_mock(const MockGeom* g, int nmocks, int side, int32_t* group_mock,
                       int64_t ngroups_total, hipStream_t s);
@@ -153,6 +154,32 @@ int build_sorted_side(const MockGeom* geom, int nmocks, int side, Order order,
 int build_curve_side(const MockGeom* geom, int nmocks, int side, const double* x, const double* y, const double* z,
                      const double* w, int nw, int64_t n, int64_t total_cells, int key_bits, SortBufs sb, SortTiles st,
                      SortedSide out, int32_t* status, hipStream_t s, PackedRows rows, int64_t xs);
+
+// The same for small one-mock requests (at most kSmallMax points a side), both
+// sides in each launch: keys and digit counts, two 9-bit passes, the second
+// writing the rows; clears the cubes and `clear` (clear_words words) on the way.
+constexpr int kSmallMax = 1 << 16;
+constexpr int kSmallTile = 1024;       // keys per workgroup
+constexpr int kSmallBits = 9, kSmallDigits = 1 << kSmallBits;
+struct SmallSide {
+    const double *x, *y, *z, *w;
+    int64_t xs;
+    int n;
+    uint32_t *key0, *key1, *val1;  // keys in input order; keys (high digit) and indices after the first pass
+    uint32_t* counts;              // [2][tiles][kSmallDigits]
+    double *row, *ow;
+    uint2* cubes;
+};
+struct SmallBuild {
+    SmallSide s[2];
+    const MockGeom* geom;
+    int32_t* status;
+    int nw;
+    int64_t total_cells;
+    uint32_t* clear;
+    int64_t clear_words;
+};
+int build_curve_small(const SmallBuild& b, int sides, hipStream_t s);
 
 // pairs.hip
 struct PairLaunch {

@@ -237,7 +237,7 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
 
     constexpr int SD = SWAP ? 1 : 0;  // the lanes' side of the geometry, the stream's
     constexpr int SS = 1 - SD;
-    const int m = uni(L.group_mock[g]);
+    const int m = L.group_mock ? uni(L.group_mock[g]) : 0;
     const_geom* const geom = (const_geom*)(L.geom + m);
     const int64_t gl = g - geom->group_off[SD];
     const int64_t p0 = geom->p_off[SD] + gl * kGroup;

@@ -83,17 +83,18 @@ __global__ void __launch_bounds__(256) k_reduce_s2(const T* __restrict__ s1, int
 
 // Counts: the pair kernel accumulates each mock's histogram directly (exact
 // integer atomics); this turns it into the reference's cumulative counts.
-__global__ void __launch_bounds__(256) k_prefix_counts(const uint64_t* __restrict__ acc, int nr, int np, int crep,
+constexpr int kPrefixThreads = 1024;  // two or three replica loads per thread instead of nine (7.2 -> 4 us)
+__global__ void __launch_bounds__(kPrefixThreads) k_prefix_counts(const uint64_t* __restrict__ acc, int nr, int np, int crep,
                                                        int64_t* __restrict__ out) {
-    __shared__ uint64_t sh[256];
+    __shared__ uint64_t sh[kPrefixThreads];
     const int m = blockIdx.x;
     const int nb = np > 0 ? nr * np : nr;
     const uint64_t* a = acc + (int64_t)m * crep * nb;
     int64_t* o = out + (int64_t)m * nb;
     // replica sums: threads split over (bin, replica stripe), then the stripes
     // are added in LDS (integer sums: exact in any order)
-    const int nbt = nb < 256 ? nb : 256;
-    const int rstride = 256 / nbt;
+    const int nbt = nb < kPrefixThreads ? nb : kPrefixThreads;
+    const int rstride = kPrefixThreads / nbt;
     for (int b0 = 0; b0 < nb; b0 += nbt) {
         const int t = threadIdx.x;
         const int b = b0 + t % nbt;
@@ -132,7 +133,7 @@ __global__ void __launch_bounds__(256) k_prefix_counts(const uint64_t* __restric
 }
 
 int launch_prefix_counts(const uint64_t* acc, int nr, int np, int nmocks, int crep, int64_t* counts, hipStream_t s) {
-    hipLaunchKernelGGL(k_prefix_counts, dim3(nmocks), dim3(256), 0, s, acc, nr, np, crep, counts);
+    hipLaunchKernelGGL(k_prefix_counts, dim3(nmocks), dim3(kPrefixThreads), 0, s, acc, nr, np, crep, counts);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
