@@ -143,3 +143,24 @@ def test_jackknife_tables(mo, n, tags):
     got = mo.npairs_jackknife_3d(p, p, rb, t, t, ns, period=1.0, weights1=w, weights2=w)
     ref = ORC.npairs_jackknife(p, p, rb, t, t, ns, period=1.0, weights1=w, weights2=w)
     np.testing.assert_allclose(got, ref, rtol=0, atol=1e-12 * ref.max())
+
+
+@pytest.mark.parametrize("n1,n2", [(1023, 1025), (1024, 1), (1, 65536), (65535, 1024), (65536, 65536), (65537, 3000)])
+def test_small_builds_agree_with_general(mo, gpu, n1, n2, monkeypatch):
+    # edges of the sort tiles and of the range that the small build takes; two samples of
+    # unlike sizes, half of the first in one spot (one digit holds whole tiles)
+    import torch
+    p1, p2 = _points(n1, "uniform", 3), _points(n2, "seam", 4)
+    p1[: n1 // 2] = p1[0]
+    w1, w2 = np.arange(1.0, n1 + 1) % 7 + 1, np.arange(1.0, n2 + 1) % 5 + 1
+    t1, t2, u1, u2 = [torch.as_tensor(a, device=gpu) for a in (p1, p2, w1, w2)]
+    rb = RB[:6]   # (sums of small whole numbers: exact in any order)
+
+    def run():
+        return (mo.npairs_3d(t1, t2, rb, period=L), mo.npairs_per_object_3d(t1, t2, rb, period=L),
+                mo.marked_npairs_3d(t1, t2, rb, period=L, weights1=u1, weights2=u2, weight_func_id=1),
+                mo.npairs_projected(t1, t1, rb, 2.0, period=L) if n1 < 2000 else mo.npairs_3d(t2, t2, rb, period=L))
+    got = run()
+    monkeypatch.setenv("HALOPAIR_NO_TILES", "1")
+    for a, b in zip(got, run()):
+        assert torch.equal(torch.as_tensor(a), torch.as_tensor(b))
