@@ -412,6 +412,8 @@ static int make_plan(const hp_request* r, int kind, Plan& P, bool tiles = true) 
         const double nlane = (double)std::max(nm[0], nm[1]);
         int mb = 1;
         while (mb < kHilbertMaxBits && (double)(1 << mb) < 1.25 * cbrt(nlane)) mb++;
+        // a small request's keys fit two 9-bit passes (up to one point per cell)
+        if (P.tiles && P.M == 1 && nlane <= (double)(P.same ? kSmallMaxSame : kSmallMax)) mb = std::min(mb, 2 * kSmallBits / 3);
         G.mbits = mb;
         for (int d = 0; d < 3; d++) G.inv_hcell[d] = (double)(1 << mb) / G.period[d];
         if (P.tiles) {
@@ -540,7 +542,8 @@ static int make_plan(const hp_request* r, int kind, Plan& P, bool tiles = true) 
             if (o == kRowMajor) S.cs = take((size_t)(P.total_cells + 1) * 4);
         }
     }
-    P.small = P.tiles && P.M == 1 && P.n[0] <= kSmallMax && P.n[s2] <= kSmallMax && P.bits_hilbert <= 2 * kSmallBits;
+    const int64_t most = P.same ? kSmallMaxSame : kSmallMax;
+    P.small = P.tiles && P.M == 1 && P.n[0] <= most && P.n[s2] <= most && P.bits_hilbert <= 2 * kSmallBits;
     if (P.tiles) {
         for (int s = 0; s <= s2; s++) {
             const size_t n = (size_t)std::max<int64_t>(P.n[s], 1);
@@ -549,7 +552,7 @@ static int make_plan(const hp_request* r, int kind, Plan& P, bool tiles = true) 
             if (P.weighted()) P.o_cw[s] = take(n * 8 * (size_t)P.nw);
             if (P.small) {
                 // keys, keys and indices after the first pass, digit counts of both
-                const size_t tiles_ = (n + kSmallTile - 1) / kSmallTile;
+                const size_t tiles_ = (n + 1023) / 1024;
                 P.o_small[s] = take(n * 12 + 2 * tiles_ * kSmallDigits * 4 + 256);
                 continue;
             }
@@ -759,7 +762,7 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
             S.xs = XS[sd];
             S.n = (int)P.n[sd];
             S.counts = reinterpret_cast<uint32_t*>(ws + P.o_small[sd]);
-            S.key0 = S.counts + 2 * ((n + kSmallTile - 1) / kSmallTile) * kSmallDigits;
+            S.key0 = S.counts + 2 * ((n + 1023) / 1024) * kSmallDigits;
             S.key1 = S.key0 + n;
             S.val1 = S.key1 + n;
             S.row = C.x;
@@ -782,6 +785,7 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
         small.geom = dgeom;
         small.status = status;
         small.nw = P.nw;
+        small.tile = small_tile(std::max(P.n[0], P.n[P.same ? 0 : 1]));
         small.total_cells = P.total_cells;
         small.clear = P.counts ? reinterpret_cast<uint32_t*>(ws + P.o_pcount) : nullptr;
         small.clear_words = P.counts ? (int64_t)P.crep * P.nb_count * 2 : 0;

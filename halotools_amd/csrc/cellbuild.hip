@@ -568,32 +568,34 @@ int build_curve_side(const MockGeom* geom, int nmocks, int side, const double* x
 }
 
 // ------------------------------------------------------------ small builds
-// A request of up to kSmallMax points a side is bound by launches and their
-// latency: three kernels build both sides (20k x 20k: 166 -> 54 us of kernels
-// per call, of which the pair kernel is 26).  At most 64 tiles a side, so a
-// workgroup adds up the digit counts of the tiles before its own itself (no
-// scan launch), and the first pass counts the second pass's digits by atomics.
-__global__ void __launch_bounds__(256) k_small_keys(const SmallBuild B) {
+// A small request is bound by launches and their latency: three kernels build
+// both sides (20k x 20k: 166 -> 71 us of kernels per call, of which the pair
+// kernel is 25).  At most 128 tiles a side, so a workgroup adds up the digit
+// counts of the tiles before its own itself (no scan launch), and the first
+// pass counts the second pass's digits by atomics.
+template <int TILE>
+__global__ void __launch_bounds__(TILE / 4) k_small_keys(const SmallBuild B) {
+    constexpr int NT = TILE / 4;
     __shared__ uint32_t h[kSmallDigits];
     const SmallSide& S = B.s[blockIdx.y];
     const MockGeom& G = B.geom[0];
-    const int tile = blockIdx.x, tiles = (S.n + kSmallTile - 1) / kSmallTile;
+    const int tile = blockIdx.x, tiles = (S.n + TILE - 1) / TILE;
     // clear what later kernels add into: this side's cubes, the second pass's
     // counts, the caller's accumulators
-    const int64_t gt = (int64_t)blockIdx.x * 256 + threadIdx.x, gn = (int64_t)gridDim.x * 256;
+    const int64_t gt = (int64_t)blockIdx.x * NT + threadIdx.x, gn = (int64_t)gridDim.x * NT;
     if (S.cubes)
         for (int64_t i = gt; i < B.total_cells; i += gn) S.cubes[i] = make_uint2(0x7fffffffu, 0u);
     for (int64_t i = gt; i < (int64_t)tiles * kSmallDigits; i += gn) S.counts[(int64_t)tiles * kSmallDigits + i] = 0u;
     if (blockIdx.y == 0)
         for (int64_t i = gt; i < B.clear_words; i += gn) B.clear[i] = 0u;
     if (tile >= tiles) return;
-    for (int i = threadIdx.x; i < kSmallDigits; i += 256) h[i] = 0u;
+    for (int i = threadIdx.x; i < kSmallDigits; i += NT) h[i] = 0u;
     __syncthreads();
     const int hb = G.mbits, hn = 1 << hb;
     bool bad = false;
 #pragma unroll
-    for (int r = 0; r < kSmallTile / 256; r++) {
-        const int p = tile * kSmallTile + r * 256 + threadIdx.x;
+    for (int r = 0; r < TILE / NT; r++) {
+        const int p = tile * TILE + r * NT + threadIdx.x;
         if (p >= S.n) break;
         const double v[3] = {S.x[p * S.xs], S.y[p * S.xs], S.z[p * S.xs]};
         uint32_t c[3];
@@ -609,21 +611,21 @@ __global__ void __launch_bounds__(256) k_small_keys(const SmallBuild B) {
     }
     if (bad) atomicOr(B.status, 1);
     __syncthreads();
-    for (int i = threadIdx.x; i < kSmallDigits; i += 256) S.counts[(int64_t)tile * kSmallDigits + i] = h[i];
+    for (int i = threadIdx.x; i < kSmallDigits; i += NT) S.counts[(int64_t)tile * kSmallDigits + i] = h[i];
 }
 
 // One stable pass over 9 bits; PASS 1 (the last) writes the points' rows and
 // their cubes' first and last rows.
-template <int PASS>
+template <int PASS, int TILE>
 __global__ void __launch_bounds__(kSmallDigits) k_small_scatter(const SmallBuild B) {
-    constexpr int WAVES = kSmallDigits / 64, kRounds = kSmallTile / WAVES / 64;
+    constexpr int WAVES = kSmallDigits / 64, kRounds = TILE / WAVES / 64;
     __shared__ uint32_t wcnt[WAVES][kSmallDigits];
     __shared__ uint32_t scan[kSmallDigits];
     const SmallSide& S = B.s[blockIdx.y];
-    const int tile = blockIdx.x, tiles = (S.n + kSmallTile - 1) / kSmallTile;
+    const int tile = blockIdx.x, tiles = (S.n + TILE - 1) / TILE;
     if (tile >= tiles) return;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int tn = min(kSmallTile, S.n - tile * kSmallTile);
+    const int tn = min(TILE, S.n - tile * TILE);
     const uint32_t* kin = PASS ? S.key1 : S.key0;
     for (int w = 0; w < WAVES; w++) wcnt[w][tid] = 0u;
     // this digit's keys in earlier tiles, and in all
@@ -640,9 +642,9 @@ __global__ void __launch_bounds__(kSmallDigits) k_small_scatter(const SmallBuild
     uint32_t kk[kRounds], rk[kRounds];
 #pragma unroll
     for (int r = 0; r < kRounds; r++) {
-        const int li = wv * (kSmallTile / WAVES) + r * 64 + lane;
+        const int li = wv * (TILE / WAVES) + r * 64 + lane;
         const bool valid = li < tn;
-        const uint32_t key = valid ? kin[tile * kSmallTile + li] : 0u;
+        const uint32_t key = valid ? kin[tile * TILE + li] : 0u;
         const uint32_t d = key & (kSmallDigits - 1);
         uint64_t peers = __ballot(valid);
 #pragma unroll
@@ -678,16 +680,16 @@ __global__ void __launch_bounds__(kSmallDigits) k_small_scatter(const SmallBuild
     const MockGeom& G = B.geom[0];
 #pragma unroll
     for (int r = 0; r < kRounds; r++) {
-        const int li = wv * (kSmallTile / WAVES) + r * 64 + lane;
+        const int li = wv * (TILE / WAVES) + r * 64 + lane;
         if (li >= tn) break;
         const uint32_t pos = wcnt[wv][kk[r] & (kSmallDigits - 1)] + rk[r];
         if (PASS == 0) {
             const uint32_t high = kk[r] >> kSmallBits;
             S.key1[pos] = high;
-            S.val1[pos] = (uint32_t)(tile * kSmallTile + li);
-            atomicAdd(S.counts + ((int64_t)tiles + pos / kSmallTile) * kSmallDigits + (high & (kSmallDigits - 1)), 1u);
+            S.val1[pos] = (uint32_t)(tile * TILE + li);
+            atomicAdd(S.counts + ((int64_t)tiles + pos / TILE) * kSmallDigits + (high & (kSmallDigits - 1)), 1u);
         } else {
-            const int64_t p = S.val1[tile * kSmallTile + li];
+            const int64_t p = S.val1[tile * TILE + li];
             const double px = S.x[p * S.xs], py = S.y[p * S.xs], pz = S.z[p * S.xs];
             reinterpret_cast<double4*>(S.row)[pos] = make_double4(px, py, pz, __longlong_as_double((long long)p));
             if (S.ow)
@@ -708,12 +710,20 @@ __global__ void __launch_bounds__(kSmallDigits) k_small_scatter(const SmallBuild
 
 int build_curve_small(const SmallBuild& b, int sides, hipStream_t s) {
     const int most = sides > 1 ? (b.s[0].n > b.s[1].n ? b.s[0].n : b.s[1].n) : b.s[0].n;
-    const unsigned tiles = (unsigned)((most + kSmallTile - 1) / kSmallTile);
+    const unsigned tiles = (unsigned)((most + b.tile - 1) / b.tile);
     // (at least a few workgroups for the clearing)
-    hipLaunchKernelGGL(k_small_keys, dim3(tiles < 16 ? 16 : tiles, sides), dim3(256), 0, s, b);
-    if (tiles == 0) return check("small");
-    hipLaunchKernelGGL(k_small_scatter<0>, dim3(tiles, sides), dim3(kSmallDigits), 0, s, b);
-    hipLaunchKernelGGL(k_small_scatter<1>, dim3(tiles, sides), dim3(kSmallDigits), 0, s, b);
+    const dim3 grid0(tiles < 16 ? 16 : tiles, sides), grid(tiles, sides);
+    if (b.tile == 1024) {
+        hipLaunchKernelGGL(k_small_keys<1024>, grid0, dim3(256), 0, s, b);
+        if (tiles == 0) return check("small");
+        hipLaunchKernelGGL((k_small_scatter<0, 1024>), grid, dim3(kSmallDigits), 0, s, b);
+        hipLaunchKernelGGL((k_small_scatter<1, 1024>), grid, dim3(kSmallDigits), 0, s, b);
+    } else {
+        hipLaunchKernelGGL(k_small_keys<2048>, grid0, dim3(512), 0, s, b);
+        if (tiles == 0) return check("small");
+        hipLaunchKernelGGL((k_small_scatter<0, 2048>), grid, dim3(kSmallDigits), 0, s, b);
+        hipLaunchKernelGGL((k_small_scatter<1, 2048>), grid, dim3(kSmallDigits), 0, s, b);
+    }
     return check("small");
 }
 

@@ -155,11 +155,17 @@ int build_curve_side(const MockGeom* geom, int nmocks, int side, const double* x
                      const double* w, int nw, int64_t n, int64_t total_cells, int key_bits, SortBufs sb, SortTiles st,
                      SortedSide out, int32_t* status, hipStream_t s, PackedRows rows, int64_t xs);
 
-// The same for small one-mock requests (at most kSmallMax points a side), both
-// sides in each launch: keys and digit counts, two 9-bit passes, the second
-// writing the rows; clears the cubes and `clear` (clear_words words) on the way.
-constexpr int kSmallMax = 1 << 16;
-constexpr int kSmallTile = 1024;       // keys per workgroup
+// The same for small one-mock requests, both sides in each launch: keys and
+// digit counts, two 9-bit passes, the second writing the rows; clears the cubes
+// and `clear` (clear_words words) on the way.  Two samples gain up to 262,144
+// points a side (131,072 with a quarter as many: 221 -> 159 us a call; 262,144:
+// 254 -> 207), one sample up to 196,608 (131,072: 184 -> 175; at 262,144 the
+// general passes' larger grids win, 225 against 232).
+constexpr int64_t kSmallMax = 1 << 18, kSmallMaxSame = 3 << 16;
+// keys per workgroup: at most 128 tiles a side, whose counts every workgroup
+// adds up (2048-key tiles at 100,000 points: 163 us a call against 160, and
+// 4096-key tiles, 64 workgroups in all, at 262,144: 244 against 232)
+inline int small_tile(int64_t n) { return n <= (1 << 17) ? 1024 : 2048; }
 constexpr int kSmallBits = 9, kSmallDigits = 1 << kSmallBits;
 struct SmallSide {
     const double *x, *y, *z, *w;
@@ -175,6 +181,7 @@ struct SmallBuild {
     const MockGeom* geom;
     int32_t* status;
     int nw;
+    int tile;                      // keys per tile, for both sides
     int64_t total_cells;
     uint32_t* clear;
     int64_t clear_words;
