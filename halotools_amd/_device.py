@@ -298,6 +298,41 @@ def backward_rows(rows, gsuffix, offsets, out=None):
     return grad
 
 
+_BOX_HEAD = 514  # doubles before the shifted rows in hp_enclose's output
+
+
+def enclose_rows(cols1, cols2):
+    """Float64 device columns of both samples shifted by their smallest coordinate
+    and the side of the enclosing cube: (columns1, columns2, side), or None where
+    the columns are not plain float64 device columns with one stride per sample
+    (the caller's elementwise path then runs)."""
+    cols = tuple(cols1) + tuple(cols2)
+    c0 = cols[0]
+    for c in cols:
+        if (type(c) is not torch.Tensor or not c.is_cuda or c.dtype != torch.float64 or c.dim() != 1
+                or c.device != c0.device or c.is_neg() or torch._C._functorch.is_functorch_wrapped_tensor(c)):
+            return None
+    n1, n2 = len(c0), len(cols[3])
+    st1, st2 = c0.stride(0), cols[3].stride(0)
+    if n1 == 0 or n2 == 0 or st1 < 1 or st2 < 1:
+        return None
+    for k in (1, 2):
+        if len(cols[k]) != n1 or cols[k].stride(0) != st1 or len(cols[k + 3]) != n2 or cols[k + 3].stride(0) != st2:
+            return None
+    ptrs = [c.data_ptr() for c in cols]
+    one = ptrs[:3] == ptrs[3:] and n1 == n2 and st1 == st2
+    m = 0 if one else n2
+    need = _BOX_HEAD + 3 * (n1 + m)
+    out = torch.empty(need, dtype=torch.float64, device=c0.device)
+    with torch.cuda.device(c0.device):
+        E.check(E.library().hp_enclose((ctypes.c_void_p * 6)(*ptrs), st1, n1, st2, m, ctypes.c_void_p(out.data_ptr()),
+                                       need, ctypes.c_void_p(torch.cuda.current_stream(c0.device).cuda_stream)))
+        lo, hi = out[:2].tolist()
+    rows1 = RowColumns(out[_BOX_HEAD:_BOX_HEAD + 3 * n1].view(n1, 3).unbind(1))
+    rows2 = rows1 if one else RowColumns(out[_BOX_HEAD + 3 * n1:].view(n2, 3).unbind(1))
+    return rows1, rows2, hi - lo
+
+
 def zheng07_tangent(log_mass, mock_id, logMmin, sigma, out):
     """out[:, 0] = Zheng07 central weights, out[:, 1] = their logMmin
     derivatives, per point of mock mock_id[i] (one library kernel; the same

@@ -1059,6 +1059,23 @@ int hp_marked_backward(const double* rows, int32_t nr, const double* gsuffix, co
     return 0;
 }
 
+int hp_enclose(const double* const* cols, int64_t stride1, int64_t n1, int64_t stride2, int64_t n2, double* out,
+               int64_t out_elems, void* stream) {
+    if (!cols || !out) return fail("null pointer");
+    const bool two = n2 > 0;
+    if (n1 < 1 || n2 < 0 || stride1 < 1 || (two && stride2 < 1)) return fail("bad sizes");
+    for (int d = 0; d < (two ? 6 : 3); d++)
+        if (!cols[d]) return fail("null pointer");
+    if (out_elems < 2 + enclose_scratch() + 3 * (n1 + n2)) return fail("output too small");
+    if ((uintptr_t)out & 15) return fail("output must be 16-byte aligned");
+    double* rows = out + 2 + enclose_scratch();
+    if (launch_enclose(cols, stride1, n1, two ? cols + 3 : cols, two ? stride2 : stride1, two ? n2 : n1, rows,
+                       two ? rows + 3 * n1 : nullptr, out, out + 2, static_cast<hipStream_t>(stream)))
+        return fail("enclose launch failed");
+    g_err.clear();
+    return 0;
+}
+
 int64_t hp_segment_sum_scratch(const int64_t* offsets, int32_t nmocks) {
     if (!offsets || nmocks < 1) return fail("bad arguments");
     for (int m = 0; m < nmocks; m++)

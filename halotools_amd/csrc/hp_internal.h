@@ -246,6 +246,12 @@ int launch_pairs(const PairLaunch& L, hipStream_t s);
 
 // reduce.hip
 int launch_prefix_counts(const uint64_t* acc, int nr, int np, int nmocks, int crep, int64_t* counts, hipStream_t s);
+// Extremes of two samples' coordinates and both samples' rows less the smallest
+// (rows2 null: one sample); scratch: enclose_scratch() doubles, 16-byte aligned.
+int64_t enclose_scratch();
+int launch_enclose(const double* const* c1, int64_t st1, int64_t n1, const double* const* c2, int64_t st2, int64_t n2,
+                   double* rows1, double* rows2, double* lohi, double* scratch, hipStream_t s);
+
 int64_t segment_sum_scratch(const int64_t* offsets, int nmocks);
 int launch_segment_sum(const double* v, const int64_t* offsets, int nmocks, double* out, double* scratch,
                        hipStream_t s);

@@ -470,6 +470,114 @@ int launch_jack_finish(double* acc, int nr, int np, int nmocks, int nsamp, bool 
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+// ------------------------------------------------------- enclosing box
+// The smallest and largest coordinate of two unperiodic samples, and both
+// samples shifted by the smallest (PC/mesh_helpers.py:17-64): a pass over the
+// points for the extremes of each workgroup's share and a pass that writes the
+// shifted (x, y, z) rows.  Bound by its two launches up to ~1e6 points (60k +
+// 240k points: 7 + 6 us, where a min, a max and a subtraction per column and
+// sample were 33 kernels and 250 us a call).  A NaN stays (comparisons with it
+// are false, so it is taken explicitly), as in the library's min and max.
+constexpr int kBoxBlocks = 256;
+
+struct BoxArgs {
+    const double* c[2][3];
+    int64_t st[2], n[2];
+    double* rows[2];      // null: the second sample is the first
+    double2* part;        // kBoxBlocks (smallest, largest)
+    double* lohi;
+};
+
+__device__ __forceinline__ void box_take(double2& e, double v) {
+    e.x = (v < e.x || v != v) ? v : e.x;
+    e.y = (v > e.y || v != v) ? v : e.y;
+}
+
+// over the workgroup; every thread gets the result
+__device__ __forceinline__ double2 box_reduce(double2 e, double2* t) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const double lo = __shfl_xor(e.x, off), hi = __shfl_xor(e.y, off);
+        e.x = (lo < e.x || lo != lo) ? lo : e.x;
+        e.y = (hi > e.y || hi != hi) ? hi : e.y;
+    }
+    const int nw = blockDim.x >> 6;
+    if ((threadIdx.x & 63) == 0) t[threadIdx.x >> 6] = e;
+    __syncthreads();
+    e = t[0];
+    for (int w = 1; w < nw; w++) {
+        const double2 o = t[w];
+        e.x = (o.x < e.x || o.x != o.x) ? o.x : e.x;
+        e.y = (o.y > e.y || o.y != o.y) ? o.y : e.y;
+    }
+    return e;
+}
+
+__global__ void __launch_bounds__(1024) k_box_extremes(const BoxArgs a) {
+    __shared__ double2 t[16];
+    double2 e = make_double2(INFINITY, -INFINITY);
+    const int64_t step = (int64_t)gridDim.x * blockDim.x;
+    for (int sd = 0; sd < 2; sd++) {
+        if (!a.rows[sd]) continue;
+        for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < a.n[sd]; i += step) {
+            const int64_t o = i * a.st[sd];
+            const double x = a.c[sd][0][o], y = a.c[sd][1][o], z = a.c[sd][2][o];
+            box_take(e, x);
+            box_take(e, y);
+            box_take(e, z);
+        }
+    }
+    e = box_reduce(e, t);
+    if (threadIdx.x == 0) a.part[blockIdx.x] = e;
+}
+
+__global__ void __launch_bounds__(kBoxBlocks) k_box_shift(const BoxArgs a, int parts) {
+    __shared__ double2 t[kBoxBlocks / 64];
+    double2 e = threadIdx.x < (unsigned)parts ? a.part[threadIdx.x] : make_double2(INFINITY, -INFINITY);
+    e = box_reduce(e, t);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        a.lohi[0] = e.x;
+        a.lohi[1] = e.y;
+    }
+    const int64_t step = (int64_t)gridDim.x * blockDim.x;
+    for (int sd = 0; sd < 2; sd++) {
+        if (!a.rows[sd]) continue;
+        for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < a.n[sd]; i += step) {
+            const int64_t o = i * a.st[sd];
+            const double x = a.c[sd][0][o], y = a.c[sd][1][o], z = a.c[sd][2][o];
+            a.rows[sd][3 * i] = x - e.x;
+            a.rows[sd][3 * i + 1] = y - e.x;
+            a.rows[sd][3 * i + 2] = z - e.x;
+        }
+    }
+}
+
+int launch_enclose(const double* const* c1, int64_t st1, int64_t n1, const double* const* c2, int64_t st2, int64_t n2,
+                   double* rows1, double* rows2, double* lohi, double* scratch, hipStream_t s) {
+    BoxArgs a;
+    for (int d = 0; d < 3; d++) {
+        a.c[0][d] = c1[d];
+        a.c[1][d] = c2[d];
+    }
+    a.st[0] = st1;
+    a.st[1] = st2;
+    a.n[0] = n1;
+    a.n[1] = n2;
+    a.rows[0] = rows1;
+    a.rows[1] = rows2;
+    a.part = reinterpret_cast<double2*>(scratch);
+    a.lohi = lohi;
+    const int64_t most = rows2 && n2 > n1 ? n2 : n1;
+    int64_t nb = (most + 1023) / 1024, nbs = (most + kBoxBlocks - 1) / kBoxBlocks;
+    if (nb > kBoxBlocks) nb = kBoxBlocks;
+    if (nbs > 2048) nbs = 2048;
+    hipLaunchKernelGGL(k_box_extremes, dim3((unsigned)nb), dim3(1024), 0, s, a);
+    hipLaunchKernelGGL(k_box_shift, dim3((unsigned)nbs), dim3(kBoxBlocks), 0, s, a, (int)nb);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+int64_t enclose_scratch() { return 2 * kBoxBlocks; }
+
 // Zheng07 central occupation of each point and its derivative with respect to
 // logMmin (empirical_models/occupation_models/zheng07_components.py:149-153):
 // u = (log_mass - logMmin[mock]) / sigma, w = 0.5 * (1 + erf(u)),

@@ -21,6 +21,7 @@ import multiprocessing
 import numpy as np
 import torch
 
+from ... import _device as D
 from ...custom_exceptions import HalotoolsError
 
 
@@ -135,8 +136,13 @@ def enclose_in_box(x1, y1, z1, x2, y2, z2, min_size=None):
 
     The subtraction runs in the input dtype (NumPy on the host or torch on the
     device, identical IEEE operations) before anything is converted to float64,
-    which is what the reference does.
+    which is what the reference does.  Float64 device samples take two library
+    kernels instead of an operation per column, with the same values.
     """
+    boxed = D.enclose_rows((x1, y1, z1), (x2, y2, z2)) if isinstance(x1, torch.Tensor) else None
+    if boxed is not None:
+        (x1, y1, z1), (x2, y2, z2), xyzmax = boxed
+        return x1, y1, z1, x2, y2, z2, _box(xyzmax, min_size)
     if isinstance(x1, torch.Tensor):
         arrs = (x1, x2, y1, y2, z1, z2)
         xyzmin = torch.stack([_min(a) for a in arrs]).min()
@@ -147,12 +153,16 @@ def enclose_in_box(x1, y1, z1, x2, y2, z2, min_size=None):
         xyzmax = np.max([np.max(x1), np.max(x2), np.max(y1), np.max(y2), np.max(z1), np.max(z2)]) - xyzmin
     x1, y1, z1 = x1 - xyzmin, y1 - xyzmin, z1 - xyzmin
     x2, y2, z2 = x2 - xyzmin, y2 - xyzmin, z2 - xyzmin
+    return x1, y1, z1, x2, y2, z2, _box(xyzmax, min_size)
+
+
+def _box(xyzmax, min_size):
     Lbox = np.array([xyzmax, xyzmax, xyzmax], dtype=float)
     if min_size is not None:
         min_size = np.atleast_1d(min_size)
         if np.any(Lbox < min_size):
             Lbox[(Lbox < min_size)] = min_size[(Lbox < min_size)]
-    return x1, y1, z1, x2, y2, z2, Lbox
+    return Lbox
 
 
 def default_cell_sizes(approx_cell1_size, approx_cell2_size, default):

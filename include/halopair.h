@@ -227,6 +227,13 @@ int hp_zheng07_tangent(const double* log_mass, const int64_t* mock_id, const dou
 int hp_segment_sum(const double* values, const int64_t* offsets, int32_t nmocks, double* out,
                    double* scratch, int64_t scratch_elems, void* stream);
 
+/* The box of one or two unperiodic samples (PC/mesh_helpers.py:17-64): out[0], out[1] = the smallest and the
+ * largest of all coordinates; the samples less the smallest, as (x, y, z) rows, start at out + 514, sample 2's
+ * after sample 1's.  cols: device pointers x1, y1, z1 (and x2, y2, z2 when n2 > 0), points stride1 / stride2
+ * doubles apart.  out: 514 + 3 * (n1 + n2) doubles on the device, 16-byte aligned; only enqueues work. */
+int hp_enclose(const double* const* cols, int64_t stride1, int64_t n1, int64_t stride2, int64_t n2, double* out,
+               int64_t out_elems, void* stream);
+
 /* Diagnostics (host only, no GPU needed; used by the CPU test-suite). */
 /* The kernels' bucketed bin lookup: out[i] = number of suffix-minimum edges of r2 below d[i];
  * info = {shift, base, table entries, multi}. */

@@ -1,0 +1,66 @@
+"""The fused enclosure of unperiodic device samples and the row contraction of the
+weight gradients, against the elementwise torch operations (equal bit for bit)."""
+import numpy as np
+import pytest
+import torch
+
+from halotools_amd import _device as D
+from halotools_amd.mock_observables.pair_counters import _process as P
+
+pytestmark = pytest.mark.gpu
+
+
+def _sample(n, layout, seed, gpu):
+    p = torch.as_tensor(np.random.default_rng([n, seed]).normal(size=(n, 3)) * 100.0 - 30.0, device=gpu)
+    if layout == "columns":
+        return p.t().contiguous().t()
+    if layout == "sliced":
+        return torch.cat([p, p], dim=1)[:, 1:4]
+    return p
+
+
+@pytest.mark.parametrize("layout", ["rows", "columns", "sliced"])
+@pytest.mark.parametrize("n1,n2", [(1, 0), (1, 1), (63, 1025), (1024, 0), (1025, 64), (300001, 7), (1000, 600000)])
+def test_enclose_equals_elementwise(gpu, monkeypatch, n1, n2, layout):
+    a = _sample(n1, layout, 0, gpu)
+    b = a if n2 == 0 else _sample(n2, "rows", 1, gpu)
+    args = P.columns(a) + P.columns(b)
+    assert D.enclose_rows(args[:3], args[3:]) is not None
+    got = P.enclose_in_box(*args, min_size=[1.0, 900.0, 2.0])
+    monkeypatch.setattr(D, "enclose_rows", lambda *k: None)
+    ref = P.enclose_in_box(*args, min_size=[1.0, 900.0, 2.0])
+    assert all(torch.equal(x, y) for x, y in zip(got[:6], ref[:6])) and np.array_equal(got[6], ref[6])
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
+def test_enclose_of_bad_values(gpu, monkeypatch, bad):
+    a = _sample(3000, "rows", 2, gpu)
+    a[1700, 1] = bad
+    args = P.columns(a) + P.columns(a)
+    got = P.enclose_in_box(*args)
+    monkeypatch.setattr(D, "enclose_rows", lambda *k: None)
+    ref = P.enclose_in_box(*args)
+    assert all(torch.equal(x.isfinite(), y.isfinite()) for x, y in zip(got[:6], ref[:6]))
+    assert np.array_equal(got[6], ref[6], equal_nan=True)
+
+
+def test_other_types_keep_the_elementwise_path(gpu):
+    a = _sample(100, "rows", 3, gpu)
+    f = P.columns(a.float())
+    assert D.enclose_rows(f, f) is None
+    assert D.enclose_rows(P.columns(a), f) is None
+    assert D.enclose_rows(P.columns(a.cpu()), P.columns(a.cpu())) is None
+    n = P.columns(torch._neg_view(a))
+    assert D.enclose_rows(n, n) is None
+
+
+@pytest.mark.parametrize("nr", [1, 2, 20, 31, 32, 33, 64, 80])
+@pytest.mark.parametrize("sizes", [[1], [63], [64], [65], [100, 0, 1, 300], [10] * 130])
+def test_row_contraction(gpu, nr, sizes):
+    # small whole numbers: exact in any order
+    off = np.concatenate([[0], np.cumsum(sizes)])
+    g = torch.Generator(device=gpu).manual_seed(nr)
+    rows = torch.randint(-9, 9, (int(off[-1]), nr), device=gpu, generator=g).double()
+    G = torch.randint(-9, 9, (len(sizes), nr), device=gpu, generator=g).double()
+    ref = (rows * torch.repeat_interleave(G, torch.as_tensor(sizes, device=gpu), dim=0)).sum(dim=1)
+    assert torch.equal(D.backward_rows(rows, G, off), ref)
