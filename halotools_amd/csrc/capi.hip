@@ -199,7 +199,7 @@ struct Plan {
     std::vector<MockGeom> geom;
     Table tr, tp;
     TileTable ttr, ttp;  // radial / rp and pi bins for the matrix-core kernels
-    size_t o_ttr = 0, o_ttp = 0;
+    size_t o_ttr = 0, o_ttp = 0, o_tqueue = 0;
     int parts_sh = 0;    // log2 of their work items per lane group
     int Kr = 0, Kp = 0, nb_count = 0;
     // workspace layout (byte offsets)
@@ -506,6 +506,8 @@ static int make_plan(const hp_request* r, int kind, Plan& P, bool tiles = true) 
     P.o_tp = take(P.tp.t.size() * sizeof(TabEntry));
     P.o_ttr = take(P.ttr.t.size() * 4);
     P.o_ttp = take(P.ttp.t.size() * 4);
+    // zeros: the work queues of the matrix-core kernels, a set per pass
+    if (P.tiles) P.o_tqueue = take(8 * kQueueWords * 4 * (P.rows2 && !P.same ? 2 : 1));
     P.o_tfirst[0] = take(((size_t)P.M + 1) * 4);
     P.o_tfirst[1] = take(((size_t)P.M + 1) * 4);
     const size_t consts_end = off;
@@ -870,7 +872,8 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
     // candidate evaluations per group, only when the caller asked for them
     L.pevals = r->evals ? reinterpret_cast<uint64_t*>(ws + P.o_pevals) : nullptr;
     if (L.pevals) launch_fill_u32(reinterpret_cast<uint32_t*>(L.pevals), 0u, P.ngroups[0] * 2, s);
-    L.queue = reinterpret_cast<uint32_t*>(ws + P.o_queue);
+    // (the matrix-core kernels' queues go up as zeros with the constants, a set per pass)
+    L.queue = reinterpret_cast<uint32_t*>(ws + (P.tiles ? P.o_tqueue : P.o_queue));
     L.mode = mode_of(P, kind, r->wfunc);
     if (kind == HP_NPAIRS_PER_OBJECT_3D) L.orows = r->counts;
     if (P.jack) {
@@ -929,6 +932,7 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
             B.strm = curve[0];
         }
         B.rows = r->rows2;
+        if (P.tiles) B.queue = L.queue + 8 * kQueueWords;
         B.pcount = nullptr;
         B.psum = nullptr;
         B.pevals = nullptr;

@@ -232,10 +232,12 @@ struct PairLaunch {
     int nsamp;
     int unit;              // jackknife: every weight is 1
     int jslots;            // LDS rows per wave for subsample tags (<= kJackSlots)
-    // persistent launches: one work-queue counter per XCD (8 words, zeroed
-    // by launch_pairs before every launch)
+    // persistent launches: one work-queue counter per XCD (8 words, zero before
+    // every launch: launch_pairs clears them, or the constants of the
+    // matrix-core kernels hold them)
     uint32_t* queue;
 };
+constexpr int kQueueWords = 16;  // matrix-core kernels: words from queue to queue (a line each)
 // LDS bytes of one wave of the matrix-core kernels for a mode, or -1 when they
 // have no such mode
 int tile_wave_bytes(int mode, int K, int Kp, int nw, int also);

@@ -169,13 +169,20 @@ static int launch_tiles(const PairLaunch& L, int lds_per_block, hipStream_t s) {
     A.tp_off = xy ? 8 * (int)std::max(L.tr.mask + 1, L.tp.mask + 1) : 0;
     A.tab_bytes = xy ? A.tp_off + 8 * ((int)L.tp.mask + 1) : 8 * ((int)L.tr.mask + 1);
     constexpr int kLdsPerCU = 160 * 1024, reg_waves = 4 * HP_TILE_WPS;
+    // The shape with the most resident waves.  Four waves go one to each SIMD
+    // and stay there; smaller workgroups spread unevenly (1M counts, 16 resident
+    // waves of four: 740 us a call, 15 single ones: 820), so they have to gain a
+    // ninth (per-object rows: 14 singles 1205, 12 in fours 1265; jackknife rows:
+    // 13 singles 1635, 12 in fours 1605).
     int waves = 0, best = 0;
+    double most = 0.0;
     for (const int w : {4, 8, 2, 1}) {
         if (L.waves > 0 && w != L.waves) continue;
         const int bytes = A.tab_bytes + w * A.wave_bytes;
         if (bytes > lds_per_block) continue;
         const int res = std::min(w * (kLdsPerCU / bytes), reg_waves);
-        if (res > best) { best = res; waves = w; }
+        const double score = res * (w >= 4 ? 1.0 : (w == 2 ? 0.85 : 0.9));
+        if (score > most) { most = score; best = res; waves = w; }
     }
     if (best == 0 && L.waves > 0) {
         PairLaunch M = L;
@@ -191,18 +198,32 @@ static int launch_tiles(const PairLaunch& L, int lds_per_block, hipStream_t s) {
         A.tail_sh = 2;
         A.tail = L.ngroups - std::min<int64_t>(L.ngroups, (int64_t)num_compute_units() * best * HP_TILE_TAIL / 16);
     }
-    const int64_t items = (A.tail << A.parts_sh) + ((L.ngroups - A.tail) << A.tail_sh);
+    A.items = (A.tail << A.parts_sh) + ((L.ngroups - A.tail) << A.tail_sh);
+    // chunks of at most 64 items, smaller where the launch has too few of them
+    A.chunk_sh = 6;
+    while (A.chunk_sh > 0 && (A.items >> (A.chunk_sh + 3)) < 4) A.chunk_sh--;
+    const int64_t per_queue = ((A.items + (8 << A.chunk_sh) - 1) >> (A.chunk_sh + 3)) << A.chunk_sh;
+    int64_t blocks = A.items > 0 ? 8 * ((per_queue + waves - 1) / waves) : 0;
+    const int64_t resident = (int64_t)num_compute_units() * (best / waves) & ~(int64_t)7;
+    A.queue = nullptr;
+    A.taken = 0;
+        // (the queues' lines cost more than they give where a wave has one or two items)
+    if (L.queue && resident > 0 && blocks > 2 * resident) {
+        blocks = resident;
+        A.queue = L.queue;
+        A.taken = (uint32_t)(blocks / 8 * waves);
+    }
     const int smem = A.tab_bytes + waves * A.wave_bytes;
     switch (L.mode) {
-        case kModeCount3D: return launch_tiles_mode<kModeCount3D>(A, waves, items, smem, also, var, s);
-        case kModeProj: return launch_tiles_mode<kModeProj>(A, waves, items, smem, also, var, s);
-        case kModeXYZ: return launch_tiles_mode<kModeXYZ>(A, waves, items, smem, also, var, s);
-        case kModeWXYZ: return launch_tiles_mode<kModeWXYZ>(A, waves, items, smem, also, var, s);
-        case kModeObj: return launch_tiles_mode<kModeObj>(A, waves, items, smem, also, var, s);
-        case kModeJack: return launch_tiles_mode<kModeJack>(A, waves, items, smem, also, var, s);
-        case kModeJac: return launch_tiles_mode<kModeJac>(A, waves, items, smem, also, var, s);
-        case kModeTan: return launch_tiles_mode<kModeTan>(A, waves, items, smem, also, var, s);
-        case kModeWSum: return launch_tiles_mode<kModeWSum>(A, waves, items, smem, also, var, s);
+        case kModeCount3D: return launch_tiles_mode<kModeCount3D>(A, waves, blocks, smem, also, var, s);
+        case kModeProj: return launch_tiles_mode<kModeProj>(A, waves, blocks, smem, also, var, s);
+        case kModeXYZ: return launch_tiles_mode<kModeXYZ>(A, waves, blocks, smem, also, var, s);
+        case kModeWXYZ: return launch_tiles_mode<kModeWXYZ>(A, waves, blocks, smem, also, var, s);
+        case kModeObj: return launch_tiles_mode<kModeObj>(A, waves, blocks, smem, also, var, s);
+        case kModeJack: return launch_tiles_mode<kModeJack>(A, waves, blocks, smem, also, var, s);
+        case kModeJac: return launch_tiles_mode<kModeJac>(A, waves, blocks, smem, also, var, s);
+        case kModeTan: return launch_tiles_mode<kModeTan>(A, waves, blocks, smem, also, var, s);
+        case kModeWSum: return launch_tiles_mode<kModeWSum>(A, waves, blocks, smem, also, var, s);
     }
     return -1;
 }

@@ -83,6 +83,10 @@ struct TileArgs {
     int parts_sh;    // log2 of the work items per lane group (cubes dealt round-robin)
     int tail_sh;     // ... of the groups from `tail` on
     int64_t tail;
+    int64_t items;
+    int chunk_sh;    // log2 of the consecutive items one XCD takes
+    uint32_t taken;  // items of each queue that the launch starts on (its waves' first ones)
+    uint32_t* queue; // work queues, one per XCD: items taken beyond those; null: every wave has one item
 };
 
 typedef const __attribute__((address_space(4))) TileArgs kernarg_tile_args;  // as the kernel receives them
@@ -212,837 +216,865 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
     float* const info = reinterpret_cast<float*>(wsm + ST::kInfoOff);  // per sub-group: low x, y, z, high x, y, z; the group's
     double* const LWT = reinterpret_cast<double*>(wsm + A.lw_off);  // lane points' weights: [nw][64]
     unsigned char* const hist = wsm + A.hist_off;
-    for (int i = lane; i < (A.wave_bytes - A.hist_off) / 4; i += 64) reinterpret_cast<uint32_t*>(hist)[i] = 0u;
     __syncthreads();  // no block-level synchronisation below
 
-    // XCD-interleaved block order, as the other count kernels (pairs_kernel.h)
-    int64_t b = blockIdx.x;
-    {
-        constexpr int64_t C = HP_XCD_CHUNK;
-        const int64_t full = ((int64_t)gridDim.x / (8 * C)) * (8 * C);
-        if (b < full) b = ((b >> 3) / C) * (8 * C) + (b & 7) * C + ((b >> 3) % C);
-    }
-    int64_t item = b * WAVES + wid;
-    int psh = A.parts_sh;
-    int64_t g = item >> psh;
-    if (g >= A.tail) {
-        // the last groups go out in smaller items, which even out the end of the launch
-        item -= A.tail << psh;
-        psh = A.tail_sh;
-        g = A.tail + (item >> psh);
-    }
-    const int parts = 1 << psh;
-    const int part = uni((int)(item & (parts - 1)));
-    if (g >= L.ngroups) return;
-
-    constexpr int SD = SWAP ? 1 : 0;  // the lanes' side of the geometry, the stream's
-    constexpr int SS = 1 - SD;
-    const int m = L.group_mock ? uni(L.group_mock[g]) : 0;
-    const_geom* const geom = (const_geom*)(L.geom + m);
-    const int64_t gl = g - geom->group_off[SD];
-    const int64_t p0 = geom->p_off[SD] + gl * kGroup;
-    const int64_t left = geom->n[SD] - gl * kGroup;
-    const int cnt = uni((int)(left < kGroup ? left : kGroup));
-    const bool act = lane < cnt;
-    const float r2xy = geom->r2xy;
-    const float Rz = geom->search[2];
-    const bool sym = L.sym != 0;
-    const bool own = L.own != 0;  // one sample, every ordered pair from its first point: the group's own points come last
-
-    // ---- the group's box, and the lane points relative to its centre
-    float hx, hy, hz;     // half sizes, with the eps margin
-    double cx, cy, cz;
-    double Bf[4], NA[4];  // per sub-group: the tile's B operand and |a|^2
-    uint32_t floor_hi;    // pairs below this high word are evaluated exactly
-    uint32_t floor_pi = 0u;  // ... (rp, pi): below this high word of dz^2
-    {
-        const float INF = __builtin_inff();
-        const float eps = geom->eps;
-        const double4 pr = reinterpret_cast<const double4*>(L.lane.x)[p0 + (act ? lane : 0)];
-        const double px = pr.x, py = pr.y, pz = pr.z;
-        // boxes of the sub-groups, one 16-lane row of the wave each
-        float xl = row_min(act ? f32_down(px) : INF) - eps, xh = row_max(act ? f32_up(px) : -INF) + eps;
-        float yl = row_min(act ? f32_down(py) : INF) - eps, yh = row_max(act ? f32_up(py) : -INF) + eps;
-        float zl = row_min(act ? f32_down(pz) : INF) - eps, zh = row_max(act ? f32_up(pz) : -INF) + eps;
-        const float bxlo = rows_min(xl), bylo = rows_min(yl), bzlo = rows_min(zl);
-        const float bxhi = rows_max(xh), byhi = rows_max(yh), bzhi = rows_max(zh);
-        const float fx = unif(0.5f * (bxlo + bxhi)), fy = unif(0.5f * (bylo + byhi)), fz = unif(0.5f * (bzlo + bzhi));
-        cx = unid((double)fx);
-        cy = unid((double)fy);
-        cz = unid((double)fz);
-        // half sizes of the box about its (rounded) centre; the eps margin covers the rounding
-        hx = unif(0.5f * (bxhi - bxlo));
-        hy = unif(0.5f * (byhi - bylo));
-        hz = unif(0.5f * (bzhi - bzlo));
-        const double ax = px - cx, ay = py - cy, az = pz - cz;
-        const double na = !act ? kFar : (XY ? ax * ax + ay * ay : ax * ax + ay * ay + az * az);
-        if ((lane & 15) == 0) {
-            float* const f = info + (lane >> 4) * 8;
-            f[0] = xl - fx; f[1] = yl - fy; f[2] = zl - fz; f[3] = xh - fx; f[4] = yh - fy; f[5] = zh - fz;
-        }
-        if (lane == 0) {
-            float* const f = info + 32;
-            f[0] = bxlo; f[1] = bylo; f[2] = bzlo; f[3] = bxhi; f[4] = byhi; f[5] = bzhi;
-            // the window of cubes (the eps margin of the box covers the rounding here)
-            const int nc = geom->ndiv[0];
-            const int j0 = geom->pbc ? -nc : 0, j1 = geom->pbc ? 2 * nc - 1 : nc - 1;
-            const float R = geom->search[0];
-            const float ix = (float)geom->inv_cell[0], iy = (float)geom->inv_cell[1], iz = (float)geom->inv_cell[2];
-            const int jx0 = max((int)floorf((bxlo - R) * ix), j0), jx1 = min((int)floorf((bxhi + R) * ix), j1);
-            const int jy0 = max((int)floorf((bylo - R) * iy), j0), jy1 = min((int)floorf((byhi + R) * iy), j1);
-            const int jz0 = max((int)floorf((bzlo - Rz) * iz), j0), jz1 = min((int)floorf((bzhi + Rz) * iz), j1);
-            const int wy = jy1 - jy0 + 1, wz = jz1 - jz0 + 1;
-            int* const w = reinterpret_cast<int*>(info) + 40;
-            w[0] = jx0; w[1] = jy0; w[2] = jz0; w[3] = wy; w[4] = wz;
-            w[5] = (jx1 >= jx0 && wy > 0 && wz > 0) ? (jx1 - jx0 + 1) * wy * wz : 0;
-            f[14] = 1.0f / (float)wy;
-            f[15] = 1.0f / (float)wz;
-            f[16] = (float)geom->cell[0]; f[17] = (float)geom->cell[1]; f[18] = (float)geom->cell[2];
-            // the slot that fills up a tile
-            SX[kStage] = 0.0;
-            SX[kSlots + kStage] = 0.0;
-            SX[2 * kSlots + kStage] = 0.0;
-            SX[3 * kSlots + kStage] = kFar;
-            ID[kStage] = 0u;
-        }
-        if (F64) {
-            const double* w = L.lane.w + (p0 + (act ? lane : 0)) * wst;
-            for (int c = 0; c < nw; c++) LWT[c * 64 + lane] = w[c];
-        }
-        // B operand: lane l holds component l / 16 of point l % 16 of the sub-group
-        SX[lane] = act ? -2.0 * ax : 0.0;
-        SX[kSlots + lane] = act ? -2.0 * ay : 0.0;
-        SX[2 * kSlots + lane] = (act && !XY) ? -2.0 * az : 0.0;
-        SX[3 * kSlots + lane] = na;
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int s = 0; s < 4; s++) {
-            const double v = SX[min(lane >> 4, 2) * kSlots + s * kSub + (lane & 15)];
-            Bf[s] = (lane >> 4) == 3 ? 1.0 : v;
-            NA[s] = SX[3 * kSlots + s * kSub + (lane & 15)];
-        }
-        __builtin_amdgcn_wave_barrier();
-        if (XY) {
-            // the lane points' z, read by the tiles
-            reinterpret_cast<double*>(wsm + A.lw_off)[nw * 64 + lane] = az;
-        }
-        // Rounding of |a|^2 + |b|^2 - 2 a.b: below 2^-47 (|a|^2 + |b|^2), with
-        // |a| <= h (half the box diagonal) and |b| <= h + R.  One unit of the
-        // high word of d is at least 2^-21 d, so the rounding stays within a
-        // unit for d >= 2^-26 S; the floor takes twice that.  The rounding of
-        // the centre and of the periodic shift (2^-52 of the box) is covered
-        // by the second term (dz^2 has only that one).
-        const float h = sqrtf(hx * hx + hy * hy + (XY ? 0.f : hz * hz)) * 1.001f, hr = h + geom->search[0] * 1.001f;
-        const double Lmax = fmax(fmax(geom->period[0], geom->period[1]), geom->period[2]);
-        const double fl2 = Lmax * Lmax * 3.5527136788005009e-15;                          // 2^-48
-        const double fl = (double)(h * h + hr * hr) * 2.9802322387695312e-08 + fl2;      // 2^-25
-        floor_hi = (uint32_t)uni((int)(__double2hiint(fl) + 1));
-        if (XY) floor_pi = (uint32_t)uni((int)(__double2hiint(fl2) + 1));
-    }
-
-    bool self_done = false;
-    const uint32_t sbase = (uint32_t)uni((int)geom->p_off[SS]);
-    const int tlo = (int)A.tr.lo, thi = (int)A.tr.hi;
-    const uint32_t tsh = A.tr.sh3, tmask = A.tr.mask << 3;
-    const int plo = (int)A.tp.lo, phi = (int)A.tp.hi;
-    const uint32_t psh3 = A.tp.sh3, pmask = A.tp.mask << 3, ptab = (uint32_t)A.tp_off;
-    const int lrow = ((lane & 3) << 2) | ((lane >> 2) & 3);   // list position of this lane's A row
-    const int brow = ((lane >> 4) << 2) | (lane & 3);         // list position of the D row this lane's row broadcasts
-    const double* const comp = SX + (lane >> 4) * kSlots;     // the component this lane holds of the A operand
-    // histogram columns: u32 rows of 32 columns, f64 rows of 16 (no two lanes of
-    // one LDS pass on one address); per lane point for object rows and Jacobians
-    const uint32_t col4 = (uint32_t)(lane & 31) * 4u, col8 = (uint32_t)(lane & 15) * 8u;
-    constexpr uint32_t TC = kTanCols, TR = 8u * TC;  // forward mode: columns of the W, dW and count rows
-    const uint32_t tcol8 = (uint32_t)(lane & (TC - 1)) * 8u, tcol4 = (uint32_t)(lane & (2 * TC - 1)) * 4u;
-    const uint32_t ccol = (uint32_t)A.ccol_sh, ccl = (uint32_t)(lane & ((1 << A.ccol_sh) - 1));
-    uint64_t evals = 0;
-    const double* const SWm = F64 ? L.strm.w + (int64_t)sbase * wst : nullptr;
-
-    // Exact bin of the pair (lane point j of the group, staged slot): the first
-    // edge not below the distance, scanning from edge k (and q along pi).  Rarely
-    // taken: what it needs is loaded here, not kept in registers through the
-    // kernel (the empty asm hides that it is the same).  rev: the pair's other
-    // orientation, (x2 + shift) - x1.
-    auto exact_bin = [&](int j, int slot, uint32_t k, uint32_t& kp, bool rev) __attribute__((always_inline)) -> uint32_t {
-        kernarg_tile_args* ap = (kernarg_tile_args*)__builtin_amdgcn_kernarg_segment_ptr();
-        const_geom* gp = geom;
-        asm volatile("" : "+s"(ap), "+s"(gp));
-        const double* ge = reinterpret_cast<const double*>(static_cast<const char*>(ap->L.ws) + ap->L.br.edges_off);
-        const int64_t first = gp->p_off[SD] + gl * kGroup;
-        const double* pl = ap->L.lane.x + (first + min(j, cnt - 1)) * 4;
-        double px = pl[0], py = pl[1], pz = pl[2];
-        const uint32_t id = ID[slot];
-        const int img = (int)(id >> kImgShift);
-        const double* r = ap->L.strm.x + (gp->p_off[SS] + (int64_t)(id & kRowMask)) * 4;
-        const int tx = (img & 3) - 1, ty = ((img >> 2) & 3) - 1, tz = (img >> 4) - 1;
-        double qx = r[0], qy = r[1], qz = r[2];
-        // the image of the stream point lies at q + t L; the reference shifts the sample-1 point
-        if ((!SWAP && !rev) || (SWAP && rev)) {
-            if (tx) px = px - (double)tx * gp->period[0];
-            if (ty) py = py - (double)ty * gp->period[1];
-            if (tz) pz = pz - (double)tz * gp->period[2];
-        } else {
-            if (tx) qx = qx + (double)tx * gp->period[0];
-            if (ty) qy = qy + (double)ty * gp->period[1];
-            if (tz) qz = qz + (double)tz * gp->period[2];
-        }
-        const double dx = px - qx, dy = py - qy, dz = pz - qz;
-        if (XY) {
-            const double* gq = reinterpret_cast<const double*>(static_cast<const char*>(ap->L.ws) + ap->L.bp.edges_off);
-            const double dz2 = dz * dz;
-            uint32_t q = 0;
-            while (gq[q] < dz2) ++q;
-            kp = q;
-            const double dxy = dx * dx + dy * dy;
-            while (ge[k] < dxy) ++k;
-        } else {
-            const double dsq = dx * dx + dy * dy + dz * dz;
-            while (ge[k] < dsq) ++k;
-        }
-        return k;
+    // Work items (lane groups or parts of them) in chunks of consecutive ones:
+    // chunk c belongs to queue c % 8, and the waves of block b work on queue
+    // b % 8 (blocks go to the XCDs round-robin, so an XCD's L2 sees one region;
+    // the counter decides who takes an item, whichever XCD it runs on).  The
+    // waves start on the first items and take the others one by one: with one
+    // item per wave a workgroup's LDS stayed taken until the longest of its
+    // waves was done, 12 of 16 waves alive on average (64-mock step 42.3 ->
+    // 38.4 ms, (rp, pi) counts of 2M points 2220 -> 1900 us, 1M counts 810 ->
+    // 745).  An addition or a look at a counter occupies its line for ~10 ns, so
+    // a wave whose queue is empty ends: moving on to the others made every wave
+    // look at eight lines (+75 us at 20k points); chunks of 64 items keep the
+    // queues even instead (256: 1M counts 763 us).
+    auto item_of = [&](int64_t t) __attribute__((always_inline)) -> int64_t {
+        return ((((t >> A.chunk_sh) << 3) + (blockIdx.x & 7)) << A.chunk_sh) + (t & ((1 << A.chunk_sh) - 1));
     };
-
-    // ---- staged points: deal them to the sub-groups, evaluate the tiles
-    // self: the slots hold the group's own points
-    int qlen = 0;
-    auto process = [&](bool self) __attribute__((always_inline)) {
-        float fx[kDealH], fy[kDealH], fz[kDealH];
-        uint64_t in[kDealH], plain[kDealH];
-#pragma unroll
-        for (int h = 0; h < kDealH; h++) {
-            const int slot = h * 64 + lane;
-            in[h] = (uint64_t)__ballot(slot < qlen);
-            fx[h] = (float)SX[slot];
-            fy[h] = (float)SX[kSlots + slot];
-            fz[h] = (float)SX[2 * kSlots + slot];
-            plain[h] = sym ? (uint64_t)__ballot((ID[slot] >> kImgShift) == (uint32_t)kHere) & in[h] : 0ull;
+    auto take = [&]() __attribute__((always_inline)) -> int64_t {
+        if (!A.queue) return -1;
+        uint32_t c = 0u;
+        if (lane == 0)
+            c = __hip_atomic_fetch_add(A.queue + (blockIdx.x & 7) * kQueueWords, 1u, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+        const int64_t it = item_of((int64_t)A.taken + (uint32_t)uni((int)c));
+        return it < A.items ? it : -1;
+    };
+    int64_t item = item_of((int64_t)(blockIdx.x >> 3) * WAVES + wid);
+    if (item >= A.items) item = take();
+    const int lane0 = lane;
+    for (; item >= 0; item = take()) {
+        // (the empty asm keeps what follows from the lane inside the loop: kept in
+        // registers from item to item, it would push the tiles' into scratch)
+        int lane = lane0;
+        kernarg_tile_args* args = (kernarg_tile_args*)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+v"(lane), "+s"(args));
+        kernarg_tile_args& A = *args;
+        const __attribute__((address_space(4))) PairLaunch& L = A.L;
+        for (int i = lane; i < (A.wave_bytes - A.hist_off) / 4; i += 64) reinterpret_cast<uint32_t*>(hist)[i] = 0u;
+        int psh = A.parts_sh;
+        int64_t g = item >> psh;
+        int64_t it = item;
+        if (g >= A.tail) {
+            // the last groups go out in smaller items, which even out the end of the launch
+            it -= A.tail << psh;
+            psh = A.tail_sh;
+            g = A.tail + (it >> psh);
         }
-        // symmetric counts: the shifted points (once), then the unshifted ones
-        // (twice); other counts: every point once
-        const bool two = sym && !self;
-        for (int sc = two ? 0 : 4; sc < 8; sc++) {
-            const int s = sc & 3;
-            uint64_t mk[kDealH], any = 0;
+        const int parts = 1 << psh;
+        const int part = uni((int)(it & (parts - 1)));
+
+        constexpr int SD = SWAP ? 1 : 0;  // the lanes' side of the geometry, the stream's
+        constexpr int SS = 1 - SD;
+        const int m = L.group_mock ? uni(L.group_mock[g]) : 0;
+        const_geom* const geom = (const_geom*)(L.geom + m);
+        const int64_t gl = g - geom->group_off[SD];
+        const int64_t p0 = geom->p_off[SD] + gl * kGroup;
+        const int64_t left = geom->n[SD] - gl * kGroup;
+        const int cnt = uni((int)(left < kGroup ? left : kGroup));
+        const bool act = lane < cnt;
+        const float r2xy = geom->r2xy;
+        const float Rz = geom->search[2];
+        const bool sym = L.sym != 0;
+        const bool own = L.own != 0;  // one sample, every ordered pair from its first point: the group's own points come last
+
+        // ---- the group's box, and the lane points relative to its centre
+        float hx, hy, hz;     // half sizes, with the eps margin
+        double cx, cy, cz;
+        double Bf[4], NA[4];  // per sub-group: the tile's B operand and |a|^2
+        uint32_t floor_hi;    // pairs below this high word are evaluated exactly
+        uint32_t floor_pi = 0u;  // ... (rp, pi): below this high word of dz^2
+        {
+            const float INF = __builtin_inff();
+            const float eps = geom->eps;
+            const double4 pr = reinterpret_cast<const double4*>(L.lane.x)[p0 + (act ? lane : 0)];
+            const double px = pr.x, py = pr.y, pz = pr.z;
+            // boxes of the sub-groups, one 16-lane row of the wave each
+            float xl = row_min(act ? f32_down(px) : INF) - eps, xh = row_max(act ? f32_up(px) : -INF) + eps;
+            float yl = row_min(act ? f32_down(py) : INF) - eps, yh = row_max(act ? f32_up(py) : -INF) + eps;
+            float zl = row_min(act ? f32_down(pz) : INF) - eps, zh = row_max(act ? f32_up(pz) : -INF) + eps;
+            const float bxlo = rows_min(xl), bylo = rows_min(yl), bzlo = rows_min(zl);
+            const float bxhi = rows_max(xh), byhi = rows_max(yh), bzhi = rows_max(zh);
+            const float fx = unif(0.5f * (bxlo + bxhi)), fy = unif(0.5f * (bylo + byhi)), fz = unif(0.5f * (bzlo + bzhi));
+            cx = unid((double)fx);
+            cy = unid((double)fy);
+            cz = unid((double)fz);
+            // half sizes of the box about its (rounded) centre; the eps margin covers the rounding
+            hx = unif(0.5f * (bxhi - bxlo));
+            hy = unif(0.5f * (byhi - bylo));
+            hz = unif(0.5f * (bzhi - bzlo));
+            const double ax = px - cx, ay = py - cy, az = pz - cz;
+            const double na = !act ? kFar : (XY ? ax * ax + ay * ay : ax * ax + ay * ay + az * az);
+            if ((lane & 15) == 0) {
+                float* const f = info + (lane >> 4) * 8;
+                f[0] = xl - fx; f[1] = yl - fy; f[2] = zl - fz; f[3] = xh - fx; f[4] = yh - fy; f[5] = zh - fz;
+            }
+            if (lane == 0) {
+                float* const f = info + 32;
+                f[0] = bxlo; f[1] = bylo; f[2] = bzlo; f[3] = bxhi; f[4] = byhi; f[5] = bzhi;
+                // the window of cubes (the eps margin of the box covers the rounding here)
+                const int nc = geom->ndiv[0];
+                const int j0 = geom->pbc ? -nc : 0, j1 = geom->pbc ? 2 * nc - 1 : nc - 1;
+                const float R = geom->search[0];
+                const float ix = (float)geom->inv_cell[0], iy = (float)geom->inv_cell[1], iz = (float)geom->inv_cell[2];
+                const int jx0 = max((int)floorf((bxlo - R) * ix), j0), jx1 = min((int)floorf((bxhi + R) * ix), j1);
+                const int jy0 = max((int)floorf((bylo - R) * iy), j0), jy1 = min((int)floorf((byhi + R) * iy), j1);
+                const int jz0 = max((int)floorf((bzlo - Rz) * iz), j0), jz1 = min((int)floorf((bzhi + Rz) * iz), j1);
+                const int wy = jy1 - jy0 + 1, wz = jz1 - jz0 + 1;
+                int* const w = reinterpret_cast<int*>(info) + 40;
+                w[0] = jx0; w[1] = jy0; w[2] = jz0; w[3] = wy; w[4] = wz;
+                w[5] = (jx1 >= jx0 && wy > 0 && wz > 0) ? (jx1 - jx0 + 1) * wy * wz : 0;
+                f[14] = 1.0f / (float)wy;
+                f[15] = 1.0f / (float)wz;
+                f[16] = (float)geom->cell[0]; f[17] = (float)geom->cell[1]; f[18] = (float)geom->cell[2];
+                // the slot that fills up a tile
+                SX[kStage] = 0.0;
+                SX[kSlots + kStage] = 0.0;
+                SX[2 * kSlots + kStage] = 0.0;
+                SX[3 * kSlots + kStage] = kFar;
+                ID[kStage] = 0u;
+            }
+            if (F64) {
+                const double* w = L.lane.w + (p0 + (act ? lane : 0)) * wst;
+                for (int c = 0; c < nw; c++) LWT[c * 64 + lane] = w[c];
+            }
+            // B operand: lane l holds component l / 16 of point l % 16 of the sub-group
+            SX[lane] = act ? -2.0 * ax : 0.0;
+            SX[kSlots + lane] = act ? -2.0 * ay : 0.0;
+            SX[2 * kSlots + lane] = (act && !XY) ? -2.0 * az : 0.0;
+            SX[3 * kSlots + lane] = na;
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const double v = SX[min(lane >> 4, 2) * kSlots + s * kSub + (lane & 15)];
+                Bf[s] = (lane >> 4) == 3 ? 1.0 : v;
+                NA[s] = SX[3 * kSlots + s * kSub + (lane & 15)];
+            }
+            __builtin_amdgcn_wave_barrier();
+            if (XY) {
+                // the lane points' z, read by the tiles
+                reinterpret_cast<double*>(wsm + A.lw_off)[nw * 64 + lane] = az;
+            }
+            // Rounding of |a|^2 + |b|^2 - 2 a.b: below 2^-47 (|a|^2 + |b|^2), with
+            // |a| <= h (half the box diagonal) and |b| <= h + R.  One unit of the
+            // high word of d is at least 2^-21 d, so the rounding stays within a
+            // unit for d >= 2^-26 S; the floor takes twice that.  The rounding of
+            // the centre and of the periodic shift (2^-52 of the box) is covered
+            // by the second term (dz^2 has only that one).
+            const float h = sqrtf(hx * hx + hy * hy + (XY ? 0.f : hz * hz)) * 1.001f, hr = h + geom->search[0] * 1.001f;
+            const double Lmax = fmax(fmax(geom->period[0], geom->period[1]), geom->period[2]);
+            const double fl2 = Lmax * Lmax * 3.5527136788005009e-15;                          // 2^-48
+            const double fl = (double)(h * h + hr * hr) * 2.9802322387695312e-08 + fl2;      // 2^-25
+            floor_hi = (uint32_t)uni((int)(__double2hiint(fl) + 1));
+            if (XY) floor_pi = (uint32_t)uni((int)(__double2hiint(fl2) + 1));
+        }
+
+        bool self_done = false;
+        const uint32_t sbase = (uint32_t)uni((int)geom->p_off[SS]);
+        const int tlo = (int)A.tr.lo, thi = (int)A.tr.hi;
+        const uint32_t tsh = A.tr.sh3, tmask = A.tr.mask << 3;
+        const int plo = (int)A.tp.lo, phi = (int)A.tp.hi;
+        const uint32_t psh3 = A.tp.sh3, pmask = A.tp.mask << 3, ptab = (uint32_t)A.tp_off;
+        const int lrow = ((lane & 3) << 2) | ((lane >> 2) & 3);   // list position of this lane's A row
+        const int brow = ((lane >> 4) << 2) | (lane & 3);         // list position of the D row this lane's row broadcasts
+        const double* const comp = SX + (lane >> 4) * kSlots;     // the component this lane holds of the A operand
+        // histogram columns: u32 rows of 32 columns, f64 rows of 16 (no two lanes of
+        // one LDS pass on one address); per lane point for object rows and Jacobians
+        const uint32_t col4 = (uint32_t)(lane & 31) * 4u, col8 = (uint32_t)(lane & 15) * 8u;
+        constexpr uint32_t TC = kTanCols, TR = 8u * TC;  // forward mode: columns of the W, dW and count rows
+        const uint32_t tcol8 = (uint32_t)(lane & (TC - 1)) * 8u, tcol4 = (uint32_t)(lane & (2 * TC - 1)) * 4u;
+        const uint32_t ccol = (uint32_t)A.ccol_sh, ccl = (uint32_t)(lane & ((1 << A.ccol_sh) - 1));
+        uint64_t evals = 0;
+        const double* const SWm = F64 ? L.strm.w + (int64_t)sbase * wst : nullptr;
+
+        // Exact bin of the pair (lane point j of the group, staged slot): the first
+        // edge not below the distance, scanning from edge k (and q along pi).  Rarely
+        // taken: what it needs is loaded here, not kept in registers through the
+        // kernel (the empty asm hides that it is the same).  rev: the pair's other
+        // orientation, (x2 + shift) - x1.
+        auto exact_bin = [&](int j, int slot, uint32_t k, uint32_t& kp, bool rev) __attribute__((always_inline)) -> uint32_t {
+            kernarg_tile_args* ap = (kernarg_tile_args*)__builtin_amdgcn_kernarg_segment_ptr();
+            const_geom* gp = geom;
+            asm volatile("" : "+s"(ap), "+s"(gp));
+            const double* ge = reinterpret_cast<const double*>(static_cast<const char*>(ap->L.ws) + ap->L.br.edges_off);
+            const int64_t first = gp->p_off[SD] + gl * kGroup;
+            const double* pl = ap->L.lane.x + (first + min(j, cnt - 1)) * 4;
+            double px = pl[0], py = pl[1], pz = pl[2];
+            const uint32_t id = ID[slot];
+            const int img = (int)(id >> kImgShift);
+            const double* r = ap->L.strm.x + (gp->p_off[SS] + (int64_t)(id & kRowMask)) * 4;
+            const int tx = (img & 3) - 1, ty = ((img >> 2) & 3) - 1, tz = (img >> 4) - 1;
+            double qx = r[0], qy = r[1], qz = r[2];
+            // the image of the stream point lies at q + t L; the reference shifts the sample-1 point
+            if ((!SWAP && !rev) || (SWAP && rev)) {
+                if (tx) px = px - (double)tx * gp->period[0];
+                if (ty) py = py - (double)ty * gp->period[1];
+                if (tz) pz = pz - (double)tz * gp->period[2];
+            } else {
+                if (tx) qx = qx + (double)tx * gp->period[0];
+                if (ty) qy = qy + (double)ty * gp->period[1];
+                if (tz) qz = qz + (double)tz * gp->period[2];
+            }
+            const double dx = px - qx, dy = py - qy, dz = pz - qz;
+            if (XY) {
+                const double* gq = reinterpret_cast<const double*>(static_cast<const char*>(ap->L.ws) + ap->L.bp.edges_off);
+                const double dz2 = dz * dz;
+                uint32_t q = 0;
+                while (gq[q] < dz2) ++q;
+                kp = q;
+                const double dxy = dx * dx + dy * dy;
+                while (ge[k] < dxy) ++k;
+            } else {
+                const double dsq = dx * dx + dy * dy + dz * dz;
+                while (ge[k] < dsq) ++k;
+            }
+            return k;
+        };
+
+        // ---- staged points: deal them to the sub-groups, evaluate the tiles
+        // self: the slots hold the group's own points
+        int qlen = 0;
+        auto process = [&](bool self) __attribute__((always_inline)) {
+            float fx[kDealH], fy[kDealH], fz[kDealH];
+            uint64_t in[kDealH], plain[kDealH];
 #pragma unroll
             for (int h = 0; h < kDealH; h++) {
-                mk[h] = !two ? in[h] : (sc < 4 ? in[h] & ~plain[h] : plain[h]);
-                any |= mk[h];
+                const int slot = h * 64 + lane;
+                in[h] = (uint64_t)__ballot(slot < qlen);
+                fx[h] = (float)SX[slot];
+                fy[h] = (float)SX[kSlots + slot];
+                fz[h] = (float)SX[2 * kSlots + slot];
+                plain[h] = sym ? (uint64_t)__ballot((ID[slot] >> kImgShift) == (uint32_t)kHere) & in[h] : 0ull;
             }
-            if (any == 0) {
-                sc |= 3;  // none of this class
-                continue;
-            }
-            uint32_t inc = (two && sc >= 4) ? 2u : 1u;
-            int n;
-            if (self) {
-                n = sym ? min(qlen, (s + 1) * kSub) : qlen;  // the group's points (up to this sub-group)
-                list[lane] = (uint8_t)lane;
-                if (lane < 2 * kSub) list[64 + lane] = (uint8_t)kStage;
-            } else {
-                // staged points near the sub-group's box
-                const float4 b0 = *reinterpret_cast<const float4*>(info + 8 * s);
-                const float2 b1 = *reinterpret_cast<const float2*>(info + 8 * s + 4);
-                n = 0;
+            // symmetric counts: the shifted points (once), then the unshifted ones
+            // (twice); other counts: every point once
+            const bool two = sym && !self;
+            for (int sc = two ? 0 : 4; sc < 8; sc++) {
+                const int s = sc & 3;
+                uint64_t mk[kDealH], any = 0;
 #pragma unroll
                 for (int h = 0; h < kDealH; h++) {
-                    const float gx = fmaxf(0.f, fmaxf(fx[h] - b0.w, b0.x - fx[h]));
-                    const float gy = fmaxf(0.f, fmaxf(fy[h] - b1.x, b0.y - fy[h]));
-                    const float gz = fmaxf(0.f, fmaxf(fz[h] - b1.y, b0.z - fz[h]));
-                    const float gxy = __builtin_fmaf(gy, gy, gx * gx);
-                    const bool near = XY ? (gxy <= r2xy && gz <= Rz) : (__builtin_fmaf(gz, gz, gxy) <= r2xy);
-                    const uint64_t mm = (uint64_t)__ballot(near) & mk[h];
-                    const uint32_t r = __builtin_amdgcn_mbcnt_hi((uint32_t)(mm >> 32),
-                                                                 __builtin_amdgcn_mbcnt_lo((uint32_t)mm, (uint32_t)n));
-                    if (__builtin_amdgcn_inverse_ballot_w64(mm)) list[r] = (uint8_t)(h * 64 + lane);
-                    n += __builtin_popcountll(mm);
+                    mk[h] = !two ? in[h] : (sc < 4 ? in[h] & ~plain[h] : plain[h]);
+                    any |= mk[h];
                 }
-                if (n == 0) continue;
-                if (lane < 2 * kSub) list[n + lane] = (uint8_t)kStage;
-                evals += (uint64_t)n * kSub;
-            }
-            __builtin_amdgcn_wave_barrier();
-            const double bs = s == 0 ? Bf[0] : (s == 1 ? Bf[1] : (s == 2 ? Bf[2] : Bf[3]));
-            const double ns = s == 0 ? NA[0] : (s == 1 ? NA[1] : (s == 2 ? NA[2] : NA[3]));
-            const dbl4 cc = {ns, ns, ns, ns};
-            // this sub-group's lane points: weights and z
-            const int lj = s * kSub + (lane & 15);
-            double lw[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-            if (F64) {
-#pragma unroll
-                for (int c = 0; c < 5; c++)
-                    if (c < nw) lw[c] = LWT[c * 64 + lj];
-            }
-            if (TAN && sym && !self && sc < 4) {
-                // symmetric sums are doubled at the end: a shifted pair counts from both sides
-                lw[0] *= 0.5;
-                lw[1] *= 0.5;
-            }
-            double za = 0.0;
-            if (XY) za = LWT[nw * 64 + lj];
-            // stream weights of the D row this lane's row broadcasts
-            double wn[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-            auto load_weights = [&](int slot) __attribute__((always_inline)) {
-                const double* w = SWm + (uint32_t)((ID[slot] & kRowMask) * (uint32_t)wst);
-#pragma unroll
-                for (int c = 0; c < 5; c++)
-                    if (c < nw) wn[c] = w[c];
-            };
-            if (F64) load_weights(list[brow]);
-            // operands one tile ahead, their slots two
-            double a = comp[list[lrow]];
-            int slot2 = list[kSub + lrow];
-            for (int t0 = 0; t0 < n; t0 += kSub) {
-                // rows: staged points list[t0 + 4 (lane / 16) + i]; columns: the sub-group's points
-                const double a1 = comp[slot2];
-                slot2 = list[t0 + 2 * kSub + lrow];
-                double zb = 0.0, wb[5];
-                if (XY) zb = SX[2 * kSlots + list[t0 + brow]];
-                if (F64) {
-                    // this tile's stream weights were loaded a tile ago
-#pragma unroll
-                    for (int c = 0; c < 5; c++) wb[c] = wn[c];
-                    load_weights(list[t0 + kSub + brow]);
+                if (any == 0) {
+                    sc |= 3;  // none of this class
+                    continue;
                 }
-                // (the next operands' reads go out before the product, which would otherwise
-                // hold them back: its result registers are reused at once)
-                __builtin_amdgcn_sched_barrier(0);
-                const dbl4 D = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bs, cc, 0, 0, 0);
-                a = a1;
-                int hi[4], hp[4];
-                uint2 ent[4], enp[4];
-                uint32_t t[4], k[4], tp[4], kp[4];
-#pragma unroll
-                for (int i = 0; i < 4; i++) hi[i] = __double2hiint(D[i]);
-                bool diag = false;
+                uint32_t inc = (two && sc >= 4) ? 2u : 1u;
+                int n;
                 if (self) {
-                    inc = sym ? 2u : 1u;
-                    diag = t0 == s * kSub;
-                    if (diag) {
-                        // inside a sub-group: ordered pairs, without a point and itself
-                        inc = 1u;
+                    n = sym ? min(qlen, (s + 1) * kSub) : qlen;  // the group's points (up to this sub-group)
+                    list[lane] = (uint8_t)lane;
+                    if (lane < 2 * kSub) list[64 + lane] = (uint8_t)kStage;
+                } else {
+                    // staged points near the sub-group's box
+                    const float4 b0 = *reinterpret_cast<const float4*>(info + 8 * s);
+                    const float2 b1 = *reinterpret_cast<const float2*>(info + 8 * s + 4);
+                    n = 0;
 #pragma unroll
-                        for (int i = 0; i < 4; i++)
-                            if ((lane >> 4) * 4 + i == (lane & 15)) hi[i] = 0x7e000000;
+                    for (int h = 0; h < kDealH; h++) {
+                        const float gx = fmaxf(0.f, fmaxf(fx[h] - b0.w, b0.x - fx[h]));
+                        const float gy = fmaxf(0.f, fmaxf(fy[h] - b1.x, b0.y - fy[h]));
+                        const float gz = fmaxf(0.f, fmaxf(fz[h] - b1.y, b0.z - fz[h]));
+                        const float gxy = __builtin_fmaf(gy, gy, gx * gx);
+                        const bool near = XY ? (gxy <= r2xy && gz <= Rz) : (__builtin_fmaf(gz, gz, gxy) <= r2xy);
+                        const uint64_t mm = (uint64_t)__ballot(near) & mk[h];
+                        const uint32_t r = __builtin_amdgcn_mbcnt_hi((uint32_t)(mm >> 32),
+                                                                     __builtin_amdgcn_mbcnt_lo((uint32_t)mm, (uint32_t)n));
+                        if (__builtin_amdgcn_inverse_ballot_w64(mm)) list[r] = (uint8_t)(h * 64 + lane);
+                        n += __builtin_popcountll(mm);
                     }
+                    if (n == 0) continue;
+                    if (lane < 2 * kSub) list[n + lane] = (uint8_t)kStage;
+                    evals += (uint64_t)n * kSub;
                 }
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const uint32_t off = ((uint32_t)med3i(hi[i], tlo, thi) >> tsh) & tmask;
-                    ent[i] = lds_entry(off);
-                }
-                if (XY) {
-                    double dz[4];
-                    dz[0] = row_bcast<0>(zb) - za;
-                    dz[1] = row_bcast<1>(zb) - za;
-                    dz[2] = row_bcast<2>(zb) - za;
-                    dz[3] = row_bcast<3>(zb) - za;
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        hp[i] = __double2hiint(dz[i] * dz[i]);
-                        const uint32_t off = (((uint32_t)med3i(hp[i], plo, phi) >> psh3) & pmask) | ptab;
-                        enp[i] = lds_entry(off);
-                    }
-                }
-#pragma unroll
-                for (int i = 0; i < 4; i++) sub_borrow(ent[i].x, (uint32_t)hi[i], ent[i].y, t[i], k[i]);
-                uint32_t tm = min(min(t[0], t[1]), min(t[2], t[3]));
-                const int hm = min(min(hi[0], hi[1]), min(hi[2], hi[3]));
-                bool odd = tm <= 2u || hm < (int)floor_hi;
-                if (XY) {
-#pragma unroll
-                    for (int i = 0; i < 4; i++) sub_borrow(enp[i].x, (uint32_t)hp[i], enp[i].y, tp[i], kp[i]);
-                    const uint32_t pm = min(min(tp[0], tp[1]), min(tp[2], tp[3]));
-                    const int qm = min(min(hp[0], hp[1]), min(hp[2], hp[3]));
-                    odd = odd || pm <= 2u || qm < (int)floor_pi;
-                }
-                if (__builtin_expect((uint64_t)__ballot(odd) != 0, 0)) {
-#pragma unroll 1
-                    for (int i = 0; i < 4; i++) {
-                        const uint32_t ti = i == 0 ? t[0] : (i == 1 ? t[1] : (i == 2 ? t[2] : t[3]));
-                        const int hv = i == 0 ? hi[0] : (i == 1 ? hi[1] : (i == 2 ? hi[2] : hi[3]));
-                        const uint32_t ek = i == 0 ? ent[0].y : (i == 1 ? ent[1].y : (i == 2 ? ent[2].y : ent[3].y));
-                        bool oi = ti <= 2u || hv < (int)floor_hi;
-                        if (XY) {
-                            const uint32_t pi = i == 0 ? tp[0] : (i == 1 ? tp[1] : (i == 2 ? tp[2] : tp[3]));
-                            const int hq = i == 0 ? hp[0] : (i == 1 ? hp[1] : (i == 2 ? hp[2] : hp[3]));
-                            oi = (oi || pi <= 2u || hq < (int)floor_pi) && hv < 0x7e000000;
-                        }
-                        if (oi) {
-                            const int slot = list[t0 + (lane >> 4) * 4 + i];
-                            const uint32_t kb = hv < (int)floor_hi || ek == 0u ? 0u : ek - 1u;
-                            uint32_t kq = 0u;
-                            uint32_t kk = exact_bin(s * kSub + (lane & 15), slot, kb, kq, false);
-                            if (MODE == kModeJac && !SWAP && L.corr != nullptr) {
-                                // Auto-count with one set of weights: the sample-2 rows take
-                                // the pair's other orientation, which across the periodic seam
-                                // may round into another bin; those disagreements are recorded,
-                                // so rows2 = rows1 + corr (as pairs_kernel.h does for every
-                                // shifted pair; only these can differ).
-                                const uint32_t id = ID[slot];
-                                uint32_t dummy = 0u;
-                                const uint32_t kr = exact_bin(s * kSub + (lane & 15), slot, kb, dummy, true);
-                                if (kr != kk && (id >> kImgShift) != (uint32_t)kHere && s * kSub + (lane & 15) < cnt) {
-                                    const int64_t sr = (int64_t)sbase + (int64_t)(id & kRowMask);
-                                    const int64_t q = __double_as_longlong(L.strm.x[sr * 4 + 3]);
-                                    double* crow = L.corr + q * K;
-                                    if (kk < (uint32_t)K)
-                                        __hip_atomic_fetch_add(crow + kk, lw[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                                    if (kr < (uint32_t)K)
-                                        __hip_atomic_fetch_add(crow + kr, -lw[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                                }
-                            }
-                            if constexpr (JK) {
-                                // A pair of two tags gives half of its weight to each.  The rows
-                                // give all of an ordered pair's to its lane point's tag, which is
-                                // the same where the pair's other order lands in the same bin;
-                                // across the periodic seam it may not, and half moves over.
-                                const uint32_t id = ID[slot];
-                                uint32_t dummy = 0u;
-                                const uint32_t kr = exact_bin(lj, slot, kb, dummy, true);
-                                if (kr != kk && (id >> kImgShift) != (uint32_t)kHere && lj < cnt) {
-                                    const double* wi = L.lane.w + (p0 + lj) * 2;
-                                    const double v = 0.5 * wi[0] * L.strm.w[((int64_t)sbase + (int64_t)(id & kRowMask)) * 2];
-                                    const int t = (int)wi[1];
-                                    double* r = L.jacc + ((int64_t)m * (L.nsamp + 1) + t) * K;
-                                    if (t >= 1 && t <= L.nsamp) {
-                                        if (kk < (uint32_t)K)
-                                            __hip_atomic_fetch_add(r + kk, -v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                                        if (kr < (uint32_t)K)
-                                            __hip_atomic_fetch_add(r + kr, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                                    }
-                                }
-                            }
-#pragma unroll
-                            for (int u = 0; u < 4; u++)
-                                if (i == u) {
-                                    k[u] = kk;
-                                    if (XY) kp[u] = kq;
-                                }
-                        }
-                    }
-                }
-                // ---- accumulate
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    // the row's stream weights (all lanes: a broadcast reads none that is masked off)
-                    double sw[5];
-                    if constexpr (F64) {
-#pragma unroll
-                        for (int c = 0; c < 5; c++)
-                            sw[c] = c >= nw ? 0.0
-                                            : (i == 0 ? row_bcast<0>(wb[c])
-                                                      : (i == 1 ? row_bcast<1>(wb[c])
-                                                                : (i == 2 ? row_bcast<2>(wb[c]) : row_bcast<3>(wb[c]))));
-                    }
-                    if constexpr (MODE == kModeCount3D) {
-                        __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hist + ((k[i] << 7) + col4)), inc,
-                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    } else if constexpr (MODE == kModeProj) {
-                        // beyond pi_max: the trash row
-                        const uint32_t kk = kp[i] == 0u ? k[i] : (uint32_t)K;
-                        __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hist + ((kk << 7) + col4)), inc,
-                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    } else if constexpr (MODE == kModeXYZ || MODE == kModeWXYZ) {
-                        // one [K][Kp] histogram per wave; pairs beyond an edge skip it
-                        if (k[i] < (uint32_t)K && kp[i] < (uint32_t)Kp) {
-                            const uint32_t cell = __umul24(k[i], (uint32_t)Kp) + kp[i];
-                            if constexpr (MODE == kModeXYZ) {
-                                __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hist) + ((cell << ccol) + ccl), inc, __ATOMIC_RELAXED,
-                                                       __HIP_MEMORY_SCOPE_WORKGROUP);
-                            } else {
-                                const double v = PROD ? lw[0] * sw[0] : wfunc_eval(L.wfunc, lw, sw);
-                                __hip_atomic_fetch_add(reinterpret_cast<double*>(hist) + cell, v, __ATOMIC_RELAXED,
-                                                       __HIP_MEMORY_SCOPE_WORKGROUP);
-                            }
-                        }
-                    } else if constexpr (MODE == kModeObj || (JK && !VAR)) {
-                        __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hist + ((k[i] << 8) + (uint32_t)lj * 4u)), 1u,
-                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    } else {
-                        if constexpr (MODE == kModeJac || JK) {
-                            __hip_atomic_fetch_add(reinterpret_cast<double*>(hist + ((k[i] << 9) + (uint32_t)lj * 8u)),
-                                                   sw[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                        } else if constexpr (MODE == kModeTan) {
-                            // pair terms w_i w_j and t_i w_j + w_i t_j (t = dw/dtheta); the
-                            // group's own pairs: ordered ones inside a sub-group count half
-                            if (k[i] < (uint32_t)K) {
-                                double wj = sw[0], tj = sw[1];
-                                if (diag) {
-                                    wj *= 0.5;
-                                    tj *= 0.5;
-                                }
-                                const double v = lw[0] * wj;
-                                const double tv = __builtin_fma(lw[0], tj, lw[1] * wj);
-                                unsigned char* const r = hist + __umul24(k[i], ALSO ? 3 * TR : 2 * TR);
-                                __hip_atomic_fetch_add(reinterpret_cast<double*>(r + tcol8), v, __ATOMIC_RELAXED,
-                                                       __HIP_MEMORY_SCOPE_WORKGROUP);
-                                __hip_atomic_fetch_add(reinterpret_cast<double*>(r + TR + tcol8), tv, __ATOMIC_RELAXED,
-                                                       __HIP_MEMORY_SCOPE_WORKGROUP);
-                                if (ALSO)
-                                    __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(r + 2 * TR + tcol4), inc,
-                                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                            }
-                        } else if constexpr (MODE == kModeWSum) {
-                            const double v = PROD ? lw[0] * sw[0] : wfunc_eval(L.wfunc, lw, sw);
-                            __hip_atomic_fetch_add(reinterpret_cast<double*>(hist + ((k[i] << 7) + col8)), v,
-                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                        }
-                        if constexpr (ALSO && MODE != kModeTan)
-                            __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(wsm + A.cnt_off + ((k[i] << 7) + col4)), 1u,
-                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    }
-                }
-            }
-            __builtin_amdgcn_wave_barrier();
-        }
-        // what was not dealt moves to the front
-        const int rest = self ? 0 : max(qlen - kDeal, 0);
-        if (rest > 0 && lane < rest) {
-            const int f = kDeal + lane;
-            const double x = SX[f], y = SX[kSlots + f], z = SX[2 * kSlots + f], nn = SX[3 * kSlots + f];
-            const uint32_t id = ID[f];
-            SX[lane] = x;
-            SX[kSlots + lane] = y;
-            SX[2 * kSlots + lane] = z;
-            SX[3 * kSlots + lane] = nn;
-            ID[lane] = id;
-        }
-        __builtin_amdgcn_wave_barrier();
-        qlen = rest;
-    };
-
-    // ---- the cubes of the curve near the group.  A lane takes one cube of the
-    // window and looks up the stretch of rows it holds; the stretches of 64 cubes
-    // form one list of rows, which is walked 64 rows at a time: a scan over the
-    // starts gives each lane its stretch.  Symmetric counts drop the rows before
-    // the group's end here (unshifted cubes), a whole stretch at a time.
-    const double4* const SR = reinterpret_cast<const double4*>(L.strm.x) + sbase;
-    int cube0 = -64;                // the next 64 cubes of the window
-    int cimg = 0;                   // the lane's cube: its image
-    bool seam = false;              // some cube of the list is a periodic image
-    int pre = 0, end = 0, run = 0;  // the lane's stretch: its place [pre, end) in the list, first row - pre
-    int at = 0, total = 0;          // list position of the next rows, rows in the list
-    // the next 64 rows: false when the group has no more.  The list is made
-    // rarely: what that needs is loaded here.
-    auto next = [&]() __attribute__((always_inline)) -> bool {
-        at += 64;
-        while (at >= total) {
-            const_geom* gp = geom;
-            asm volatile("" : "+s"(gp));
-            const int cb = gp->cbits, nc = 1 << cb;  // cubes per dimension
-            const int* const w = reinterpret_cast<const int*>(info) + 40;
-            const int wy = w[3], wz = w[4], ncubes = uni(w[5]);
-            cube0 += 64;
-            if ((cube0 << psh) + part >= ncubes) return false;
-            // cube ci of the window: z fastest (quotients from reciprocals: exact
-            // for the few thousand cubes of a window, and one more test for more)
-            const int ci = ((cube0 + lane) << psh) + part;
-            int cxy = (int)((float)ci * info[47]);
-            int jz = ci - cxy * wz;
-            if (jz < 0) { jz += wz; cxy--; }
-            if (jz >= wz) { jz -= wz; cxy++; }
-            int jx = (int)((float)cxy * info[46]);
-            int jy = cxy - jx * wy;
-            if (jy < 0) { jy += wy; jx--; }
-            if (jy >= wy) { jy -= wy; jx++; }
-            jx += w[0];
-            jy += w[1];
-            jz += w[2];
-            const float cxf = info[48], cyf = info[49], czf = info[50];
-            const float gx = fmaxf(0.f, fmaxf((float)jx * cxf - info[35], info[32] - (float)(jx + 1) * cxf));
-            const float gy = fmaxf(0.f, fmaxf((float)jy * cyf - info[36], info[33] - (float)(jy + 1) * cyf));
-            const float gz = fmaxf(0.f, fmaxf((float)jz * czf - info[37], info[34] - (float)(jz + 1) * czf));
-            at = 0;
-            total = 0;
-            const bool has = ci < ncubes && (XY ? gx * gx + gy * gy : gx * gx + gy * gy + gz * gz) <= r2xy;
-            if ((uint64_t)__ballot(has) == 0) continue;
-            // image: 0, 1, 2 for -L, 0, +L per dimension, two bits each
-            const int ux = (jx >> cb) + 1, uy = (jy >> cb) + 1, uz = (jz >> cb) + 1;
-            cimg = ux | (uy << 2) | (uz << 4);
-            int len = 0;
-            run = 0;
-            if (has) {
-                const int cm = nc - 1;
-                const uint2 c = (L.strm.cubes + gp->cell_off)[(uint32_t)(((((jx & cm) << cb) + (jy & cm)) << cb) + (jz & cm))];
-                run = (int)c.x;
-                if (sym && cimg == kHere) run = max(run, (int)(gp->p_off[SD] + gl * kGroup + cnt));
-                len = max((int)c.y - run, 0);
-            }
-            seam = (uint64_t)__ballot(len > 0 && cimg != kHere) != 0;
-            pre = wave_prefix(len);
-            total = __builtin_amdgcn_readlane(pre, 63);
-            end = len > 0 ? pre : -1;
-            pre -= len;
-            run -= pre + (int)sbase;
-        }
-        return true;
-    };
-    // this lane's row of the list (relative to the mock's first) and its image;
-    // a row past the end repeats the last one
-    auto fetch = [&](uint32_t& jj, int& img) __attribute__((always_inline)) {
-        mark[lane] = 0;
-        __builtin_amdgcn_wave_barrier();
-        if (pre < at + 64 && end > at) mark[max(pre - at, 0)] = (uint8_t)lane;
-        __builtin_amdgcn_wave_barrier();
-        const int sg = wave_scan_max((int)mark[lane]) << 2;
-        jj = (uint32_t)(min(at + lane, total - 1) + __builtin_amdgcn_ds_bpermute(sg, run));
-        img = seam ? __builtin_amdgcn_ds_bpermute(sg, cimg) : kHere;
-    };
-    const uint32_t own0 = (uint32_t)(p0 - (int64_t)sbase);  // the group's first row, in one sample
-    bool more = next();
-    double4 row = make_double4(0.0, 0.0, 0.0, 0.0);
-    uint32_t jn = 0;
-    int imgn = kHere, nn = 0;  // the rows being loaded: indices, images, how many
-    bool seamn = false;
-    if (more) {
-        fetch(jn, imgn);
-        nn = total - at;
-        seamn = seam;
-        row = SR[jn];
-    }
-    for (;;) {
-        bool self = false;
-        if (more) {
-            const double4 sr = row;
-            const uint32_t jj = jn;
-            const int img = imgn, nrow = nn;
-            double x = sr.x - cx, y = sr.y - cy, z = sr.z - cz;
-            if (seamn) {
-                const_geom* gp = geom;
-                asm volatile("" : "+s"(gp));
-                x = sr.x - __builtin_fma((double)(1 - (img & 3)), gp->period[0], cx);
-                y = sr.y - __builtin_fma((double)(1 - ((img >> 2) & 3)), gp->period[1], cy);
-                z = sr.z - __builtin_fma((double)(1 - (img >> 4)), gp->period[2], cz);
-            }
-            more = next();
-            if (more) {
-                fetch(jn, imgn);
-                nn = total - at;
-                seamn = seam;
-                row = SR[jn];
-            }
-            const float gx = fmaxf(0.f, fabsf((float)x) - hx);
-            const float gy = fmaxf(0.f, fabsf((float)y) - hy);
-            const float gz = fmaxf(0.f, fabsf((float)z) - hz);
-            const float gxy = __builtin_fmaf(gy, gy, gx * gx);
-            // (the group's own rows wait for the end)
-            const bool ok = lane < nrow && !(own && jj - own0 < (uint32_t)cnt && img == kHere) && (XY ? (gxy <= r2xy && gz <= Rz) : (__builtin_fmaf(gz, gz, gxy) <= r2xy));
-            const uint64_t mk = (uint64_t)__ballot(ok);
-            if (ok) {
-                const uint32_t slot = __builtin_amdgcn_mbcnt_hi(
-                    (uint32_t)(mk >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mk, (uint32_t)qlen));
-                SX[slot] = x;
-                SX[kSlots + slot] = y;
-                SX[2 * kSlots + slot] = z;
-                SX[3 * kSlots + slot] = XY ? x * x + y * y : x * x + y * y + z * z;
-                ID[slot] = jj | ((uint32_t)img << kImgShift);
-            }
-            __builtin_amdgcn_wave_barrier();
-            qlen += __builtin_popcountll(mk);
-        } else if (qlen == 0) {
-            if (!(sym || own) || part != 0 || self_done) break;
-            // One sample, last: the group's own points.  Symmetric counts take each
-            // unordered pair of different sub-groups twice and the ordered pairs
-            // inside a sub-group once, other passes every ordered pair once; each
-            // point with itself (distance 0: bin 0) is added here.
-            const double4 pr = reinterpret_cast<const double4*>(L.lane.x)[p0 + (act ? lane : 0)];
-            const double ax = pr.x - cx, ay = pr.y - cy, az = pr.z - cz;
-            SX[lane] = act ? ax : 0.0;
-            SX[kSlots + lane] = act ? ay : 0.0;
-            SX[2 * kSlots + lane] = act ? az : 0.0;
-            SX[3 * kSlots + lane] = !act ? kFar : (XY ? ax * ax + ay * ay : ax * ax + ay * ay + az * az);
-            // (the lanes' rows are the stream's: one sample)
-            ID[lane] = (uint32_t)(p0 + (act ? lane : 0) - (int64_t)sbase) | ((uint32_t)kHere << kImgShift);
-            evals += (uint64_t)cnt * cnt;
-            if constexpr (MODE == kModeTan) {
-                if (act) {
-                    const double w = LWT[lane], t = LWT[64 + lane];
-                    __hip_atomic_fetch_add(reinterpret_cast<double*>(hist + tcol8), 0.5 * (w * w), __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_WORKGROUP);
-                    __hip_atomic_fetch_add(reinterpret_cast<double*>(hist + TR + tcol8), w * t, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_WORKGROUP);
-                }
-                if (ALSO && lane == 0) *reinterpret_cast<uint32_t*>(hist + 2 * TR) += (uint32_t)cnt;
-            } else if constexpr (MODE == kModeObj || (JK && !VAR)) {
-                if (act) reinterpret_cast<uint32_t*>(hist)[lane] += 1u;
-            } else if constexpr (MODE == kModeJac || JK) {
-                if (act) reinterpret_cast<double*>(hist)[lane] += LWT[lane];
-            } else if constexpr (MODE == kModeWSum || MODE == kModeWXYZ) {
-                if (act) {
-                    double w[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+                __builtin_amdgcn_wave_barrier();
+                const double bs = s == 0 ? Bf[0] : (s == 1 ? Bf[1] : (s == 2 ? Bf[2] : Bf[3]));
+                const double ns = s == 0 ? NA[0] : (s == 1 ? NA[1] : (s == 2 ? NA[2] : NA[3]));
+                const dbl4 cc = {ns, ns, ns, ns};
+                // this sub-group's lane points: weights and z
+                const int lj = s * kSub + (lane & 15);
+                double lw[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+                if (F64) {
 #pragma unroll
                     for (int c = 0; c < 5; c++)
-                        if (c < nw) w[c] = LWT[c * 64 + lane];
-                    const double v = PROD ? w[0] * w[0] : wfunc_eval(L.wfunc, w, w);
-                    __hip_atomic_fetch_add(reinterpret_cast<double*>(hist + (MODE == kModeWSum ? col8 : 0u)), v,
-                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        if (c < nw) lw[c] = LWT[c * 64 + lj];
                 }
-            } else {
-                if (lane == 0) *reinterpret_cast<uint32_t*>(hist) += (uint32_t)cnt;
+                if (TAN && sym && !self && sc < 4) {
+                    // symmetric sums are doubled at the end: a shifted pair counts from both sides
+                    lw[0] *= 0.5;
+                    lw[1] *= 0.5;
+                }
+                double za = 0.0;
+                if (XY) za = LWT[nw * 64 + lj];
+                // stream weights of the D row this lane's row broadcasts
+                double wn[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+                auto load_weights = [&](int slot) __attribute__((always_inline)) {
+                    const double* w = SWm + (uint32_t)((ID[slot] & kRowMask) * (uint32_t)wst);
+#pragma unroll
+                    for (int c = 0; c < 5; c++)
+                        if (c < nw) wn[c] = w[c];
+                };
+                if (F64) load_weights(list[brow]);
+                // operands one tile ahead, their slots two
+                double a = comp[list[lrow]];
+                int slot2 = list[kSub + lrow];
+                for (int t0 = 0; t0 < n; t0 += kSub) {
+                    // rows: staged points list[t0 + 4 (lane / 16) + i]; columns: the sub-group's points
+                    const double a1 = comp[slot2];
+                    slot2 = list[t0 + 2 * kSub + lrow];
+                    double zb = 0.0, wb[5];
+                    if (XY) zb = SX[2 * kSlots + list[t0 + brow]];
+                    if (F64) {
+                        // this tile's stream weights were loaded a tile ago
+#pragma unroll
+                        for (int c = 0; c < 5; c++) wb[c] = wn[c];
+                        load_weights(list[t0 + kSub + brow]);
+                    }
+                    // (the next operands' reads go out before the product, which would otherwise
+                    // hold them back: its result registers are reused at once)
+                    __builtin_amdgcn_sched_barrier(0);
+                    const dbl4 D = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bs, cc, 0, 0, 0);
+                    a = a1;
+                    int hi[4], hp[4];
+                    uint2 ent[4], enp[4];
+                    uint32_t t[4], k[4], tp[4], kp[4];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) hi[i] = __double2hiint(D[i]);
+                    bool diag = false;
+                    if (self) {
+                        inc = sym ? 2u : 1u;
+                        diag = t0 == s * kSub;
+                        if (diag) {
+                            // inside a sub-group: ordered pairs, without a point and itself
+                            inc = 1u;
+#pragma unroll
+                            for (int i = 0; i < 4; i++)
+                                if ((lane >> 4) * 4 + i == (lane & 15)) hi[i] = 0x7e000000;
+                        }
+                    }
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const uint32_t off = ((uint32_t)med3i(hi[i], tlo, thi) >> tsh) & tmask;
+                        ent[i] = lds_entry(off);
+                    }
+                    if (XY) {
+                        double dz[4];
+                        dz[0] = row_bcast<0>(zb) - za;
+                        dz[1] = row_bcast<1>(zb) - za;
+                        dz[2] = row_bcast<2>(zb) - za;
+                        dz[3] = row_bcast<3>(zb) - za;
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            hp[i] = __double2hiint(dz[i] * dz[i]);
+                            const uint32_t off = (((uint32_t)med3i(hp[i], plo, phi) >> psh3) & pmask) | ptab;
+                            enp[i] = lds_entry(off);
+                        }
+                    }
+#pragma unroll
+                    for (int i = 0; i < 4; i++) sub_borrow(ent[i].x, (uint32_t)hi[i], ent[i].y, t[i], k[i]);
+                    uint32_t tm = min(min(t[0], t[1]), min(t[2], t[3]));
+                    const int hm = min(min(hi[0], hi[1]), min(hi[2], hi[3]));
+                    bool odd = tm <= 2u || hm < (int)floor_hi;
+                    if (XY) {
+#pragma unroll
+                        for (int i = 0; i < 4; i++) sub_borrow(enp[i].x, (uint32_t)hp[i], enp[i].y, tp[i], kp[i]);
+                        const uint32_t pm = min(min(tp[0], tp[1]), min(tp[2], tp[3]));
+                        const int qm = min(min(hp[0], hp[1]), min(hp[2], hp[3]));
+                        odd = odd || pm <= 2u || qm < (int)floor_pi;
+                    }
+                    if (__builtin_expect((uint64_t)__ballot(odd) != 0, 0)) {
+#pragma unroll 1
+                        for (int i = 0; i < 4; i++) {
+                            const uint32_t ti = i == 0 ? t[0] : (i == 1 ? t[1] : (i == 2 ? t[2] : t[3]));
+                            const int hv = i == 0 ? hi[0] : (i == 1 ? hi[1] : (i == 2 ? hi[2] : hi[3]));
+                            const uint32_t ek = i == 0 ? ent[0].y : (i == 1 ? ent[1].y : (i == 2 ? ent[2].y : ent[3].y));
+                            bool oi = ti <= 2u || hv < (int)floor_hi;
+                            if (XY) {
+                                const uint32_t pi = i == 0 ? tp[0] : (i == 1 ? tp[1] : (i == 2 ? tp[2] : tp[3]));
+                                const int hq = i == 0 ? hp[0] : (i == 1 ? hp[1] : (i == 2 ? hp[2] : hp[3]));
+                                oi = (oi || pi <= 2u || hq < (int)floor_pi) && hv < 0x7e000000;
+                            }
+                            if (oi) {
+                                const int slot = list[t0 + (lane >> 4) * 4 + i];
+                                const uint32_t kb = hv < (int)floor_hi || ek == 0u ? 0u : ek - 1u;
+                                uint32_t kq = 0u;
+                                uint32_t kk = exact_bin(s * kSub + (lane & 15), slot, kb, kq, false);
+                                if (MODE == kModeJac && !SWAP && L.corr != nullptr) {
+                                    // Auto-count with one set of weights: the sample-2 rows take
+                                    // the pair's other orientation, which across the periodic seam
+                                    // may round into another bin; those disagreements are recorded,
+                                    // so rows2 = rows1 + corr (as pairs_kernel.h does for every
+                                    // shifted pair; only these can differ).
+                                    const uint32_t id = ID[slot];
+                                    uint32_t dummy = 0u;
+                                    const uint32_t kr = exact_bin(s * kSub + (lane & 15), slot, kb, dummy, true);
+                                    if (kr != kk && (id >> kImgShift) != (uint32_t)kHere && s * kSub + (lane & 15) < cnt) {
+                                        const int64_t sr = (int64_t)sbase + (int64_t)(id & kRowMask);
+                                        const int64_t q = __double_as_longlong(L.strm.x[sr * 4 + 3]);
+                                        double* crow = L.corr + q * K;
+                                        if (kk < (uint32_t)K)
+                                            __hip_atomic_fetch_add(crow + kk, lw[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                                        if (kr < (uint32_t)K)
+                                            __hip_atomic_fetch_add(crow + kr, -lw[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                                    }
+                                }
+                                if constexpr (JK) {
+                                    // A pair of two tags gives half of its weight to each.  The rows
+                                    // give all of an ordered pair's to its lane point's tag, which is
+                                    // the same where the pair's other order lands in the same bin;
+                                    // across the periodic seam it may not, and half moves over.
+                                    const uint32_t id = ID[slot];
+                                    uint32_t dummy = 0u;
+                                    const uint32_t kr = exact_bin(lj, slot, kb, dummy, true);
+                                    if (kr != kk && (id >> kImgShift) != (uint32_t)kHere && lj < cnt) {
+                                        const double* wi = L.lane.w + (p0 + lj) * 2;
+                                        const double v = 0.5 * wi[0] * L.strm.w[((int64_t)sbase + (int64_t)(id & kRowMask)) * 2];
+                                        const int t = (int)wi[1];
+                                        double* r = L.jacc + ((int64_t)m * (L.nsamp + 1) + t) * K;
+                                        if (t >= 1 && t <= L.nsamp) {
+                                            if (kk < (uint32_t)K)
+                                                __hip_atomic_fetch_add(r + kk, -v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                                            if (kr < (uint32_t)K)
+                                                __hip_atomic_fetch_add(r + kr, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                                        }
+                                    }
+                                }
+#pragma unroll
+                                for (int u = 0; u < 4; u++)
+                                    if (i == u) {
+                                        k[u] = kk;
+                                        if (XY) kp[u] = kq;
+                                    }
+                            }
+                        }
+                    }
+                    // ---- accumulate
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        // the row's stream weights (all lanes: a broadcast reads none that is masked off)
+                        double sw[5];
+                        if constexpr (F64) {
+#pragma unroll
+                            for (int c = 0; c < 5; c++)
+                                sw[c] = c >= nw ? 0.0
+                                                : (i == 0 ? row_bcast<0>(wb[c])
+                                                          : (i == 1 ? row_bcast<1>(wb[c])
+                                                                    : (i == 2 ? row_bcast<2>(wb[c]) : row_bcast<3>(wb[c]))));
+                        }
+                        if constexpr (MODE == kModeCount3D) {
+                            __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hist + ((k[i] << 7) + col4)), inc,
+                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        } else if constexpr (MODE == kModeProj) {
+                            // beyond pi_max: the trash row
+                            const uint32_t kk = kp[i] == 0u ? k[i] : (uint32_t)K;
+                            __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hist + ((kk << 7) + col4)), inc,
+                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        } else if constexpr (MODE == kModeXYZ || MODE == kModeWXYZ) {
+                            // one [K][Kp] histogram per wave; pairs beyond an edge skip it
+                            if (k[i] < (uint32_t)K && kp[i] < (uint32_t)Kp) {
+                                const uint32_t cell = __umul24(k[i], (uint32_t)Kp) + kp[i];
+                                if constexpr (MODE == kModeXYZ) {
+                                    __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hist) + ((cell << ccol) + ccl), inc, __ATOMIC_RELAXED,
+                                                           __HIP_MEMORY_SCOPE_WORKGROUP);
+                                } else {
+                                    const double v = PROD ? lw[0] * sw[0] : wfunc_eval(L.wfunc, lw, sw);
+                                    __hip_atomic_fetch_add(reinterpret_cast<double*>(hist) + cell, v, __ATOMIC_RELAXED,
+                                                           __HIP_MEMORY_SCOPE_WORKGROUP);
+                                }
+                            }
+                        } else if constexpr (MODE == kModeObj || (JK && !VAR)) {
+                            __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hist + ((k[i] << 8) + (uint32_t)lj * 4u)), 1u,
+                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        } else {
+                            if constexpr (MODE == kModeJac || JK) {
+                                __hip_atomic_fetch_add(reinterpret_cast<double*>(hist + ((k[i] << 9) + (uint32_t)lj * 8u)),
+                                                       sw[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                            } else if constexpr (MODE == kModeTan) {
+                                // pair terms w_i w_j and t_i w_j + w_i t_j (t = dw/dtheta); the
+                                // group's own pairs: ordered ones inside a sub-group count half
+                                if (k[i] < (uint32_t)K) {
+                                    double wj = sw[0], tj = sw[1];
+                                    if (diag) {
+                                        wj *= 0.5;
+                                        tj *= 0.5;
+                                    }
+                                    const double v = lw[0] * wj;
+                                    const double tv = __builtin_fma(lw[0], tj, lw[1] * wj);
+                                    unsigned char* const r = hist + __umul24(k[i], ALSO ? 3 * TR : 2 * TR);
+                                    __hip_atomic_fetch_add(reinterpret_cast<double*>(r + tcol8), v, __ATOMIC_RELAXED,
+                                                           __HIP_MEMORY_SCOPE_WORKGROUP);
+                                    __hip_atomic_fetch_add(reinterpret_cast<double*>(r + TR + tcol8), tv, __ATOMIC_RELAXED,
+                                                           __HIP_MEMORY_SCOPE_WORKGROUP);
+                                    if (ALSO)
+                                        __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(r + 2 * TR + tcol4), inc,
+                                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                                }
+                            } else if constexpr (MODE == kModeWSum) {
+                                const double v = PROD ? lw[0] * sw[0] : wfunc_eval(L.wfunc, lw, sw);
+                                __hip_atomic_fetch_add(reinterpret_cast<double*>(hist + ((k[i] << 7) + col8)), v,
+                                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                            }
+                            if constexpr (ALSO && MODE != kModeTan)
+                                __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(wsm + A.cnt_off + ((k[i] << 7) + col4)), 1u,
+                                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        }
+                    }
+                }
+                __builtin_amdgcn_wave_barrier();
             }
-            if constexpr (ALSO && MODE != kModeTan) {
-                if (lane == 0) *reinterpret_cast<uint32_t*>(wsm + A.cnt_off) += (uint32_t)cnt;
+            // what was not dealt moves to the front
+            const int rest = self ? 0 : max(qlen - kDeal, 0);
+            if (rest > 0 && lane < rest) {
+                const int f = kDeal + lane;
+                const double x = SX[f], y = SX[kSlots + f], z = SX[2 * kSlots + f], nn = SX[3 * kSlots + f];
+                const uint32_t id = ID[f];
+                SX[lane] = x;
+                SX[kSlots + lane] = y;
+                SX[2 * kSlots + lane] = z;
+                SX[3 * kSlots + lane] = nn;
+                ID[lane] = id;
             }
             __builtin_amdgcn_wave_barrier();
-            qlen = cnt;
-            self = true;
-            self_done = true;
-        }
-        if (qlen >= kDeal || !more) process(self);
-    }
-    __builtin_amdgcn_wave_barrier();
-
-    // ---- the group's results
-    // columns are summed starting at a lane's own one (a bank per lane), counts
-    // go to the mock's accumulators
-    uint64_t* const cacc =
-        L.pcount ? L.pcount + ((int64_t)m * L.crep + (int64_t)(gl % L.crep)) * ((MODE == kModeXYZ) ? K * Kp : K) : nullptr;
-    if constexpr (MODE == kModeXYZ) {
-        const uint32_t* h = reinterpret_cast<const uint32_t*>(hist);
-        for (int k = lane; k < K * Kp; k += 64) {
-            uint64_t tot = 0;
-            for (int c = 0; c < (1 << ccol); c++) tot += h[(k << ccol) + ((c + lane) & ((1 << ccol) - 1))];
-            if (tot) __hip_atomic_fetch_add(cacc + k, tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-    } else if constexpr (MODE == kModeCount3D || MODE == kModeProj || ALSO) {
-        const uint32_t* h = reinterpret_cast<const uint32_t*>(wsm + A.cnt_off);
-        constexpr int step = TAN ? 3 * (int)TR / 4 : 32, nc = TAN ? 2 * (int)TC : 32;
-        for (int k = lane; k < K; k += 64) {
-            uint64_t tot = 0;
-            for (int c = 0; c < nc; c++) tot += h[k * step + ((c + lane) & (nc - 1))];
-            if (tot) __hip_atomic_fetch_add(cacc + k, tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-    }
-    if constexpr (MODE == kModeWXYZ) {
-        const double* h = reinterpret_cast<const double*>(hist);
-        double* dst = L.psum + ((g << psh) + part) * (int64_t)K * Kp;
-        for (int k = lane; k < K * Kp; k += 64) dst[k] = h[k];
-    }
-    if constexpr (MODE == kModeWSum || MODE == kModeTan) {
-        const double* h = reinterpret_cast<const double*>(hist);
-        constexpr int nc = TAN ? (int)TC : 16;
-        constexpr int step = TAN ? (ALSO ? 3 : 2) * (int)TC : 16;
-        const double sc = (TAN && sym) ? 2.0 : 1.0;
-        for (int k = lane; k < K; k += 64) {
-            double v = 0.0, tv = 0.0;
-            for (int c = 0; c < nc; c++) {
-                v += h[k * step + ((c + lane) & (nc - 1))];
-                if (TAN) tv += h[k * step + nc + ((c + lane) & (nc - 1))];
-            }
-            const int64_t at_ = ((g << psh) + part) * K + k;
-            if (L.psum) L.psum[at_] = sc * v;
-            if (TAN) L.ptan[at_] = sc * tv;
-        }
-    }
-    if constexpr (JK) {
-        // sums of the lane points' rows by tag, one distinct tag at a time: lane
-        // k adds up bin k of the points that carry it.  (A group of very many
-        // tags leaves the loop and adds point by point.)
-        const int tag = act ? (int)L.lane.w[(p0 + lane) * 2 + 1] : 0;
-        const double wl = (VAR && act) ? LWT[lane] : 1.0;
-        uint64_t todo = (uint64_t)__ballot(act && tag >= 1 && tag <= L.nsamp);
-        auto value = [&](int k, int j) __attribute__((always_inline)) -> double {
-            if (VAR) return LWT[j] * reinterpret_cast<const double*>(hist)[k * 64 + j];
-            return (double)reinterpret_cast<const uint32_t*>(hist)[k * 64 + j];
+            qlen = rest;
         };
-        for (int round = 0; round < 8 && todo; round++) {
-            const int t = __builtin_amdgcn_readlane(tag, __builtin_ctzll(todo));
-            const uint64_t mine = (uint64_t)__ballot(tag == t) & todo;
-            todo &= ~mine;
-            double* r = L.jacc + ((int64_t)m * (L.nsamp + 1) + t) * K;
-            for (int k0 = 0; k0 < K; k0 += 64) {
-                const int k = k0 + lane;
-                double sum = 0.0;
-                for (int c = 0; c < 64; c++) {
-                    const int j = (c + lane) & 63;  // a bank per lane
-                    if (((mine >> j) & 1) && k < K) sum += value(k, j);
+
+        // ---- the cubes of the curve near the group.  A lane takes one cube of the
+        // window and looks up the stretch of rows it holds; the stretches of 64 cubes
+        // form one list of rows, which is walked 64 rows at a time: a scan over the
+        // starts gives each lane its stretch.  Symmetric counts drop the rows before
+        // the group's end here (unshifted cubes), a whole stretch at a time.
+        const double4* const SR = reinterpret_cast<const double4*>(L.strm.x) + sbase;
+        int cube0 = -64;                // the next 64 cubes of the window
+        int cimg = 0;                   // the lane's cube: its image
+        bool seam = false;              // some cube of the list is a periodic image
+        int pre = 0, end = 0, run = 0;  // the lane's stretch: its place [pre, end) in the list, first row - pre
+        int at = 0, total = 0;          // list position of the next rows, rows in the list
+        // the next 64 rows: false when the group has no more.  The list is made
+        // rarely: what that needs is loaded here.
+        auto next = [&]() __attribute__((always_inline)) -> bool {
+            at += 64;
+            while (at >= total) {
+                const_geom* gp = geom;
+                asm volatile("" : "+s"(gp));
+                const int cb = gp->cbits, nc = 1 << cb;  // cubes per dimension
+                const int* const w = reinterpret_cast<const int*>(info) + 40;
+                const int wy = w[3], wz = w[4], ncubes = uni(w[5]);
+                cube0 += 64;
+                if ((cube0 << psh) + part >= ncubes) return false;
+                // cube ci of the window: z fastest (quotients from reciprocals: exact
+                // for the few thousand cubes of a window, and one more test for more)
+                const int ci = ((cube0 + lane) << psh) + part;
+                int cxy = (int)((float)ci * info[47]);
+                int jz = ci - cxy * wz;
+                if (jz < 0) { jz += wz; cxy--; }
+                if (jz >= wz) { jz -= wz; cxy++; }
+                int jx = (int)((float)cxy * info[46]);
+                int jy = cxy - jx * wy;
+                if (jy < 0) { jy += wy; jx--; }
+                if (jy >= wy) { jy -= wy; jx++; }
+                jx += w[0];
+                jy += w[1];
+                jz += w[2];
+                const float cxf = info[48], cyf = info[49], czf = info[50];
+                const float gx = fmaxf(0.f, fmaxf((float)jx * cxf - info[35], info[32] - (float)(jx + 1) * cxf));
+                const float gy = fmaxf(0.f, fmaxf((float)jy * cyf - info[36], info[33] - (float)(jy + 1) * cyf));
+                const float gz = fmaxf(0.f, fmaxf((float)jz * czf - info[37], info[34] - (float)(jz + 1) * czf));
+                at = 0;
+                total = 0;
+                const bool has = ci < ncubes && (XY ? gx * gx + gy * gy : gx * gx + gy * gy + gz * gz) <= r2xy;
+                if ((uint64_t)__ballot(has) == 0) continue;
+                // image: 0, 1, 2 for -L, 0, +L per dimension, two bits each
+                const int ux = (jx >> cb) + 1, uy = (jy >> cb) + 1, uz = (jz >> cb) + 1;
+                cimg = ux | (uy << 2) | (uz << 4);
+                int len = 0;
+                run = 0;
+                if (has) {
+                    const int cm = nc - 1;
+                    const uint2 c = (L.strm.cubes + gp->cell_off)[(uint32_t)(((((jx & cm) << cb) + (jy & cm)) << cb) + (jz & cm))];
+                    run = (int)c.x;
+                    if (sym && cimg == kHere) run = max(run, (int)(gp->p_off[SD] + gl * kGroup + cnt));
+                    len = max((int)c.y - run, 0);
                 }
-                if (k < K && sum != 0.0) __hip_atomic_fetch_add(r + k, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                seam = (uint64_t)__ballot(len > 0 && cimg != kHere) != 0;
+                pre = wave_prefix(len);
+                total = __builtin_amdgcn_readlane(pre, 63);
+                end = len > 0 ? pre : -1;
+                pre -= len;
+                run -= pre + (int)sbase;
+            }
+            return true;
+        };
+        // this lane's row of the list (relative to the mock's first) and its image;
+        // a row past the end repeats the last one
+        auto fetch = [&](uint32_t& jj, int& img) __attribute__((always_inline)) {
+            mark[lane] = 0;
+            __builtin_amdgcn_wave_barrier();
+            if (pre < at + 64 && end > at) mark[max(pre - at, 0)] = (uint8_t)lane;
+            __builtin_amdgcn_wave_barrier();
+            const int sg = wave_scan_max((int)mark[lane]) << 2;
+            jj = (uint32_t)(min(at + lane, total - 1) + __builtin_amdgcn_ds_bpermute(sg, run));
+            img = seam ? __builtin_amdgcn_ds_bpermute(sg, cimg) : kHere;
+        };
+        const uint32_t own0 = (uint32_t)(p0 - (int64_t)sbase);  // the group's first row, in one sample
+        bool more = next();
+        double4 row = make_double4(0.0, 0.0, 0.0, 0.0);
+        uint32_t jn = 0;
+        int imgn = kHere, nn = 0;  // the rows being loaded: indices, images, how many
+        bool seamn = false;
+        if (more) {
+            fetch(jn, imgn);
+            nn = total - at;
+            seamn = seam;
+            row = SR[jn];
+        }
+        for (;;) {
+            bool self = false;
+            if (more) {
+                const double4 sr = row;
+                const uint32_t jj = jn;
+                const int img = imgn, nrow = nn;
+                double x = sr.x - cx, y = sr.y - cy, z = sr.z - cz;
+                if (seamn) {
+                    const_geom* gp = geom;
+                    asm volatile("" : "+s"(gp));
+                    x = sr.x - __builtin_fma((double)(1 - (img & 3)), gp->period[0], cx);
+                    y = sr.y - __builtin_fma((double)(1 - ((img >> 2) & 3)), gp->period[1], cy);
+                    z = sr.z - __builtin_fma((double)(1 - (img >> 4)), gp->period[2], cz);
+                }
+                more = next();
+                if (more) {
+                    fetch(jn, imgn);
+                    nn = total - at;
+                    seamn = seam;
+                    row = SR[jn];
+                }
+                const float gx = fmaxf(0.f, fabsf((float)x) - hx);
+                const float gy = fmaxf(0.f, fabsf((float)y) - hy);
+                const float gz = fmaxf(0.f, fabsf((float)z) - hz);
+                const float gxy = __builtin_fmaf(gy, gy, gx * gx);
+                // (the group's own rows wait for the end)
+                const bool ok = lane < nrow && !(own && jj - own0 < (uint32_t)cnt && img == kHere) && (XY ? (gxy <= r2xy && gz <= Rz) : (__builtin_fmaf(gz, gz, gxy) <= r2xy));
+                const uint64_t mk = (uint64_t)__ballot(ok);
+                if (ok) {
+                    const uint32_t slot = __builtin_amdgcn_mbcnt_hi(
+                        (uint32_t)(mk >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mk, (uint32_t)qlen));
+                    SX[slot] = x;
+                    SX[kSlots + slot] = y;
+                    SX[2 * kSlots + slot] = z;
+                    SX[3 * kSlots + slot] = XY ? x * x + y * y : x * x + y * y + z * z;
+                    ID[slot] = jj | ((uint32_t)img << kImgShift);
+                }
+                __builtin_amdgcn_wave_barrier();
+                qlen += __builtin_popcountll(mk);
+            } else if (qlen == 0) {
+                if (!(sym || own) || part != 0 || self_done) break;
+                // One sample, last: the group's own points.  Symmetric counts take each
+                // unordered pair of different sub-groups twice and the ordered pairs
+                // inside a sub-group once, other passes every ordered pair once; each
+                // point with itself (distance 0: bin 0) is added here.
+                const double4 pr = reinterpret_cast<const double4*>(L.lane.x)[p0 + (act ? lane : 0)];
+                const double ax = pr.x - cx, ay = pr.y - cy, az = pr.z - cz;
+                SX[lane] = act ? ax : 0.0;
+                SX[kSlots + lane] = act ? ay : 0.0;
+                SX[2 * kSlots + lane] = act ? az : 0.0;
+                SX[3 * kSlots + lane] = !act ? kFar : (XY ? ax * ax + ay * ay : ax * ax + ay * ay + az * az);
+                // (the lanes' rows are the stream's: one sample)
+                ID[lane] = (uint32_t)(p0 + (act ? lane : 0) - (int64_t)sbase) | ((uint32_t)kHere << kImgShift);
+                evals += (uint64_t)cnt * cnt;
+                if constexpr (MODE == kModeTan) {
+                    if (act) {
+                        const double w = LWT[lane], t = LWT[64 + lane];
+                        __hip_atomic_fetch_add(reinterpret_cast<double*>(hist + tcol8), 0.5 * (w * w), __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_WORKGROUP);
+                        __hip_atomic_fetch_add(reinterpret_cast<double*>(hist + TR + tcol8), w * t, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_WORKGROUP);
+                    }
+                    if (ALSO && lane == 0) *reinterpret_cast<uint32_t*>(hist + 2 * TR) += (uint32_t)cnt;
+                } else if constexpr (MODE == kModeObj || (JK && !VAR)) {
+                    if (act) reinterpret_cast<uint32_t*>(hist)[lane] += 1u;
+                } else if constexpr (MODE == kModeJac || JK) {
+                    if (act) reinterpret_cast<double*>(hist)[lane] += LWT[lane];
+                } else if constexpr (MODE == kModeWSum || MODE == kModeWXYZ) {
+                    if (act) {
+                        double w[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                        for (int c = 0; c < 5; c++)
+                            if (c < nw) w[c] = LWT[c * 64 + lane];
+                        const double v = PROD ? w[0] * w[0] : wfunc_eval(L.wfunc, w, w);
+                        __hip_atomic_fetch_add(reinterpret_cast<double*>(hist + (MODE == kModeWSum ? col8 : 0u)), v,
+                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    }
+                } else {
+                    if (lane == 0) *reinterpret_cast<uint32_t*>(hist) += (uint32_t)cnt;
+                }
+                if constexpr (ALSO && MODE != kModeTan) {
+                    if (lane == 0) *reinterpret_cast<uint32_t*>(wsm + A.cnt_off) += (uint32_t)cnt;
+                }
+                __builtin_amdgcn_wave_barrier();
+                qlen = cnt;
+                self = true;
+                self_done = true;
+            }
+            if (qlen >= kDeal || !more) process(self);
+        }
+        __builtin_amdgcn_wave_barrier();
+
+        // ---- the group's results
+        // columns are summed starting at a lane's own one (a bank per lane), counts
+        // go to the mock's accumulators
+        uint64_t* const cacc =
+            L.pcount ? L.pcount + ((int64_t)m * L.crep + (int64_t)(gl % L.crep)) * ((MODE == kModeXYZ) ? K * Kp : K) : nullptr;
+        if constexpr (MODE == kModeXYZ) {
+            const uint32_t* h = reinterpret_cast<const uint32_t*>(hist);
+            for (int k = lane; k < K * Kp; k += 64) {
+                uint64_t tot = 0;
+                for (int c = 0; c < (1 << ccol); c++) tot += h[(k << ccol) + ((c + lane) & ((1 << ccol) - 1))];
+                if (tot) __hip_atomic_fetch_add(cacc + k, tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        } else if constexpr (MODE == kModeCount3D || MODE == kModeProj || ALSO) {
+            const uint32_t* h = reinterpret_cast<const uint32_t*>(wsm + A.cnt_off);
+            constexpr int step = TAN ? 3 * (int)TR / 4 : 32, nc = TAN ? 2 * (int)TC : 32;
+            for (int k = lane; k < K; k += 64) {
+                uint64_t tot = 0;
+                for (int c = 0; c < nc; c++) tot += h[k * step + ((c + lane) & (nc - 1))];
+                if (tot) __hip_atomic_fetch_add(cacc + k, tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
-        if (todo && ((todo >> lane) & 1)) {
-            double* r = L.jacc + ((int64_t)m * (L.nsamp + 1) + tag) * K;
-            for (int k = 0; k < K; k++) {
-                const double v = VAR ? wl * reinterpret_cast<const double*>(hist)[k * 64 + lane]
-                                     : (double)reinterpret_cast<const uint32_t*>(hist)[k * 64 + lane];
-                if (v != 0.0) __hip_atomic_fetch_add(r + k, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if constexpr (MODE == kModeWXYZ) {
+            const double* h = reinterpret_cast<const double*>(hist);
+            double* dst = L.psum + ((g << psh) + part) * (int64_t)K * Kp;
+            for (int k = lane; k < K * Kp; k += 64) dst[k] = h[k];
+        }
+        if constexpr (MODE == kModeWSum || MODE == kModeTan) {
+            const double* h = reinterpret_cast<const double*>(hist);
+            constexpr int nc = TAN ? (int)TC : 16;
+            constexpr int step = TAN ? (ALSO ? 3 : 2) * (int)TC : 16;
+            const double sc = (TAN && sym) ? 2.0 : 1.0;
+            for (int k = lane; k < K; k += 64) {
+                double v = 0.0, tv = 0.0;
+                for (int c = 0; c < nc; c++) {
+                    v += h[k * step + ((c + lane) & (nc - 1))];
+                    if (TAN) tv += h[k * step + nc + ((c + lane) & (nc - 1))];
+                }
+                const int64_t at_ = ((g << psh) + part) * K + k;
+                if (L.psum) L.psum[at_] = sc * v;
+                if (TAN) L.ptan[at_] = sc * tv;
             }
         }
-    }
-    if constexpr (MODE == kModeObj || MODE == kModeJac) {
-        if (act) {
-            // the lane point's row at its input position
-            const int64_t q = __double_as_longlong(L.lane.x[(p0 + lane) * 4 + 3]);
-            if constexpr (MODE == kModeObj) {
-                int64_t* r = L.orows + q * K;
-                int64_t sum = 0;
+        if constexpr (JK) {
+            // sums of the lane points' rows by tag, one distinct tag at a time: lane
+            // k adds up bin k of the points that carry it.  (A group of very many
+            // tags leaves the loop and adds point by point.)
+            const int tag = act ? (int)L.lane.w[(p0 + lane) * 2 + 1] : 0;
+            const double wl = (VAR && act) ? LWT[lane] : 1.0;
+            uint64_t todo = (uint64_t)__ballot(act && tag >= 1 && tag <= L.nsamp);
+            auto value = [&](int k, int j) __attribute__((always_inline)) -> double {
+                if (VAR) return LWT[j] * reinterpret_cast<const double*>(hist)[k * 64 + j];
+                return (double)reinterpret_cast<const uint32_t*>(hist)[k * 64 + j];
+            };
+            for (int round = 0; round < 8 && todo; round++) {
+                const int t = __builtin_amdgcn_readlane(tag, __builtin_ctzll(todo));
+                const uint64_t mine = (uint64_t)__ballot(tag == t) & todo;
+                todo &= ~mine;
+                double* r = L.jacc + ((int64_t)m * (L.nsamp + 1) + t) * K;
+                for (int k0 = 0; k0 < K; k0 += 64) {
+                    const int k = k0 + lane;
+                    double sum = 0.0;
+                    for (int c = 0; c < 64; c++) {
+                        const int j = (c + lane) & 63;  // a bank per lane
+                        if (((mine >> j) & 1) && k < K) sum += value(k, j);
+                    }
+                    if (k < K && sum != 0.0) __hip_atomic_fetch_add(r + k, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+            }
+            if (todo && ((todo >> lane) & 1)) {
+                double* r = L.jacc + ((int64_t)m * (L.nsamp + 1) + tag) * K;
                 for (int k = 0; k < K; k++) {
-                    sum += (int64_t)reinterpret_cast<const uint32_t*>(hist)[k * 64 + lane];
-                    r[k] = sum;
-                }
-            } else if (L.rows) {
-                double* r = L.rows + q * K;
-                for (int k = 0; k < K; k++) r[k] = reinterpret_cast<const double*>(hist)[k * 64 + lane];
-            }
-        }
-        if constexpr (MODE == kModeJac && !SWAP) {
-            if (L.psum) {
-                const double w = act ? LWT[lane] : 0.0;
-                for (int k = 0; k < K; k++) {
-                    const double tot = wave_sum_f64(act ? w * reinterpret_cast<const double*>(hist)[k * 64 + lane] : 0.0);
-                    if (lane == 0) L.psum[g * K + k] = tot;
+                    const double v = VAR ? wl * reinterpret_cast<const double*>(hist)[k * 64 + lane]
+                                         : (double)reinterpret_cast<const uint32_t*>(hist)[k * 64 + lane];
+                    if (v != 0.0) __hip_atomic_fetch_add(r + k, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
             }
         }
+        if constexpr (MODE == kModeObj || MODE == kModeJac) {
+            if (act) {
+                // the lane point's row at its input position
+                const int64_t q = __double_as_longlong(L.lane.x[(p0 + lane) * 4 + 3]);
+                if constexpr (MODE == kModeObj) {
+                    int64_t* r = L.orows + q * K;
+                    int64_t sum = 0;
+                    for (int k = 0; k < K; k++) {
+                        sum += (int64_t)reinterpret_cast<const uint32_t*>(hist)[k * 64 + lane];
+                        r[k] = sum;
+                    }
+                } else if (L.rows) {
+                    double* r = L.rows + q * K;
+                    for (int k = 0; k < K; k++) r[k] = reinterpret_cast<const double*>(hist)[k * 64 + lane];
+                }
+            }
+            if constexpr (MODE == kModeJac && !SWAP) {
+                if (L.psum) {
+                    const double w = act ? LWT[lane] : 0.0;
+                    for (int k = 0; k < K; k++) {
+                        const double tot = wave_sum_f64(act ? w * reinterpret_cast<const double*>(hist)[k * 64 + lane] : 0.0);
+                        if (lane == 0) L.psum[g * K + k] = tot;
+                    }
+                }
+            }
+        }
+        if (L.pevals && lane == 0)
+            __hip_atomic_fetch_add(reinterpret_cast<unsigned long long*>(L.pevals + g), (unsigned long long)evals,
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_wave_barrier();
     }
-    if (L.pevals && lane == 0)
-        __hip_atomic_fetch_add(reinterpret_cast<unsigned long long*>(L.pevals + g), (unsigned long long)evals,
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 template <int MODE, int VAR, int ALSO, int WAVES>
-static int launch_tiles_w(const TileArgs& A, int64_t items, int smem, hipStream_t s) {
-    hipLaunchKernelGGL((k_tiles<MODE, VAR, ALSO, WAVES>), dim3((unsigned)((items + WAVES - 1) / WAVES)),
-                       dim3(WAVES * 64), (size_t)smem, s, A);
+static int launch_tiles_w(const TileArgs& A, int64_t blocks, int smem, hipStream_t s) {
+    hipLaunchKernelGGL((k_tiles<MODE, VAR, ALSO, WAVES>), dim3((unsigned)blocks), dim3(WAVES * 64), (size_t)smem, s, A);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 template <int MODE, int VAR, int ALSO>
-static int launch_tiles_v(const TileArgs& A, int waves, int64_t items, int smem, hipStream_t s) {
-    if (items <= 0) return 0;
-    if (waves == 8) return launch_tiles_w<MODE, VAR, ALSO, 8>(A, items, smem, s);
-    if (waves == 4) return launch_tiles_w<MODE, VAR, ALSO, 4>(A, items, smem, s);
-    if (waves == 2) return launch_tiles_w<MODE, VAR, ALSO, 2>(A, items, smem, s);
-    return launch_tiles_w<MODE, VAR, ALSO, 1>(A, items, smem, s);
+static int launch_tiles_v(const TileArgs& A, int waves, int64_t blocks, int smem, hipStream_t s) {
+    if (blocks <= 0) return 0;
+    if (waves == 8) return launch_tiles_w<MODE, VAR, ALSO, 8>(A, blocks, smem, s);
+    if (waves == 4) return launch_tiles_w<MODE, VAR, ALSO, 4>(A, blocks, smem, s);
+    if (waves == 2) return launch_tiles_w<MODE, VAR, ALSO, 2>(A, blocks, smem, s);
+    return launch_tiles_w<MODE, VAR, ALSO, 1>(A, blocks, smem, s);
 }
 
 // One launch of mode MODE; each mode is instantiated in its own translation
 // unit (pairs_tile_*.hip).
 template <int MODE>
-int launch_tiles_mode(const TileArgs& A, int waves, int64_t items, int smem, int also, int var, hipStream_t s) {
+int launch_tiles_mode(const TileArgs& A, int waves, int64_t blocks, int smem, int also, int var, hipStream_t s) {
     if constexpr (MODE == kModeWSum) {
         if (var == 2)
-            return also ? launch_tiles_v<MODE, 2, 1>(A, waves, items, smem, s)
-                        : launch_tiles_v<MODE, 2, 0>(A, waves, items, smem, s);
+            return also ? launch_tiles_v<MODE, 2, 1>(A, waves, blocks, smem, s)
+                        : launch_tiles_v<MODE, 2, 0>(A, waves, blocks, smem, s);
     }
     if constexpr (MODE == kModeWSum || MODE == kModeJac) {
         if (var)
-            return also ? launch_tiles_v<MODE, 1, 1>(A, waves, items, smem, s)
-                        : launch_tiles_v<MODE, 1, 0>(A, waves, items, smem, s);
-        return also ? launch_tiles_v<MODE, 0, 1>(A, waves, items, smem, s)
-                    : launch_tiles_v<MODE, 0, 0>(A, waves, items, smem, s);
+            return also ? launch_tiles_v<MODE, 1, 1>(A, waves, blocks, smem, s)
+                        : launch_tiles_v<MODE, 1, 0>(A, waves, blocks, smem, s);
+        return also ? launch_tiles_v<MODE, 0, 1>(A, waves, blocks, smem, s)
+                    : launch_tiles_v<MODE, 0, 0>(A, waves, blocks, smem, s);
     } else if constexpr (MODE == kModeWXYZ) {
-        if (var == 2) return launch_tiles_v<MODE, 2, 0>(A, waves, items, smem, s);
-        return var ? launch_tiles_v<MODE, 1, 0>(A, waves, items, smem, s)
-                   : launch_tiles_v<MODE, 0, 0>(A, waves, items, smem, s);
+        if (var == 2) return launch_tiles_v<MODE, 2, 0>(A, waves, blocks, smem, s);
+        return var ? launch_tiles_v<MODE, 1, 0>(A, waves, blocks, smem, s)
+                   : launch_tiles_v<MODE, 0, 0>(A, waves, blocks, smem, s);
     } else if constexpr (MODE == kModeXYZ || MODE == kModeJack) {
-        return var ? launch_tiles_v<MODE, 1, 0>(A, waves, items, smem, s)
-                   : launch_tiles_v<MODE, 0, 0>(A, waves, items, smem, s);
+        return var ? launch_tiles_v<MODE, 1, 0>(A, waves, blocks, smem, s)
+                   : launch_tiles_v<MODE, 0, 0>(A, waves, blocks, smem, s);
     } else if constexpr (MODE == kModeTan) {
-        return also ? launch_tiles_v<MODE, 0, 1>(A, waves, items, smem, s)
-                    : launch_tiles_v<MODE, 0, 0>(A, waves, items, smem, s);
+        return also ? launch_tiles_v<MODE, 0, 1>(A, waves, blocks, smem, s)
+                    : launch_tiles_v<MODE, 0, 0>(A, waves, blocks, smem, s);
     } else {
-        return launch_tiles_v<MODE, 0, 0>(A, waves, items, smem, s);
+        return launch_tiles_v<MODE, 0, 0>(A, waves, blocks, smem, s);
     }
 }
 

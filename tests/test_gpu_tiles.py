@@ -165,3 +165,25 @@ def test_small_builds_agree_with_general(mo, gpu, n1, n2, monkeypatch):
     monkeypatch.setenv("HALOPAIR_NO_TILES", "1")
     for a, b in zip(got, run()):
         assert torch.equal(torch.as_tensor(a), torch.as_tensor(b))
+
+
+@pytest.mark.parametrize("n1,n2", [(800001, 0), (650000, 70001)])
+def test_queued_items_agree_with_general(mo, gpu, n1, n2, monkeypatch):
+    # more lane groups than two per resident wave: waves take them from queues
+    import torch
+    g = torch.Generator(device=gpu).manual_seed(n1)
+    t1 = torch.rand((n1, 3), dtype=torch.float64, device=gpu, generator=g) * 400.0
+    t1[: n1 // 8] = 200.0 + 0.01 * (t1[: n1 // 8] - 200.0)   # items of very unlike cost
+    t2 = t1 if n2 == 0 else torch.rand((n2, 3), dtype=torch.float64, device=gpu, generator=g) * 400.0
+    u1 = torch.randint(1, 9, (n1,), device=gpu, generator=g).double()
+    u2 = u1 if n2 == 0 else torch.randint(1, 9, (n2,), device=gpu, generator=g).double()
+    rb, pi, kw = np.array([0.02, 0.1, 1.0, 4.0]), np.array([0.0, 0.5, 3.0]), dict(period=400.0)
+
+    def run():
+        return (mo.npairs_3d(t1, t2, rb, **kw), mo.npairs_xy_z(t1, t2, rb, pi, **kw),
+                mo.npairs_per_object_3d(t1, t2, rb, **kw), mo.npairs_projected(t1, t2, rb, 3.0, **kw),
+                mo.marked_npairs_3d(t1, t2, rb, weights1=u1, weights2=u2, weight_func_id=1, **kw))
+    got = run()
+    monkeypatch.setenv("HALOPAIR_NO_TILES", "1")
+    for a, b in zip(got, run()):
+        assert torch.equal(torch.as_tensor(a), torch.as_tensor(b))
