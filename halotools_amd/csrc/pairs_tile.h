@@ -190,6 +190,7 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
     constexpr int kDeal = deal_of(MODE, VAR), kDealH = kDeal / 64;
     using ST = Stage<kDeal>;
     constexpr int kStage = ST::kStage, kSlots = ST::kSlots;
+    constexpr int kPad = (F64 ? 3 : 2) * kSub;  // a list is read this far past its end
     extern __shared__ __align__(16) unsigned char lds[];
     const PairLaunch& L = A.L;
     const int lane = threadIdx.x & 63;
@@ -468,7 +469,7 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                 if (self) {
                     n = sym ? min(qlen, (s + 1) * kSub) : qlen;  // the group's points (up to this sub-group)
                     list[lane] = (uint8_t)lane;
-                    if (lane < 2 * kSub) list[64 + lane] = (uint8_t)kStage;
+                    if (lane < kPad) list[64 + lane] = (uint8_t)kStage;
                 } else {
                     // staged points near the sub-group's box
                     const float4 b0 = *reinterpret_cast<const float4*>(info + 8 * s);
@@ -488,7 +489,7 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                         n += __builtin_popcountll(mm);
                     }
                     if (n == 0) continue;
-                    if (lane < 2 * kSub) list[n + lane] = (uint8_t)kStage;
+                    if (lane < kPad) list[n + lane] = (uint8_t)kStage;
                     evals += (uint64_t)n * kSub;
                 }
                 __builtin_amdgcn_wave_barrier();
@@ -512,13 +513,21 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                 if (XY) za = LWT[nw * 64 + lj];
                 // stream weights of the D row this lane's row broadcasts
                 double wn[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-                auto load_weights = [&](int slot) __attribute__((always_inline)) {
-                    const double* w = SWm + (uint32_t)((ID[slot] & kRowMask) * (uint32_t)wst);
+                auto load_weights = [&](uint32_t row) __attribute__((always_inline)) {
+                    const double* w = SWm + (uint32_t)(row * (uint32_t)wst);
 #pragma unroll
                     for (int c = 0; c < 5; c++)
                         if (c < nw) wn[c] = w[c];
                 };
-                if (F64) load_weights(list[brow]);
+                // (loaded a tile ahead, their rows two and the slots three: the chain of
+                // reads does not hold up a tile)
+                uint32_t wrow = 0u;
+                int wslot = 0;
+                if (F64) {
+                    load_weights(ID[list[brow]] & kRowMask);
+                    wrow = ID[list[kSub + brow]] & kRowMask;
+                    wslot = list[2 * kSub + brow];
+                }
                 // operands one tile ahead, their slots two
                 double a = comp[list[lrow]];
                 int slot2 = list[kSub + lrow];
@@ -532,7 +541,9 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                         // this tile's stream weights were loaded a tile ago
 #pragma unroll
                         for (int c = 0; c < 5; c++) wb[c] = wn[c];
-                        load_weights(list[t0 + kSub + brow]);
+                        load_weights(wrow);
+                        wrow = ID[wslot] & kRowMask;
+                        wslot = list[t0 + 3 * kSub + brow];
                     }
                     // (the next operands' reads go out before the product, which would otherwise
                     // hold them back: its result registers are reused at once)
