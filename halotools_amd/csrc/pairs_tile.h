@@ -434,6 +434,8 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
             return k;
         };
 
+        const uint32_t own0 = (uint32_t)(p0 - (int64_t)sbase);  // the group's first row, in one sample
+
         // ---- staged points: deal them to the sub-groups, evaluate the tiles
         // self: the slots hold the group's own points
         int qlen = 0;
@@ -612,9 +614,13 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                             if (oi) {
                                 const int slot = list[t0 + (lane >> 4) * 4 + i];
                                 const uint32_t kb = hv < (int)floor_hi || ek == 0u ? 0u : ek - 1u;
-                                uint32_t kq = 0u;
-                                uint32_t kk = exact_bin(s * kSub + (lane & 15), slot, kb, kq, false);
-                                if (MODE == kModeJac && !SWAP && L.corr != nullptr) {
+                                uint32_t kq = 0u, kk = 0u;
+                                // (a Jacobian's points meet themselves in the tiles, at
+                                // distance 0: 64 exact evaluations per group otherwise)
+                                const bool itself = MODE == kModeJac && L.lane.x == L.strm.x &&
+                                                    ID[slot] == (own0 + (uint32_t)lj | ((uint32_t)kHere << kImgShift));
+                                if (!itself) kk = exact_bin(lj, slot, kb, kq, false);
+                                if (MODE == kModeJac && !SWAP && L.corr != nullptr && !itself) {
                                     // Auto-count with one set of weights: the sample-2 rows take
                                     // the pair's other orientation, which across the periodic seam
                                     // may round into another bin; those disagreements are recorded,
@@ -830,7 +836,6 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
             jj = (uint32_t)(min(at + lane, total - 1) + __builtin_amdgcn_ds_bpermute(sg, run));
             img = seam ? __builtin_amdgcn_ds_bpermute(sg, cimg) : kHere;
         };
-        const uint32_t own0 = (uint32_t)(p0 - (int64_t)sbase);  // the group's first row, in one sample
         bool more = next();
         double4 row = make_double4(0.0, 0.0, 0.0, 0.0);
         uint32_t jn = 0;
