@@ -160,6 +160,7 @@ static TileTable make_tile_table(const std::vector<double>& e, int K) {
         T.spec.hi = (uint32_t)((base + nb - 1) << shift);
         T.spec.sh3 = (uint32_t)shift - 3;
         T.spec.mask = n - 1;
+        T.spec.first = hiword(e[0]);
         T.spec.ok = 1;
         return T;
     }

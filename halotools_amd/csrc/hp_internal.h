@@ -63,6 +63,7 @@ struct TileSpec {
     uint32_t lo, hi; // clamp: first value of the lowest and of the highest bucket
     uint32_t sh3;    // shift - 3 (entries are 8 bytes)
     uint32_t mask;   // entries - 1 (a power of two)
+    uint32_t first;  // high word of the smallest edge
     int32_t ok;      // the edges fit such a table
 };
 

@@ -112,8 +112,13 @@ static int tile_layout(int mode, int K, int Kp, int nw, int also, int var, TileA
         case kModeXYZ:
             // few cells (wp: one pi bin) in up to 32 columns, so that the lanes of
             // one LDS pass rarely meet on one cell
-            while (A.ccol_sh < 5 && (K * Kp * 4 << (A.ccol_sh + 1)) <= 4096) A.ccol_sh++;
-            h = K * Kp * 4 << A.ccol_sh;
+            if (var) {
+                while (A.ccol_sh < 5 && (K * Kp * 4 << (A.ccol_sh + 1)) <= 4096) A.ccol_sh++;
+                h = K * Kp * 4 << A.ccol_sh;
+            } else {
+                while (A.ccol_sh < 5 && ((K + 1) * (Kp + 1) * 4 << (A.ccol_sh + 1)) <= 4096) A.ccol_sh++;
+                h = (K + 1) * (Kp + 1) * 4 << A.ccol_sh;
+            }
             break;
         case kModeWXYZ: h = K * Kp * 8; break;
         case kModeObj: h = (K + 1) * 256; break;

@@ -164,12 +164,28 @@ __device__ __forceinline__ uint2 lds_entry(uint32_t off) {
     const unsigned long long v = *(lds_u64*)(uintptr_t)off;
     return make_uint2((uint32_t)v, (uint32_t)(v >> 32));
 }
+// t = e - c; the address step: lo, or hi where e < c
+__device__ __forceinline__ void edge_step(uint32_t e, uint32_t c, uint32_t lo, uint32_t hi, uint32_t& t, uint32_t& step) {
+    asm("v_sub_co_u32_e32 %0, vcc, %2, %3\n\tv_cndmask_b32_e32 %1, %4, %5, vcc"
+        : "=&v"(t), "=v"(step)
+        : "v"(e), "v"(c), "v"(lo), "v"(hi)
+        : "vcc");
+}
 // t = e - c, kout = k + (e < c): one subtraction with borrow, one addition with carry
 __device__ __forceinline__ void sub_borrow(uint32_t e, uint32_t c, uint32_t k, uint32_t& t, uint32_t& kout) {
     asm("v_sub_co_u32_e32 %0, vcc, %2, %3\n\tv_addc_co_u32_e32 %1, vcc, 0, %4, vcc"
         : "=&v"(t), "=v"(kout)
         : "v"(e), "v"(c), "v"(k)
         : "vcc");
+}
+// additions at a byte offset of the workgroup's LDS
+__device__ __forceinline__ void lds_add(uint32_t off, uint32_t v) {
+    typedef __attribute__((address_space(3))) uint32_t lds_u32;
+    __hip_atomic_fetch_add((lds_u32*)(uintptr_t)off, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void lds_add(uint32_t off, double v) {
+    typedef __attribute__((address_space(3))) double lds_f64;
+    __hip_atomic_fetch_add((lds_f64*)(uintptr_t)off, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 // VAR: product marks compiled in (kModeWSum, kModeWXYZ: 1; 2: two weights per
@@ -199,15 +215,31 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
     const int nw = !F64 ? 0 : (TAN ? 2 : ((MODE == kModeJac || PROD || JK) ? 1 : (VAR == 2 ? 2 : L.nw)));
     const int wst = JK ? 2 : nw;  // doubles per weight row (jackknife: weight and tag)
     unsigned char* const wsm = lds + A.tab_bytes + wid * A.wave_bytes;
-    // entries of the tables: k becomes the byte offset of the bin's row (column)
+    // Bytes from a bin's histogram row to the next (and from a pi bin to the
+    // next): the tables' entries hold the bin's offset, so that a pair's address
+    // takes a select and an addition per table, and rows of pairs beyond the
+    // last edge exist and are not read (adding under a mask costs more than
+    // their space: per-object rows 1195 -> 1266 us).  Where many pairs would
+    // meet on a few such cells (one histogram column), the bins' numbers are kept
+    // instead and those pairs masked off ((rp, pi) counts 1905 -> 2090 us without).
+    constexpr uint32_t TC = kTanCols, TR = 8u * TC;  // forward mode: columns of the W, dW and count rows
+    constexpr bool CELL = MODE == kModeWXYZ || (MODE == kModeXYZ && VAR);
+    const uint32_t rbytes = CELL ? 1u
+                            : MODE == kModeXYZ ? (uint32_t)(Kp + 1) << (2 + A.ccol_sh)
+                            : (MODE == kModeObj || (JK && !VAR)) ? 256u
+                            : (MODE == kModeJac || JK) ? 512u
+                            : TAN ? (ALSO ? 3u : 2u) * TR : 128u;
+    const uint32_t pbytes = CELL ? 1u : (MODE == kModeXYZ ? 4u << A.ccol_sh : 0x10000u);
     {
         const uint2* gt = reinterpret_cast<const uint2*>(static_cast<const char*>(L.ws) + A.tr.off);
         uint2* st = reinterpret_cast<uint2*>(lds);
-        for (int i = threadIdx.x; i <= (int)A.tr.mask; i += WAVES * 64) st[i] = gt[i];
+        for (int i = threadIdx.x; i <= (int)A.tr.mask; i += WAVES * 64)
+            st[i] = make_uint2(gt[i].x, gt[i].y * rbytes);
         if (XY) {
             const uint2* gp = reinterpret_cast<const uint2*>(static_cast<const char*>(L.ws) + A.tp.off);
             uint2* sp = reinterpret_cast<uint2*>(lds + A.tp_off);
-            for (int i = threadIdx.x; i <= (int)A.tp.mask; i += WAVES * 64) sp[i] = gp[i];
+            for (int i = threadIdx.x; i <= (int)A.tp.mask; i += WAVES * 64)
+                sp[i] = make_uint2(gp[i].x, gp[i].y * pbytes);
         }
     }
     double* const SX = reinterpret_cast<double*>(wsm);  // x[kSlots], y, z, n
@@ -285,8 +317,9 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
         float hx, hy, hz;     // half sizes, with the eps margin
         double cx, cy, cz;
         double Bf[4], NA[4];  // per sub-group: the tile's B operand and |a|^2
-        uint32_t floor_hi;    // pairs below this high word are evaluated exactly
-        uint32_t floor_pi = 0u;  // ... (rp, pi): below this high word of dz^2
+        int floor_hi;         // pairs below this high word are evaluated exactly
+        int floor_pi = 0;     // ... (rp, pi): below this high word of dz^2
+        bool low;             // ... which only matters where an edge is not above it
         {
             const float INF = __builtin_inff();
             const float eps = geom->eps;
@@ -368,8 +401,13 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
             const double Lmax = fmax(fmax(geom->period[0], geom->period[1]), geom->period[2]);
             const double fl2 = Lmax * Lmax * 3.5527136788005009e-15;                          // 2^-48
             const double fl = (double)(h * h + hr * hr) * 2.9802322387695312e-08 + fl2;      // 2^-25
-            floor_hi = (uint32_t)uni((int)(__double2hiint(fl) + 1));
-            if (XY) floor_pi = (uint32_t)uni((int)(__double2hiint(fl2) + 1));
+            floor_hi = uni(__double2hiint(fl) + 1);
+            // (below every edge, all of them lie in the first bin)
+            low = CELL || floor_hi + 2 >= (int)A.tr.first;
+            if (XY) {
+                floor_pi = uni(__double2hiint(fl2) + 1);
+                low = low || floor_pi + 2 >= (int)A.tp.first;
+            }
         }
 
         bool self_done = false;
@@ -384,9 +422,10 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
         // histogram columns: u32 rows of 32 columns, f64 rows of 16 (no two lanes of
         // one LDS pass on one address); per lane point for object rows and Jacobians
         const uint32_t col4 = (uint32_t)(lane & 31) * 4u, col8 = (uint32_t)(lane & 15) * 8u;
-        constexpr uint32_t TC = kTanCols, TR = 8u * TC;  // forward mode: columns of the W, dW and count rows
         const uint32_t tcol8 = (uint32_t)(lane & (TC - 1)) * 8u, tcol4 = (uint32_t)(lane & (2 * TC - 1)) * 4u;
         const uint32_t ccol = (uint32_t)A.ccol_sh, ccl = (uint32_t)(lane & ((1 << A.ccol_sh) - 1));
+        const uint32_t hbase = (uint32_t)(A.tab_bytes + wid * A.wave_bytes + A.hist_off);
+        const uint32_t cbase = (uint32_t)(A.tab_bytes + wid * A.wave_bytes + A.cnt_off);
         uint64_t evals = 0;
         const double* const SWm = F64 ? L.strm.w + (int64_t)sbase * wst : nullptr;
 
@@ -500,6 +539,12 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                 const dbl4 cc = {ns, ns, ns, ns};
                 // this sub-group's lane points: weights and z
                 const int lj = s * kSub + (lane & 15);
+                // the first bin's address for this lane, the second's, the one past the last edge
+                const uint32_t adr0 = CELL ? 0u : hbase + (MODE == kModeXYZ ? ccl * 4u
+                                               : (MODE == kModeObj || (JK && !VAR)) ? (uint32_t)lj * 4u
+                                               : (MODE == kModeJac || JK) ? (uint32_t)lj * 8u
+                                               : TAN ? tcol8 : (MODE == kModeWSum ? col8 : col4));
+                const uint32_t adr1 = adr0 + rbytes, trash = adr0 + (uint32_t)K * rbytes;
                 double lw[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
                 if (F64) {
 #pragma unroll
@@ -552,9 +597,9 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                     __builtin_amdgcn_sched_barrier(0);
                     const dbl4 D = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bs, cc, 0, 0, 0);
                     a = a1;
-                    int hi[4], hp[4];
+                    int hi[4], hp[4], c[4];
                     uint2 ent[4], enp[4];
-                    uint32_t t[4], k[4], tp[4], kp[4];
+                    uint32_t t[4], st[4], tp[4], sp[4], adr[4], pad[4];  // (addresses: row, pi part)
 #pragma unroll
                     for (int i = 0; i < 4; i++) hi[i] = __double2hiint(D[i]);
                     bool diag = false;
@@ -571,8 +616,8 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                     }
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
-                        const uint32_t off = ((uint32_t)med3i(hi[i], tlo, thi) >> tsh) & tmask;
-                        ent[i] = lds_entry(off);
+                        c[i] = med3i(hi[i], tlo, thi);
+                        ent[i] = lds_entry(((uint32_t)c[i] >> tsh) & tmask);
                     }
                     if (XY) {
                         double dz[4];
@@ -588,32 +633,50 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                         }
                     }
 #pragma unroll
-                    for (int i = 0; i < 4; i++) sub_borrow(ent[i].x, (uint32_t)hi[i], ent[i].y, t[i], k[i]);
-                    uint32_t tm = min(min(t[0], t[1]), min(t[2], t[3]));
-                    const int hm = min(min(hi[0], hi[1]), min(hi[2], hi[3]));
-                    bool odd = tm <= 2u || hm < (int)floor_hi;
+                    for (int i = 0; i < 4; i++) {
+                        // (the clamped value: rounding may leave a square below zero)
+                        if (CELL) {
+                            sub_borrow(ent[i].x, (uint32_t)hi[i], ent[i].y, t[i], adr[i]);
+                        } else {
+                            edge_step(ent[i].x, (uint32_t)c[i], adr0, adr1, t[i], st[i]);
+                            adr[i] = ent[i].y + st[i];
+                        }
+                    }
+                    uint64_t odd = (uint64_t)__ballot(min(min(t[0], t[1]), min(t[2], t[3])) <= 2u);
                     if (XY) {
 #pragma unroll
-                        for (int i = 0; i < 4; i++) sub_borrow(enp[i].x, (uint32_t)hp[i], enp[i].y, tp[i], kp[i]);
-                        const uint32_t pm = min(min(tp[0], tp[1]), min(tp[2], tp[3]));
-                        const int qm = min(min(hp[0], hp[1]), min(hp[2], hp[3]));
-                        odd = odd || pm <= 2u || qm < (int)floor_pi;
+                        for (int i = 0; i < 4; i++) {
+                            if (CELL) {
+                                sub_borrow(enp[i].x, (uint32_t)hp[i], enp[i].y, tp[i], pad[i]);
+                            } else {
+                                edge_step(enp[i].x, (uint32_t)hp[i], 0u, pbytes, tp[i], sp[i]);
+                                pad[i] = enp[i].y + sp[i];
+                            }
+                        }
+                        odd |= (uint64_t)__ballot(min(min(tp[0], tp[1]), min(tp[2], tp[3])) <= 2u);
                     }
-                    if (__builtin_expect((uint64_t)__ballot(odd) != 0, 0)) {
+                    if (CELL || low) {
+                        if (!CELL) asm volatile("");  // (a branch: most groups have no use for this)
+                        odd |= (uint64_t)__ballot(min(min(hi[0], hi[1]), min(hi[2], hi[3])) < floor_hi);
+                        if (XY) odd |= (uint64_t)__ballot(min(min(hp[0], hp[1]), min(hp[2], hp[3])) < floor_pi);
+                    }
+                    if (__builtin_expect(odd != 0, 0)) {
 #pragma unroll 1
                         for (int i = 0; i < 4; i++) {
                             const uint32_t ti = i == 0 ? t[0] : (i == 1 ? t[1] : (i == 2 ? t[2] : t[3]));
                             const int hv = i == 0 ? hi[0] : (i == 1 ? hi[1] : (i == 2 ? hi[2] : hi[3]));
-                            const uint32_t ek = i == 0 ? ent[0].y : (i == 1 ? ent[1].y : (i == 2 ? ent[2].y : ent[3].y));
-                            bool oi = ti <= 2u || hv < (int)floor_hi;
+                            const uint32_t eo = i == 0 ? ent[0].y : (i == 1 ? ent[1].y : (i == 2 ? ent[2].y : ent[3].y));
+                            bool oi = ti <= 2u || (low && hv < floor_hi);
                             if (XY) {
                                 const uint32_t pi = i == 0 ? tp[0] : (i == 1 ? tp[1] : (i == 2 ? tp[2] : tp[3]));
                                 const int hq = i == 0 ? hp[0] : (i == 1 ? hp[1] : (i == 2 ? hp[2] : hp[3]));
-                                oi = (oi || pi <= 2u || hq < (int)floor_pi) && hv < 0x7e000000;
+                                oi = (oi || pi <= 2u || (low && hq < floor_pi)) && hv < 0x7e000000;
                             }
                             if (oi) {
                                 const int slot = list[t0 + (lane >> 4) * 4 + i];
-                                const uint32_t kb = hv < (int)floor_hi || ek == 0u ? 0u : ek - 1u;
+                                // (a bin's number from its offset, exactly: both are far below 2^22)
+                                const uint32_t ek = (uint32_t)((float)eo / (float)rbytes + 0.5f);
+                                const uint32_t kb = (low && hv < floor_hi) || ek == 0u ? 0u : ek - 1u;
                                 uint32_t kq = 0u, kk = 0u;
                                 // (a Jacobian's points meet themselves in the tiles, at
                                 // distance 0: 64 exact evaluations per group otherwise)
@@ -663,8 +726,8 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
 #pragma unroll
                                 for (int u = 0; u < 4; u++)
                                     if (i == u) {
-                                        k[u] = kk;
-                                        if (XY) kp[u] = kq;
+                                        adr[u] = adr0 + kk * rbytes;
+                                        if (XY) pad[u] = kq * pbytes;
                                     }
                             }
                         }
@@ -683,61 +746,40 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                                                                     : (i == 2 ? row_bcast<2>(wb[c]) : row_bcast<3>(wb[c]))));
                         }
                         if constexpr (MODE == kModeCount3D) {
-                            __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hist + ((k[i] << 7) + col4)), inc,
-                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                            lds_add(adr[i], inc);
                         } else if constexpr (MODE == kModeProj) {
-                            // beyond pi_max: the trash row
-                            const uint32_t kk = kp[i] == 0u ? k[i] : (uint32_t)K;
-                            __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hist + ((kk << 7) + col4)), inc,
-                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                        } else if constexpr (MODE == kModeXYZ || MODE == kModeWXYZ) {
-                            // one [K][Kp] histogram per wave; pairs beyond an edge skip it
-                            if (k[i] < (uint32_t)K && kp[i] < (uint32_t)Kp) {
-                                const uint32_t cell = __umul24(k[i], (uint32_t)Kp) + kp[i];
-                                if constexpr (MODE == kModeXYZ) {
-                                    __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hist) + ((cell << ccol) + ccl), inc, __ATOMIC_RELAXED,
-                                                           __HIP_MEMORY_SCOPE_WORKGROUP);
-                                } else {
-                                    const double v = PROD ? lw[0] * sw[0] : wfunc_eval(L.wfunc, lw, sw);
-                                    __hip_atomic_fetch_add(reinterpret_cast<double*>(hist) + cell, v, __ATOMIC_RELAXED,
-                                                           __HIP_MEMORY_SCOPE_WORKGROUP);
-                                }
+                            lds_add(min(adr[i] + pad[i], trash), inc);  // beyond pi_max: the row past the last edge
+                        } else if constexpr (MODE == kModeXYZ && !VAR) {
+                            lds_add(adr[i] + pad[i], inc);
+                        } else if constexpr (CELL) {
+                            if (adr[i] < (uint32_t)K && pad[i] < (uint32_t)Kp) {
+                                const uint32_t cell = __umul24(adr[i], (uint32_t)Kp) + pad[i];
+                                if constexpr (MODE == kModeXYZ)
+                                    lds_add((cell << (ccol + 2)) + (hbase + ccl * 4u), inc);
+                                else
+                                    lds_add(cell * 8u + hbase, PROD ? lw[0] * sw[0] : wfunc_eval(L.wfunc, lw, sw));
                             }
                         } else if constexpr (MODE == kModeObj || (JK && !VAR)) {
-                            __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hist + ((k[i] << 8) + (uint32_t)lj * 4u)), 1u,
-                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                        } else {
-                            if constexpr (MODE == kModeJac || JK) {
-                                __hip_atomic_fetch_add(reinterpret_cast<double*>(hist + ((k[i] << 9) + (uint32_t)lj * 8u)),
-                                                       sw[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                            } else if constexpr (MODE == kModeTan) {
-                                // pair terms w_i w_j and t_i w_j + w_i t_j (t = dw/dtheta); the
-                                // group's own pairs: ordered ones inside a sub-group count half
-                                if (k[i] < (uint32_t)K) {
-                                    double wj = sw[0], tj = sw[1];
-                                    if (diag) {
-                                        wj *= 0.5;
-                                        tj *= 0.5;
-                                    }
-                                    const double v = lw[0] * wj;
-                                    const double tv = __builtin_fma(lw[0], tj, lw[1] * wj);
-                                    unsigned char* const r = hist + __umul24(k[i], ALSO ? 3 * TR : 2 * TR);
-                                    __hip_atomic_fetch_add(reinterpret_cast<double*>(r + tcol8), v, __ATOMIC_RELAXED,
-                                                           __HIP_MEMORY_SCOPE_WORKGROUP);
-                                    __hip_atomic_fetch_add(reinterpret_cast<double*>(r + TR + tcol8), tv, __ATOMIC_RELAXED,
-                                                           __HIP_MEMORY_SCOPE_WORKGROUP);
-                                    if (ALSO)
-                                        __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(r + 2 * TR + tcol4), inc,
-                                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                            lds_add(adr[i], 1u);
+                        } else if constexpr (MODE == kModeJac || JK) {
+                            lds_add(adr[i], sw[0]);
+                            if (ALSO) lds_add(((adr[i] - adr0) >> 2) + cbase + col4, 1u);
+                        } else if constexpr (MODE == kModeTan) {
+                            // pair terms w_i w_j and t_i w_j + w_i t_j (t = dw/dtheta); the
+                            // group's own pairs: ordered ones inside a sub-group count half
+                            if (adr[i] < trash) {
+                                double wj = sw[0], tj = sw[1];
+                                if (diag) {
+                                    wj *= 0.5;
+                                    tj *= 0.5;
                                 }
-                            } else if constexpr (MODE == kModeWSum) {
-                                const double v = PROD ? lw[0] * sw[0] : wfunc_eval(L.wfunc, lw, sw);
-                                __hip_atomic_fetch_add(reinterpret_cast<double*>(hist + ((k[i] << 7) + col8)), v,
-                                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                                lds_add(adr[i], lw[0] * wj);
+                                lds_add(adr[i] + TR, __builtin_fma(lw[0], tj, lw[1] * wj));
+                                if (ALSO) lds_add(adr[i] + (2 * TR + tcol4 - tcol8), inc);
                             }
-                            if constexpr (ALSO && MODE != kModeTan)
-                                __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(wsm + A.cnt_off + ((k[i] << 7) + col4)), 1u,
-                                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        } else {
+                            lds_add(adr[i], PROD ? lw[0] * sw[0] : wfunc_eval(L.wfunc, lw, sw));
+                            if (MODE == kModeWSum && ALSO) lds_add(adr[i] - adr0 + cbase + col4, 1u);
                         }
                     }
                 }
@@ -948,7 +990,8 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
             const uint32_t* h = reinterpret_cast<const uint32_t*>(hist);
             for (int k = lane; k < K * Kp; k += 64) {
                 uint64_t tot = 0;
-                for (int c = 0; c < (1 << ccol); c++) tot += h[(k << ccol) + ((c + lane) & ((1 << ccol) - 1))];
+                const uint32_t cell = CELL ? (uint32_t)k : (uint32_t)k + (uint32_t)k / (uint32_t)Kp;  // (rows of Kp + 1)
+                for (int c = 0; c < (1 << ccol); c++) tot += h[(cell << ccol) + ((c + lane) & ((1 << ccol) - 1))];
                 if (tot) __hip_atomic_fetch_add(cacc + k, tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         } else if constexpr (MODE == kModeCount3D || MODE == kModeProj || ALSO) {
