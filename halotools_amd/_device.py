@@ -333,6 +333,28 @@ def enclose_rows(cols1, cols2):
     return rows1, rows2, hi - lo
 
 
+def tag_stats(t1, t2, n_samples):
+    """((smallest, largest, missing), the same of t2) of int64 device tags, or None
+    where they are not plain contiguous ones or n_samples is not in [1, 65536]."""
+    if not isinstance(n_samples, (int, np.integer)) or not 1 <= n_samples <= 65536:
+        return None
+    for t in (t1, t2):
+        if (type(t) is not torch.Tensor or not t.is_cuda or t.dtype != torch.int64 or t.dim() != 1 or len(t) == 0
+                or not t.is_contiguous() or t.device != t1.device
+                or torch._C._functorch.is_functorch_wrapped_tensor(t)):
+            return None
+    one = t1.data_ptr() == t2.data_ptr() and len(t1) == len(t2)
+    need = 6 + 512 * (2 + (int(n_samples) + 63) // 64)
+    out = torch.empty(need, dtype=torch.int64, device=t1.device)
+    with torch.cuda.device(t1.device):
+        E.check(E.library().hp_tag_stats(
+            ctypes.c_void_p(t1.data_ptr()), len(t1), None if one else ctypes.c_void_p(t2.data_ptr()), len(t2),
+            int(n_samples), ctypes.c_void_p(out.data_ptr()), need,
+            ctypes.c_void_p(torch.cuda.current_stream(t1.device).cuda_stream)))
+        host = out[:6].tolist()
+    return tuple(host[:3]), tuple(host[:3] if one else host[3:])
+
+
 def zheng07_tangent(log_mass, mock_id, logMmin, sigma, out):
     """out[:, 0] = Zheng07 central weights, out[:, 1] = their logMmin
     derivatives, per point of mock mock_id[i] (one library kernel; the same

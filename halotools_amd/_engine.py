@@ -35,7 +35,7 @@ EXPORTED_SYMBOLS = (
     "hp_marked_npairs_xy_z", "hp_npairs_jackknife_3d", "hp_npairs_jackknife_xy_z", "hp_marked_backward",
     "hp_segment_sum_scratch", "hp_segment_sum", "hp_debug_bin_lookup", "hp_debug_hilbert",
     "hp_debug_tile_lookup",
-    "hp_npairs_3d_noalloc", "hp_zheng07_tangent", "hp_enclose",
+    "hp_npairs_3d_noalloc", "hp_zheng07_tangent", "hp_enclose", "hp_tag_stats",
 )
 
 
@@ -130,6 +130,9 @@ def library():
     lib.hp_enclose.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_int64, ctypes.c_int64, ctypes.c_int64,
                                ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]
     lib.hp_enclose.restype = ctypes.c_int
+    lib.hp_tag_stats.argtypes = [ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_int32,
+                                 ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]
+    lib.hp_tag_stats.restype = ctypes.c_int
     lib.hp_debug_bin_lookup.argtypes = [ctypes.POINTER(ctypes.c_double), ctypes.c_int32,
                                         ctypes.POINTER(ctypes.c_double), ctypes.c_int64,
                                         ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32)]

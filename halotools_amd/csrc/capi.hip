@@ -1081,6 +1081,19 @@ int hp_enclose(const double* const* cols, int64_t stride1, int64_t n1, int64_t s
     return 0;
 }
 
+int hp_tag_stats(const int64_t* tags1, int64_t n1, const int64_t* tags2, int64_t n2, int32_t n_samples, int64_t* out,
+                 int64_t out_elems, void* stream) {
+    if (!tags1 || !out) return fail("null pointer");
+    if (n1 < 1 || (tags2 && n2 < 1)) return fail("bad sizes");
+    const int64_t need = tag_scratch(n_samples);
+    if (need < 0) return fail("n_samples out of range");
+    if (out_elems < 6 + need) return fail("output too small");
+    if (launch_tag_stats(tags1, n1, tags2, n2, n_samples, out, out + 6, static_cast<hipStream_t>(stream)))
+        return fail("tag launch failed");
+    g_err.clear();
+    return 0;
+}
+
 int64_t hp_segment_sum_scratch(const int64_t* offsets, int32_t nmocks) {
     if (!offsets || nmocks < 1) return fail("bad arguments");
     for (int m = 0; m < nmocks; m++)

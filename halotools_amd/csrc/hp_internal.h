@@ -255,6 +255,12 @@ int64_t enclose_scratch();
 int launch_enclose(const double* const* c1, int64_t st1, int64_t n1, const double* const* c2, int64_t st2, int64_t n2,
                    double* rows1, double* rows2, double* lohi, double* scratch, hipStream_t s);
 
+// Smallest and largest tag of one or two samples (t2 null: one) and the number of
+// tags 1 .. nsamp missing; scratch: tag_scratch(nsamp) words (< 0: too many tags).
+int64_t tag_scratch(int nsamp);
+int launch_tag_stats(const int64_t* t1, int64_t n1, const int64_t* t2, int64_t n2, int nsamp, int64_t* out,
+                     int64_t* scratch, hipStream_t s);
+
 int64_t segment_sum_scratch(const int64_t* offsets, int nmocks);
 int launch_segment_sum(const double* v, const int64_t* offsets, int nmocks, double* out, double* scratch,
                        hipStream_t s);

@@ -74,17 +74,20 @@ def _process_weights_jtags(sample1, sample2, weights1, weights2, jtags1, jtags2,
     """PC/npairs_jackknife_3d.py:217-276 (identical in PC/npairs_jackknife_xy_z.py:202-261)."""
     weights1 = _as_weights(weights1, sample1, "weights1")
     weights2 = _as_weights(weights2, sample2, "weights2")
+    shared = jtags2 is jtags1
     jtags1 = _as_tags(jtags1, sample1, "jtags1")
-    jtags2 = _as_tags(jtags2, sample2, "jtags2")
-    if _min(jtags1) < 1:
+    jtags2 = _as_tags(jtags1 if shared else jtags2, sample2, "jtags2")
+    # device tags: one pass and one copy back for all the checks
+    stats = D.tag_stats(jtags1, jtags2, N_samples)
+    if (stats[0][0] if stats else _min(jtags1)) < 1:
         raise HalotoolsError("jtags1 must be >= 1")
-    if _min(jtags2) < 1:
+    if (stats[1][0] if stats else _min(jtags2)) < 1:
         raise HalotoolsError("jtags2 must be >= 1")
-    if _max(jtags1) > N_samples:
+    if (stats[0][1] if stats else _max(jtags1)) > N_samples:
         raise HalotoolsError("jtags1 must be <= N_samples")
-    if _max(jtags2) > N_samples:
+    if (stats[1][1] if stats else _max(jtags2)) > N_samples:
         raise HalotoolsError("jtags2 must be <= N_samples")
-    covers = _covers_all(jtags1, N_samples)
+    covers = stats[0][2] == 0 if stats else _covers_all(jtags1, N_samples)
     if not covers:
         warn("Warning: sample1 does not contain points in every jackknife sample.")
     # the reference tests jtags1 again for its sample2 warning (PC/npairs_jackknife_3d.py:273-274)

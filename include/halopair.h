@@ -234,6 +234,12 @@ int hp_segment_sum(const double* values, const int64_t* offsets, int32_t nmocks,
 int hp_enclose(const double* const* cols, int64_t stride1, int64_t n1, int64_t stride2, int64_t n2, double* out,
                int64_t out_elems, void* stream);
 
+/* Jackknife tags of one or two samples (tags2 null: one), int64 on the device: out[0..2] = smallest, largest, number
+ * of the tags 1 .. n_samples that do not occur in sample 1, out[3..5] in sample 2 (PC/npairs_jackknife_3d.py:251-276).
+ * 1 <= n_samples <= 65536; out: 6 + 512 * (2 + (n_samples + 63) / 64) words on the device; only enqueues work. */
+int hp_tag_stats(const int64_t* tags1, int64_t n1, const int64_t* tags2, int64_t n2, int32_t n_samples, int64_t* out,
+                 int64_t out_elems, void* stream);
+
 /* Diagnostics (host only, no GPU needed; used by the CPU test-suite). */
 /* The kernels' bucketed bin lookup: out[i] = number of suffix-minimum edges of r2 below d[i];
  * info = {shift, base, table entries, multi}. */

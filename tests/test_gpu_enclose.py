@@ -64,3 +64,18 @@ def test_row_contraction(gpu, nr, sizes):
     G = torch.randint(-9, 9, (len(sizes), nr), device=gpu, generator=g).double()
     ref = (rows * torch.repeat_interleave(G, torch.as_tensor(sizes, device=gpu), dim=0)).sum(dim=1)
     assert torch.equal(D.backward_rows(rows, G, off), ref)
+
+
+@pytest.mark.parametrize("nsamp", [1, 63, 64, 65, 125, 1000, 65536])
+@pytest.mark.parametrize("n1,n2", [(1, 0), (1023, 5), (1025, 70000), (300001, 0)])
+def test_tag_stats(gpu, n1, n2, nsamp):
+    rng = np.random.default_rng([n1, nsamp])
+    t = [rng.integers(1, nsamp + 1, n) for n in (n1, max(n2, 1))]
+    t[0][n1 // 2] = -7
+    t[1][0] = nsamp + (2 ** 40 if n2 else 0)
+    d = [torch.as_tensor(a, device=gpu) for a in t]
+    got = D.tag_stats(d[0], d[1] if n2 else d[0], nsamp)
+    ref = [(a.min(), a.max(), nsamp - len(np.unique(a[(a >= 1) & (a <= nsamp)]))) for a in (t if n2 else [t[0]] * 2)]
+    assert got == tuple(ref)
+    assert D.tag_stats(d[0].int(), d[0], nsamp) is None and D.tag_stats(d[0][::2], d[0], nsamp) is None or n1 < 3
+    assert D.tag_stats(d[0], d[0], 65537) is None and D.tag_stats(d[0], d[0], 0) is None
