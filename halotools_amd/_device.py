@@ -156,7 +156,7 @@ def launch(res, stream=None):
 
 def prepare(kind, mocks, s1, s2, r2, p2=None, same=False, w1=None, w2=None, nw=0, wfunc=0,
             want_counts=True, want_sums=False, rows1=False, rows2=False, want_evals=False,
-            also_counts=False, device=None, pair_events=None, build_events=None, tile_waves=0, tangent=False,
+            also_counts=False, seam_check=False, device=None, pair_events=None, build_events=None, tile_waves=0, tangent=False,
             jtags1=None, jtags2=None, n_samples=0):
     """Build a request with all of its output and scratch buffers allocated.
 
@@ -166,6 +166,7 @@ def prepare(kind, mocks, s1, s2, r2, p2=None, same=False, w1=None, w2=None, nw=0
     pair_events, build_events : optional (start, end) HIP event handles recorded
         around the pair kernel(s) and around the cell build
     tile_waves : wavefronts per pair-kernel workgroup (1, 2, 4, 8; 0 = library default)
+    seam_check : marked id 1 auto-count with rows1 only: status bit 4 where rows2 would differ
     tangent : marked id 1 with (w, dw/dtheta) weights: also res.tangents, d(sums)/dtheta
     jtags1, jtags2, n_samples : jackknife kinds: int32 device tags (1..n_samples);
         w1 / w2 are then optional (n,) weights and res.sums has shape
@@ -205,6 +206,8 @@ def prepare(kind, mocks, s1, s2, r2, p2=None, same=False, w1=None, w2=None, nw=0
             flags |= E.HP_ALSO_COUNTS
         if tangent:
             flags |= E.HP_TANGENT
+        if seam_check:
+            flags |= E.HP_SEAM_CHECK
     req = E.HpRequest()
     req.kind = kind
     req.flags = flags

@@ -28,6 +28,7 @@ HP_ROWS2 = 4
 HP_NO_SUMS = 8
 HP_ALSO_COUNTS = 16
 HP_TANGENT = 32
+HP_SEAM_CHECK = 64
 
 EXPORTED_SYMBOLS = (
     "hp_last_error", "hp_abi_version", "hp_workspace_size", "hp_npairs_3d",

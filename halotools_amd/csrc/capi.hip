@@ -187,6 +187,7 @@ struct Side {
 
 struct Plan {
     int kind = 0, flags = 0, M = 0;
+    bool seam = false;
     bool same = false, marked = false, rows1 = false, rows2 = false, sums = false, counts = false;
     int nw = 0;
     int64_t n[2] = {0, 0};
@@ -282,6 +283,7 @@ static int make_plan(const hp_request* r, int kind, Plan& P, bool tiles = true) 
     P.obj = (kind == HP_NPAIRS_PER_OBJECT_3D);
     P.rows1 = P.marked && (r->flags & HP_ROWS1);
     P.rows2 = P.marked && (r->flags & HP_ROWS2);
+    P.seam = P.marked && (r->flags & HP_SEAM_CHECK);
     P.sums = P.marked && !(r->flags & HP_NO_SUMS);
     P.counts = (!P.marked && !P.obj && !P.jack) || (P.marked && (r->flags & HP_ALSO_COUNTS));
     P.tangent = P.marked && (r->flags & HP_TANGENT);
@@ -305,6 +307,8 @@ static int make_plan(const hp_request* r, int kind, Plan& P, bool tiles = true) 
         if (P.nw < 1 || P.nw > 5) return fail("weights per point must be in 1..5");
         if ((P.rows1 || P.rows2) && (r->wfunc != 1 || P.nw != 1))
             return fail("per-point rows (HP_ROWS1/2) need weight_func_id 1 with one weight per point");
+        if (P.seam && (!P.same || !P.rows1 || P.rows2))
+            return fail("HP_SEAM_CHECK needs HP_SAME_SAMPLES and HP_ROWS1 without HP_ROWS2");
         if (P.tangent && (r->wfunc != 1 || P.nw != 2 || P.rows1 || P.rows2))
             return fail("HP_TANGENT needs weight_func_id 1 with (w, dw/dtheta) per point and no rows");
     }
@@ -895,6 +899,7 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
         L.corr = corr;
         launch_fill_u32(reinterpret_cast<uint32_t*>(corr), 0u, P.n[0] * (int64_t)P.Kr * 2, s);
     }
+    L.seam = P.seam ? status : nullptr;
     L.crep = P.crep;
     if (P.counts && !P.small)
         launch_fill_u32(reinterpret_cast<uint32_t*>(L.pcount), 0u, (int64_t)P.M * P.crep * P.nb_count * 2, s);
@@ -938,6 +943,7 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
         B.psum = nullptr;
         B.pevals = nullptr;
         B.hkey = nullptr;
+        B.seam = nullptr;
         B.hrows = nullptr;
         // with SAME_SAMPLES the side-1 rows of the geometry equal the side-0 rows
         if (launch_pairs(B, s)) return fail("pair kernel (swapped) launch failed");

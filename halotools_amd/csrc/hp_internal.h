@@ -216,6 +216,7 @@ struct PairLaunch {
     int64_t* orows;        // per-object mode: [n_lane_total][nr] cumulative counts (input order)
     double* rows;          // [n_lane_total][nr] (original order) or nullptr
     double* corr;          // auto-counts: rows2 - rows1 corrections from seam pairs, or nullptr
+    int32_t* seam;         // instead of corr: the status word, bit 4 set where corr would not be zero
     uint64_t* pevals;      // [ngroups]
     // symmetric auto-counts: the Hilbert order keys of the stream points, the
     // fourth word of each 32-byte stream row ((Hilbert key << 32) | input

@@ -683,22 +683,23 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                                 const bool itself = MODE == kModeJac && L.lane.x == L.strm.x &&
                                                     ID[slot] == (own0 + (uint32_t)lj | ((uint32_t)kHere << kImgShift));
                                 if (!itself) kk = exact_bin(lj, slot, kb, kq, false);
-                                if (MODE == kModeJac && !SWAP && L.corr != nullptr && !itself) {
+                                if (MODE == kModeJac && !SWAP && (L.corr != nullptr || L.seam != nullptr) && !itself) {
                                     // Auto-count with one set of weights: the sample-2 rows take
                                     // the pair's other orientation, which across the periodic seam
                                     // may round into another bin; those disagreements are recorded,
                                     // so rows2 = rows1 + corr (as pairs_kernel.h does for every
-                                    // shifted pair; only these can differ).
+                                    // shifted pair; only these can differ), or that there is one.
                                     const uint32_t id = ID[slot];
                                     uint32_t dummy = 0u;
                                     const uint32_t kr = exact_bin(s * kSub + (lane & 15), slot, kb, dummy, true);
                                     if (kr != kk && (id >> kImgShift) != (uint32_t)kHere && s * kSub + (lane & 15) < cnt) {
+                                        if (L.seam) atomicOr(L.seam, 4);
                                         const int64_t sr = (int64_t)sbase + (int64_t)(id & kRowMask);
                                         const int64_t q = __double_as_longlong(L.strm.x[sr * 4 + 3]);
                                         double* crow = L.corr + q * K;
-                                        if (kk < (uint32_t)K)
+                                        if (L.corr && kk < (uint32_t)K)
                                             __hip_atomic_fetch_add(crow + kk, lw[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                                        if (kr < (uint32_t)K)
+                                        if (L.corr && kr < (uint32_t)K)
                                             __hip_atomic_fetch_add(crow + kr, -lw[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                                     }
                                 }

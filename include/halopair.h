@@ -64,6 +64,10 @@ enum hp_flags {
     HP_ROWS2 = 4,        /* marked id 1: write rows2 = d sums / d weights2 per point   */
     HP_NO_SUMS = 8,      /* marked: skip the weighted sums (rows only)                */
     HP_ALSO_COUNTS = 16, /* marked: also produce the unweighted counts of npairs_3d   */
+    HP_SEAM_CHECK = 64,  /* HP_SAME_SAMPLES and HP_ROWS1 without HP_ROWS2: bit 4 of    */
+                         /* the status word tells that rows2 would differ from rows1  */
+                         /* (a pair across the periodic seam whose two orientations   */
+                         /* round into different bins); clear, rows1 serves for both  */
     HP_TANGENT = 32      /* marked, weight_func_id 1 with nw = 2 weights per point    */
                          /* (w, dw/dtheta): sums of w1*w2 and `tangents`, the sums of */
                          /* t1*w2 + w1*t2 = d(sums)/dtheta (forward-mode derivative)  */

@@ -187,3 +187,35 @@ def test_queued_items_agree_with_general(mo, gpu, n1, n2, monkeypatch):
     monkeypatch.setenv("HALOPAIR_NO_TILES", "1")
     for a, b in zip(got, run()):
         assert torch.equal(torch.as_tensor(a), torch.as_tensor(b))
+
+
+@pytest.mark.parametrize("tiles", [True, False])
+@pytest.mark.parametrize("seam", [True, False])
+def test_seam_check(gpu, seam, tiles, monkeypatch):
+    # the status bit tells whether rows2 would differ, and the gradient has it either way
+    import torch
+
+    from halotools_amd import _device as D
+    from halotools_amd import _engine as E
+    from halotools_amd.autodiff import marked_npairs_3d_product
+    if not tiles:
+        monkeypatch.setenv("HALOPAIR_NO_TILES", "1")
+    xi, xj, r = _seam_pair()
+    pts = np.random.default_rng(3).uniform(0, 1, (700, 3))
+    if seam:
+        pts[10], pts[20] = [xi, 0.5, 0.5], [xj, 0.5, 0.5]
+    rb = np.array([0.5 * r, r, 0.2])
+    t = torch.as_tensor(pts, device=gpu)
+    w = torch.randint(1, 9, (700,), device=gpu).double().requires_grad_(True)
+    args = dict(same=True, w1=w.detach().reshape(-1, 1), nw=1, wfunc=1, want_counts=False, want_sums=True, device=gpu)
+    mock = [dict(n1=700, n2=700, period=[1.0] * 3, pbc=True)]
+    chk = D.run(E.HP_MARKED_NPAIRS_3D, mock, t.unbind(1), t.unbind(1), rb * rb, rows1=True, seam_check=True, **args)
+    full = D.run(E.HP_MARKED_NPAIRS_3D, mock, t.unbind(1), t.unbind(1), rb * rb, rows1=True, rows2=True, **args)
+    assert (int(chk.status.item()) & 0xFFFFFFFF) == (4 if seam else 0)
+    assert torch.equal(chk.rows1, full.rows1) and torch.equal(full.rows1, full.rows2) == (not seam)
+    c = torch.tensor([1.0, 2.0, 4.0], dtype=torch.float64, device=gpu)
+    (marked_npairs_3d_product(t, t, rb, w, w, period=1.0) * c).sum().backward()
+    G = torch.tensor([7.0, 6.0, 4.0], dtype=torch.float64, device=gpu)
+    assert torch.equal(w.grad, ((full.rows1 + full.rows2) * G).sum(dim=1))
+    with pytest.raises(E.EngineError):
+        D.run(E.HP_MARKED_NPAIRS_3D, mock, t.unbind(1), t.unbind(1), rb * rb, rows1=True, rows2=True, seam_check=True, **args)
