@@ -751,6 +751,7 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
     // matrix-core kernels: one curve-ordered copy of each side, the stream side's with its cubes
     SortedSide curve[2] = {};
     SmallBuild small = {};
+    const int64_t count_words = P.counts ? (int64_t)P.M * P.crep * P.nb_count * 2 : 0;  // cleared by the build
     for (int sd = 0; P.tiles && sd < (P.same ? 1 : 2); sd++) {
         SortedSide& C = curve[sd];
         C.x = reinterpret_cast<double*>(ws + P.o_crow[sd]);
@@ -785,7 +786,8 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
         st.tile = P.tile[sd];
         st.ntiles = P.ntiles[sd];
         if (build_curve_side(dgeom, P.M, sd, X[sd], Y[sd], Z[sd], P.weighted() ? W[sd] : nullptr, P.nw, P.n[sd],
-                             P.total_cells, P.bits_hilbert, sb, st, C, status, s, rows, XS[sd]))
+                             P.total_cells, P.bits_hilbert, sb, st, C, status, s, rows, XS[sd],
+                             reinterpret_cast<uint32_t*>(ws + P.o_pcount), sd == 0 ? count_words : 0))
             return fail("cell build launch failed");
     }
     if (P.small) {
@@ -795,7 +797,7 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
         small.tile = small_tile(std::max(P.n[0], P.n[P.same ? 0 : 1]));
         small.total_cells = P.total_cells;
         small.clear = P.counts ? reinterpret_cast<uint32_t*>(ws + P.o_pcount) : nullptr;
-        small.clear_words = P.counts ? (int64_t)P.crep * P.nb_count * 2 : 0;
+        small.clear_words = count_words;
         if (build_curve_small(small, P.same ? 1 : 2, s)) return fail("cell build launch failed");
     }
     for (int sd = 0; sd < 2; sd++) {
@@ -901,7 +903,7 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
     }
     L.seam = P.seam ? status : nullptr;
     L.crep = P.crep;
-    if (P.counts && !P.small)
+    if (P.counts && !P.tiles)
         launch_fill_u32(reinterpret_cast<uint32_t*>(L.pcount), 0u, (int64_t)P.M * P.crep * P.nb_count * 2, s);
     int rc = 0;
     phase.begin("halopair: pair kernels");

@@ -440,9 +440,10 @@ int sort_tile(int64_t n) {
 
 // The counting-sort passes of one order: keys from kin0 (or sb.keys[0]), the
 // permutation into perm; returns the buffer that ends up with the sorted keys,
-// or null on a bad tile shape.
+// or null on a bad tile shape.  counted: the first pass's digits are counted.
 static uint32_t* sort_passes(const uint32_t* kin0, const MockGeom* geom, int nmocks, int side, int key_bits,
-                             SortBufs sb, SortTiles st, uint32_t* perm, bool global_ids, hipStream_t s) {
+                             SortBufs sb, SortTiles st, uint32_t* perm, bool global_ids, hipStream_t s,
+                             bool counted = false) {
     const int tile = st.tile, ntiles = st.ntiles;
     if ((tile != kSortTile && tile != kSortTileLarge) || ntiles <= 0) return nullptr;
     const int passes = key_bits <= 0 ? 1 : (key_bits + kRadixBits - 1) / kRadixBits;
@@ -450,7 +451,9 @@ static uint32_t* sort_passes(const uint32_t* kin0, const MockGeom* geom, int nmo
     for (int pass = 0; pass < passes; pass++) {
         const int shift = pass * kRadixBits;
         const uint32_t* kin = (pass == 0 && kin0) ? kin0 : sb.keys[cur];
-        if (tile == kSortTileLarge)
+        if (pass == 0 && counted) {
+            // (k_curve_keys)
+        } else if (tile == kSortTileLarge)
             hipLaunchKernelGGL(k_radix_hist<kSortTileLarge>, dim3(ntiles), dim3(256), 0, s, kin, geom, st.first,
                                nmocks, side, shift, sb.tile_counts, ntiles);
         else
@@ -552,15 +555,67 @@ __global__ void k_gather_curve(const uint32_t* __restrict__ perm, const uint32_t
     if (last) c->y = (uint32_t)(q + 1);
 }
 
+// The Hilbert keys of one mock, the digit counts of the first pass and the
+// clearing of what later kernels add into, in one launch: at 1M points the count
+// and the two fills were 11 us and three launches of their own beside the keys'
+// 16.  A workgroup takes one sort tile, two points a thread.
+__global__ void __launch_bounds__(1024) k_curve_keys(const MockGeom* __restrict__ geom, const double* __restrict__ x,
+                                                     const double* __restrict__ y, const double* __restrict__ z,
+                                                     int64_t n, int64_t xs, uint32_t* __restrict__ keys,
+                                                     int32_t* __restrict__ status, PackedRows rows,
+                                                     uint32_t* __restrict__ tile_counts, uint32_t* __restrict__ cubes,
+                                                     int64_t cube_words, uint32_t* __restrict__ clear,
+                                                     int64_t clear_words) {
+    __shared__ uint32_t h[kRadixDigits];
+    const int64_t gt = blockIdx.x * (int64_t)1024 + threadIdx.x, gn = (int64_t)gridDim.x * 1024;
+    for (int64_t i = gt; i < cube_words; i += gn) cubes[i] = 0u;
+    for (int64_t i = gt; i < clear_words; i += gn) clear[i] = 0u;
+    if (threadIdx.x < kRadixDigits) h[threadIdx.x] = 0u;
+    __syncthreads();
+    const MockGeom& G = geom[0];
+    const int hb = G.mbits, hn = 1 << hb;
+    bool bad = false;
+#pragma unroll
+    for (int r = 0; r < kSortTile / 1024; r++) {
+        const int64_t p = blockIdx.x * (int64_t)kSortTile + r * 1024 + threadIdx.x;
+        if (p >= n) break;
+        const double px = x[p * xs], py = y[p * xs], pz = z[p * xs];
+        cell_index(px, G.inv_cell[0], G.ndiv[0], bad, G.period[0], G.pbc);
+        cell_index(py, G.inv_cell[1], G.ndiv[1], bad, G.period[1], G.pbc);
+        cell_index(pz, G.inv_cell[2], G.ndiv[2], bad, G.period[2], G.pbc);
+        bool dummy = false;
+        const int hx = cell_index(px, G.inv_hcell[0], hn, dummy, G.period[0], 0);
+        const int hy = cell_index(py, G.inv_hcell[1], hn, dummy, G.period[1], 0);
+        const int hz = cell_index(pz, G.inv_hcell[2], hn, dummy, G.period[2], 0);
+        const uint32_t key = hilbert3((uint32_t)hx, (uint32_t)hy, (uint32_t)hz, hb);
+        keys[p] = key;
+        atomicAdd(&h[key & (kRadixDigits - 1)], 1u);
+        if (rows.p)
+            *reinterpret_cast<double4*>(rows.p + p * rows.stride) = make_double4(px, py, pz, __hiloint2double(0, (int)key));
+    }
+    if (bad && status) atomicOr(status, 1);
+    __syncthreads();
+    if (threadIdx.x < kRadixDigits) tile_counts[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = h[threadIdx.x];
+}
+
 int build_curve_side(const MockGeom* geom, int nmocks, int side, const double* x, const double* y, const double* z,
                      const double* w, int nw, int64_t n, int64_t total_cells, int key_bits, SortBufs sb, SortTiles st,
-                     SortedSide out, int32_t* status, hipStream_t s, PackedRows rows, int64_t xs) {
-    if (out.cubes && launch_fill_u32(reinterpret_cast<uint32_t*>(out.cubes), 0u, 2 * total_cells, s)) return -1;
+                     SortedSide out, int32_t* status, hipStream_t s, PackedRows rows, int64_t xs, uint32_t* clear,
+                     int64_t clear_words) {
+    // (batches and the large tiles of tens of millions of points: the launches are nothing there)
+    const bool fused = nmocks == 1 && st.tile == kSortTile && n > 0 && st.ntiles == (n + kSortTile - 1) / kSortTile;
+    if (!fused && clear_words > 0 && launch_fill_u32(clear, 0u, clear_words, s)) return -1;
+    if (!fused && out.cubes && launch_fill_u32(reinterpret_cast<uint32_t*>(out.cubes), 0u, 2 * total_cells, s)) return -1;
     if (n <= 0) return 0;
     const unsigned nb = (unsigned)((n + 255) / 256);
-    hipLaunchKernelGGL(k_keys, dim3(nb), dim3(256), 0, s, geom, nmocks, side, (int)kHilbert, x, y, z, n, sb.keys[0],
-                       status, (uint32_t*)nullptr, (const double*)nullptr, 0, rows, xs);
-    const uint32_t* keys = sort_passes(nullptr, geom, nmocks, side, key_bits, sb, st, out.perm, false, s);
+    if (fused)
+        hipLaunchKernelGGL(k_curve_keys, dim3((unsigned)st.ntiles), dim3(1024), 0, s, geom, x, y, z, n, xs, sb.keys[0],
+                           status, rows, sb.tile_counts, reinterpret_cast<uint32_t*>(out.cubes),
+                           out.cubes ? 2 * total_cells : 0, clear, clear_words);
+    else
+        hipLaunchKernelGGL(k_keys, dim3(nb), dim3(256), 0, s, geom, nmocks, side, (int)kHilbert, x, y, z, n, sb.keys[0],
+                           status, (uint32_t*)nullptr, (const double*)nullptr, 0, rows, xs);
+    const uint32_t* keys = sort_passes(nullptr, geom, nmocks, side, key_bits, sb, st, out.perm, false, s, fused);
     if (!keys) return -1;
     hipLaunchKernelGGL(k_gather_curve, dim3(nb), dim3(256), 0, s, out.perm, keys, n, geom, nmocks, side, x, y, z, xs,
                        rows, w, nw, out.x, out.w, out.cubes);

@@ -154,7 +154,8 @@ int build_sorted_side(const MockGeom* geom, int nmocks, int side, Order order,
 // pass writes them), or none: the gather reads the caller's coordinates.
 int build_curve_side(const MockGeom* geom, int nmocks, int side, const double* x, const double* y, const double* z,
                      const double* w, int nw, int64_t n, int64_t total_cells, int key_bits, SortBufs sb, SortTiles st,
-                     SortedSide out, int32_t* status, hipStream_t s, PackedRows rows, int64_t xs);
+                     SortedSide out, int32_t* status, hipStream_t s, PackedRows rows, int64_t xs,
+                     uint32_t* clear, int64_t clear_words);
 
 // The same for small one-mock requests, both sides in each launch: keys and
 // digit counts, two 9-bit passes, the second writing the rows; clears the cubes
