@@ -61,7 +61,6 @@ class _MarkedProductSums(torch.autograd.Function):
         ctx.rows2 = res.rows1 if same and res.rows2 is None else res.rows2
         ctx.offsets1 = plan["offsets1"]
         ctx.offsets2 = plan["offsets2"]
-        ctx.plan_res = res
         ctx.need = (need1, need2)
         return res.sums
 

@@ -196,3 +196,22 @@ def test_seam_correction_non_integer_weights(gpu):
     np.testing.assert_array_equal(elim.rows1.cpu().numpy(), swapped.rows1.cpu().numpy())
     np.testing.assert_allclose(r2e, r2s, rtol=1e-13, atol=1e-13 * np.abs(r2s).max())
     np.testing.assert_allclose(elim.sums.cpu().numpy(), swapped.sums.cpu().numpy(), rtol=1e-13)
+
+
+def test_gradient_steps_hold_no_memory(ad, gpu):
+    # nothing of a step outlives it, without the garbage collector's help
+    import gc
+    s = random_sample(20000, seed=8)
+    w = torch.tensor(np.random.default_rng(1).uniform(0, 1, 20000), device=gpu, requires_grad=True)
+    rb = np.array([0.02, 0.05])
+    used = []
+    gc.collect()
+    gc.disable()
+    try:
+        for _ in range(3):
+            w.grad = None
+            ad.marked_npairs_3d_product(s, s, rb, w, w, period=1.0).sum().backward()
+            used.append(torch.cuda.memory_allocated(gpu))
+    finally:
+        gc.enable()
+    assert used[0] == used[1] == used[2]
