@@ -624,13 +624,14 @@ int build_curve_side(const MockGeom* geom, int nmocks, int side, const double* x
 
 // ------------------------------------------------------------ small builds
 // A small request is bound by launches and their latency: three kernels build
-// both sides (20k x 20k: 166 -> 71 us of kernels per call, of which the pair
-// kernel is 25).  At most 128 tiles a side, so a workgroup adds up the digit
+// both sides (20k x 20k: 166 -> 66 us of kernels per call, of which the pair
+// kernel is 25; the keys' workgroups have a thread per key, 10.4 -> 5.2 us against
+// four keys a thread).  At most 128 tiles a side, so a workgroup adds up the digit
 // counts of the tiles before its own itself (no scan launch), and the first
 // pass counts the second pass's digits by atomics.
 template <int TILE>
-__global__ void __launch_bounds__(TILE / 4) k_small_keys(const SmallBuild B) {
-    constexpr int NT = TILE / 4;
+__global__ void __launch_bounds__(1024) k_small_keys(const SmallBuild B) {
+    constexpr int NT = 1024;
     __shared__ uint32_t h[kSmallDigits];
     const SmallSide& S = B.s[blockIdx.y];
     const MockGeom& G = B.geom[0];
@@ -769,12 +770,12 @@ int build_curve_small(const SmallBuild& b, int sides, hipStream_t s) {
     // (at least a few workgroups for the clearing)
     const dim3 grid0(tiles < 16 ? 16 : tiles, sides), grid(tiles, sides);
     if (b.tile == 1024) {
-        hipLaunchKernelGGL(k_small_keys<1024>, grid0, dim3(256), 0, s, b);
+        hipLaunchKernelGGL(k_small_keys<1024>, grid0, dim3(1024), 0, s, b);
         if (tiles == 0) return check("small");
         hipLaunchKernelGGL((k_small_scatter<0, 1024>), grid, dim3(kSmallDigits), 0, s, b);
         hipLaunchKernelGGL((k_small_scatter<1, 1024>), grid, dim3(kSmallDigits), 0, s, b);
     } else {
-        hipLaunchKernelGGL(k_small_keys<2048>, grid0, dim3(512), 0, s, b);
+        hipLaunchKernelGGL(k_small_keys<2048>, grid0, dim3(1024), 0, s, b);
         if (tiles == 0) return check("small");
         hipLaunchKernelGGL((k_small_scatter<0, 2048>), grid, dim3(kSmallDigits), 0, s, b);
         hipLaunchKernelGGL((k_small_scatter<1, 2048>), grid, dim3(kSmallDigits), 0, s, b);
