@@ -585,9 +585,12 @@ static int make_plan(const hp_request* r, int kind, Plan& P, bool tiles = true) 
     const int64_t gA = std::max<int64_t>(P.ngroups[0], 1);
     // Small requests split each lane group into work items until the chip has
     // HP_TILE_ITEMS waves per CU to run (rows per lane point are written once,
-    // so those stay whole).
+    // so those stay whole), twice that where up to four items per group give it:
+    // a second round evens out the first (200k generic marks 390 -> 369 us, wp of
+    // 500k 1000 -> 963); eight and sixteen items per group cost more in their own
+    // starts than that gains (60k points: 470 -> 485).
     if (P.tiles && mode != kModeObj && mode != kModeJac)
-        while (P.parts_sh < 4 && (gA << P.parts_sh) < 256 * HP_TILE_ITEMS) P.parts_sh++;
+        while (P.parts_sh < 4 && (gA << P.parts_sh) < 256 * HP_TILE_ITEMS * (P.parts_sh < 2 ? 2 : 1)) P.parts_sh++;
     const int64_t gP = gA << P.parts_sh;  // rows of FP64 partials
     // count accumulators: up to kCountReplicas copies per mock (a group adds
     // into copy group % crep), so the atomics of many groups spread over cache
@@ -1166,8 +1169,11 @@ int hp_debug_tile_lookup(const double* r2, int32_t K, const double* d, int64_t n
         const int32_t h = (int32_t)hiword(d[i]) + off;
         const int32_t c = std::max((int32_t)T.spec.lo, std::min(h, (int32_t)T.spec.hi));
         const size_t at = (size_t)(((uint32_t)c >> (T.spec.sh3 + 3)) & T.spec.mask);
-        const uint32_t edge = T.t[2 * at], t = edge - (uint32_t)h;
-        out[i] = t <= 2u ? -1 : (int32_t)(T.t[2 * at + 1] + (edge < (uint32_t)h ? 1u : 0u));
+        // (kernels subtract the word, or the clamped one)
+        const uint32_t edge = T.t[2 * at], k = T.t[2 * at + 1];
+        const uint32_t t = std::min(edge - (uint32_t)h, edge - (uint32_t)c);
+        const uint32_t k1 = k + (edge < (uint32_t)h ? 1u : 0u), k2 = k + (edge < (uint32_t)c ? 1u : 0u);
+        out[i] = t <= 2u ? -1 : (k1 == k2 ? (int32_t)k1 : -2);
     }
     return 0;
 }

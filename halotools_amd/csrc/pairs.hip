@@ -99,7 +99,7 @@ static int num_compute_units() {
 
 // LDS layout of one wave of the matrix-core kernels: the stage, the weights of
 // staged and lane points (and the lanes' z for (rp, pi) bins), the histogram.
-static int tile_layout(int mode, int K, int Kp, int nw, int also, int var, TileArgs& A) {
+static int tile_layout(int mode, int K, int Kp, int nw, int also, int var, bool many, TileArgs& A) {
     const bool xy = (mode == kModeXYZ || mode == kModeWXYZ || mode == kModeProj);
     A.lw_off = align16(deal_of(mode, var) == 64 ? Stage<64>::kTileBytes : Stage<128>::kTileBytes);
     A.ccol_sh = 0;
@@ -111,12 +111,15 @@ static int tile_layout(int mode, int K, int Kp, int nw, int also, int var, TileA
         case kModeProj: h = (K + 1) * 128; break;
         case kModeXYZ:
             // few cells (wp: one pi bin) in up to 32 columns, so that the lanes of
-            // one LDS pass rarely meet on one cell
+            // one LDS pass rarely meet on one cell; half the space where the launch
+            // has more items than waves, which are then 16 a CU instead of 12 (wp
+            // edges, 500k points: 750 -> 670 us; at 100k, two items a wave, 16 x 4
+            // cells lose 219 -> 234)
             if (var) {
                 while (A.ccol_sh < 5 && (K * Kp * 4 << (A.ccol_sh + 1)) <= 4096) A.ccol_sh++;
                 h = K * Kp * 4 << A.ccol_sh;
             } else {
-                while (A.ccol_sh < 5 && ((K + 1) * (Kp + 1) * 4 << (A.ccol_sh + 1)) <= 4096) A.ccol_sh++;
+                while (A.ccol_sh < 5 && ((K + 1) * (Kp + 1) * 4 << (A.ccol_sh + 1)) <= (many ? 2048 : 4096)) A.ccol_sh++;
                 h = (K + 1) * (Kp + 1) * 4 << A.ccol_sh;
             }
             break;
@@ -156,7 +159,7 @@ static int tile_var(int mode, int K, int Kp, int wfunc, int nw, int swap, int un
 int tile_wave_bytes(int mode, int K, int Kp, int nw, int also) {
     TileArgs A;
     if ((int64_t)K * std::max(Kp, 1) > 65536) return -1;
-    return tile_layout(mode, K, Kp, nw, also, tile_var(mode, K, Kp, 0, nw, 0, 0), A);
+    return tile_layout(mode, K, Kp, nw, also, tile_var(mode, K, Kp, 0, nw, 0, 0), false, A);
 }
 
 // Matrix-core kernels: workgroup shape (the waves per workgroup that keep the
@@ -169,7 +172,8 @@ static int launch_tiles(const PairLaunch& L, int lds_per_block, hipStream_t s) {
     const bool xy = (L.mode == kModeXYZ || L.mode == kModeWXYZ || L.mode == kModeProj);
     const int also = L.also_count ? 1 : 0;
     const int var = tile_var(L.mode, L.br.nbins, L.bp.nbins, L.wfunc, L.nw, L.swap, L.unit);
-    if (tile_layout(L.mode, L.br.nbins, L.bp.nbins, L.nw, also, var, A) < 0) return -1;
+    const bool many = (L.ngroups << L.parts_sh) >= (int64_t)num_compute_units() * 32;
+    if (tile_layout(L.mode, L.br.nbins, L.bp.nbins, L.nw, also, var, many, A) < 0) return -1;
     // tables of 2^n entries, the pi table at a multiple of its size
     A.tp_off = xy ? 8 * (int)std::max(L.tr.mask + 1, L.tp.mask + 1) : 0;
     A.tab_bytes = xy ? A.tp_off + 8 * ((int)L.tp.mask + 1) : 8 * ((int)L.tr.mask + 1);
