@@ -624,7 +624,7 @@ int build_curve_side(const MockGeom* geom, int nmocks, int side, const double* x
 
 // ------------------------------------------------------------ small builds
 // A small request is bound by launches and their latency: three kernels build
-// both sides (20k x 20k: 166 -> 66 us of kernels per call, of which the pair
+// both sides (20k x 20k: 166 -> 64 us of kernels per call, of which the pair
 // kernel is 25; the keys' workgroups have a thread per key, 10.4 -> 5.2 us against
 // four keys a thread).  At most 128 tiles a side, so a workgroup adds up the digit
 // counts of the tiles before its own itself (no scan launch), and the first
@@ -670,13 +670,33 @@ __global__ void __launch_bounds__(1024) k_small_keys(const SmallBuild B) {
     for (int i = threadIdx.x; i < kSmallDigits; i += NT) S.counts[(int64_t)tile * kSmallDigits + i] = h[i];
 }
 
+// Exclusive sums over the workgroup's kSmallDigits threads.
+__device__ __forceinline__ uint32_t small_scan(uint32_t v, uint32_t* tot) {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    uint32_t inc = v;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t u = __shfl_up(inc, off);
+        if (lane >= off) inc += u;
+    }
+    if (lane == 63) tot[wv] = inc;
+    __syncthreads();
+    uint32_t run = inc - v;
+    for (int w = 0; w < kSmallDigits / 64; w++) run += w < wv ? tot[w] : 0u;
+    return run;
+}
+
 // One stable pass over 9 bits; PASS 1 (the last) writes the points' rows and
-// their cubes' first and last rows.
+// their cubes' first and last rows, from the tile staged in digit order: a
+// tile's points of one cube follow each other there, and only its first and
+// last one touch the cube's entry (two atomics for every point took most of the
+// pass: 37 us at 60k + 240k points).
 template <int PASS, int TILE>
 __global__ void __launch_bounds__(kSmallDigits) k_small_scatter(const SmallBuild B) {
     constexpr int WAVES = kSmallDigits / 64, kRounds = TILE / WAVES / 64;
     __shared__ uint32_t wcnt[WAVES][kSmallDigits];
-    __shared__ uint32_t scan[kSmallDigits];
+    __shared__ uint32_t tot[2][kSmallDigits / 64];
+    __shared__ uint32_t skey[PASS ? TILE : 1], sval[PASS ? TILE : 1], sbase[PASS ? kSmallDigits : 1];
     const SmallSide& S = B.s[blockIdx.y];
     const int tile = blockIdx.x, tiles = (S.n + TILE - 1) / TILE;
     if (tile >= tiles) return;
@@ -717,16 +737,15 @@ __global__ void __launch_bounds__(kSmallDigits) k_small_scatter(const SmallBuild
         kk[r] = key;
         rk[r] = c + ahead;
     }
-    // exclusive prefix of the digit totals, then this digit's place for every wave
-    scan[tid] = all;
-    __syncthreads();
-    for (int off = 1; off < kSmallDigits; off <<= 1) {
-        const uint32_t u = tid >= off ? scan[tid - off] : 0u;
-        __syncthreads();
-        scan[tid] += u;
-        __syncthreads();
+    // the digit's first position, the tile's first one in it, then every wave's
+    uint32_t run = small_scan(all, tot[0]) + before;
+    uint32_t here = 0;
+    for (int w = 0; w < WAVES; w++) here += wcnt[w][tid];
+    if (PASS) {
+        const uint32_t first = small_scan(here, tot[1]);
+        sbase[tid] = run - first;  // from a staged place to its position
+        run = first;
     }
-    uint32_t run = scan[tid] - all + before;
     for (int w = 0; w < WAVES; w++) {
         const uint32_t c = wcnt[w][tid];
         wcnt[w][tid] = run;
@@ -745,20 +764,39 @@ __global__ void __launch_bounds__(kSmallDigits) k_small_scatter(const SmallBuild
             S.val1[pos] = (uint32_t)(tile * TILE + li);
             atomicAdd(S.counts + ((int64_t)tiles + pos / TILE) * kSmallDigits + (high & (kSmallDigits - 1)), 1u);
         } else {
-            const int64_t p = S.val1[tile * TILE + li];
-            const double px = S.x[p * S.xs], py = S.y[p * S.xs], pz = S.z[p * S.xs];
+            skey[pos] = kk[r];
+            sval[pos] = S.val1[tile * TILE + li];
+        }
+    }
+    if (PASS == 0) return;
+    __syncthreads();
+    const int hn = 1 << G.mbits, sh = G.mbits - G.cbits;
+    auto cube_of = [&](double x, double y, double z) {
+        bool bad = false;
+        const int cx = cell_index(x, G.inv_hcell[0], hn, bad, G.period[0], 0) >> sh;
+        const int cy = cell_index(y, G.inv_hcell[1], hn, bad, G.period[1], 0) >> sh;
+        const int cz = cell_index(z, G.inv_hcell[2], hn, bad, G.period[2], 0) >> sh;
+        return (((cx << G.cbits) + cy) << G.cbits) + cz;
+    };
+#pragma unroll
+    for (int r = 0; r < TILE / kSmallDigits; r++) {
+        const int i = r * kSmallDigits + tid;
+        const bool in = i < tn;
+        const uint32_t pos = in ? sbase[skey[i] & (kSmallDigits - 1)] + (uint32_t)i : 0u;
+        const int64_t p = in ? sval[i] : 0u;
+        const double px = S.x[p * S.xs], py = S.y[p * S.xs], pz = S.z[p * S.xs];
+        if (in) {
             reinterpret_cast<double4*>(S.row)[pos] = make_double4(px, py, pz, __longlong_as_double((long long)p));
             if (S.ow)
                 for (int k = 0; k < B.nw; k++) S.ow[(int64_t)pos * B.nw + k] = S.w[p * B.nw + k];
-            if (S.cubes) {
-                bool bad = false;
-                const int hn = 1 << G.mbits, sh = G.mbits - G.cbits;
-                const int cx = cell_index(px, G.inv_hcell[0], hn, bad, G.period[0], 0) >> sh;
-                const int cy = cell_index(py, G.inv_hcell[1], hn, bad, G.period[1], 0) >> sh;
-                const int cz = cell_index(pz, G.inv_hcell[2], hn, bad, G.period[2], 0) >> sh;
-                uint2* c = S.cubes + (((((int64_t)cx << G.cbits) + cy) << G.cbits) + cz);
-                atomicMin(&c->x, pos);
-                atomicMax(&c->y, pos + 1u);
+        }
+        if (S.cubes) {
+            // (a wave's 64 staged points: their neighbours' cubes from the lanes beside them)
+            const int c = in ? cube_of(px, py, pz) : -1;
+            const int up = __shfl_up(c, 1), down = __shfl_down(c, 1);
+            if (in) {
+                if (lane == 0 || up != c) atomicMin(&S.cubes[c].x, pos);
+                if (lane == 63 || down != c) atomicMax(&S.cubes[c].y, pos + 1u);
             }
         }
     }
