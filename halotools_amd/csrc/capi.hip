@@ -216,7 +216,7 @@ struct Plan {
     int row_stride[2] = {4, 4}, row_nw[2] = {0, 0};
     size_t o_keys_row = 0;           // row-major keys of a side sorted in both orders
     bool tiles = false;  // matrix-core kernels on the curve-ordered rows
-    bool small = false;  // ... built by the launches for small requests
+    bool small[2] = {false, false};  // ... side built by the launches for small requests
     size_t o_small[2] = {0, 0};
     size_t o_crow[2] = {0, 0}, o_cw[2] = {0, 0}, o_cperm[2] = {0, 0}, o_cubes[2] = {0, 0};
     bool sym = false;  // auto-count (unweighted or tangent): symmetric evaluation
@@ -550,14 +550,19 @@ static int make_plan(const hp_request* r, int kind, Plan& P, bool tiles = true) 
         }
     }
     const int64_t most = P.same ? kSmallMaxSame : kSmallMax;
-    P.small = P.tiles && P.M == 1 && P.n[0] <= most && P.n[s2] <= most && P.bits_hilbert <= 2 * kSmallBits;
+    P.small[0] = P.small[1] = P.tiles && P.M == 1 && P.n[0] <= most && P.n[s2] <= most && P.bits_hilbert <= 2 * kSmallBits;
+    // one small sample beside a large one (150k x 1M projected: 460 -> 446 us a call, 10k x 2M: 501 -> 468): its
+    // curve may be coarser than the other's, but not than the cubes
+    for (int s = 0; s <= s2 && !P.small[s]; s++)
+        P.small[s] = P.tiles && P.M == 1 && !P.same && P.n[s] > 0 && P.n[s] <= kSmallMaxSame &&
+                     P.geom[0].cbits <= 2 * kSmallBits / 3;
     if (P.tiles) {
         for (int s = 0; s <= s2; s++) {
             const size_t n = (size_t)std::max<int64_t>(P.n[s], 1);
             nmax = std::max<int64_t>(nmax, (int64_t)n);
             P.o_crow[s] = take(n * 32);
             if (P.weighted()) P.o_cw[s] = take(n * 8 * (size_t)P.nw);
-            if (P.small) {
+            if (P.small[s]) {
                 // keys, keys and indices after the first pass, digit counts of both
                 const size_t tiles_ = (n + 1023) / 1024;
                 P.o_small[s] = take(n * 12 + 2 * tiles_ * kSmallDigits * 4 + 256);
@@ -754,6 +759,7 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
     // matrix-core kernels: one curve-ordered copy of each side, the stream side's with its cubes
     SortedSide curve[2] = {};
     SmallBuild small = {};
+    int nsmall = 0;
     const int64_t count_words = P.counts ? (int64_t)P.M * P.crep * P.nb_count * 2 : 0;  // cleared by the build
     for (int sd = 0; P.tiles && sd < (P.same ? 1 : 2); sd++) {
         SortedSide& C = curve[sd];
@@ -762,8 +768,13 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
         C.perm = reinterpret_cast<uint32_t*>(ws + P.o_cperm[sd]);
         C.cubes = P.o_cubes[sd] ? reinterpret_cast<uint2*>(ws + P.o_cubes[sd]) : nullptr;
         C.xs = 4;
-        if (P.small) {
-            SmallSide& S = small.s[sd];
+        if (P.small[sd]) {
+            SmallSide& S = small.s[nsmall++];
+            small.tile = std::max(small.tile, small_tile(P.n[sd]));
+            if (sd == 0) {
+                small.clear = reinterpret_cast<uint32_t*>(ws + P.o_pcount);
+                small.clear_words = count_words;
+            }
             const size_t n = (size_t)std::max<int64_t>(P.n[sd], 1);
             C.perm = nullptr;
             S.x = X[sd];
@@ -793,15 +804,12 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
                              reinterpret_cast<uint32_t*>(ws + P.o_pcount), sd == 0 ? count_words : 0))
             return fail("cell build launch failed");
     }
-    if (P.small) {
+    if (nsmall > 0) {
         small.geom = dgeom;
         small.status = status;
         small.nw = P.nw;
-        small.tile = small_tile(std::max(P.n[0], P.n[P.same ? 0 : 1]));
         small.total_cells = P.total_cells;
-        small.clear = P.counts ? reinterpret_cast<uint32_t*>(ws + P.o_pcount) : nullptr;
-        small.clear_words = count_words;
-        if (build_curve_small(small, P.same ? 1 : 2, s)) return fail("cell build launch failed");
+        if (build_curve_small(small, nsmall, s)) return fail("cell build launch failed");
     }
     for (int sd = 0; sd < 2; sd++) {
         for (int o = 0; o < 2; o++) {

@@ -648,6 +648,7 @@ __global__ void __launch_bounds__(1024) k_small_keys(const SmallBuild B) {
     for (int i = threadIdx.x; i < kSmallDigits; i += NT) h[i] = 0u;
     __syncthreads();
     const int hb = G.mbits, hn = 1 << hb;
+    const int drop = max(3 * hb - 2 * kSmallBits, 0);  // a coarser curve beside a large sample's
     bool bad = false;
 #pragma unroll
     for (int r = 0; r < TILE / NT; r++) {
@@ -661,7 +662,7 @@ __global__ void __launch_bounds__(1024) k_small_keys(const SmallBuild B) {
             if (G.pbc && (v[d] < 0.0 || v[d] > G.period[d])) bad = true;
             c[d] = (uint32_t)cell_index(v[d], G.inv_hcell[d], hn, dummy, G.period[d], 0);
         }
-        const uint32_t key = hilbert3(c[0], c[1], c[2], hb);
+        const uint32_t key = hilbert3(c[0], c[1], c[2], hb) >> drop;
         S.key0[p] = key;
         atomicAdd(&h[key & (kSmallDigits - 1)], 1u);
     }

@@ -160,9 +160,9 @@ int build_curve_side(const MockGeom* geom, int nmocks, int side, const double* x
 // The same for small one-mock requests, both sides in each launch: keys and
 // digit counts, two 9-bit passes, the second writing the rows; clears the cubes
 // and `clear` (clear_words words) on the way.  Two samples gain up to 262,144
-// points a side (131,072 with a quarter as many: 221 -> 159 us a call; 262,144:
-// 254 -> 207), one sample up to 196,608 (131,072: 184 -> 175; at 262,144 the
-// general passes' larger grids win, 225 against 232).
+// points a side (131,072 with a quarter as many: 221 -> 147 us a call; 262,144:
+// 254 -> 191), one sample up to 196,608 (131,072: 184 -> 161; at 262,144 the
+// general passes' larger grids won, 225 against 232).
 constexpr int64_t kSmallMax = 1 << 18, kSmallMaxSame = 3 << 16;
 // keys per workgroup: at most 128 tiles a side, whose counts every workgroup
 // adds up (2048-key tiles at 100,000 points: 163 us a call against 160, and

@@ -17,15 +17,16 @@
 // in FP64, and binned with its "<=".  Every pair therefore lands in the bin
 // the reference puts it in.
 //
-// What bounds it: instruction issue.  The MFMA (65 cycles per 256 pairs; it does
-// not overlap other waves' VALU work here) replaces 8 FP64 instructions of 4.5
-// cycles per 64 pairs, the bin takes 7 instructions and two LDS accesses instead
-// of 12 and two, and sub-groups of 16 evaluate 2.4 pairs per pair in range where
-// groups of 64 evaluated 4.4 (1M clustered points, 20 edges to 50 Mpc/h: 6.3e8
-// instead of 1.18e9 evaluations).  Measured against the kernels of pairs_kernel.h
-// on the whole call: that count 1192 -> 782 us, 20k x 20k 344 -> 228 us, 2M
-// (rp, pi) 2782 -> 2192 us, 150k x 1M projected 1011 -> 528 us, 200k generic
-// marks 935 -> 574 us, per-object rows of 1M 1621 -> 1324 us.
+// What bounds it: instruction issue (1M clustered points, 20 edges to 50 Mpc/h:
+// vector instructions 65 % and the matrix product 14 % of the issue slots, 13 of
+// 16 waves alive on average).  The MFMA (65 cycles per 256 pairs; it does not
+// overlap other waves' VALU work here) replaces 8 FP64 instructions of 4.5 cycles
+// per 64 pairs, the bin takes 6 instructions and two LDS accesses instead of 12
+// and two, and sub-groups of 16 evaluate 2.4 pairs per pair in range where groups
+// of 64 evaluated 4.4 (6.3e8 instead of 1.18e9 evaluations there).  Pair kernels
+// against those of pairs_kernel.h: that count 1.04 -> 0.55 ms, 2M (rp, pi) 2.5 ->
+// 1.65 ms, per-object rows of 1M 1.49 -> 1.04 ms, the 64-mock forward-mode pass
+// 49 -> 35 ms, Jacobian rows of 1M 2.7 -> 1.9 ms.
 #pragma once
 
 #include "pairs_kernel.h"
@@ -60,7 +61,7 @@ struct Stage {
 static constexpr int kStage = kDeal + 64;         // staged points
 static constexpr int kSlots = kStage + 1;         // and one that no pair bins
 static constexpr int kIdOff = 4 * kSlots * 8;     // after x, y, z, squared norm: stream index and image of each
-static constexpr int kListOff = kIdOff + (kSlots + 3) / 4 * 16;            // slots dealt to a sub-group, two tiles of padding
+static constexpr int kListOff = kIdOff + (kSlots + 3) / 4 * 16;            // slots dealt to a sub-group, three tiles of padding
 static constexpr int kMarkOff = kListOff + kDeal + 3 * kSub;    // 64: starts of stretches
 static constexpr int kInfoOff = (kMarkOff + 64 + 15) / 16 * 16; // boxes of the sub-groups and the group, the cube window
 static constexpr int kTileBytes = kInfoOff + 4 * 32 + 32 + 48;
