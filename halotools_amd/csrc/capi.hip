@@ -593,9 +593,12 @@ static int make_plan(const hp_request* r, int kind, Plan& P, bool tiles = true) 
     // so those stay whole), twice that where up to four items per group give it:
     // a second round evens out the first (200k generic marks 390 -> 369 us, wp of
     // 500k 1000 -> 963); eight and sixteen items per group cost more in their own
-    // starts than that gains (60k points: 470 -> 485).
+    // starts than that gains (60k points: 470 -> 485).  At most 16 items per group,
+    // 128 where each still walks a long stream (2,000 points against 1M: 440 -> 241
+    // us a call, 10,000 against 2M 435 -> 402; 16,000 alone with 32: 110 -> 120).
+    const int most_sh = P.n[s2] >= (1 << 17) ? 7 : 4;
     if (P.tiles && mode != kModeObj && mode != kModeJac)
-        while (P.parts_sh < 4 && (gA << P.parts_sh) < 256 * HP_TILE_ITEMS * (P.parts_sh < 2 ? 2 : 1)) P.parts_sh++;
+        while (P.parts_sh < most_sh && (gA << P.parts_sh) < 256 * HP_TILE_ITEMS * (P.parts_sh < 2 ? 2 : 1)) P.parts_sh++;
     const int64_t gP = gA << P.parts_sh;  // rows of FP64 partials
     // count accumulators: up to kCountReplicas copies per mock (a group adds
     // into copy group % crep), so the atomics of many groups spread over cache

@@ -147,7 +147,7 @@ def test_jackknife_tables(mo, n, tags):
 
 @pytest.mark.parametrize("n1,n2", [(1023, 1025), (1024, 1), (1, 65536), (65535, 1024), (65536, 65536), (65537, 3000),
                                    (131072, 131073), (196609, 65536), (262144, 5000), (262145, 262144),
-                                   (300000, 1), (63, 300001), (196608, 300000), (300000, 1500)])
+                                   (300000, 1), (63, 300001), (2000, 131072), (196608, 300000), (300000, 1500)])
 def test_small_builds_agree_with_general(mo, gpu, n1, n2, monkeypatch):
     # edges of the sort tiles and of the range that the small build takes; two samples of
     # unlike sizes, half of the first in one spot (one digit holds whole tiles)
