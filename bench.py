@@ -28,8 +28,8 @@ HBM_PEAK_GBPS = 8000.0
 ALG_BUILD_BYTES = 76
 # HBM bytes per launch of the pair kernel on this workload: rocprofv3
 # FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0, the factors being what the same
-# counters read for a plain 256 MiB copy (profiles/k_pairs_count3d_clustered_1M.md)
-PAIR_KERNEL_TRAFFIC_BYTES = 5.843e8
+# counters read for a plain 256 MiB copy (profiles/k_tiles_cases.md)
+PAIR_KERNEL_TRAFFIC_BYTES = 2.164e8
 
 
 def _progress(msg):
@@ -721,13 +721,14 @@ def main():
         "fp64_peak_frac": achieved / FP64_PEAK_TFLOPS,
         "cell_build": _build_rate(n, build_s),
         "numpy_in_out_ms_per_call": numpy_io_ms,
-        # compute-bound on the FP64 vector ALU (a distance threshold, not a
-        # contraction, so no MFMA); MI355X's FP64 peak is 78.6 TFLOP/s
+        # bound by instruction issue: squared distances on the FP64 matrix
+        # cores, bins and the walk on the vector ALU; MI355X's FP64 peak is 78.6
+        # TFLOP/s for both
         "roofline": {"bound": "fp64-valu", "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / FP64_PEAK_TFLOPS, "traffic": PAIR_KERNEL_TRAFFIC_BYTES,
                      "traffic_source": "rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE of this kernel on this "
                                        "workload, scaled by a plain copy's readings "
-                                       "(profiles/k_pairs_count3d_clustered_1M.md)"},
+                                       "(profiles/k_tiles_cases.md)"},
         "batched_64_mocks": batched,
         "cell_build_64_mocks": build64,
         "headline_host_phases": host_phases,

@@ -591,7 +591,7 @@ static int make_plan(const hp_request* r, int kind, Plan& P, bool tiles = true) 
     // Small requests split each lane group into work items until the chip has
     // HP_TILE_ITEMS waves per CU to run (rows per lane point are written once,
     // so those stay whole), twice that where up to four items per group give it:
-    // a second round evens out the first (200k generic marks 390 -> 369 us, wp of
+    // later items even out the first ones (200k generic marks 390 -> 369 us, wp of
     // 500k 1000 -> 963); eight and sixteen items per group cost more in their own
     // starts than that gains (60k points: 470 -> 485).  At most 16 items per group,
     // 128 where each still walks a long stream (2,000 points against 1M: 440 -> 241
