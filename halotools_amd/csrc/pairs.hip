@@ -149,7 +149,9 @@ static int tile_var(int mode, int K, int Kp, int wfunc, int nw, int swap, int un
     switch (mode) {
         case kModeXYZ: return K * Kp > 256 ? 1 : 0;  // cells in one column or two: their LDS bounds the waves
         case kModeWSum:
-        case kModeWXYZ: return (wfunc == 1 && nw == 1) ? 1 : (nw == 2 ? 2 : 0);
+        // the number of weights compiled in where it is small: five rows of them cost
+        // registers (sums of marks, id 2, of 400k points: 591 -> 406 us; (rp, pi) 1204 -> 787)
+        case kModeWXYZ: return (wfunc == 1 && nw == 1) ? 1 : (nw == 2 ? 2 : (nw == 1 ? 3 : 0));
         case kModeJac: return swap;
         case kModeJack: return unit ? 0 : 1;
     }

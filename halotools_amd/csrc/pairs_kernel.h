@@ -35,41 +35,69 @@ namespace hp {
 
 // ------------------------------------------------------------- marking functions
 // PC/marked_cpairs/marking_functions.pyx:14-217 (ids 1-17).
-__device__ __forceinline__ double wfunc_eval(int id, const double* a, const double* b) {
-    switch (id) {
-        case 1: return a[0] * b[0];
-        case 2: return a[0] + b[0];
-        case 3: return a[0] == b[0] ? a[1] * b[1] : 0.0;
-        case 4: return a[0] != b[0] ? a[1] * b[1] : 0.0;
-        case 5: return b[0] > a[0] ? a[1] * b[1] : 0.0;
-        case 6: return b[0] < a[0] ? a[1] * b[1] : 0.0;
-        case 7: return b[0] > (a[0] + a[1]) ? b[1] : 0.0;
-        case 8: return b[0] < (a[0] + a[1]) ? b[1] : 0.0;  // '+' as in the reference (:104-115)
-        case 9: return fabs(a[0] - b[0]) < a[1] ? b[1] : 0.0;
-        case 10: return fabs(a[0] - b[0]) > a[1] ? b[1] : 0.0;
-        case 11: return b[0] > a[0] * a[1] ? b[1] : 0.0;
-        case 12: return a[0] * b[0] * (a[1] * b[1] + a[2] * b[2] + a[3] * b[3]);
-        case 13: {
-            const double c = a[1] * b[1] + a[2] * b[2] + a[3] * b[3];
-            return a[0] * b[0] * (a[1] * b[1] + a[2] * b[2] + a[3] * b[3]) * c;
-        }
-        case 14: return a[0] * b[0] * (a[1] * b[1] + a[2] * b[2]);
-        case 15: {
-            const double c = a[1] * b[1] + a[2] * b[2];
-            return a[0] * b[0] * (a[1] * b[1] + a[2] * b[2]) * c;
-        }
-        case 16: {
-            if (a[4] != b[4]) return 0.0;
-            const double c = a[1] * b[1] + a[2] * b[2] + a[3] * b[3];
-            return a[0] * b[0] * (a[1] * b[1] + a[2] * b[2] + a[3] * b[3]) * c;
-        }
-        case 17: {
-            if (a[4] == b[4]) return 0.0;
-            const double c = a[1] * b[1] + a[2] * b[2] + a[3] * b[3];
-            return a[0] * b[0] * (a[1] * b[1] + a[2] * b[2] + a[3] * b[3]) * c;
-        }
-        default: return 0.0;
+template <int ID>
+__device__ __forceinline__ double wfunc_one(const double* a, const double* b) {
+    if constexpr (ID == 1) return a[0] * b[0];
+    if constexpr (ID == 2) return a[0] + b[0];
+    if constexpr (ID == 3) return a[0] == b[0] ? a[1] * b[1] : 0.0;
+    if constexpr (ID == 4) return a[0] != b[0] ? a[1] * b[1] : 0.0;
+    if constexpr (ID == 5) return b[0] > a[0] ? a[1] * b[1] : 0.0;
+    if constexpr (ID == 6) return b[0] < a[0] ? a[1] * b[1] : 0.0;
+    if constexpr (ID == 7) return b[0] > (a[0] + a[1]) ? b[1] : 0.0;
+    if constexpr (ID == 8) return b[0] < (a[0] + a[1]) ? b[1] : 0.0;  // '+' as in the reference (:104-115)
+    if constexpr (ID == 9) return fabs(a[0] - b[0]) < a[1] ? b[1] : 0.0;
+    if constexpr (ID == 10) return fabs(a[0] - b[0]) > a[1] ? b[1] : 0.0;
+    if constexpr (ID == 11) return b[0] > a[0] * a[1] ? b[1] : 0.0;
+    if constexpr (ID == 12) return a[0] * b[0] * (a[1] * b[1] + a[2] * b[2] + a[3] * b[3]);
+    if constexpr (ID == 13 || ID == 16 || ID == 17) {
+        const double c = a[1] * b[1] + a[2] * b[2] + a[3] * b[3];
+        const double v = a[0] * b[0] * (a[1] * b[1] + a[2] * b[2] + a[3] * b[3]) * c;
+        if constexpr (ID == 16) return a[4] != b[4] ? 0.0 : v;
+        if constexpr (ID == 17) return a[4] == b[4] ? 0.0 : v;
+        return v;
     }
+    if constexpr (ID == 14) return a[0] * b[0] * (a[1] * b[1] + a[2] * b[2]);
+    if constexpr (ID == 15) {
+        const double c = a[1] * b[1] + a[2] * b[2];
+        return a[0] * b[0] * (a[1] * b[1] + a[2] * b[2]) * c;
+    }
+    return 0.0;
+}
+
+template <int ID>
+struct WfuncId {
+    static constexpr int value = ID;
+};
+
+// f(WfuncId<id>{}) for a marking function known when the kernel runs
+template <typename F>
+__device__ __forceinline__ void wfunc_switch(int id, F f) {
+    switch (id) {
+        case 1: return f(WfuncId<1>{});
+        case 2: return f(WfuncId<2>{});
+        case 3: return f(WfuncId<3>{});
+        case 4: return f(WfuncId<4>{});
+        case 5: return f(WfuncId<5>{});
+        case 6: return f(WfuncId<6>{});
+        case 7: return f(WfuncId<7>{});
+        case 8: return f(WfuncId<8>{});
+        case 9: return f(WfuncId<9>{});
+        case 10: return f(WfuncId<10>{});
+        case 11: return f(WfuncId<11>{});
+        case 12: return f(WfuncId<12>{});
+        case 13: return f(WfuncId<13>{});
+        case 14: return f(WfuncId<14>{});
+        case 15: return f(WfuncId<15>{});
+        case 16: return f(WfuncId<16>{});
+        case 17: return f(WfuncId<17>{});
+        default: return f(WfuncId<0>{});
+    }
+}
+
+__device__ __forceinline__ double wfunc_eval(int id, const double* a, const double* b) {
+    double v = 0.0;
+    wfunc_switch(id, [&](auto k) __attribute__((always_inline)) { v = wfunc_one<decltype(k)::value>(a, b); });
+    return v;
 }
 
 // ------------------------------------------------------------- helpers

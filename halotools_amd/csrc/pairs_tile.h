@@ -189,8 +189,8 @@ __device__ __forceinline__ void lds_add(uint32_t off, double v) {
     __hip_atomic_fetch_add((lds_f64*)(uintptr_t)off, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// VAR: product marks compiled in (kModeWSum, kModeWXYZ: 1; 2: two weights per
-// point); the swapped Jacobian pass (kModeJac: lanes are sample 2, the stream is
+// VAR: product marks compiled in (kModeWSum, kModeWXYZ: 1; 2, 3: other marks of
+// two or one weights per point; 0: any); the swapped Jacobian pass (kModeJac: lanes are sample 2, the stream is
 // sample 1).  ALSO: plain
 // counts beside the sums.
 template <int MODE, int VAR, int ALSO, int WAVES>
@@ -213,7 +213,11 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
     const int lane = threadIdx.x & 63;
     const int wid = uni(threadIdx.x >> 6);
     const int K = L.br.nbins, Kp = XY ? L.bp.nbins : 1;
-    const int nw = !F64 ? 0 : (TAN ? 2 : ((MODE == kModeJac || PROD || JK) ? 1 : (VAR == 2 ? 2 : L.nw)));
+    const int nw = !F64                             ? 0
+                   : TAN || VAR == 2                ? 2
+                   : (MODE == kModeJac || JK)       ? 1
+                   : (VAR == 1 || VAR == 3)         ? 1
+                                                    : L.nw;
     const int wst = JK ? 2 : nw;  // doubles per weight row (jackknife: weight and tag)
     unsigned char* const wsm = lds + A.tab_bytes + wid * A.wave_bytes;
     // Bytes from a bin's histogram row to the next (and from a pi bin to the
@@ -735,6 +739,24 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                         }
                     }
                     // ---- accumulate
+                    // generic marks: one choice of the function for the tile's four rows (a
+                    // choice per row took more issue slots than the marks themselves)
+                    double mv[4] = {0.0, 0.0, 0.0, 0.0};
+                    if constexpr ((MODE == kModeWSum || MODE == kModeWXYZ) && !PROD) {
+                        wfunc_switch(L.wfunc, [&](auto id) __attribute__((always_inline)) {
+#pragma unroll
+                            for (int i = 0; i < 4; i++) {
+                                double bw[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                                for (int c = 0; c < 5; c++)
+                                    if (c < nw)
+                                        bw[c] = i == 0 ? row_bcast<0>(wb[c])
+                                                : (i == 1 ? row_bcast<1>(wb[c])
+                                                          : (i == 2 ? row_bcast<2>(wb[c]) : row_bcast<3>(wb[c])));
+                                mv[i] = wfunc_one<decltype(id)::value>(lw, bw);
+                            }
+                        });
+                    }
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
                         // the row's stream weights (all lanes: a broadcast reads none that is masked off)
@@ -759,7 +781,7 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                                 if constexpr (MODE == kModeXYZ)
                                     lds_add((cell << (ccol + 2)) + (hbase + ccl * 4u), inc);
                                 else
-                                    lds_add(cell * 8u + hbase, PROD ? lw[0] * sw[0] : wfunc_eval(L.wfunc, lw, sw));
+                                    lds_add(cell * 8u + hbase, PROD ? lw[0] * sw[0] : mv[i]);
                             }
                         } else if constexpr (MODE == kModeObj || (JK && !VAR)) {
                             lds_add(adr[i], 1u);
@@ -780,7 +802,7 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                                 if (ALSO) lds_add(adr[i] + (2 * TR + tcol4 - tcol8), inc);
                             }
                         } else {
-                            lds_add(adr[i], PROD ? lw[0] * sw[0] : wfunc_eval(L.wfunc, lw, sw));
+                            lds_add(adr[i], PROD ? lw[0] * sw[0] : mv[i]);
                             if (MODE == kModeWSum && ALSO) lds_add(adr[i] - adr0 + cbase + col4, 1u);
                         }
                     }
@@ -1117,6 +1139,9 @@ int launch_tiles_mode(const TileArgs& A, int waves, int64_t blocks, int smem, in
         if (var == 2)
             return also ? launch_tiles_v<MODE, 2, 1>(A, waves, blocks, smem, s)
                         : launch_tiles_v<MODE, 2, 0>(A, waves, blocks, smem, s);
+        if (var == 3)
+            return also ? launch_tiles_v<MODE, 3, 1>(A, waves, blocks, smem, s)
+                        : launch_tiles_v<MODE, 3, 0>(A, waves, blocks, smem, s);
     }
     if constexpr (MODE == kModeWSum || MODE == kModeJac) {
         if (var)
@@ -1126,6 +1151,7 @@ int launch_tiles_mode(const TileArgs& A, int waves, int64_t blocks, int smem, in
                     : launch_tiles_v<MODE, 0, 0>(A, waves, blocks, smem, s);
     } else if constexpr (MODE == kModeWXYZ) {
         if (var == 2) return launch_tiles_v<MODE, 2, 0>(A, waves, blocks, smem, s);
+        if (var == 3) return launch_tiles_v<MODE, 3, 0>(A, waves, blocks, smem, s);
         return var ? launch_tiles_v<MODE, 1, 0>(A, waves, blocks, smem, s)
                    : launch_tiles_v<MODE, 0, 0>(A, waves, blocks, smem, s);
     } else if constexpr (MODE == kModeXYZ || MODE == kModeJack) {
