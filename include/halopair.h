@@ -249,7 +249,8 @@ int hp_tag_stats(const int64_t* tags1, int64_t n1, const int64_t* tags2, int64_t
  * info = {shift, base, table entries, multi}. */
 int hp_debug_bin_lookup(const double* r2, int32_t K, const double* d, int64_t n, int32_t* out, int32_t* info);
 /* The matrix-core pair kernels' lookup when the high word of d[i] is off by `off` units: out[i] = the bin,
- * or -1 where the kernels evaluate the pair exactly (-2: the word and the clamped word disagree); info = {1 if the edges fit such a table, shift, entries}. */
+ * -1 where the kernels evaluate the pair exactly, -2 where the word and the clamped word would disagree;
+ * info = {1 if the edges fit such a table, shift, entries}. */
 int hp_debug_tile_lookup(const double* r2, int32_t K, const double* d, int64_t n, int32_t off, int32_t* out,
                          int32_t* info);
 /* Hilbert index of cell (x, y, z) on a 2^bits grid: the lane-group order of the pair kernels. */
