@@ -220,3 +220,23 @@ def test_seam_check(gpu, seam, tiles, monkeypatch):
     assert torch.equal(w.grad, ((full.rows1 + full.rows2) * G).sum(dim=1))
     with pytest.raises(E.EngineError):
         D.run(E.HP_MARKED_NPAIRS_3D, mock, t.unbind(1), t.unbind(1), rb * rb, rows1=True, rows2=True, seam_check=True, **args)
+
+
+@pytest.mark.parametrize("tags", ["slabs", "random"])
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 0.0])
+def test_jackknife_weights_that_are_not_finite(mo, value, tags, monkeypatch):
+    # a pair's weight is the product of its two: bins without a pair of the infinite point stay finite
+    # (sums of small whole numbers: the finite ones are exact)
+    rng = np.random.default_rng(31)
+    n, ns = 500, 4
+    p = rng.uniform(0, 1, (n, 3))
+    t = 1 + np.minimum((p[:, 0] * ns).astype(int), ns - 1) if tags == "slabs" else rng.integers(1, ns + 1, n)
+    w = rng.integers(1, 5, n).astype(float)
+    w[40] = value
+    w[7] = 0.0
+    rb = np.array([0.01, 0.02, 0.05, 0.1, 0.2])
+    kw = dict(period=1.0, weights1=w, weights2=w)
+    got = mo.npairs_jackknife_3d(p, p, rb, t, t, ns, **kw)
+    monkeypatch.setenv("HALOPAIR_NO_TILES", "1")
+    ref = mo.npairs_jackknife_3d(p, p, rb, t, t, ns, **kw)
+    assert np.array_equal(got, ref, equal_nan=True)
