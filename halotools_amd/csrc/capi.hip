@@ -152,7 +152,9 @@ static TileTable make_tile_table(const std::vector<double>& e, int K) {
             if (upto - below == 1 && upto < K && (int64_t)((hiword(e[(size_t)upto]) - 1) >> shift) == base + b)
                 fits = false;
             const size_t at = (size_t)((base + b) & (n - 1));
-            T.t[2 * at] = hiword(e[(size_t)below]) + 1;
+            // (no word is past the last entry, that of a NaN neither: pairs of a point
+            // that is not finite stay within the histogram)
+            T.t[2 * at] = below < K ? hiword(e[(size_t)below]) + 1 : 0xffffffffu;
             T.t[2 * at + 1] = (uint32_t)below;
         }
         if (!fits) continue;

@@ -55,3 +55,12 @@ def test_a_high_word_two_off_at_an_edge_is_caught():
                                    np.nextafter(np.array([0.5, 1.0, 2.0, 4.0]), 0)])  # edges that end a bucket
 def test_edges_that_share_a_bucket_do_not_fit(edges):
     assert not E.debug_tile_lookup(edges * edges, np.array([0.5]))[1]
+
+
+@pytest.mark.parametrize("edges", FITS, ids=range(len(FITS)))
+def test_words_beyond_every_number_take_the_row_past_the_last_edge(edges):
+    # a coordinate that is not a number reaches the kernels (they report it): the row its
+    # pairs are added to must be one of the histogram's
+    d = np.array([np.inf, np.nan, np.finfo(float).max])
+    out, fits = E.debug_tile_lookup(edges * edges, d)
+    assert fits and np.array_equal(out, np.full(3, len(edges)))
