@@ -166,7 +166,7 @@ def prepare(kind, mocks, s1, s2, r2, p2=None, same=False, w1=None, w2=None, nw=0
     pair_events, build_events : optional (start, end) HIP event handles recorded
         around the pair kernel(s) and around the cell build
     tile_waves : wavefronts per pair-kernel workgroup (1, 2, 4, 8; 0 = library default)
-    seam_check : marked id 1 auto-count with rows1 only: status bit 4 where rows2 would differ
+    seam_check : marked id 1 auto-count with rows1 only: status bit 4 where rows2 would differ (see seam_rows)
     tangent : marked id 1 with (w, dw/dtheta) weights: also res.tangents, d(sums)/dtheta
     jtags1, jtags2, n_samples : jackknife kinds: int32 device tags (1..n_samples);
         w1 / w2 are then optional (n,) weights and res.sums has shape
@@ -286,6 +286,15 @@ def prepare(kind, mocks, s1, s2, r2, p2=None, same=False, w1=None, w2=None, nw=0
     res.workspace = ws
     res.cbuf = cbuf
     return res
+
+
+def seam_rows(res):
+    """rows2 of a seam_check request whose status has bit 4, on the current stream."""
+    res.rows2 = torch.empty_like(res.rows1)
+    res.req.rows2 = res.rows2.data_ptr()
+    res.req.stream = torch.cuda.current_stream(res.device).cuda_stream
+    E.check(E.library().hp_seam_rows(ctypes.byref(res.req)))
+    return res.rows2
 
 
 def backward_rows(rows, gsuffix, offsets, out=None):

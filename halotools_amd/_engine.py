@@ -36,7 +36,7 @@ EXPORTED_SYMBOLS = (
     "hp_marked_npairs_xy_z", "hp_npairs_jackknife_3d", "hp_npairs_jackknife_xy_z", "hp_marked_backward",
     "hp_segment_sum_scratch", "hp_segment_sum", "hp_debug_bin_lookup", "hp_debug_hilbert",
     "hp_debug_tile_lookup",
-    "hp_npairs_3d_noalloc", "hp_zheng07_tangent", "hp_enclose", "hp_tag_stats",
+    "hp_npairs_3d_noalloc", "hp_zheng07_tangent", "hp_enclose", "hp_tag_stats", "hp_seam_rows",
 )
 
 
@@ -112,7 +112,7 @@ def library():
     lib.hp_workspace_size.restype = ctypes.c_size_t
     for name in ("hp_npairs_3d", "hp_npairs_projected", "hp_npairs_xy_z", "hp_marked_npairs_3d",
                  "hp_npairs_per_object_3d", "hp_marked_npairs_xy_z", "hp_npairs_jackknife_3d",
-                 "hp_npairs_jackknife_xy_z", "hp_npairs_3d_noalloc"):
+                 "hp_npairs_jackknife_xy_z", "hp_npairs_3d_noalloc", "hp_seam_rows"):
         fn = getattr(lib, name)
         fn.argtypes = [ctypes.POINTER(HpRequest)]
         fn.restype = ctypes.c_int

@@ -17,7 +17,7 @@ sample-2 weights, with the pair arithmetic still (x1 - shift) - x2, so bin
 membership is the forward's, bit for bit.  An auto-count with one set of weights
 makes no second rows: both orientations of a pair round into one bin, except now
 and then across the periodic seam, which the pass reports (the second rows are
-then made as well).  The sums are
+then the first with the corrections that the pass recorded).  The sums are
 W_k = sum_{s <= k} sum_i w1_i rows1[i, s].
 
 Backward.  With upstream g = dL/dW and G(s) = sum_{k >= s} g_k, the hand-written
@@ -44,21 +44,17 @@ class _MarkedProductSums(torch.autograd.Function):
         need1 = ctx.needs_input_grad[0]
         need2 = ctx.needs_input_grad[1]
         same = plan["same_weights"]
-        args = dict(w1=w1.detach().reshape(-1, 1).contiguous(),
-                    w2=None if same else w2.detach().reshape(-1, 1).contiguous(), nw=1, wfunc=1,
-                    want_counts=False, want_sums=True, rows1=True,
-                    device=plan["device"], tile_waves=plan.get("tile_waves", 0))
         res = D.run(E.HP_MARKED_NPAIRS_3D, plan["mocks"], plan["s1"], plan["s2"], plan["r2"], same=same,
-                    rows2=need2 and not same, seam_check=same, **args)
+                    w1=w1.detach().reshape(-1, 1).contiguous(),
+                    w2=None if same else w2.detach().reshape(-1, 1).contiguous(), nw=1, wfunc=1,
+                    want_counts=False, want_sums=True, rows1=True, rows2=need2 and not same, seam_check=same,
+                    device=plan["device"], tile_waves=plan.get("tile_waves", 0))
         status = int(res.cbuf[-1].item()) & 0xFFFFFFFF
-        if status == 4:
-            # some pair across the seam is binned by its order: sample 2 has rows of its own
-            res = D.run(E.HP_MARKED_NPAIRS_3D, plan["mocks"], plan["s1"], plan["s2"], plan["r2"], same=same,
-                        rows2=True, **args)
-        elif status:
+        if status & ~4:
             raise ValueError("All points must be finite and lie inside the periodic box [0, period]")
         ctx.rows1 = res.rows1
-        ctx.rows2 = res.rows1 if same and res.rows2 is None else res.rows2
+        # (status 4: some pair across the seam is binned by its order, sample 2 has rows of its own)
+        ctx.rows2 = res.rows2 if not same else (D.seam_rows(res) if status else res.rows1)
         ctx.offsets1 = plan["offsets1"]
         ctx.offsets2 = plan["offsets2"]
         ctx.need = (need1, need2)

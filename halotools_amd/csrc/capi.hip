@@ -213,7 +213,7 @@ struct Plan {
     size_t o_keys[2] = {0, 0}, o_vals[2] = {0, 0}, o_tiles = 0, o_digits = 0;
     size_t o_pcount = 0, o_psum = 0, o_pevals = 0, o_red = 0, o_status = 0;
     bool elim = false;
-    size_t o_corr = 0, o_rows_tmp = 0;
+    size_t o_corr = 0, o_cflag = 0, o_rows_tmp = 0;
     size_t o_rows[2] = {0, 0};       // packed coordinate rows of each side with a row-major order
     int row_stride[2] = {4, 4}, row_nw[2] = {0, 0};
     size_t o_keys_row = 0;           // row-major keys of a side sorted in both orders
@@ -617,8 +617,10 @@ static int make_plan(const hp_request* r, int kind, Plan& P, bool tiles = true) 
     P.o_red = take((size_t)red * 8);
     // auto-count with shared weights: rows2 = rows1 + seam corrections, no swapped pass
     P.elim = P.rows2 && P.same && P.marked && r->wfunc == 1;
-    if (P.elim) {
+    // (HP_SEAM_CHECK: the corrections stay in the workspace for hp_seam_rows)
+    if (P.elim || P.seam) {
         P.o_corr = take((size_t)std::max<int64_t>(P.n[0], 1) * (size_t)P.Kr * 8);
+        if (P.tiles) P.o_cflag = take((size_t)gA * 4);
         if (!P.rows1) P.o_rows_tmp = take((size_t)std::max<int64_t>(P.n[0], 1) * (size_t)P.Kr * 8);
     }
     // unweighted auto-counts evaluate each unshifted unordered pair once; they
@@ -704,6 +706,16 @@ struct PhaseRange {
     }
     ~PhaseRange() { end(); }
 };
+
+// rows2 of an auto-count from its rows1 and the corrections its pair pass left
+static int seam_rows(const Plan& P, char* ws, const double* rows1, double* rows2, hipStream_t s) {
+    const double* corr = reinterpret_cast<const double*>(ws + P.o_corr);
+    if (!P.tiles) return launch_add_rows(rows1, corr, rows2, P.n[0] * (int64_t)P.Kr, s);
+    return launch_seam_rows(reinterpret_cast<const MockGeom*>(ws + P.o_geom),
+                            P.M > 1 ? reinterpret_cast<const int32_t*>(ws + P.o_gm[0]) : nullptr, P.ngroups[0],
+                            reinterpret_cast<const double*>(ws + P.o_crow[0]), P.Kr, rows1, corr,
+                            reinterpret_cast<const uint32_t*>(ws + P.o_cflag), rows2, s);
+}
 
 static int run(const hp_request* r, int kind, bool tiles = true) {
     PhaseRange phase;
@@ -911,11 +923,14 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
         L.rows = P.rows1 ? r->rows1 : nullptr;
     }
     double* corr = nullptr;
-    if (P.elim) {
+    if (P.elim || P.seam) {
         corr = reinterpret_cast<double*>(ws + P.o_corr);
         if (!P.rows1) L.rows = reinterpret_cast<double*>(ws + P.o_rows_tmp);
         L.corr = corr;
-        launch_fill_u32(reinterpret_cast<uint32_t*>(corr), 0u, P.n[0] * (int64_t)P.Kr * 2, s);
+        if (P.tiles)
+            L.cflag = reinterpret_cast<uint32_t*>(ws + P.o_cflag);
+        else
+            launch_fill_u32(reinterpret_cast<uint32_t*>(corr), 0u, P.n[0] * (int64_t)P.Kr * 2, s);
     }
     L.seam = P.seam ? status : nullptr;
     L.crep = P.crep;
@@ -933,7 +948,7 @@ static int run(const hp_request* r, int kind, bool tiles = true) {
         if (rc) return fail("pair kernel launch failed");
     }
     if (P.elim) {
-        if (launch_add_rows(L.rows, corr, r->rows2, P.n[0] * (int64_t)P.Kr, s)) return fail("row add launch failed");
+        if (seam_rows(P, ws, L.rows, r->rows2, s)) return fail("row add launch failed");
     } else if (P.rows2) {
         // pass B: lanes are sample 2, the stream is sample 1 (same arithmetic,
         // (x1 - x2shift) - x2, with the shift applied to the sample-1 point)
@@ -1078,6 +1093,17 @@ int hp_marked_npairs_xy_z(const hp_request* req) { return run(req, HP_MARKED_NPA
 int hp_npairs_jackknife_3d(const hp_request* req) { return run(req, HP_NPAIRS_JACKKNIFE_3D); }
 int hp_npairs_jackknife_xy_z(const hp_request* req) { return run(req, HP_NPAIRS_JACKKNIFE_XY_Z); }
 
+int hp_seam_rows(const hp_request* req) {
+    Plan P;
+    if (make_plan(req, HP_MARKED_NPAIRS_3D, P)) return -1;
+    if (!P.seam) return fail("hp_seam_rows takes a request with HP_SEAM_CHECK");
+    if (!req->workspace || req->workspace_bytes < P.total) return fail("workspace too small");
+    if (P.n[0] > 0 && (!req->rows1 || !req->rows2)) return fail("rows1 and rows2 must not be null");
+    if (seam_rows(P, static_cast<char*>(req->workspace), req->rows1, req->rows2, static_cast<hipStream_t>(req->stream)))
+        return fail("row add launch failed");
+    g_err.clear();
+    return 0;
+}
 int hp_marked_backward(const double* rows, int32_t nr, const double* gsuffix, const int64_t* offsets,
                        int32_t nmocks, double* grad, void* stream) {
     if (!rows || !gsuffix || !offsets || !grad) return fail("null pointer");

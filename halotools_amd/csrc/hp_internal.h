@@ -216,8 +216,10 @@ struct PairLaunch {
     double* ptan;          // tangent mode: [ngroups][nr]
     int64_t* orows;        // per-object mode: [n_lane_total][nr] cumulative counts (input order)
     double* rows;          // [n_lane_total][nr] (original order) or nullptr
-    double* corr;          // auto-counts: rows2 - rows1 corrections from seam pairs, or nullptr
-    int32_t* seam;         // instead of corr: the status word, bit 4 set where corr would not be zero
+    double* corr;          // auto-counts: rows2 - rows1, corrections from seam pairs, or nullptr; in input
+                           // order, zeroed (matrix-core kernels: in the lanes' order, rows of flagged groups)
+    uint32_t* cflag;       // matrix-core kernels: per lane group, whether its corr rows are written
+    int32_t* seam;         // the status word, bit 4 set where some correction is made, or nullptr
     uint64_t* pevals;      // [ngroups]
     // symmetric auto-counts: the Hilbert order keys of the stream points, the
     // fourth word of each 32-byte stream row ((Hilbert key << 32) | input
@@ -269,6 +271,8 @@ int launch_segment_sum(const double* v, const int64_t* offsets, int nmocks, doub
 int launch_rows_dot(const double* rows, int nr, const double* gsuffix, const int64_t* offsets,
                     int nmocks, double* grad, hipStream_t s);
 int launch_add_rows(const double* a, const double* b, double* out, int64_t n, hipStream_t s);
+int launch_seam_rows(const MockGeom* geom, const int32_t* group_mock, int64_t ngroups, const double* lane_rows, int nr,
+                     const double* rows1, const double* corr, const uint32_t* cflag, double* rows2, hipStream_t s);
 int launch_pack_jack(const double* w, const int32_t* tags, int64_t n, int nsamp, double* out, int32_t* status,
                      hipStream_t s);
 // total: row 0 (all pairs) is the sum of the subsample rows

@@ -816,9 +816,8 @@ __global__ void __launch_bounds__(WAVES * 64, (kWavesPerSimd<MODE, VAR>)) k_pair
                     const double ry = rsys ? (by[u] + rshy) - py : py - by[u];
                     const double rz = rszs ? (bz[u] + rshz) - pz : pz - bz[u];
                     const uint32_t ar = addr_of(rx, ry, rz);
-                    if (ar != a[u] && L.seam) {
-                        if (lw[0] != 0.0) atomicOr(L.seam, 4);
-                    } else if (ar != a[u]) {
+                    if (ar != a[u]) {
+                        if (L.seam) atomicOr(L.seam, 4);
                         const uint32_t sf = a[u] / step_r, sr = ar / step_r;
                         double* crow = L.corr + (int64_t)sload_u32_at(SP, sbase + (off[u] >> 3)) * Kr + k0;
                         if (sf < (uint32_t)kc)
@@ -975,7 +974,7 @@ __global__ void __launch_bounds__(WAVES * 64, (kWavesPerSimd<MODE, VAR>)) k_pair
                         rsxs = sxs; rsys = sys; rszs = szs;
                         rax = ax; ray = ay; raz = az;
                         rinc = (sym && img == 13) ? 2u : 1u;
-                        rcorr = MODE == kModeJac && !SWAP && (L.corr != nullptr || L.seam != nullptr) && img != 13;
+                        rcorr = MODE == kModeJac && !SWAP && L.corr != nullptr && img != 13;
                         rhalf = MODE == kModeTan && sym && img != 13;
                         if (JK) rl0 = (sym && img == 13) ? 2.0 * lw[0] : lw[0];
                         if (MODE == kModeTan) {

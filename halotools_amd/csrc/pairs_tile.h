@@ -419,6 +419,7 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
         }
 
         bool self_done = false;
+        [[maybe_unused]] bool tied = false;  // Jacobian: the group's rows of corr are in use
         const uint32_t sbase = (uint32_t)uni((int)geom->p_off[SS]);
         const int tlo = (int)A.tr.lo, thi = (int)A.tr.hi;
         const uint32_t tsh = A.tr.sh3, tmask = A.tr.mask << 3;
@@ -669,6 +670,7 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                         if (XY) odd |= (uint64_t)__ballot(min(min(hp[0], hp[1]), min(hp[2], hp[3])) < floor_pi);
                     }
                     if (__builtin_expect(odd != 0, 0)) {
+                        [[maybe_unused]] uint32_t ties = 0u;  // Jacobian: this lane's pairs whose other order has a bin of its own
 #pragma unroll 1
                         for (int i = 0; i < 4; i++) {
                             const uint32_t ti = i == 0 ? t[0] : (i == 1 ? t[1] : (i == 2 ? t[2] : t[3]));
@@ -691,25 +693,13 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                                 const bool itself = MODE == kModeJac && L.lane.x == L.strm.x &&
                                                     ID[slot] == (own0 + (uint32_t)lj | ((uint32_t)kHere << kImgShift));
                                 if (!itself) kk = exact_bin(lj, slot, kb, kq, false);
-                                if (MODE == kModeJac && !SWAP && (L.corr != nullptr || L.seam != nullptr) && !itself) {
+                                if (MODE == kModeJac && !SWAP && L.corr != nullptr && (ID[slot] >> kImgShift) != (uint32_t)kHere) {
                                     // Auto-count with one set of weights: the sample-2 rows take
                                     // the pair's other orientation, which across the periodic seam
-                                    // may round into another bin; those disagreements are recorded,
-                                    // so rows2 = rows1 + corr (as pairs_kernel.h does for every
-                                    // shifted pair; only these can differ), or that there is one.
-                                    const uint32_t id = ID[slot];
+                                    // may round into another bin (only these pairs can differ).
                                     uint32_t dummy = 0u;
                                     const uint32_t kr = exact_bin(s * kSub + (lane & 15), slot, kb, dummy, true);
-                                    if (kr != kk && (id >> kImgShift) != (uint32_t)kHere && s * kSub + (lane & 15) < cnt) {
-                                        if (L.seam) atomicOr(L.seam, 4);
-                                        const int64_t sr = (int64_t)sbase + (int64_t)(id & kRowMask);
-                                        const int64_t q = __double_as_longlong(L.strm.x[sr * 4 + 3]);
-                                        double* crow = L.corr + q * K;
-                                        if (L.corr && kk < (uint32_t)K)
-                                            __hip_atomic_fetch_add(crow + kk, lw[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                                        if (L.corr && kr < (uint32_t)K)
-                                            __hip_atomic_fetch_add(crow + kr, -lw[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                                    }
+                                    if (kr != kk && s * kSub + (lane & 15) < cnt) ties |= 1u << i;
                                 }
                                 if constexpr (JK) {
                                     // A pair of two tags gives half of its weight to each.  The rows
@@ -738,6 +728,32 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                                         adr[u] = adr0 + kk * rbytes;
                                         if (XY) pad[u] = kq * pbytes;
                                     }
+                            }
+                        }
+                        if constexpr (MODE == kModeJac && !SWAP) {
+                            // Such a pair moves the partner's weight from one bin to the other
+                            // in the lane point's own row of corr, rows2 = rows1 + corr.  This
+                            // wave alone has these rows: it clears them at the group's first
+                            // such pair, and most groups never touch them.
+                            if ((uint64_t)__ballot(ties != 0u) != 0) {
+                                double* const crow = L.corr + p0 * K;
+                                if (!tied) {
+                                    for (int e = lane; e < cnt * K; e += 64) crow[e] = 0.0;
+                                    __threadfence();
+                                    tied = true;
+                                }
+#pragma unroll 1
+                                for (int i = 0; i < 4; i++) {
+                                    if (!((ties >> i) & 1u)) continue;
+                                    const int slot = list[t0 + (lane >> 4) * 4 + i];
+                                    uint32_t dummy = 0u;
+                                    const uint32_t kf = exact_bin(lj, slot, 0u, dummy, false);
+                                    const uint32_t kr = exact_bin(lj, slot, 0u, dummy, true);
+                                    const double w = SWm[ID[slot] & kRowMask];
+                                    double* const r = crow + lj * K;
+                                    if (kf < (uint32_t)K) __hip_atomic_fetch_add(r + kf, -w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                                    if (kr < (uint32_t)K) __hip_atomic_fetch_add(r + kr, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                                }
                             }
                         }
                     }
@@ -1102,6 +1118,10 @@ __global__ void __launch_bounds__(WAVES * 64, HP_TILE_WPS) k_tiles(const TileArg
                 }
             }
             if constexpr (MODE == kModeJac && !SWAP) {
+                if (L.corr && lane == 0) {
+                    L.cflag[g] = tied ? 1u : 0u;
+                    if (tied && L.seam) atomicOr(L.seam, 4);
+                }
                 if (L.psum) {
                     const double w = act ? LWT[lane] : 0.0;
                     for (int k = 0; k < K; k++) {

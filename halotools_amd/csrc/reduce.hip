@@ -462,6 +462,35 @@ int launch_add_rows(const double* a, const double* b, double* out, int64_t n, hi
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+// The sample-2 rows of an auto-count with one set of weights from the matrix-core
+// pass: a lane group's rows1, with its corrections where it wrote any (corr in
+// the lanes' order; a lane row's fourth word is the point's input position).  A
+// wave per group; bound by the rows' one read and write (1M x 20: 320 MB).
+__global__ void __launch_bounds__(256) k_seam_rows(const MockGeom* __restrict__ geom, const int32_t* __restrict__ group_mock,
+                                                   int64_t ngroups, const double* __restrict__ lane_rows, int nr,
+                                                   const double* __restrict__ rows1, const double* __restrict__ corr,
+                                                   const uint32_t* __restrict__ cflag, double* __restrict__ rows2) {
+    const int64_t g = blockIdx.x * (int64_t)4 + (threadIdx.x >> 6);
+    if (g >= ngroups) return;
+    const MockGeom& G = geom[group_mock ? group_mock[g] : 0];
+    const int64_t gl = g - G.group_off[0], p0 = G.p_off[0] + gl * kGroup, left = G.n[0] - gl * kGroup;
+    const int total = (int)(left < kGroup ? left : kGroup) * nr;
+    const bool tied = cflag[g] != 0u;
+    for (int e = threadIdx.x & 63; e < total; e += 64) {
+        const int r = e / nr;
+        const int64_t q = __double_as_longlong(lane_rows[(p0 + r) * 4 + 3]) * nr + (e - r * nr);
+        rows2[q] = tied ? rows1[q] + corr[p0 * nr + e] : rows1[q];
+    }
+}
+
+int launch_seam_rows(const MockGeom* geom, const int32_t* group_mock, int64_t ngroups, const double* lane_rows, int nr,
+                     const double* rows1, const double* corr, const uint32_t* cflag, double* rows2, hipStream_t s) {
+    if (ngroups <= 0) return 0;
+    hipLaunchKernelGGL(k_seam_rows, dim3((unsigned)((ngroups + 3) / 4)), dim3(256), 0, s, geom, group_mock, ngroups,
+                       lane_rows, nr, rows1, corr, cflag, rows2);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
 // ------------------------------------------------------------ jackknife
 // (w, tag) rows for the pair kernel: the weight (1 when none is given) and the
 // subsample tag as a double (exact below 2^53).  Tags outside [1, nsamp] set

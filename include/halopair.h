@@ -67,7 +67,8 @@ enum hp_flags {
     HP_SEAM_CHECK = 64,  /* HP_SAME_SAMPLES and HP_ROWS1 without HP_ROWS2: bit 4 of    */
                          /* the status word tells that rows2 would differ from rows1  */
                          /* (a pair across the periodic seam whose two orientations   */
-                         /* round into different bins); clear, rows1 serves for both  */
+                         /* round into different bins): hp_seam_rows then makes it;   */
+                         /* clear, rows1 serves for both                              */
     HP_TANGENT = 32      /* marked, weight_func_id 1 with nw = 2 weights per point    */
                          /* (w, dw/dtheta): sums of w1*w2 and `tangents`, the sums of */
                          /* t1*w2 + w1*t2 = d(sums)/dtheta (forward-mode derivative)  */
@@ -243,6 +244,10 @@ int hp_enclose(const double* const* cols, int64_t stride1, int64_t n1, int64_t s
  * 1 <= n_samples <= 65536; out: 6 + 512 * (2 + (n_samples + 63) / 64) words on the device; only enqueues work. */
 int hp_tag_stats(const int64_t* tags1, int64_t n1, const int64_t* tags2, int64_t n2, int32_t n_samples, int64_t* out,
                  int64_t out_elems, void* stream);
+
+/* rows2 of a finished request with HP_SEAM_CHECK (the same fields, `workspace` and `rows1` as the pair pass left
+ * them, `rows2` set): rows1 and the pass's corrections, one pass over the rows; only enqueues work. */
+int hp_seam_rows(const hp_request* req);
 
 /* Diagnostics (host only, no GPU needed; used by the CPU test-suite). */
 /* The kernels' bucketed bin lookup: out[i] = number of suffix-minimum edges of r2 below d[i];

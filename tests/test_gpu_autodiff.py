@@ -215,3 +215,41 @@ def test_gradient_steps_hold_no_memory(ad, gpu):
     finally:
         gc.enable()
     assert used[0] == used[1] == used[2]
+
+
+def _tied(n, L, step, seed):
+    """Points on a decimal lattice, whose pairs across the seam often bin by their order."""
+    return np.random.default_rng(seed).integers(0, int(L / step), (n, 3)) * step
+
+
+@pytest.mark.parametrize("kernel", ["tiles", "general"])
+@pytest.mark.parametrize("sizes", [[3000], [65, 1, 0, 2500, 64, 700]], ids=["one", "batch"])
+def test_tied_seam_pairs_take_one_pass(gpu, sizes, kernel, monkeypatch):
+    # the second rows come from the corrections of the one pair pass: no second request, the
+    # swapped pass's rows (sums of small whole numbers: exact in any order)
+    from halotools_amd import _device as D, _engine as E
+    from halotools_amd.batch import MockBatch
+    if kernel == "general":
+        monkeypatch.setenv("HALOPAIR_NO_TILES", "1")
+    L, rb = 10.0, np.array([0.3, 0.7, 1.1, 1.5])
+    pts = [torch.tensor(_tied(n, L, 0.1, i), device=gpu) for i, n in enumerate(sizes)]
+    n = sum(sizes)
+    w = torch.randint(1, 9, (n,), device=gpu, generator=torch.Generator(device=gpu).manual_seed(1)).double()
+    cols = tuple(torch.cat(pts)[:, k].contiguous() for k in range(3))
+    mocks = [dict(n1=m, n2=m, period=[L] * 3, pbc=True) for m in sizes]
+    swapped = D.run(E.HP_MARKED_NPAIRS_3D, mocks, cols, tuple(c.clone() for c in cols), rb * rb, same=False,
+                    w1=w.reshape(-1, 1), w2=w.clone().reshape(-1, 1), nw=1, wfunc=1, want_counts=False, want_sums=True,
+                    rows1=True, rows2=True, device=gpu)
+    elim = D.run(E.HP_MARKED_NPAIRS_3D, mocks, cols, cols, rb * rb, same=True, w1=w.reshape(-1, 1), nw=1, wfunc=1,
+                 want_counts=False, want_sums=True, rows2=True, device=gpu)
+    assert not torch.equal(swapped.rows1, swapped.rows2) and torch.equal(elim.rows2, swapped.rows2)
+    calls = []
+    real = D.run
+    monkeypatch.setattr(D, "run", lambda *a, **k: calls.append(1) or real(*a, **k))
+    wt = w.clone().requires_grad_(True)
+    W = MockBatch(pts, L, rb, device=gpu).marked_npairs_3d_product(wt)
+    c = torch.arange(1.0, W.numel() + 1, device=gpu, dtype=torch.float64).reshape(W.shape)
+    (W * c).sum().backward()
+    assert len(calls) == 1
+    G = torch.flip(torch.cumsum(torch.flip(c, [1]), 1), [1]).repeat_interleave(torch.tensor(sizes, device=gpu), dim=0)
+    assert torch.equal(wt.grad, ((swapped.rows1 + swapped.rows2) * G).sum(dim=1))
