@@ -807,7 +807,8 @@ __global__ void __launch_bounds__(WAVES * 64, (kWavesPerSimd<MODE, VAR>)) k_pair
                 // one; record the rare disagreements so rows2 = rows1 + corr (the
                 // swapped pass's rows, exactly for sums of small integers and to
                 // the rounding of the row sums otherwise: corr is added with
-                // atomics from many waves, in no fixed order).
+                // atomics from many waves, in no fixed order), and that there is
+                // one where the caller asks that.
                 const uint32_t* __restrict__ SP = L.strm.perm;
 #pragma unroll
                 for (int u = 0; u < B; u++) {
