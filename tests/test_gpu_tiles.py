@@ -240,3 +240,46 @@ def test_jackknife_weights_that_are_not_finite(mo, value, tags, monkeypatch):
     monkeypatch.setenv("HALOPAIR_NO_TILES", "1")
     ref = mo.npairs_jackknife_3d(p, p, rb, t, t, ns, **kw)
     assert np.array_equal(got, ref, equal_nan=True)
+
+
+def _seconds(f, reps=9):
+    import time
+
+    import torch
+    times = []
+    for _ in range(reps + 2):
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+        f()
+        torch.cuda.synchronize()
+        times.append(time.perf_counter() - t0)
+    return float(np.median(times[2:]))
+
+
+@pytest.mark.parametrize("ns", [1, 8, 511, 512, 513, 1024, 1025, 5000])
+def test_many_subsamples(mo, ns, monkeypatch):
+    # the table's total over parts of the subsamples (whole numbers: exact in any order)
+    rng = np.random.default_rng(ns)
+    p = rng.uniform(0, 1, (700, 3))
+    t = rng.integers(1, ns + 1, 700)
+    w = rng.integers(1, 5, 700).astype(float)
+    rb = np.linspace(0.01, 0.2, 33)
+    run = lambda: [mo.npairs_jackknife_3d(p, p, rb, t, t, ns, period=1.0, **kw)
+                   for kw in ({}, dict(weights1=w, weights2=w))]
+    got = run()
+    monkeypatch.setenv("HALOPAIR_NO_TILES", "1")
+    for a, b in zip(got, run()):
+        assert np.array_equal(a, b)
+
+
+def test_many_subsamples_cost_no_more_than_in_the_general_kernels(mo, gpu, monkeypatch):
+    # 300 points, 65536 subsamples: the tables' total and output are the work (2.7 times the
+    # general kernels' call with the total in one workgroup, 0.4 times in parts)
+    import torch
+    p = torch.rand((300, 3), dtype=torch.float64, device=gpu)
+    t = torch.randint(1, 65537, (300,), device=gpu)
+    rb = np.logspace(-2, -1, 15)
+    run = lambda: mo.npairs_jackknife_3d(p, p, rb, t, t, 65536, period=1.0)
+    tiles = _seconds(run)
+    monkeypatch.setenv("HALOPAIR_NO_TILES", "1")
+    assert tiles < 1.4 * _seconds(run)
