@@ -757,28 +757,38 @@ __global__ void __launch_bounds__(1024) k_tag_parts(const TagArgs a) {
     for (int w = threadIdx.x; w < a.words; w += blockDim.x) p[2 + w] = (int64_t)bits[w];
 }
 
-__global__ void __launch_bounds__(256) k_tag_join(const TagArgs a, int blocks) {
+__global__ void __launch_bounds__(1024) k_tag_join(const TagArgs a, int blocks) {
     extern __shared__ unsigned long long bits[];
-    __shared__ int64_t t[8];
+    __shared__ int64_t t[32];
     __shared__ int seen;
     const int sd = blockIdx.x;
     const int64_t* part = a.part + (int64_t)sd * kTagBlocks * (2 + a.words);
     if (threadIdx.x == 0) seen = 0;
-    for (int w = threadIdx.x; w < a.words; w += 256) bits[w] = 0ull;
+    for (int w = threadIdx.x; w < a.words; w += 1024) bits[w] = 0ull;
     __syncthreads();
     int64_t lo = INT64_MAX, hi = INT64_MIN;
-    for (int b = threadIdx.x; b < blocks; b += 256) {
+    for (int b = threadIdx.x; b < blocks; b += 1024) {
         const int64_t* p = part + (int64_t)b * (2 + a.words);
         lo = p[0] < lo ? p[0] : lo;
         hi = p[1] > hi ? p[1] : hi;
     }
-    for (int i = threadIdx.x; i < blocks * a.words; i += 256) {
-        const int b = i / a.words, w = i - b * a.words;
-        const unsigned long long v = (unsigned long long)part[(int64_t)b * (2 + a.words) + 2 + w];
-        if (v) atomicOr(&bits[w], v);
+    // (eight loads in flight: one by one in 256 threads, a call on 1M tags of 65536 took 424 us, now 109)
+    const int cells = blocks * a.words;
+    for (int i0 = threadIdx.x; i0 < cells; i0 += 8 * 1024) {
+        unsigned long long v[8];
+        int w[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const int i = i0 + u * 1024, b = i / a.words;
+            w[u] = i - b * a.words;
+            v[u] = i < cells ? (unsigned long long)part[(int64_t)b * (2 + a.words) + 2 + w[u]] : 0ull;
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (v[u]) atomicOr(&bits[w[u]], v[u]);
     }
     tag_minmax(lo, hi, t);  // (waits for the bitmap too)
-    for (int w = threadIdx.x; w < a.words; w += 256) atomicAdd(&seen, __popcll(bits[w]));
+    for (int w = threadIdx.x; w < a.words; w += 1024) atomicAdd(&seen, __popcll(bits[w]));
     __syncthreads();
     if (threadIdx.x == 0) {
         a.out[3 * sd] = lo;
@@ -806,7 +816,7 @@ int launch_tag_stats(const int64_t* t1, int64_t n1, const int64_t* t2, int64_t n
     if (nb > kTagBlocks) nb = kTagBlocks;
     const size_t lds = (size_t)a.words * 8;
     hipLaunchKernelGGL(k_tag_parts, dim3((unsigned)nb, sides), dim3(1024), lds, s, a);
-    hipLaunchKernelGGL(k_tag_join, dim3(sides), dim3(256), lds, s, a, (int)nb);
+    hipLaunchKernelGGL(k_tag_join, dim3(sides), dim3(1024), lds, s, a, (int)nb);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

@@ -79,3 +79,25 @@ def test_tag_stats(gpu, n1, n2, nsamp):
     assert got == tuple(ref)
     assert D.tag_stats(d[0].int(), d[0], nsamp) is None and D.tag_stats(d[0][::2], d[0], nsamp) is None or n1 < 3
     assert D.tag_stats(d[0], d[0], 65537) is None and D.tag_stats(d[0], d[0], 0) is None
+
+
+def test_tag_stats_cost_no_more_than_the_elementwise_checks(gpu):
+    # 1M tags, bitmaps of 65536 in 256 workgroups to join: twice the elementwise checks with
+    # one load in flight per thread, half of them with eight
+    from tests.test_gpu_tiles import _seconds
+    t = torch.randint(1, 65537, (1000000,), device=gpu)
+    elementwise = _seconds(lambda: (t.min().item(), t.max().item(),
+                                    (torch.bincount(t, minlength=65537)[1:] > 0).all().item()))
+    assert _seconds(lambda: D.tag_stats(t, t, 65536)) < 1.4 * elementwise
+
+
+@pytest.mark.parametrize("nsamp", [8191, 8192, 65535, 65536])
+@pytest.mark.parametrize("n1,n2", [(262143, 300), (1000003, 0)])
+def test_tag_stats_of_many_tags(gpu, n1, n2, nsamp):
+    rng = np.random.default_rng([n1, nsamp])
+    t = [rng.integers(1, nsamp + 1, n) for n in (n1, max(n2, 1))]
+    t[0][t[0] == nsamp] = 1   # the last tag does not occur
+    d = [torch.as_tensor(a, device=gpu) for a in t]
+    got = D.tag_stats(d[0], d[1] if n2 else d[0], nsamp)
+    ref = [(a.min(), a.max(), nsamp - len(np.unique(a))) for a in (t if n2 else [t[0]] * 2)]
+    assert got == tuple(ref)
