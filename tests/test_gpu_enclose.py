@@ -101,3 +101,14 @@ def test_tag_stats_of_many_tags(gpu, n1, n2, nsamp):
     got = D.tag_stats(d[0], d[1] if n2 else d[0], nsamp)
     ref = [(a.min(), a.max(), nsamp - len(np.unique(a))) for a in (t if n2 else [t[0]] * 2)]
     assert got == tuple(ref)
+
+
+def test_tag_stats_leave_other_tags_to_the_elementwise_path(gpu):
+    d = torch.arange(1, 9, device=gpu)
+    assert D.tag_stats(d.int(), d, 8) is None
+    assert D.tag_stats(d, d.int(), 8) is None
+    assert D.tag_stats(d[::2], d, 8) is None
+    assert D.tag_stats(d, d[::2], 8) is None
+    assert D.tag_stats(d[:0], d, 8) is None
+    assert D.tag_stats(d.cpu(), d, 8) is None
+    assert D.tag_stats(d, d, 8) is not None
