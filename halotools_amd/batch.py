@@ -102,7 +102,11 @@ class MockBatch(object):
         """Autotune cell edges and the tile shape on this batch's own mocks.
 
         One representative (the largest mock) per density bucket of the tuner's
-        cache key is timed; every mock of the bucket then uses its result.
+        cache key is timed; every mock of the bucket then uses its result, if
+        that makes the batch's own pass clearly faster than the library's
+        choices do (a shape that suits one mock may not suit their launch:
+        Jacobian rows of 500k points in four-wave groups 1002 -> 954 us, of four
+        such mocks 2650 -> 2900).
         Returns {bucket key: ((target, waves), timings)}.
         """
         done = {}
@@ -115,6 +119,16 @@ class MockBatch(object):
             pts = self.rows[a:b]
             done[k] = autotune.tune(pts, self.period, self.rbins, kind=kind, device=self.device, **kw)
         self._apply_tuning(kind)
+        if done and 0.0 in kw.get("targets", autotune.TARGETS) and 0 in kw.get("waves", autotune.WAVES):
+            own = [dict(m, cell=[0.0] * 3) for m in self.mocks]
+            reps = kw.get("reps", 2)
+            t_own = autotune.seconds(autotune.request(kind, own, self.cols, self.rbins, 0, self.device), reps,
+                                     self.device)
+            t = autotune.seconds(autotune.request(kind, self.mocks, self.cols, self.rbins,
+                                                  self._kind_waves.get(kind, 0), self.device), reps, self.device)
+            if t_own <= (1.0 + autotune.MARGIN) * t:
+                self.mocks = own
+                self._kind_waves.pop(kind, None)
         return done
 
     def npairs_3d(self, build_events=None, pair_events=None):

@@ -232,3 +232,27 @@ def test_zheng07_tangent_kernel_matches_torch(gpu):
         assert torch.equal(out[:, 0], w) and torch.equal(out[:, 1], dw), sigma
     with pytest.raises(ValueError):
         D.zheng07_tangent(log_mass, mock_id, logMmin, 0.3, torch.empty((3, 2), dtype=torch.float64, device=gpu))
+
+
+@pytest.mark.parametrize("gain", [False, True])
+def test_tuned_settings_stay_only_if_the_batch_gains(data, gpu, tmp_path, monkeypatch, gain):
+    # every mock alone is fastest with (8 points a cell, 4 waves); the batch's pass is not, or is
+    from halotools_amd import autotune
+    from halotools_amd.batch import MockBatch
+    monkeypatch.setenv("HALOTOOLS_AMD_TUNE_CACHE", str(tmp_path / "tune.json"))
+    monkeypatch.setattr(autotune, "_CACHE", {})
+    sizes, pts = data[:2]
+    b = MockBatch(pts, L, RB, device=gpu)
+    before = b.npairs_3d().clone()
+
+    def seconds(res, reps, device):
+        autotune.D.launch(res)
+        marr = res.keep[0]
+        tuned = res.req.tile_waves == 4 and any(m.cell[0] > 0 for m in marr)
+        return 0.5 if tuned and (len(marr) == 1 or gain) else 1.0
+
+    monkeypatch.setattr(autotune, "seconds", seconds)
+    b.tune(autotune.TANGENT, targets=(0.0, 8.0), waves=(0, 4))
+    assert b.waves_for(autotune.TANGENT) == (4 if gain else 0)
+    assert any(m["cell"][0] > 0 for m in b.mocks) == gain
+    assert torch.equal(b.npairs_3d(), before)
