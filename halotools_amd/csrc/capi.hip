@@ -717,11 +717,26 @@ static int seam_rows(const Plan& P, char* ws, const double* rows1, double* rows2
                             reinterpret_cast<const uint32_t*>(ws + P.o_cflag), rows2, s);
 }
 
-static int run(const hp_request* r, int kind, bool tiles = true) {
+// The plan for a workspace of `room` bytes: the general kernels' where the
+// matrix-core kernels' needs more (their sorted copies of two different samples
+// are larger: 500k x 500k points 75 MiB against 44).  The smaller one if neither
+// fits.
+static int plan_for(const hp_request* r, int kind, size_t room, Plan& P) {
+    if (make_plan(r, kind, P)) return -1;
+    if (P.tiles && P.total > room) {
+        Plan G;
+        if (make_plan(r, kind, G, false)) return -1;
+        if (G.total < P.total) P = std::move(G);
+    }
+    return 0;
+}
+
+static int run(const hp_request* r, int kind) {
     PhaseRange phase;
     phase.begin("halopair: plan");
     Plan P;
-    if (make_plan(r, kind, P, tiles)) return -1;
+    if (!r) return fail("null request");
+    if (plan_for(r, kind, r->workspace ? r->workspace_bytes : SIZE_MAX, P)) return -1;
     if (!r->workspace) return fail("workspace must not be null");
     if (r->workspace_bytes < P.total) return fail("workspace too small");
     if (P.n[0] > 0 && (!r->x1 || !r->y1 || !r->z1)) return fail("sample1 coordinates must not be null");
@@ -1065,14 +1080,7 @@ int hp_npairs_3d_noalloc(const hp_request* req) {
     if (req->workspace || req->workspace_bytes)
         return fail("hp_npairs_3d_noalloc takes no workspace (workspace must be NULL and workspace_bytes 0)");
     Plan P;
-    if (make_plan(req, HP_NPAIRS_3D, P)) return -1;
-    bool tiles = true;
-    if (P.total > (size_t)HP_NOALLOC_SCRATCH_BYTES) {
-        // the other kernels' sorted copies of two different samples are smaller
-        P = Plan();
-        if (make_plan(req, HP_NPAIRS_3D, P, false)) return -1;
-        tiles = false;
-    }
+    if (plan_for(req, HP_NPAIRS_3D, HP_NOALLOC_SCRATCH_BYTES, P)) return -1;
     if (P.total > (size_t)HP_NOALLOC_SCRATCH_BYTES)
         return fail("hp_npairs_3d_noalloc: the request needs " + std::to_string(P.total) +
                     " bytes of scratch, more than the library's fixed " +
@@ -1083,7 +1091,7 @@ int hp_npairs_3d_noalloc(const hp_request* req) {
     hp_request r = *req;
     r.workspace = ptr;
     r.workspace_bytes = (size_t)HP_NOALLOC_SCRATCH_BYTES;
-    return run(&r, HP_NPAIRS_3D, tiles);
+    return run(&r, HP_NPAIRS_3D);
 }
 int hp_npairs_projected(const hp_request* req) { return run(req, HP_NPAIRS_PROJECTED); }
 int hp_npairs_xy_z(const hp_request* req) { return run(req, HP_NPAIRS_XY_Z); }
@@ -1095,7 +1103,8 @@ int hp_npairs_jackknife_xy_z(const hp_request* req) { return run(req, HP_NPAIRS_
 
 int hp_seam_rows(const hp_request* req) {
     Plan P;
-    if (make_plan(req, HP_MARKED_NPAIRS_3D, P)) return -1;
+    if (!req) return fail("null request");
+    if (plan_for(req, HP_MARKED_NPAIRS_3D, req->workspace ? req->workspace_bytes : SIZE_MAX, P)) return -1;
     if (!P.seam) return fail("hp_seam_rows takes a request with HP_SEAM_CHECK");
     if (!req->workspace || req->workspace_bytes < P.total) return fail("workspace too small");
     if (P.n[0] > 0 && (!req->rows1 || !req->rows2)) return fail("rows1 and rows2 must not be null");

@@ -141,7 +141,8 @@ const char* hp_last_error(void);
 /* ABI version of the loaded library (HP_ABI_VERSION). */
 int hp_abi_version(void);
 
-/* Bytes of workspace the request needs (pointers in `req` are not read). */
+/* Bytes of workspace the request needs (pointers in `req` are not read).  A call with a smaller workspace that the
+ * general pair kernels' plan still fits (two different samples: about 0.6 times) runs those, with the same results. */
 size_t hp_workspace_size(const hp_request* req);
 
 /* npairs_3d: cumulative int64 counts[m][k] of ordered pairs with
@@ -157,7 +158,9 @@ int hp_npairs_3d(const hp_request* req);
  * a fixed HP_NOALLOC_SCRATCH_BYTES (64 MiB) array that every GPU the library
  * runs on holds from module load until the process ends.  A request fits when
  * hp_workspace_size(req) <= HP_NOALLOC_SCRATCH_BYTES (an auto-count of about
- * 720K points with 20 bins); a larger one returns an error.  The current HIP
+ * 720K points with 20 bins, two samples of about 430K each), and two different
+ * samples also when the general pair kernels' plan does (about 720K each); a
+ * larger one returns an error.  The current HIP
  * device's array is used (the stream must belong to that device), and it keeps
  * the last call's contents: calls that overlap on one GPU race. */
 int hp_npairs_3d_noalloc(const hp_request* req);

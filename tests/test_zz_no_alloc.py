@@ -52,3 +52,29 @@ def test_noalloc_rejects_requests_beyond_its_scratch(gpu):
                     np.array([1.0, 4.0]), same=True, device=gpu)
     with pytest.raises(E.EngineError, match="more than the library's fixed"):
         _noalloc(res, gpu)
+
+
+def test_two_samples_beyond_the_matrix_core_plan(gpu):
+    # 500k x 500k: 75 MiB for the matrix-core kernels, 44 MiB for the general ones, which
+    # a fixed scratch or a caller's workspace of 64 MiB holds
+    import torch
+    from halotools_amd import _device as D
+    from halotools_amd import _engine as E
+    rng = np.random.default_rng(78)
+    s1, s2 = [tuple(torch.tensor(rng.uniform(0, 300.0, (3, 500000)), device=gpu).unbind(0)) for _ in range(2)]
+    args = (E.HP_NPAIRS_3D, [dict(n1=500000, n2=500000, period=[300.0] * 3, pbc=True)], s1, s2,
+            np.logspace(-1, np.log10(2), 6) ** 2)
+    ref = D.run(*args, device=gpu)
+    assert ref.req.workspace_bytes > 64 << 20
+    for run in (_noalloc, lambda res, gpu: E.check(res.fn(ctypes.byref(res.req)))):
+        got = D.prepare(*args, device=gpu)
+        got.cbuf.fill_(-1)
+        got.req.workspace_bytes = 64 << 20
+        got.req.stream = torch.cuda.current_stream(gpu).cuda_stream
+        run(got, gpu)
+        torch.cuda.synchronize()
+        assert int(got.status.item()) & 0xFFFFFFFF == 0
+        assert torch.equal(got.counts, ref.counts) and int(ref.counts[0, -1].item()) > 0
+    got.req.workspace_bytes = 32 << 20
+    with pytest.raises(E.EngineError, match="workspace too small"):
+        E.check(got.fn(ctypes.byref(got.req)))
