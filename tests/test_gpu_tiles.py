@@ -283,3 +283,134 @@ def test_many_subsamples_cost_no_more_than_in_the_general_kernels(mo, gpu, monke
     tiles = _seconds(run)
     monkeypatch.setenv("HALOPAIR_NO_TILES", "1")
     assert tiles < 1.4 * _seconds(run)
+
+
+@pytest.mark.parametrize("n1,n2", [(1, 0), (15, 0), (16, 0), (17, 0), (63, 0), (64, 0), (65, 0), (129, 0), (1000, 0),
+                                   (1, 64), (17, 1), (65, 200), (200, 65), (64, 1000)])
+@pytest.mark.parametrize("kind", ["uniform", "clumps", "lattice", "seam"])
+def test_forward_mode_agrees_with_general(gpu, n1, n2, kind, monkeypatch):
+    # weights and tangents that are small whole numbers: every term and its halves are exact
+    import torch
+
+    from halotools_amd import _device as D
+    from halotools_amd import _engine as E
+    same = n2 == 0
+    rng = np.random.default_rng([n1, n2])
+    p = [torch.as_tensor(_points(n, kind, i), device=gpu) for i, n in enumerate((n1, n2 or n1))]
+    w = [torch.as_tensor(rng.integers(-8, 9, (len(x), 2)).astype(float), device=gpu) for x in p]
+    rb = np.array([2.5, 5.0, 7.5, 10.0, 12.5]) if kind == "lattice" else RB
+
+    def run():
+        res = D.run(E.HP_MARKED_NPAIRS_3D, [dict(n1=n1, n2=n2 or n1, period=[L] * 3, pbc=True)], p[0].unbind(1),
+                    p[0 if same else 1].unbind(1), rb * rb, same=same, w1=w[0], w2=None if same else w[1], nw=2,
+                    wfunc=1, want_counts=False, want_sums=True, also_counts=True, tangent=True, device=gpu)
+        return res.counts, res.sums, res.tangents
+    got = run()
+    monkeypatch.setenv("HALOPAIR_NO_TILES", "1")
+    for a, b in zip(got, run()):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("n1,n2", [(800001, 0), (650000, 600001)])
+def test_queued_items_of_every_mode_agree_with_general(mo, gpu, n1, n2, monkeypatch):
+    # the passes that test_queued_items_agree_with_general leaves out: one-column (rp, pi) cells, generic
+    # marks, Jacobian rows and their swapped pass (a queue set of its own), jackknife rows
+    import torch
+
+    from halotools_amd import _device as D
+    from halotools_amd import _engine as E
+    g = torch.Generator(device=gpu).manual_seed(n1)
+    box = 400.0
+    t1 = torch.rand((n1, 3), dtype=torch.float64, device=gpu, generator=g) * box
+    t1[: n1 // 8] = 200.0 + 0.01 * (t1[: n1 // 8] - 200.0)   # items of very unlike cost
+    t2 = t1 if n2 == 0 else torch.rand((n2, 3), dtype=torch.float64, device=gpu, generator=g) * box
+    u1 = torch.randint(1, 9, (n1, 2), device=gpu, generator=g).double()
+    u2 = u1 if n2 == 0 else torch.randint(1, 9, (n2, 2), device=gpu, generator=g).double()
+    s1, s2 = u1[:, 0].contiguous(), u2[:, 0].contiguous()
+    rb, kw = np.array([0.02, 0.1, 1.0, 4.0]), dict(period=box)
+    wide, pi = np.linspace(0.05, 3.0, 17), np.linspace(0.0, 3.0, 17)
+    marks = lambda a, b, i: dict(weights1=a, weights2=b, weight_func_id=i, **kw)
+    tags = 1 + torch.clamp((t1[:, 0] / box * 5).long(), max=4)
+
+    def run():
+        out = [mo.npairs_xy_z(t1, t2, wide, pi, **kw), mo.marked_npairs_xy_z(t1, t2, wide, pi, **marks(s1, s2, 1)),
+               mo.marked_npairs_xy_z(t1, t2, rb, pi[:3], **marks(u1, u2, 5)),
+               mo.marked_npairs_3d(t1, t2, rb, **marks(u1, u2, 9)), mo.marked_npairs_3d(t1, t2, rb, **marks(s1, s2, 2))]
+        res = D.run(E.HP_MARKED_NPAIRS_3D, [dict(n1=n1, n2=n2 or n1, period=[box] * 3, pbc=True)], t1.unbind(1),
+                    t2.unbind(1), rb * rb, same=n2 == 0, w1=s1.reshape(-1, 1),
+                    w2=None if n2 == 0 else s2.reshape(-1, 1), nw=1, wfunc=1, want_counts=False, want_sums=True,
+                    rows1=True, rows2=True, also_counts=True, device=gpu)
+        out += [res.sums, res.counts, res.rows1, res.rows2]
+        if n2 == 0:
+            out += [mo.npairs_jackknife_3d(t1, t1, rb, tags, tags, 5, **kw),
+                    mo.npairs_jackknife_3d(t1, t1, rb, tags, tags, 5, weights1=s1, weights2=s1, **kw)]
+        return out
+    got = run()
+    monkeypatch.setenv("HALOPAIR_NO_TILES", "1")
+    for a, b in zip(got, run()):
+        assert torch.equal(torch.as_tensor(a), torch.as_tensor(b))
+
+
+@pytest.mark.parametrize("clustered", [False, True])
+def test_jackknife_rows_by_their_subsamples_own_counts(mo, gpu, clustered):
+    # each subsample's row against the cross-counts of its points with all points, in both
+    # orders (row 0 is the rows' sum, so the rows' sum says nothing about them)
+    import torch
+    g = torch.Generator(device=gpu).manual_seed(3)
+    n, box = 800001, 400.0
+    t = torch.rand((n, 3), dtype=torch.float64, device=gpu, generator=g) * box
+    if clustered:
+        t[: n // 8] = 200.0 + 0.01 * (t[: n // 8] - 200.0)
+    sub = torch.clamp((t / box * 5).long(), max=4)
+    tags = 1 + (sub[:, 0] * 5 + sub[:, 1]) * 5 + sub[:, 2]
+    rb = np.array([0.02, 0.1, 1.0, 4.0])
+    jk = mo.npairs_jackknife_3d(t, t, rb, tags, tags, 125, period=box)
+    assert torch.equal(jk[0], mo.npairs_3d(t, t, rb, period=box).double())
+    for s in (1, 2, 31, 63, 94, 125):
+        own = t[tags == s]
+        both = mo.npairs_3d(own, t, rb, period=box) + mo.npairs_3d(t, own, rb, period=box)
+        assert torch.equal(jk[0] - jk[s], 0.5 * both.double()), s
+
+
+@pytest.mark.parametrize("layout", ["columns", "f32", "rows"])
+@pytest.mark.parametrize("n1,n2", [(196609, 0), (270001, 262145), (300000, 1000)])
+def test_large_builds_of_one_mock(mo, gpu, n1, n2, layout, monkeypatch):
+    # one mock beyond the small builds: packed rows of columns, both sort tiles (a stable
+    # sort: the same rows, hence the same bits), against the general kernels
+    import torch
+    t = [torch.as_tensor(_points(n, "seam" if i else "uniform", 5), device=gpu) for i, n in enumerate((n1, n2 or 1))]
+    if layout == "columns":
+        t = [x.t().contiguous().t() for x in t]
+    elif layout == "f32":
+        t = [x.to(torch.float32).clamp(0, float(np.nextafter(np.float32(L), np.float32(0)))) for x in t]
+    p, q = t[0], t[1] if n2 else t[0]
+    w = [torch.rand((len(x),), dtype=torch.float64, device=gpu, generator=torch.Generator(device=gpu).manual_seed(9))
+         for x in t]
+    rb = RB[:6]
+
+    def run():
+        return (mo.npairs_3d(p, q, rb, period=L), mo.npairs_per_object_3d(p, q, rb, period=L),
+                mo.marked_npairs_3d(p, q, rb, period=L, weights1=w[0], weights2=w[1 if n2 else 0], weight_func_id=1))
+    monkeypatch.setenv("HALOPAIR_SORT_TILE", "2048")
+    small = run()
+    monkeypatch.setenv("HALOPAIR_SORT_TILE", "8192")
+    large = run()
+    for a, b in zip(small, large):
+        assert torch.equal(torch.as_tensor(a), torch.as_tensor(b))
+    monkeypatch.setenv("HALOPAIR_NO_TILES", "1")
+    ref = run()
+    assert torch.equal(small[0], ref[0]) and torch.equal(small[1], ref[1])
+    np.testing.assert_allclose(torch.as_tensor(small[2]).cpu(), torch.as_tensor(ref[2]).cpu(), rtol=1e-12)
+
+
+@pytest.mark.parametrize("box", [(200.0, 30.0, 25.0), (25.0, 200.0, 30.0), (30.0, 25.0, 600.0), (300.0, 280.0, 24.0)])
+@pytest.mark.parametrize("n1,n2", [(2000, 0), (300, 5000)])
+def test_elongated_boxes(mo, n1, n2, box):
+    # the curve's cubes have as many along each side of the box as along the others
+    rng = np.random.default_rng([n1, int(box[0])])
+    p1 = rng.uniform(0, 1, (n1, 3)) * box
+    p2 = p1 if n2 == 0 else rng.uniform(0, 1, (n2, 3)) * box
+    rb, kw = np.logspace(-1, np.log10(7.9), 10), dict(period=list(box))
+    assert np.array_equal(mo.npairs_3d(p1, p2, rb, **kw), ORC.npairs_3d(p1, p2, rb, **kw))
+    assert np.array_equal(mo.npairs_xy_z(p1, p2, rb, PI[:3], **kw), ORC.npairs_xy_z(p1, p2, rb, PI[:3], **kw))
+    assert np.array_equal(mo.npairs_per_object_3d(p1, p2, rb, **kw), ORC.npairs_per_object_3d(p1, p2, rb, **kw))
