@@ -724,7 +724,7 @@ def main():
         # bound by instruction issue: squared distances on the FP64 matrix
         # cores, bins and the walk on the vector ALU; MI355X's FP64 peak is 78.6
         # TFLOP/s for both
-        "roofline": {"bound": "fp64-valu", "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
+        "roofline": {"bound": "instruction-issue", "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / FP64_PEAK_TFLOPS, "traffic": PAIR_KERNEL_TRAFFIC_BYTES,
                      "traffic_source": "rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE of this kernel on this "
                                        "workload, scaled by a plain copy's readings "

@@ -241,6 +241,11 @@ static size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 #ifndef HP_TILE_ITEMS
 #define HP_TILE_ITEMS 16
 #endif
+// Default edge of the curve's cubes: this part of the search length, or of a lane
+// group's size where that is longer (the nearest 2^c per side).  Calls in us with
+// half and with twice the first: 1M points, 50 Mpc/h 724, 770, 745; 2M 1835, 1848,
+// 1995; (rp, pi) of 2M 1466, 1462, 1433; 150k x 1M 335, 333, 329; of the second:
+// 1M points, 5 Mpc/h 234, 262, 244; 5M 825, 823, 990.
 #ifndef HP_CUBE_R
 #define HP_CUBE_R 0.6
 #define HP_CUBE_G 0.5
@@ -357,11 +362,11 @@ static int make_plan(const hp_request* r, int kind, Plan& P, bool tiles = true) 
     if (!(Rxy == Rxy) || !(Rz == Rz)) return fail("bins must not be NaN");
     P.nb_count = xyz ? P.Kr * P.Kp : P.Kr;
 
-    // (the jackknife tables of an auto-count; cross-counts stay with pairs_kernel.h)
     // The matrix-core kernels (pairs_tile.h) take what their bucket tables and the
-    // LDS hold: bins that buckets of 1/16 octave or finer part, and a wave's
-    // histogram beside its stage at 7 waves per CU or more.  Wider or denser
-    // binnings and the jackknife tables stay with pairs_kernel.h.
+    // LDS hold: bins that at most 512 buckets of an octave or finer part, one edge
+    // in each, and a wave's stage and histogram of at most 23 KB (6 waves per CU,
+    // 4 in workgroups of four).  Wider or denser binnings, two-sample and (rp, pi)
+    // jackknife tables stay with pairs_kernel.h.
     const int mode = mode_of(P, kind, r->wfunc);
     {
         const int wb = tile_wave_bytes(mode, P.Kr, P.Kp, P.nw, P.counts ? 1 : 0);

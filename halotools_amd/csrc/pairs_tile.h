@@ -19,8 +19,9 @@
 //
 // What bounds it: instruction issue (1M clustered points, 20 edges to 50 Mpc/h:
 // vector instructions 65 % and the matrix product 14 % of the issue slots, 13 of
-// 16 waves alive on average).  The MFMA (65 cycles per 256 pairs; it does not
-// overlap other waves' VALU work here) replaces 8 FP64 instructions of 4.5 cycles
+// 16 waves alive on average).  The MFMA (65 cycles per 256 pairs, next to none of
+// which other waves' VALU work fills: with 16 integer additions 112 to 119, 43 to
+// 47 alone) replaces 8 FP64 instructions of 4.5 cycles
 // per 64 pairs, the bin takes 6 instructions and two LDS accesses instead of 12
 // and two, and sub-groups of 16 evaluate 2.4 pairs per pair in range where groups
 // of 64 evaluated 4.4 (6.3e8 instead of 1.18e9 evaluations there).  Pair kernels
