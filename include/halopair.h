@@ -99,8 +99,8 @@ typedef struct hp_request {
     int32_t nr;                /* number of radial / rp edges                          */
     int32_t np;                /* xy_z: number of pi edges; projected: 1               */
     int32_t tile_waves;        /* pair-kernel workgroup: 1, 2, 4 or 8 wavefronts of 64 */
-                               /* lane points; 0 = library default (8, fewer if the    */
-                               /* histograms do not fit in LDS)                        */
+                               /* lane points; 0 = the library's choice (the shape     */
+                               /* whose LDS keeps the most waves resident)             */
     const double* r2;          /* host [nr]: rbins*rbins (or rp_bins*rp_bins)          */
     const double* p2;          /* host [np]: pi_bins*pi_bins, or {pi_max*pi_max}        */
     double search[3];          /* reserved, not read: the search lengths follow from   */
@@ -113,7 +113,8 @@ typedef struct hp_request {
     double* rows1;             /* HP_ROWS1: [n1_total][nr] per-bin (not cumulative)     */
     double* rows2;             /* HP_ROWS2: [n2_total][nr]                              */
     int64_t* evals;            /* optional [nmocks]: candidate pairs evaluated          */
-    int32_t* status;           /* optional [1]: 0, or 1 when a point is outside its box */
+    int32_t* status;           /* optional [1]: 0, or bits: 1 a point outside its box,  */
+                               /* 2 a tag outside 1..n_samples, 4 see HP_SEAM_CHECK    */
     void* workspace;           /* device scratch                                       */
     size_t workspace_bytes;
     void* stream;              /* hipStream_t; NULL = default stream                   */
